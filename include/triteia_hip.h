@@ -286,6 +286,14 @@ TRITEIA_HIP_API int triteia_hip_sgmv_routed_bf16(void* y, long y_stride, const v
                                  int n_adapters, int d_in, int d_out, float scale, const void* plan, int prob_n,
                                  int accumulate, int dev, void* stream);
 
+/* Quantise, prune and pack a dense fp16 weight [prob_k, prob_m] (row-major) with one fp16 scale per column: of every
+ * aligned group of 4 along k the two entries of largest magnitude are kept (of equal ones the later), as
+ * clamp(round(w / scale) + 8, 0, 15) - 8.  Writes qweight and meta in the layouts above, and meta_raw int16
+ * [prob_m, prob_k/16], the metadata words before the kernel's re-layout.  prob_k % 32 == 0, prob_m % 64 == 0.
+ * Replaces sparse_low_precision_linear.pack (triteia/python/nn/linear.py:79-141, torch on the host's side there). */
+TRITEIA_HIP_API int triteia_hip_pack_2_4(const void* weight, const void* scales, void* qweight, void* meta, void* meta_raw, int prob_k,
+                         int prob_m, int dev, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

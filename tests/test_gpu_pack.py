@@ -1,0 +1,31 @@
+"""The packing kernel against the torch codec, byte for byte (the CPU tests hold the codec exact against the oracle)."""
+import pytest
+import torch
+
+from triteia_amd.python.ops.utils.sparsity import mask_creator, prune_pack_2_4
+
+pytestmark = pytest.mark.gpu
+
+
+# edges: half a column block (m % 128 = 64), a single packed row, packed rows that leave wavefronts of a block idle
+@pytest.mark.parametrize("k,m", [(32, 64), (64, 192), (288, 128), (512, 320), (4096, 1024)])
+@pytest.mark.parametrize("values", ["normal", "ties", "special"])
+def test_pack_kernel_gives_the_codecs_bytes(k, m, values):
+    g = torch.Generator().manual_seed(k * m)
+    w = torch.randn((k, m), generator=g).to(torch.float16)
+    s = (w.abs().amax(0, keepdim=True) * (2 / 15))
+    if values == "ties":               # few distinct magnitudes of either sign, zeros among them: ties in most groups
+        w = torch.randint(-3, 4, (k, m), generator=g).to(torch.float16)
+        s = torch.full((1, m), 0.5, dtype=torch.float16)
+    elif values == "special":          # what a broken checkpoint holds: zero scales, infinities, NaNs, tiny and huge values
+        pool = torch.tensor([0.0, -0.0, 1.0, -65504.0, 6e-8, float("inf"), float("-inf"), float("nan")], dtype=torch.float16)
+        w = pool[torch.randint(0, len(pool), (k, m), generator=g)]
+        s[:, ::3] = 0.0
+    w, s = w.cuda(), s.cuda()
+    got = prune_pack_2_4(w, s)
+    # (an explicit mask takes the codec's own steps on the same device)
+    want = prune_pack_2_4(w, s, mask=mask_creator(w.t().contiguous()))
+    for a, b, name in zip(got, want, ("qweight", "meta", "scales", "meta_raw")):
+        assert a.dtype == b.dtype and a.shape == b.shape
+        # (the scales are handed through: compared as bytes, for their NaNs)
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8)), name

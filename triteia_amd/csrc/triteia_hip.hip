@@ -12,6 +12,7 @@
 
 #include "lora.hip.h"
 #include "lora_mfma.hip.h"
+#include "pack.hip.h"
 #include "route_plan.hip.h"
 #include "sparse24_gemm.hip.h"
 #include "sparse24_share.hip.h"
@@ -1420,6 +1421,25 @@ int triteia_hip_sgmv_routed_bf16(void* y, long y_stride, const void* x, long x_s
                                  int n_adapters, int d_in, int d_out, float scale, const void* plan, int prob_n,
                                  int accumulate, int dev, void* stream) {
   return sgmv_routed_impl<bf16_t>(y, y_stride, x, x_stride, w_base, w_stride, n_adapters, d_in, d_out, scale, plan, prob_n, accumulate, dev, stream);
+}
+
+int triteia_hip_pack_2_4(const void* weight, const void* scales, void* qweight, void* meta, void* meta_raw, int prob_k, int prob_m,
+                         int dev, void* stream) {
+  if (prob_k < 0 || prob_m < 0 || prob_k % 32 != 0 || prob_m % 64 != 0)
+    return fail(TRITEIA_HIP_ERR_PROB_SHAPE, "pack_2_4: k=%d, m=%d need k %% 32 == 0 and m %% 64 == 0", prob_k, prob_m);
+  if (prob_k == 0 || prob_m == 0) return TRITEIA_HIP_OK;
+  if (!weight || !scales || !qweight || !meta || !meta_raw) return fail(TRITEIA_HIP_ERR_ARGUMENT, "pack_2_4: null tensor pointer");
+  if ((reinterpret_cast<uintptr_t>(weight) | reinterpret_cast<uintptr_t>(scales)) % 4 != 0 ||
+      (reinterpret_cast<uintptr_t>(qweight) | reinterpret_cast<uintptr_t>(meta)) % 8 != 0 || reinterpret_cast<uintptr_t>(meta_raw) % 4 != 0)
+    return fail(TRITEIA_HIP_ERR_ARGUMENT, "pack_2_4: weight, scales and meta_raw need 4-byte, qweight and meta 8-byte alignment");
+  const long row_blocks = (prob_k / 32 + kPackRows - 1) / kPackRows;
+  if (row_blocks > 65535) return fail(TRITEIA_HIP_ERR_PROB_SHAPE, "pack_2_4: k=%d is too long", prob_k);
+  DeviceGuard g(dev);
+  if (!g.ok) return fail(TRITEIA_HIP_ERR_RUNTIME, "cannot select device %d", dev);
+  hipLaunchKernelGGL(pack_2_4_kernel, dim3((prob_m + kPackCols - 1) / kPackCols, (unsigned)row_blocks), dim3(64 * kPackRows), 0,
+                     static_cast<hipStream_t>(stream), static_cast<const _Float16*>(weight), static_cast<const _Float16*>(scales), prob_k,
+                     prob_m, static_cast<uint32_t*>(qweight), static_cast<uint32_t*>(meta), static_cast<uint32_t*>(meta_raw));
+  return check_launch("pack_2_4_kernel");
 }
 
 }  // extern "C"

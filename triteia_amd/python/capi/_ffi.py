@@ -56,6 +56,7 @@ SIGNATURES = {
     "triteia_hip_bgmv_store_bf16": (_c_int, [_c_vp] * 4 + [_c_int] * 5 + [_c_float, _c_int, _c_vp]),
     "triteia_hip_sgmv_store": (_c_int, [_c_vp] * 4 + [_c_int] * 5 + [_c_vp]),
     "triteia_hip_sgmv_store_bf16": (_c_int, [_c_vp] * 4 + [_c_int] * 5 + [_c_vp]),
+    "triteia_hip_pack_2_4": (_c_int, [_c_vp] * 5 + [_c_int] * 3 + [_c_vp]),
 }
 
 _lib = None

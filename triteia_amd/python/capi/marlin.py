@@ -219,3 +219,23 @@ def sbmm_2_4_planned(A, B, meta, C, s, plan, accumulate=False):
         _ffi.ptr(A), _ffi.ptr(B), _ffi.ptr(meta), _ffi.ptr(C), _ffi.ptr(s), _ffi.ptr(plan), n_deltas, prob_m, prob_n,
         prob_k, 1 if accumulate else 0, _ffi.device_index(A), _ffi.stream_of(A))
     _raise(err, prob_m, prob_n, prob_k, -1, -1, -1)
+
+
+def pack_2_4(weight, scales):
+    """Quantise, prune and pack a dense weight on the GPU in one pass.  weight fp16 [k, m], scales fp16 [1, m];
+    k % 32 == 0, m % 64 == 0.  Returns (qweight int32 [k/32, 2m], meta int16 [m, k/16], meta_raw int16 [m, k/16])."""
+    _ffi.require_gpu(weight=weight, scales=scales)
+    _ffi.require_dtype(weight, torch.float16, "weight")
+    _ffi.require_dtype(scales, torch.float16, "scales")
+    k, m = weight.shape
+    if scales.numel() != m:
+        raise RuntimeError(f"scales has {scales.numel()} entries, expected {m}")
+    # (pairs of columns are read as one word: a view that starts at an odd element is copied)
+    weight, scales = (t.clone() if t.data_ptr() % 4 else t for t in (weight, scales))
+    qweight = torch.empty((k // 32, 2 * m), dtype=torch.int32, device=weight.device)
+    meta, meta_raw = (torch.empty((m, k // 16), dtype=torch.int16, device=weight.device) for _ in range(2))
+    err = _ffi.lib().triteia_hip_pack_2_4(
+        _ffi.ptr(weight), _ffi.ptr(scales), _ffi.ptr(qweight), _ffi.ptr(meta), _ffi.ptr(meta_raw), k, m,
+        _ffi.device_index(weight), _ffi.stream_of(weight))
+    _raise(err, m, 0, k, -1, -1, -1)
+    return qweight, meta, meta_raw

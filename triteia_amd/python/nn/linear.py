@@ -2,7 +2,7 @@ import torch
 import torch.nn as nn
 
 from triteia_amd.python.capi import mul_2_4
-from triteia_amd.python.ops.utils.sparsity import mask_creator, meta_raw, pack_2_4, positions_from_mask
+from triteia_amd.python.ops.utils.sparsity import prune_pack_2_4
 
 
 class sparse_low_precision_linear(nn.Module):
@@ -56,12 +56,7 @@ class sparse_low_precision_linear(nn.Module):
         dev = B.device if isinstance(B, torch.Tensor) else self.qweight.device
         w = weight.to(dev)
         s = scales.to(dev).reshape(1, m)
-        mask = mask_creator(w.t().contiguous(), n=2, m=4)
-        lo, hi = positions_from_mask(mask)
-        q = torch.clamp(torch.round(w / s).to(torch.int64) + 8, 0, 15) - 8
-        qt = q.t().reshape(m, k // 4, 4)
-        kept = torch.stack([qt.gather(-1, lo.unsqueeze(-1)).squeeze(-1), qt.gather(-1, hi.unsqueeze(-1)).squeeze(-1)], -1)
-        qweight, meta, s16 = pack_2_4(kept.reshape(m, k // 2), lo, hi, s)
+        qweight, meta, s16, raw = prune_pack_2_4(w, s)
         self.qweight.copy_(qweight)
         self.meta.copy_(meta)        # (the buffer, or the tensor a caller has put in its place)
         self.scale.copy_(s16)
@@ -69,7 +64,7 @@ class sparse_low_precision_linear(nn.Module):
             B[:, :] = qweight.to(B.device)
         if isinstance(s_attr, torch.Tensor):
             s_attr[:, :] = s16.to(s_attr.device)
-        self.meta_raw = meta_raw(lo, hi)
+        self.meta_raw = raw
 
 
 class multi_delta_linear(nn.Module):

@@ -9,7 +9,7 @@ and packing records the kept positions explicitly, so a kept value of -8
 import numpy as np
 import torch
 
-from .sparsity import mask_creator, meta_raw, pack_2_4, positions_from_mask
+from .sparsity import mask_creator, pack_2_4, prune_pack_2_4
 
 
 def _randn(shape, generator, device, dtype=torch.float16):
@@ -34,15 +34,8 @@ def fp16_to_sparse(weights, scale, device="cuda", mask=None):
     `meta_raw` is the metadata before the kernel's re-layout: int16 [m, k/16], row = output column."""
     weights = weights.to(device)
     scale = scale.to(device).reshape(1, -1)
-    k, m = weights.shape
-    if mask is None:
-        mask = mask_creator(weights.t().contiguous(), n=2, m=4)
-    lo, hi = positions_from_mask(mask)
-    q = torch.clamp(torch.round(weights / scale).to(torch.int64) + 8, 0, 15) - 8          # [k, m]
-    qt = q.t().reshape(m, k // 4, 4)
-    kept = torch.stack([qt.gather(-1, lo.unsqueeze(-1)).squeeze(-1), qt.gather(-1, hi.unsqueeze(-1)).squeeze(-1)], -1)
-    qweight, meta, s = pack_2_4(kept.reshape(m, k // 2), lo, hi, scale)
-    return weights, qweight, s, meta, meta_raw(lo, hi)
+    qweight, meta, s, raw = prune_pack_2_4(weights, scale, mask)
+    return weights, qweight, s, meta, raw
 
 
 def gen_sparse_quant4_NT(m, k, groupsize=-1, device="cuda", prune_n=2, prune_m=4, generator=None):

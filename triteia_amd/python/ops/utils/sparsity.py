@@ -133,6 +133,29 @@ def pack_2_4(q: torch.Tensor, lo: torch.Tensor, hi: torch.Tensor, scales: torch.
     return qweight, pack_meta(lo, hi), scales.reshape(1, m).to(torch.float16).contiguous()
 
 
+def prune_pack_2_4(weight: torch.Tensor, scale: torch.Tensor, mask: torch.Tensor = None):
+    """Quantise a [k, m] weight with per-column `scale` [1, m], keep 2 of every 4 entries along k (by `mask` [m, k],
+    else the two of largest magnitude) and pack them.
+
+    Returns (qweight, meta, scales fp16 [1, m], meta_raw).  An fp16 weight on the GPU whose positions come from its own
+    magnitudes is packed by one kernel (triteia_amd/csrc/pack.hip.h), bit for bit as the torch codec below."""
+    k, m = weight.shape
+    if (mask is None and weight.is_cuda and weight.device == scale.device and weight.dtype == scale.dtype == torch.float16
+            and k % 32 == 0 and m % 64 == 0 and weight.numel() > 0 and scale.numel() == m):
+        from triteia_amd.python.capi import pack_2_4 as pack_on_gpu
+        s16 = scale.reshape(1, m).contiguous()
+        qweight, meta, raw = pack_on_gpu(weight.contiguous(), s16)
+        return qweight, meta, s16, raw
+    if mask is None:
+        mask = mask_creator(weight.t().contiguous(), n=2, m=4)
+    lo, hi = positions_from_mask(mask)
+    q = torch.clamp(torch.round(weight / scale).to(torch.int64) + 8, 0, 15) - 8          # [k, m]
+    qt = q.t().reshape(m, k // 4, 4)
+    kept = torch.stack([qt.gather(-1, lo.unsqueeze(-1)).squeeze(-1), qt.gather(-1, hi.unsqueeze(-1)).squeeze(-1)], -1)
+    qweight, meta, s16 = pack_2_4(kept.reshape(m, k // 2), lo, hi, scale)
+    return qweight, meta, s16, meta_raw(lo, hi)
+
+
 GROUP_K = 128   # dense k per scale group (groupsize 64 in the launchers' unit of compressed k)
 _GROUP_SCALE_ORDER = [i * 8 + j for i in range(8) for j in (0, 4, 1, 5, 2, 6, 3, 7)]
 
