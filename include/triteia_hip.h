@@ -286,6 +286,22 @@ TRITEIA_HIP_API int triteia_hip_sgmv_routed_bf16(void* y, long y_stride, const v
                                  int n_adapters, int d_in, int d_out, float scale, const void* plan, int prob_n,
                                  int accumulate, int dev, void* stream);
 
+/* The LoRA pair on adapters as they are stored and on the batch's own indices, in two launches:
+ *   y[t] (+)= scale * (x[t] @ A[i]) @ B[i],   i = indices[t] in [0, n_adapters)
+ * A [n_adapters, k, r], B [n_adapters, r, m] row-major, fp16 (bf16 = 1: bf16) like x and y; indices int32 (index64 = 1:
+ * int64), any order.  accumulate = 1 adds to y; 0 stores, and tokens without an adapter get zeros.  The shrink leaves the
+ * routing and the intermediate in `scratch` for the expand, which takes the same sizes and the same `accumulate`.
+ * triteia_hip_lora_scratch_bytes is 0 for what this pair does not take: more than 4096 tokens or 1024 adapters,
+ * k % 32 != 0, r % 8 != 0, r > 128 or r > k (and the expand needs m % 8 == 0).
+ * Replaces lora_bgmv / lora_sgmv (triteia/python/ops/matmul/lora.py:22-105), which transpose every adapter respectively
+ * build a segment table on the host on each call. */
+TRITEIA_HIP_API size_t triteia_hip_lora_scratch_bytes(int n_tokens, int n_adapters, int k, int r);
+TRITEIA_HIP_API int triteia_hip_lora_shrink(const void* x, long x_stride, const void* a, const void* indices, int index64, int n_tokens,
+                            int n_adapters, int k, int r, int accumulate, void* scratch, size_t scratch_bytes, int bf16, int dev,
+                            void* stream);
+TRITEIA_HIP_API int triteia_hip_lora_expand(void* y, long y_stride, const void* b, const void* scratch, int n_tokens, int n_adapters, int k,
+                            int r, int m, float scale, int accumulate, int bf16, int dev, void* stream);
+
 /* Quantise, prune and pack a dense fp16 weight [prob_k, prob_m] (row-major) with one fp16 scale per column: of every
  * aligned group of 4 along k the two entries of largest magnitude are kept (of equal ones the later), as
  * clamp(round(w / scale) + 8, 0, 15) - 8.  Writes qweight and meta in the layouts above, and meta_raw int16

@@ -12,6 +12,7 @@
 
 #include "lora.hip.h"
 #include "lora_mfma.hip.h"
+#include "lora_routed.hip.h"
 #include "pack.hip.h"
 #include "route_plan.hip.h"
 #include "sparse24_gemm.hip.h"
@@ -1421,6 +1422,139 @@ int triteia_hip_sgmv_routed_bf16(void* y, long y_stride, const void* x, long x_s
                                  int n_adapters, int d_in, int d_out, float scale, const void* plan, int prob_n,
                                  int accumulate, int dev, void* stream) {
   return sgmv_routed_impl<bf16_t>(y, y_stride, x, x_stride, w_base, w_stride, n_adapters, d_in, d_out, scale, plan, prob_n, accumulate, dev, stream);
+}
+
+}  // extern "C"
+
+namespace {
+
+// How the LoRA pair on raw indices cuts a batch.
+struct LoraCut {
+  int r16, nt, splits, max_tiles;
+  size_t perm_at, partial_at, total;   // bytes into the scratch
+};
+// Tiles of 16 tokens where the adapters have few each (what a tile reads is its adapter, however full it is), of 64 from
+// 32 tokens per adapter on (32 at ranks above 64, whose sums take the registers): 256 tokens over 32 adapters of rank 16
+// 11.2 us in tiles of 16 against 15.0 in tiles of 64, 2000 over 8 of rank 64 27.5 in tiles of 64, 27.5 / 28.5 in 16 / 32.
+// K in as many shares as make about 192 workgroups on the bound on the tiles, at most 8 (the expand reads every share
+// once per 256 columns), each share at least one step of 32 for every wavefront.  Shrink + expand at 1 / 2 / 4 / 8 / 16
+// shares: 100 tokens over 32 of rank 16 on 4096 x 11008 (39 tiles) 11.8 / 9.8 / 8.5 / 8.4 / 9.1 us, 16 tokens on
+// 4096 x 4096 (17 tiles) 8.9 / 7.7 / 6.9 / 6.8 / 7.4, 1000 over 8 of rank 64 (24 tiles) 34 / 26 / 21 / 19.5 / 26.7, 2000
+// (40 tiles) 40.5 / 32.4 / 27.5 / 32.7 / 44.
+LoraCut lora_cut(int n_tokens, int n_adapters, int k, int r) {
+  LoraCut c;
+  c.r16 = r <= 16 ? 1 : r <= 32 ? 2 : r <= 64 ? 4 : 8;
+  const int groups = n_adapters < n_tokens ? n_adapters : n_tokens;
+  c.nt = n_tokens < 32 * groups ? 1 : (c.r16 == 8 ? 2 : 4);
+  c.max_tiles = lora_max_tiles(n_tokens, n_adapters, 16 * c.nt);
+  const int steps = k / 32;
+  int splits = 192 / c.max_tiles;
+  splits = splits < 1 ? 1 : splits > 8 ? 8 : splits;
+  int per = (steps + splits - 1) / splits;
+  if (per < 4) per = 4;
+  c.splits = (steps + per - 1) / per;
+  c.perm_at = sizeof(int4) * (size_t)c.max_tiles;
+  c.partial_at = (c.perm_at + sizeof(int) * (size_t)n_tokens + 255) / 256 * 256;
+  c.total = c.partial_at + sizeof(float) * (size_t)c.splits * (size_t)n_tokens * (size_t)r;
+  return c;
+}
+bool lora_routed_takes(int n_tokens, int n_adapters, int k, int r) {
+  return n_tokens > 0 && n_tokens <= kLoraMaxTokens && n_adapters > 0 && n_adapters <= kLoraMaxAdapters && k > 0 && k % 32 == 0 && r > 0 &&
+         r % 8 == 0 && r <= kLoraMaxNarrow && r <= k;
+}
+
+template <class T>
+LoraArgs<T> lora_args(const LoraCut& c, void* scratch, int n_tokens, int n_adapters, int k, int r, int accumulate) {
+  LoraArgs<T> a;
+  memset(&a, 0, sizeof(a));
+  a.n_tokens = n_tokens;
+  a.n_adapters = n_adapters;
+  a.k = k;
+  a.r = r;
+  a.splits = c.splits;
+  a.accumulate = accumulate;
+  char* p = static_cast<char*>(scratch);
+  a.tiles = reinterpret_cast<int4*>(p);
+  a.perm = reinterpret_cast<int*>(p + c.perm_at);
+  a.partial = reinterpret_cast<float*>(p + c.partial_at);
+  return a;
+}
+
+#define LORA_PICK(KERNEL_, T_, GRID_)                                                                             \
+  do {                                                                                                            \
+    if (c.r16 == 1 && c.nt == 1) hipLaunchKernelGGL((KERNEL_<T_, 1, 1>), GRID_, dim3(256), 0, st, a);             \
+    else if (c.r16 == 1) hipLaunchKernelGGL((KERNEL_<T_, 1, 4>), GRID_, dim3(256), 0, st, a);                     \
+    else if (c.r16 == 2 && c.nt == 1) hipLaunchKernelGGL((KERNEL_<T_, 2, 1>), GRID_, dim3(256), 0, st, a);        \
+    else if (c.r16 == 2) hipLaunchKernelGGL((KERNEL_<T_, 2, 4>), GRID_, dim3(256), 0, st, a);                     \
+    else if (c.r16 == 4 && c.nt == 1) hipLaunchKernelGGL((KERNEL_<T_, 4, 1>), GRID_, dim3(256), 0, st, a);        \
+    else if (c.r16 == 4) hipLaunchKernelGGL((KERNEL_<T_, 4, 4>), GRID_, dim3(256), 0, st, a);                     \
+    else if (c.nt == 1) hipLaunchKernelGGL((KERNEL_<T_, 8, 1>), GRID_, dim3(256), 0, st, a);                      \
+    else hipLaunchKernelGGL((KERNEL_<T_, 8, 2>), GRID_, dim3(256), 0, st, a);                                     \
+  } while (0)
+
+template <class T>
+int lora_shrink_impl(const void* x, long x_stride, const void* w, const void* indices, int index64, int n_tokens, int n_adapters, int k,
+                     int r, int accumulate, void* scratch, hipStream_t st) {
+  const LoraCut c = lora_cut(n_tokens, n_adapters, k, r);
+  LoraArgs<T> a = lora_args<T>(c, scratch, n_tokens, n_adapters, k, r, accumulate);
+  a.x = static_cast<const T*>(x);
+  a.x_stride = x_stride;
+  a.a = static_cast<const T*>(w);
+  a.indices = indices;
+  a.index64 = index64;
+  LORA_PICK(lora_shrink_kernel, T, dim3(c.max_tiles, c.splits));
+  return check_launch("lora_shrink_kernel");
+}
+template <class T>
+int lora_expand_impl(void* y, long y_stride, const void* w, const void* scratch, int n_tokens, int n_adapters, int k, int r, int m,
+                     float scale, int accumulate, hipStream_t st) {
+  const LoraCut c = lora_cut(n_tokens, n_adapters, k, r);
+  LoraArgs<T> a = lora_args<T>(c, const_cast<void*>(scratch), n_tokens, n_adapters, k, r, accumulate);
+  a.y = static_cast<T*>(y);
+  a.y_stride = y_stride;
+  a.b = static_cast<const T*>(w);
+  a.m = m;
+  a.scale = scale;
+  LORA_PICK(lora_expand_kernel, T, dim3(c.max_tiles, (m + kLoraExpandCols - 1) / kLoraExpandCols));
+  return check_launch("lora_expand_kernel");
+}
+#undef LORA_PICK
+
+}  // namespace
+
+extern "C" {
+
+size_t triteia_hip_lora_scratch_bytes(int n_tokens, int n_adapters, int k, int r) {
+  return lora_routed_takes(n_tokens, n_adapters, k, r) ? lora_cut(n_tokens, n_adapters, k, r).total : 0;
+}
+
+int triteia_hip_lora_shrink(const void* x, long x_stride, const void* a, const void* indices, int index64, int n_tokens, int n_adapters,
+                            int k, int r, int accumulate, void* scratch, size_t scratch_bytes, int bf16, int dev, void* stream) {
+  if (n_tokens == 0) return TRITEIA_HIP_OK;
+  if (!lora_routed_takes(n_tokens, n_adapters, k, r))
+    return fail(TRITEIA_HIP_ERR_KERN_SHAPE, "lora_shrink: tokens=%d adapters=%d k=%d r=%d", n_tokens, n_adapters, k, r);
+  if (!x || !a || !indices || !scratch) return fail(TRITEIA_HIP_ERR_ARGUMENT, "lora_shrink: null tensor pointer");
+  if (scratch_bytes < triteia_hip_lora_scratch_bytes(n_tokens, n_adapters, k, r) || reinterpret_cast<uintptr_t>(scratch) % 16 != 0)
+    return fail(TRITEIA_HIP_ERR_ARGUMENT, "lora_shrink: the scratch must be 16-byte aligned and hold %zu bytes (got %zu)",
+                triteia_hip_lora_scratch_bytes(n_tokens, n_adapters, k, r), scratch_bytes);
+  DeviceGuard g(dev);
+  if (!g.ok) return fail(TRITEIA_HIP_ERR_RUNTIME, "cannot select device %d", dev);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  return bf16 ? lora_shrink_impl<bf16_t>(x, x_stride, a, indices, index64, n_tokens, n_adapters, k, r, accumulate, scratch, st)
+              : lora_shrink_impl<_Float16>(x, x_stride, a, indices, index64, n_tokens, n_adapters, k, r, accumulate, scratch, st);
+}
+
+int triteia_hip_lora_expand(void* y, long y_stride, const void* b, const void* scratch, int n_tokens, int n_adapters, int k, int r, int m,
+                            float scale, int accumulate, int bf16, int dev, void* stream) {
+  if (n_tokens == 0 || m == 0) return TRITEIA_HIP_OK;
+  if (!lora_routed_takes(n_tokens, n_adapters, k, r) || m < 0 || m % 8 != 0)
+    return fail(TRITEIA_HIP_ERR_KERN_SHAPE, "lora_expand: tokens=%d adapters=%d k=%d r=%d m=%d", n_tokens, n_adapters, k, r, m);
+  if (!y || !b || !scratch) return fail(TRITEIA_HIP_ERR_ARGUMENT, "lora_expand: null tensor pointer");
+  DeviceGuard g(dev);
+  if (!g.ok) return fail(TRITEIA_HIP_ERR_RUNTIME, "cannot select device %d", dev);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  return bf16 ? lora_expand_impl<bf16_t>(y, y_stride, b, scratch, n_tokens, n_adapters, k, r, m, scale, accumulate, st)
+              : lora_expand_impl<_Float16>(y, y_stride, b, scratch, n_tokens, n_adapters, k, r, m, scale, accumulate, st);
 }
 
 int triteia_hip_pack_2_4(const void* weight, const void* scales, void* qweight, void* meta, void* meta_raw, int prob_k, int prob_m,

@@ -118,3 +118,43 @@ def sgmv_routed(y, x, weights, plan, scale=1.0, accumulate=True):
     _check(fn(
         _ffi.ptr(y), y.stride(0), _ffi.ptr(x), x.stride(0), _ffi.ptr(weights), d_in * d_out, n_adapters, d_in, d_out,
         float(scale), _ffi.ptr(plan), x.size(0), 1 if accumulate else 0, _ffi.device_index(x), _ffi.stream_of(x)))
+
+
+def lora_scratch(n_tokens, weights_A):
+    """Scratch for `lora_shrink` on `n_tokens` tokens (uint8 tensor), or None if the pair does not take the shape."""
+    n_adapters, k, r = weights_A.shape
+    nbytes = _ffi.lib().triteia_hip_lora_scratch_bytes(n_tokens, n_adapters, k, r)
+    return torch.empty(nbytes, dtype=torch.uint8, device=weights_A.device) if nbytes else None
+
+
+def lora_shrink(x, weights_A, indices, scratch, accumulate):
+    """The first of the two launches of y[t] (+)= scale * (x[t] @ A[i]) @ B[i], i = indices[t]: routes the tokens and
+    leaves x @ A in `scratch` (from `lora_scratch`) for `lora_expand` with the same `accumulate` (False: y is
+    stored, and tokens without an adapter get zeros).
+
+    weights_A [n_adapters, k, r] fp16 or bf16 (as x), contiguous; indices int32 or int64, any order."""
+    n_adapters, k, r = weights_A.shape
+    n_tokens = x.size(0)
+    _ffi.require_gpu(x=x, weights_A=weights_A, indices=indices, scratch=scratch)
+    dtype = _lora_dtype(x, weights_A=weights_A)
+    if indices.dtype not in (torch.int32, torch.int64):
+        raise RuntimeError(f"indices must be torch.int32 or torch.int64, got {indices.dtype}")
+    if x.dim() != 2 or x.size(1) != k or indices.dim() != 1 or indices.size(0) != n_tokens:
+        raise RuntimeError("shape mismatch between x, weights_A and indices")
+    _check(_ffi.lib().triteia_hip_lora_shrink(
+        _ffi.ptr(x), k, _ffi.ptr(weights_A), _ffi.ptr(indices), 1 if indices.dtype == torch.int64 else 0, n_tokens, n_adapters, k, r,
+        1 if accumulate else 0, _ffi.ptr(scratch), scratch.numel(), 1 if dtype == torch.bfloat16 else 0, _ffi.device_index(x),
+        _ffi.stream_of(x)))
+
+
+def lora_expand(y, weights_B, scratch, k, accumulate, scale=1.0):
+    """The second launch: y [tokens, m] from the scratch of `lora_shrink` (whose A had k rows), weights_B
+    [n_adapters, r, m] contiguous."""
+    _ffi.require_gpu(y=y, weights_B=weights_B, scratch=scratch)
+    dtype = _lora_dtype(y, weights_B=weights_B)
+    n_adapters, r, m = weights_B.shape
+    if y.dim() != 2 or y.size(1) != m:
+        raise RuntimeError("shape mismatch between y and weights_B")
+    _check(_ffi.lib().triteia_hip_lora_expand(
+        _ffi.ptr(y), m, _ffi.ptr(weights_B), _ffi.ptr(scratch), y.size(0), n_adapters, k, r, m, float(scale), 1 if accumulate else 0,
+        1 if dtype == torch.bfloat16 else 0, _ffi.device_index(y), _ffi.stream_of(y)))

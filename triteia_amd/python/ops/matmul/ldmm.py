@@ -5,7 +5,7 @@ delta indices[t] - M; -1 means base model only.
 """
 import torch
 
-from triteia_amd.python.capi import route_plan, routed_workspace, sbmm_2_4_routed, sgmv_routed
+from triteia_amd.python.capi import lora_expand, lora_scratch, lora_shrink, route_plan, routed_workspace, sbmm_2_4_routed, sgmv_routed
 from .lora import lora_forloop
 from .sbmm import sbmm_4bit_2_4_forloop
 
@@ -41,12 +41,27 @@ def baseline_ldmm(indices, x, LwA, LwB, DeltaW, metas, ss, base_weight=None, deb
     return y.to(x.dtype)
 
 
+def _lora_steps(x, A, B, indices):
+    """(shrink(), expand(y)) for the LoRA tokens, y += (x @ A[i]) @ B[i], with their buffers allocated here: the pair of
+    launches that routes by itself, or a plan and the routed SGMV kernels for the shapes it does not take."""
+    scratch = lora_scratch(x.shape[0], A) if x.shape[0] > 0 and B.shape[2] % 8 == 0 else None
+    if scratch is not None:
+        return (lambda: lora_shrink(x, A, indices, scratch, True)), (lambda y: lora_expand(y, B, scratch, A.shape[1], True))
+    plan = routed_workspace(x.shape[0], A.shape[0], x.device)
+    v = torch.empty((x.shape[0], A.shape[2]), dtype=torch.float16, device=x.device)
+
+    def shrink():
+        route_plan(indices, A.shape[0], workspace=plan)
+        sgmv_routed(v, x, A, plan, accumulate=False)
+    return shrink, (lambda y: sgmv_routed(y, v, B, plan))
+
+
 def ldmm(indices, x, LwA, LwB, DeltaW, metas, ss, base_weight=None, debug=False):
     """One routed LoRA pass (shrink + expand) for the LoRA tokens plus one routed sparse pass for
     the delta tokens, both accumulating in place into the base output; no gathers, no host
     synchronisation.  The reference routes the LoRA tokens through BGMV, which wants every
-    adapter transposed on each call (ldmm.py:93-105); the routed SGMV kernels
-    read LwA / LwB as they are, one routing pass serving both of its stages.
+    adapter transposed on each call (ldmm.py:93-105); the kernels here read LwA / LwB
+    as they are, one routing pass serving both of its stages.
 
     indices int [B]; x [B, H1]; LwA [M, H1, R]; LwB [M, R, H2]; DeltaW / metas / ss the stacked
     packed deltas.  Returns [B, H2] in x.dtype."""
@@ -56,8 +71,7 @@ def ldmm(indices, x, LwA, LwB, DeltaW, metas, ss, base_weight=None, debug=False)
     idx32 = indices.to(torch.int32)
     if M > 0:
         A16, B16 = LwA.to(torch.float16).contiguous(), LwB.to(torch.float16).contiguous()
-        ws = routed_workspace(x_.shape[0], M, x_.device)
-        v = torch.empty((x_.shape[0], LwA.shape[2]), dtype=torch.float16, device=x_.device)
+        shrink, expand = _lora_steps(x_, A16, B16, idx32)
     if M > 0 and base_weight is not None:
         # Routing and the LoRA shrink need only x: they run on a side stream beside the base GEMM (a
         # library GEMM of a few hundred tokens leaves CUs idle); the expand follows the GEMM.  All
@@ -69,28 +83,26 @@ def ldmm(indices, x, LwA, LwB, DeltaW, metas, ss, base_weight=None, debug=False)
         # step measured 30 us longer on 256 tokens x 4096 x 11008; launched eagerly the order makes no difference)
         y = torch.matmul(x_, base_weight.t())
         with torch.cuda.stream(side):
-            plan = route_plan(idx32, M, workspace=ws)      # skips -1 and every index >= M (the delta tokens)
-            sgmv_routed(v, x_, A16, plan, accumulate=False)
+            shrink()                                       # skips -1 and every index >= M (the delta tokens)
         if DeltaW.shape[0] > 0:
             # LoRA tokens and delta tokens are different rows of y (disjoint index ranges): the expand stays
             # on the side stream, beside the delta kernel, and joins at the end
             side.wait_stream(cur)
             with torch.cuda.stream(side):
-                sgmv_routed(y, v, B16, plan)
+                expand(y)
             sbmm_2_4_routed(x_, DeltaW, metas, y, ss, idx32, index_offset=M, accumulate=True)
             cur.wait_stream(side)
             return y.to(x.dtype)
         cur.wait_stream(side)
-        sgmv_routed(y, v, B16, plan)
+        expand(y)
     else:
         if base_weight is not None:
             y = torch.matmul(x_, base_weight.t())
         else:
-            y = torch.zeros(x_.shape[0], LwB.shape[2], dtype=x_.dtype, device=x_.device)
+            y = torch.zeros(x_.shape[0], LwB.shape[2], dtype=x_.dtype, device=x.device)
         if M > 0:
-            plan = route_plan(idx32, M, workspace=ws)
-            sgmv_routed(v, x_, A16, plan, accumulate=False)
-            sgmv_routed(y, v, B16, plan)
+            shrink()
+            expand(y)
     if DeltaW.shape[0] > 0:
         sbmm_2_4_routed(x_, DeltaW, metas, y, ss, idx32, index_offset=M, accumulate=True)
     return y.to(x.dtype)

@@ -2,13 +2,33 @@
 (triteia/python/ops/matmul/lora.py:4-105)."""
 import torch
 
-from triteia_amd.python.capi import add_lora_bgmv, add_lora_sgmv_cutlass, route_plan, sgmv_routed
+from triteia_amd.python.capi import add_lora_bgmv, add_lora_sgmv_cutlass, lora_expand, lora_scratch, lora_shrink, route_plan, sgmv_routed
 
 
 def _base(x, out_features, base_weight):
     if base_weight is not None:
         return torch.matmul(x, base_weight.t())
     return torch.zeros(x.shape[0], out_features, dtype=x.dtype, device=x.device)
+
+
+def _lora_by_indices(weights_A, weights_B, x, indices, base_weight, scale=1.0):
+    """The pair of launches that takes adapters, tokens and indices as they are (capi.lora_shrink / lora_expand); None
+    for the shapes and types that it leaves to the kernels of the reference's own interfaces."""
+    if not (weights_A.dim() == weights_B.dim() == 3 and x.dim() == 2 and indices.dim() == 1 and x.size(0) > 0
+            and weights_A.is_contiguous() and weights_B.is_contiguous() and indices.dtype in (torch.int32, torch.int64)
+            and weights_A.size(0) == weights_B.size(0) and weights_A.size(2) == weights_B.size(1) and weights_B.size(2) % 8 == 0
+            and x.dtype == weights_A.dtype == weights_B.dtype and x.dtype in (torch.float16, torch.bfloat16)
+            and x.size(1) == weights_A.size(1) and indices.size(0) == x.size(0)):
+        return None
+    scratch = lora_scratch(x.size(0), weights_A)
+    if scratch is None:
+        return None
+    accumulate = base_weight is not None
+    lora_shrink(x.contiguous(), weights_A, indices.contiguous(), scratch, accumulate)
+    # (without a base weight every row is written by the kernel: tokens without an adapter get zeros)
+    y = torch.matmul(x, base_weight.t()) if accumulate else torch.empty((x.size(0), weights_B.size(2)), dtype=x.dtype, device=x.device)
+    lora_expand(y, weights_B, scratch, weights_A.size(1), accumulate, scale)
+    return y
 
 
 def lora_forloop(weights_A, weights_B, x, indices, base_weight=None):
@@ -26,6 +46,10 @@ def lora_forloop(weights_A, weights_B, x, indices, base_weight=None):
 def lora_bgmv(weights_A, weights_B, x, indices, base_weight=None, layer_idx=0, scale=1.0):
     """BGMV: one adapter look-up per token (lora.py:22-48).  Tokens with index -1 are skipped
     inside the kernel, so no gather / scatter is needed."""
+    if layer_idx == 0:          # (these weights have one layer: any other index is for the interface below to refuse)
+        y = _lora_by_indices(weights_A, weights_B, x, indices, base_weight, scale)
+        if y is not None:
+            return y
     y = _base(x, weights_B.shape[2], base_weight)
     weights_A_T = weights_A.transpose(1, 2).contiguous().unsqueeze(1)
     weights_B_T = weights_B.transpose(1, 2).contiguous().unsqueeze(1)
@@ -34,7 +58,12 @@ def lora_bgmv(weights_A, weights_B, x, indices, base_weight=None, layer_idx=0, s
 
 
 def lora_sgmv(weights_A, weights_B, x, indices, base_weight=None, layer_idx=0):
-    """SGMV on a host-built segment table, as lora.py:50-105 (needs ascending grouped indices)."""
+    """SGMV (lora.py:50-105).  The tokens are grouped on the device, in any order; shapes that the pair of launches behind
+    that does not take go to a host-built segment table, as in the reference, and need ascending grouped indices."""
+    if layer_idx == 0:
+        y = _lora_by_indices(weights_A, weights_B, x, indices, base_weight)
+        if y is not None:
+            return y
     y = _base(x, weights_B.shape[2], base_weight)
     if torch.all(indices == -1):
         return y
@@ -55,6 +84,10 @@ def lora_sgmv(weights_A, weights_B, x, indices, base_weight=None, layer_idx=0):
 def lora_sgmv_routed(weights_A, weights_B, x, indices, base_weight=None, plan=None):
     """SGMV with device-side grouping: any index order, no host synchronisation; `plan`
     (from capi.route_plan with n_deltas = number of adapters) can be shared with other ops."""
+    if plan is None:
+        y = _lora_by_indices(weights_A, weights_B, x, indices, base_weight)
+        if y is not None:
+            return y
     y = _base(x, weights_B.shape[2], base_weight)
     n_adapters, _, rank = weights_A.shape
     if plan is None:
