@@ -1,16 +1,19 @@
-"""Build recipe for libtriteia_hip.so (gfx950) -- run as `python -m triteia_amd.build`.
+"""Build recipe for libtriteia_hip.so (gfx950) and the torch binding of its ops -- run as `python -m triteia_amd.build`.
 
-hipcc cross-compiles without a GPU, so this works in a CPU-only container.  The
-library is built in-tree at triteia_amd/lib/libtriteia_hip.so.
+hipcc cross-compiles without a GPU, so this works in a CPU-only container.  Both are built in-tree:
+triteia_amd/lib/libtriteia_hip.so (kernels and C ABI) and triteia_amd/lib/triteia_torch.so (host code only).
 """
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 SRC = os.path.join(HERE, "csrc", "triteia_hip.hip")
 LIB_DIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIB_DIR, "libtriteia_hip.so")
+TORCH_SRC = os.path.join(HERE, "csrc", "torch_ops.cpp")
+TORCH_LIB = os.path.join(LIB_DIR, "triteia_torch.so")
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
@@ -55,14 +58,35 @@ def build(verbose: bool = True, extra_flags=()) -> str:
         raise RuntimeError(f"hipcc failed ({res.returncode}):\n{err}")
     if verbose and err.strip():
         print(err, file=sys.stderr)
+    build_torch_binding(verbose=verbose)
     return LIB
 
 
+def build_torch_binding(verbose: bool = True) -> str:
+    """The ops' native call path (host code, no device code): g++ against the installed torch and the library above."""
+    import torch
+    root = os.path.dirname(torch.__file__)
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{root}/include",
+           f"-I{root}/include/torch/csrc/api/include", f"-I{rocm}/include", f"-I{sysconfig.get_paths()['include']}", TORCH_SRC, "-o", TORCH_LIB,
+           f"-L{root}/lib", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", f"-L{LIB_DIR}", "-ltriteia_hip",
+           "-Wl,-rpath,$ORIGIN"]
+    if verbose:
+        print("[triteia_amd.build]", " ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed ({res.returncode}):\n{res.stderr}")
+    return TORCH_LIB
+
+
 def ensure_built(verbose: bool = True) -> str:
-    """The built library's path; compiles it first if (and only if) there is none in the tree.  For tests,
-    smoke runs and benchmarks, which load what is built; `build()` itself compiles every time."""
+    """The built library's path; compiles it (and the torch binding) first if (and only if) it is not in the tree.  For
+    tests, smoke runs and benchmarks, which load what is built; `build()` itself compiles every time."""
     if not os.path.exists(LIB):
         build(verbose=verbose)
+    elif not os.path.exists(TORCH_LIB):
+        build_torch_binding(verbose=verbose)
     return LIB
 
 

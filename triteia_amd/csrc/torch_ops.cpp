@@ -1,0 +1,252 @@
+// The ops' ordinary case from Python to the C ABI in one native call: argument checks, output and scratch from torch's
+// caching allocator, the current stream, the launches.  (The same steps through ctypes and torch's Python API cost 15 - 20 us
+// a call, more than most decode-size kernels take on the GPU; here 4 - 6 us.)
+//
+// Every function returns None for whatever is not the ordinary case -- another device, type, layout or shape, a pair
+// of sizes that the library refuses -- before it has launched anything; the Python op then takes its own path, which
+// checks the arguments one by one and raises the reference's error texts.  Nothing is kept between calls.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "../../include/triteia_hip.h"
+
+namespace {
+
+using at::Tensor;
+
+struct Args {
+  PyObject* const* v;
+  Py_ssize_t n;
+  bool tensor(int i) const { return i < n && THPVariable_Check(v[i]); }
+  const Tensor& operator[](int i) const { return THPVariable_Unpack(v[i]); }
+  bool none(int i) const { return i < n && v[i] == Py_None; }
+};
+
+bool on(const Tensor& t, const Tensor& ref, at::ScalarType type, int64_t dim) {
+  return t.scalar_type() == type && t.dim() == dim && t.device() == ref.device() && t.layout() == at::kStrided;
+}
+bool dense_on(const Tensor& t, const Tensor& ref, at::ScalarType type, int64_t dim) { return on(t, ref, type, dim) && t.is_contiguous(); }
+
+// the current stream of x's device, and that device current for what follows
+struct Place {
+  c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard;
+  int dev;
+  c10::hip::HIPStreamMasqueradingAsCUDA stream;
+  explicit Place(const Tensor& x)
+      : guard(x.device()), dev(x.device().index()), stream(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(x.device().index())) {}
+  void* handle() const { return stream.stream(); }
+};
+
+Tensor scratch_bytes(size_t bytes, const Tensor& like) {
+  return at::empty({(int64_t)((bytes + 255) / 256 * 256)}, like.options().dtype(at::kByte));
+}
+
+// sizes that fit the library's ints, on a GPU
+bool sizes_ok(std::initializer_list<int64_t> sizes) {
+  for (int64_t s : sizes)
+    if (s <= 0 || s > 0x7fffffff) return false;
+  return true;
+}
+
+// stacked packed matrices: q [n, k/32, 2m], meta [n, m, k/16], s [n, 1, m]
+bool packed_ok(const Tensor& q, const Tensor& meta, const Tensor& s, const Tensor& x, int64_t n, int64_t k, int64_t m) {
+  return dense_on(q, x, at::kInt, 3) && dense_on(meta, x, at::kShort, 3) && dense_on(s, x, at::kHalf, 3) && m % 128 == 0 && k % 64 == 0 &&
+         sizes_ok({n, k, m}) && q.size(0) == n && q.size(1) == k / 32 && q.size(2) == 2 * m && meta.size(0) == n && meta.size(1) == m &&
+         meta.size(2) == k / 16 && s.size(0) == n && s.size(1) == 1 && s.size(2) == m;
+}
+
+bool base_ok(const Args& a, int i, const Tensor& x, int64_t k, int64_t m) {
+  return a.none(i) || (a.tensor(i) && on(a[i], x, x.scalar_type(), 2) && a[i].size(0) == m && a[i].size(1) == k);
+}
+
+// matmul(qweight, x, meta, s): ops.matmul_4bit_2_4
+Tensor matmul(const Args& a) {
+  if (a.n != 4 || !a.tensor(0) || !a.tensor(1) || !a.tensor(2) || !a.tensor(3)) return {};
+  const Tensor &q = a[0], &x = a[1], &meta = a[2], &s = a[3];
+  if (!x.is_cuda() || x.dim() < 1 || x.scalar_type() != at::kHalf || s.dim() != 2) return {};
+  const int64_t k = x.size(-1), m = s.size(1), rows = k > 0 ? x.numel() / k : 0;
+  if (!sizes_ok({k, m, rows}) || m % 128 != 0 || k % 64 != 0 || s.size(0) != 1 || !dense_on(q, x, at::kInt, 2) || !dense_on(meta, x, at::kShort, 2) ||
+      !dense_on(s, x, at::kHalf, 2) || q.size(0) != k / 32 || q.size(1) != 2 * m || meta.size(0) != m || meta.size(1) != k / 16)
+    return {};
+  const Place at_(x);
+  const Tensor xc = x.is_contiguous() ? x : x.contiguous();
+  c10::SmallVector<int64_t, 5> shape(x.sizes().begin(), x.sizes().end());
+  shape.back() = m;
+  Tensor y = at::empty(shape, x.options());
+  const size_t split = triteia_hip_bmm_scratch_bytes(m, 1, rows, k);
+  const Tensor scratch = split ? scratch_bytes(split, x) : Tensor();
+  return triteia_hip_bmm_2_4_tokens_scratch(xc.data_ptr(), q.data_ptr(), meta.data_ptr(), y.data_ptr(), s.data_ptr(), m, 1, rows, k,
+                                            split ? scratch.data_ptr() : nullptr, split, at_.dev, at_.handle())
+             ? Tensor()
+             : y;
+}
+
+// bmm(qweights, xs, metas, ss): ops.bmm_4bit_2_4
+Tensor bmm(const Args& a) {
+  if (a.n != 4 || !a.tensor(0) || !a.tensor(1) || !a.tensor(2) || !a.tensor(3)) return {};
+  const Tensor &q = a[0], &x = a[1], &meta = a[2], &s = a[3];
+  if (!x.is_cuda() || x.dim() != 3 || x.scalar_type() != at::kHalf || s.dim() != 3) return {};
+  const int64_t n = x.size(0), tokens = x.size(1), k = x.size(2), m = s.size(2);
+  if (!sizes_ok({tokens}) || !packed_ok(q, meta, s, x, n, k, m)) return {};
+  const Place at_(x);
+  const Tensor xc = x.is_contiguous() ? x : x.contiguous();
+  Tensor y = at::empty({n, tokens, m}, x.options());
+  const size_t split = triteia_hip_bmm_scratch_bytes(m, n, tokens, k);
+  const Tensor scratch = split ? scratch_bytes(split, x) : Tensor();
+  return triteia_hip_bmm_2_4_tokens_scratch(xc.data_ptr(), q.data_ptr(), meta.data_ptr(), y.data_ptr(), s.data_ptr(), m, n, tokens, k,
+                                            split ? scratch.data_ptr() : nullptr, split, at_.dev, at_.handle())
+             ? Tensor()
+             : y;
+}
+
+// y (+)= the routed product of x [tokens, k]; false: refused, nothing launched
+bool routed(const Tensor& x, const Tensor& q, const Tensor& meta, const Tensor& s, const Tensor& indices, Tensor& y, int offset,
+            bool accumulate, const Place& at_) {
+  const int64_t tokens = x.size(0), k = x.size(1), m = y.size(1), n = q.size(0);
+  Tensor ws;
+  size_t bytes = 0;
+  if (!triteia_hip_routed_in_kernel(tokens, n, m, k)) {     // (a batch that is routed inside the kernel needs no plan)
+    bytes = triteia_hip_sbmm_routed_workspace_bytes(tokens, n);
+    ws = scratch_bytes(bytes, x);
+  }
+  return triteia_hip_sbmm_2_4_routed(x.data_ptr(), q.data_ptr(), meta.data_ptr(), y.data_ptr(), s.data_ptr(), indices.data_ptr(), offset, n,
+                                     m, tokens, k, bytes ? ws.data_ptr() : nullptr, bytes, accumulate, at_.dev, at_.handle()) == 0;
+}
+
+// sbmm(qweights, xs, metas, ss, indices, base or None): ops.sbmm_4bit_2_4_native
+Tensor sbmm(const Args& a) {
+  if (a.n != 6) return {};
+  for (int i = 0; i < 5; i++)
+    if (!a.tensor(i)) return {};
+  const Tensor &q = a[0], &x = a[1], &meta = a[2], &s = a[3], &indices = a[4];
+  if (!x.is_cuda() || x.dim() != 2 || x.scalar_type() != at::kHalf || s.dim() != 3) return {};
+  const int64_t tokens = x.size(0), k = x.size(1), m = s.size(2);
+  if (!sizes_ok({tokens}) || !packed_ok(q, meta, s, x, q.size(0), k, m) || !base_ok(a, 5, x, k, m)) return {};
+  if (indices.device() != x.device() || indices.dim() != 1 || indices.size(0) != tokens || !indices.is_contiguous() ||
+      !at::isIntegralType(indices.scalar_type(), false))
+    return {};
+  const Place at_(x);
+  const Tensor xc = x.is_contiguous() ? x : x.contiguous();
+  const Tensor idx = indices.scalar_type() == at::kInt ? indices : indices.to(at::kInt);
+  const bool base = !a.none(5);
+  Tensor y = base ? at::matmul(xc, a[5].t()) : at::zeros({tokens, m}, x.options());
+  return routed(xc, q, meta, s, idx, y, 0, base, at_) ? y : Tensor();
+}
+
+bool lora_ok(const Tensor& A, const Tensor& B, const Tensor& x, const Tensor& indices) {
+  return x.is_cuda() && x.dim() == 2 && (x.scalar_type() == at::kHalf || x.scalar_type() == at::kBFloat16) &&
+         dense_on(A, x, x.scalar_type(), 3) && dense_on(B, x, x.scalar_type(), 3) && indices.device() == x.device() && indices.dim() == 1 &&
+         indices.is_contiguous() && (indices.scalar_type() == at::kInt || indices.scalar_type() == at::kLong) &&
+         sizes_ok({x.size(0), x.size(1), A.size(0), A.size(2), B.size(2)}) && indices.size(0) == x.size(0) && A.size(1) == x.size(1) &&
+         B.size(0) == A.size(0) && B.size(1) == A.size(2) && B.size(2) % 8 == 0;
+}
+size_t lora_bytes(const Tensor& A, const Tensor& x) { return triteia_hip_lora_scratch_bytes(x.size(0), A.size(0), A.size(1), A.size(2)); }
+bool lora_shrink(const Tensor& x, const Tensor& A, const Tensor& indices, const Tensor& scratch, bool accumulate, int dev, void* stream) {
+  return triteia_hip_lora_shrink(x.data_ptr(), x.size(1), A.data_ptr(), indices.data_ptr(), indices.scalar_type() == at::kLong, x.size(0), A.size(0),
+                                 A.size(1), A.size(2), accumulate, scratch.data_ptr(), scratch.numel(), x.scalar_type() == at::kBFloat16, dev,
+                                 stream) == 0;
+}
+bool lora_expand(const Tensor& y, const Tensor& A, const Tensor& B, const Tensor& scratch, double scale, bool accumulate, int dev, void* stream) {
+  return triteia_hip_lora_expand(y.data_ptr(), y.size(1), B.data_ptr(), scratch.data_ptr(), y.size(0), B.size(0), A.size(1), B.size(1), y.size(1),
+                                 (float)scale, accumulate, y.scalar_type() == at::kBFloat16, dev, stream) == 0;
+}
+
+// lora(weights_A, weights_B, x, indices, base or None, scale): ops.lora_bgmv / lora_sgmv / lora_sgmv_routed
+Tensor lora(const Args& a) {
+  if (a.n != 6 || !a.tensor(0) || !a.tensor(1) || !a.tensor(2) || !a.tensor(3)) return {};
+  const Tensor &A = a[0], &B = a[1], &x = a[2], &indices = a[3];
+  const double scale = PyFloat_AsDouble(a.v[5]);
+  if (PyErr_Occurred()) { PyErr_Clear(); return {}; }
+  if (!lora_ok(A, B, x, indices) || !base_ok(a, 4, x, x.size(1), B.size(2))) return {};
+  const size_t bytes = lora_bytes(A, x);
+  if (bytes == 0) return {};
+  const Place at_(x);
+  const Tensor xc = x.is_contiguous() ? x : x.contiguous();
+  const Tensor scratch = scratch_bytes(bytes, x);
+  const bool base = !a.none(4);
+  if (!lora_shrink(xc, A, indices, scratch, base, at_.dev, at_.handle())) return {};
+  // (without a base weight every row is written by the expand: tokens without an adapter get zeros)
+  Tensor y = base ? at::matmul(xc, a[4].t()) : at::empty({x.size(0), B.size(2)}, x.options());
+  return lora_expand(y, A, B, scratch, scale, base, at_.dev, at_.handle()) ? y : Tensor();
+}
+
+// ldmm(indices, x, LwA, LwB, DeltaW, metas, ss, base or None): ops.ldmm.  One stream: with the LoRA pair at 10 us, a side
+// stream for it beside the base GEMM costs more in events than it hides (256 tokens over 32 adapters of rank 16 and 32
+// deltas of 4096 x 11008: 148 us on one stream, 149 with the shrink on a side stream, 153 with the expand there as well;
+// 38 against 75 and 84 us of host time).
+Tensor ldmm(const Args& a) {
+  if (a.n != 8) return {};
+  for (int i = 0; i < 7; i++)
+    if (!a.tensor(i)) return {};
+  const Tensor &indices = a[0], &x = a[1], &A = a[2], &B = a[3], &q = a[4], &meta = a[5], &s = a[6];
+  if (x.scalar_type() != at::kHalf || indices.scalar_type() != at::kInt || !lora_ok(A, B, x, indices) || s.dim() != 3) return {};
+  const int64_t k = x.size(1), m = B.size(2);
+  const size_t bytes = lora_bytes(A, x);
+  if (bytes == 0 || !packed_ok(q, meta, s, x, q.size(0), k, m) || !base_ok(a, 7, x, k, m)) return {};
+  const Place at_(x);
+  const Tensor xc = x.is_contiguous() ? x : x.contiguous();
+  const Tensor scratch = scratch_bytes(bytes, x);
+  const bool base = !a.none(7);
+  if (!lora_shrink(xc, A, indices, scratch, base, at_.dev, at_.handle())) return {};
+  // (without a base weight the expand stores the adapters' rows and zeros in all others, the deltas' among them)
+  Tensor y = base ? at::matmul(xc, a[7].t()) : at::empty({x.size(0), m}, x.options());
+  if (!lora_expand(y, A, B, scratch, 1.0, base, at_.dev, at_.handle())) return {};
+  return routed(xc, q, meta, s, indices, y, A.size(0), true, at_) ? y : Tensor();
+}
+
+PyObject* wrap(Tensor&& t) {
+  if (!t.defined()) Py_RETURN_NONE;
+  return THPVariable_Wrap(std::move(t));
+}
+
+template <Tensor (*F)(const Args&)>
+PyObject* call(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  try {
+    return wrap(F(Args{v, n}));
+  } catch (const std::exception& e) {
+    PyErr_SetString(PyExc_RuntimeError, e.what());
+    return nullptr;
+  }
+}
+
+// pack(weight, scales): (qweight, meta, meta_raw) of ops.utils.sparsity.prune_pack_2_4, or None
+PyObject* pack(PyObject*, PyObject* const* v, Py_ssize_t n) {
+  try {
+    const Args a{v, n};
+    if (n != 2 || !a.tensor(0) || !a.tensor(1)) Py_RETURN_NONE;
+    const Tensor &w = a[0], &s = a[1];
+    if (!w.is_cuda() || !dense_on(w, w, at::kHalf, 2) || !dense_on(s, w, at::kHalf, 2)) Py_RETURN_NONE;
+    const int64_t k = w.size(0), m = w.size(1);
+    if (!sizes_ok({k, m}) || k % 32 != 0 || m % 64 != 0 || s.numel() != m ||
+        (reinterpret_cast<uintptr_t>(w.data_ptr()) | reinterpret_cast<uintptr_t>(s.data_ptr())) % 4 != 0)
+      Py_RETURN_NONE;
+    const Place at_(w);
+    Tensor q = at::empty({k / 32, 2 * m}, w.options().dtype(at::kInt));
+    Tensor meta = at::empty({m, k / 16}, w.options().dtype(at::kShort)), raw = at::empty({m, k / 16}, w.options().dtype(at::kShort));
+    if (triteia_hip_pack_2_4(w.data_ptr(), s.data_ptr(), q.data_ptr(), meta.data_ptr(), raw.data_ptr(), k, m, at_.dev, at_.handle()))
+      Py_RETURN_NONE;
+    PyObject* out = PyTuple_New(3);
+    if (!out) return nullptr;
+    PyTuple_SET_ITEM(out, 0, THPVariable_Wrap(std::move(q)));
+    PyTuple_SET_ITEM(out, 1, THPVariable_Wrap(std::move(meta)));
+    PyTuple_SET_ITEM(out, 2, THPVariable_Wrap(std::move(raw)));
+    return out;
+  } catch (const std::exception& e) {
+    PyErr_SetString(PyExc_RuntimeError, e.what());
+    return nullptr;
+  }
+}
+
+#define METHOD(NAME_, FN_) {NAME_, reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(FN_)), METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {METHOD("matmul", (call<matmul>)), METHOD("bmm", (call<bmm>)), METHOD("sbmm", (call<sbmm>)), METHOD("lora", (call<lora>)), METHOD("ldmm", (call<ldmm>)),
+                         METHOD("pack", pack), {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "triteia_torch", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit_triteia_torch(void) { return PyModule_Create(&module); }

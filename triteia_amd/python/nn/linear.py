@@ -2,6 +2,7 @@ import torch
 import torch.nn as nn
 
 from triteia_amd.python.capi import mul_2_4
+from triteia_amd.python.capi._native import native
 from triteia_amd.python.ops.utils.sparsity import prune_pack_2_4
 
 
@@ -25,6 +26,9 @@ class sparse_low_precision_linear(nn.Module):
         self.register_buffer("workspace", torch.zeros(outfeatures // 128 * 16, dtype=torch.int32))
 
     def forward(self, x):
+        C = native().matmul(self.qweight, x, self.meta, self.scale)
+        if C is not None:
+            return C
         C = torch.empty(x.shape[:-1] + (self.outfeatures,), dtype=x.dtype, device=x.device)
         x2 = x.reshape(-1, x.shape[-1])
         x2 = x2 if x2.is_contiguous() else x2.contiguous()
@@ -109,6 +113,10 @@ class multi_delta_linear(nn.Module):
         from triteia_amd.python.capi import sbmm_2_4_planned, sbmm_2_4_routed
         x2 = x.reshape(-1, x.shape[-1])
         x2 = x2 if x2.is_contiguous() else x2.contiguous()
+        if plan is None:
+            y = native().sbmm(self.qweight, x2, self.meta, self.scale, indices, self.base)
+            if y is not None:
+                return y.view(x.shape[:-1] + (self.outfeatures,))
         if self.base is not None:
             y = torch.matmul(x2, self.base.t())
         else:

@@ -2,7 +2,8 @@
 (triteia/python/ops/matmul/lora.py:4-105)."""
 import torch
 
-from triteia_amd.python.capi import add_lora_bgmv, add_lora_sgmv_cutlass, lora_expand, lora_scratch, lora_shrink, route_plan, sgmv_routed
+from triteia_amd.python.capi import add_lora_bgmv, add_lora_sgmv_cutlass, route_plan, sgmv_routed
+from triteia_amd.python.capi._native import native
 
 
 def _base(x, out_features, base_weight):
@@ -14,21 +15,7 @@ def _base(x, out_features, base_weight):
 def _lora_by_indices(weights_A, weights_B, x, indices, base_weight, scale=1.0):
     """The pair of launches that takes adapters, tokens and indices as they are (capi.lora_shrink / lora_expand); None
     for the shapes and types that it leaves to the kernels of the reference's own interfaces."""
-    if not (weights_A.dim() == weights_B.dim() == 3 and x.dim() == 2 and indices.dim() == 1 and x.size(0) > 0
-            and weights_A.is_contiguous() and weights_B.is_contiguous() and indices.dtype in (torch.int32, torch.int64)
-            and weights_A.size(0) == weights_B.size(0) and weights_A.size(2) == weights_B.size(1) and weights_B.size(2) % 8 == 0
-            and x.dtype == weights_A.dtype == weights_B.dtype and x.dtype in (torch.float16, torch.bfloat16)
-            and x.size(1) == weights_A.size(1) and indices.size(0) == x.size(0)):
-        return None
-    scratch = lora_scratch(x.size(0), weights_A)
-    if scratch is None:
-        return None
-    accumulate = base_weight is not None
-    lora_shrink(x.contiguous(), weights_A, indices.contiguous(), scratch, accumulate)
-    # (without a base weight every row is written by the kernel: tokens without an adapter get zeros)
-    y = torch.matmul(x, base_weight.t()) if accumulate else torch.empty((x.size(0), weights_B.size(2)), dtype=x.dtype, device=x.device)
-    lora_expand(y, weights_B, scratch, weights_A.size(1), accumulate, scale)
-    return y
+    return native().lora(weights_A, weights_B, x, indices, base_weight, scale)
 
 
 def lora_forloop(weights_A, weights_B, x, indices, base_weight=None):

@@ -7,6 +7,7 @@ device and accepts any order.
 """
 import torch
 
+from triteia_amd.python.capi._native import native
 from triteia_amd.python.capi import mul_2_4, sbmm_2_4, sbmm_2_4_multilaunch, sbmm_2_4_routed
 
 
@@ -69,6 +70,9 @@ def sbmm_4bit_2_4_native(qweights, xs, metas, ss, indices, base_weight=None):
     """Single-launch routed sbmm (sbmm.py:89-142): tokens are grouped by index on the device, each
     delta's weights are read once, and the result is accumulated straight into the base output.
     No host synchronisation; indices may come in any order."""
+    y = native().sbmm(qweights, xs, metas, ss, indices, base_weight)
+    if y is not None:
+        return y
     y = _base(xs, ss.shape[2], base_weight)
     if indices.dtype != torch.int32:
         indices = indices.to(torch.int32)

@@ -2,6 +2,7 @@ import torch
 
 from triteia_amd.python.capi import mul_2_4
 from triteia_amd.python.capi._ffi import lock_workspace
+from triteia_amd.python.capi._native import native
 
 
 def matmul_4bit_2_4(qweight, x, meta, s):
@@ -9,6 +10,9 @@ def matmul_4bit_2_4(qweight, x, meta, s):
 
     qweight int32 [k/32, 2m], x fp16 [..., k], meta int16 [m, k/16], s fp16 [1, m] (or [k/128, m], grouped)
     -> fp16 [..., m]."""
+    C = native().matmul(qweight, x, meta, s)
+    if C is not None:
+        return C
     # every element of C is written by the kernel (unless k = 0); the lock workspace is never touched
     alloc = torch.empty if x.shape[-1] > 0 else torch.zeros
     C = alloc((x.shape[:-1] + (s.shape[1],)), dtype=x.dtype, device=x.device)

@@ -140,12 +140,12 @@ def prune_pack_2_4(weight: torch.Tensor, scale: torch.Tensor, mask: torch.Tensor
     Returns (qweight, meta, scales fp16 [1, m], meta_raw).  An fp16 weight on the GPU whose positions come from its own
     magnitudes is packed by one kernel (triteia_amd/csrc/pack.hip.h), bit for bit as the torch codec below."""
     k, m = weight.shape
-    if (mask is None and weight.is_cuda and weight.device == scale.device and weight.dtype == scale.dtype == torch.float16
-            and k % 32 == 0 and m % 64 == 0 and weight.numel() > 0 and scale.numel() == m):
-        from triteia_amd.python.capi import pack_2_4 as pack_on_gpu
+    if mask is None and weight.is_cuda and weight.dtype == torch.float16 and scale.numel() == m:
+        from triteia_amd.python.capi._native import native
         s16 = scale.reshape(1, m).contiguous()
-        qweight, meta, raw = pack_on_gpu(weight.contiguous(), s16)
-        return qweight, meta, s16, raw
+        packed = native().pack(weight.contiguous(), s16)
+        if packed is not None:
+            return packed[0], packed[1], s16, packed[2]
     if mask is None:
         mask = mask_creator(weight.t().contiguous(), n=2, m=4)
     lo, hi = positions_from_mask(mask)
