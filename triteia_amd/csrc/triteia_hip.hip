@@ -398,6 +398,46 @@ static unsigned plan_wide_grid(Sparse24Args& b, long rows, int m, int tok, int p
   }
   return (unsigned)wide_grid_units(rows, m, b.xcd_swizzle);
 }
+// Uniform launches: an XCD takes a block of column groups x a block of token tiles (order 4) where that makes its
+// L2 fetch fewer bytes than a run of column groups for every tile (order 1).  While the `window` workgroups that an XCD
+// holds at a time (32 CUs x 1 or 2) walk K, its L2 fetches the packed weights of their distinct column groups and the
+// activations of their distinct tiles once each: with units numbered column group first, a window of W units over
+// blocks of c column groups fetches c x (weights of a column group) + W / c x (activations of a tile), least near
+// c = sqrt(W x tile / column group).  Measured (order 1 -> the rule): 4096 x 4096 with 640 / 1024 / 1536 / 2048 tokens
+// 28.3 -> 27.1, 32.1 -> 30.6, 43.8 -> 41.6, 50.5 -> 46.8 us; 8192 x 8192 with 1000 tokens 81.2 -> 79.7 us; 11008 x 4096 with
+// 1280 tokens 92.5 -> 88.6 us; 4096 x 11008 and 8192 x 28672 the same either way (blocks of 14 column groups on the
+// latter, which a count over the whole launch instead of the window would pick, measured 1.7 % slower).
+// The sums do not depend on which workgroup takes which unit.  Returns the c of order 4, 0 = the layer's own order.
+static long wide_uniform_blocks(long rows, int m, int k, int tok, long window) {
+  if (wide_unit_order(m) != 1 || knobs().xcd_cgs < 0) return 0;
+  const long cgs = (m / 128 + 3) / 4, cg_pad = (cgs + 7) / 8 * 8;
+  const double w_cg = 512.0 * k * 0.375, x_tile = (double)tok * k * 2.0;
+  auto fetched = [&](long xc) {
+    const long tbs = 8 / (cg_pad / xc);
+    long slots = xc * ((rows + tbs - 1) / tbs);
+    if (slots > window) slots = window;
+    return (double)xc * w_cg + (double)((slots + xc - 1) / xc) * x_tile;
+  };
+  long best = cg_pad / 8;
+  double best_bytes = fetched(best);
+  for (long xc = 1; xc <= cg_pad; xc++) {
+    if (cg_pad % xc != 0 || cg_pad / xc > 8 || 8 % (cg_pad / xc) != 0) continue;
+    if (knobs().xcd_cgs > 0) {                                             // (forced, for measurements)
+      if (xc == knobs().xcd_cgs) best = xc;
+      continue;
+    }
+    if (fetched(xc) < 0.95 * best_bytes) { best = xc; best_bytes = fetched(xc); }
+  }
+  return best != cg_pad / 8 || knobs().xcd_cgs > 0 ? best : 0;
+}
+// How long a uniform launch of 64-token tiles on workgroups of four wavefronts is, in workgroups that its busiest CU runs:
+// workgroups are dealt to the XCDs by the order of the units, and the 32 CUs of an XCD share its own.
+static long wide64_cu_rounds(long rows, int m, int k) {
+  const long cgs = (m / 128 + 3) / 4, cg_pad = (cgs + 7) / 8 * 8;
+  const long xc = wide_uniform_blocks(rows, m, k, kWideTokens, 64);
+  const long per_xcd = xc ? wide_block_grid_units(rows, m, xc) / 8 : wide_unit_order(m) == 1 ? rows * (cg_pad / 8) : (rows * cgs + 7) / 8;
+  return (per_xcd + 31) / 32;
+}
 // (`plan_tokens`, `plan_deltas`: the batch behind a plan's list of tiles, for the order of its units; 0 for uniform groups)
 int launch_wide(const Sparse24Args& a, hipStream_t st, int tok = kWideTokens, int plan_tokens = 0, int plan_deltas = 0) {
   if (a.n_groups <= 0 || a.m == 0 || a.k == 0) return TRITEIA_HIP_OK;
@@ -411,44 +451,14 @@ int launch_wide(const Sparse24Args& a, hipStream_t st, int tok = kWideTokens, in
   b.xcd_swizzle = wide_unit_order(a.m);
   unsigned grid = a.tiles && plan_tokens > 0 ? plan_wide_grid(b, (long)a.n_groups * chunks, a.m, tok, plan_tokens, plan_deltas, 64)
                                              : (unsigned)wide_grid_units((long)a.n_groups * chunks, a.m, b.xcd_swizzle);
-  // Uniform launches: an XCD takes a block of column groups x a block of token tiles (order 4) where that makes its
-  // L2 fetch fewer bytes than a run of column groups for every tile (order 1).  While the workgroups that an XCD holds at
-  // a time (32 CUs x 1 or 2) walk K, its L2 fetches the packed weights of their distinct column groups and the
-  // activations of their distinct tiles once each: with units numbered column group first, a window of W units over
-  // blocks of c column groups fetches c x (weights of a column group) + W / c x (activations of a tile), least near
-  // c = sqrt(W x tile / column group).  Measured (order 1 -> the rule): 4096 x 4096 with 640 / 1024 / 1536 / 2048 tokens
-  // 28.3 -> 27.1, 32.1 -> 30.6, 43.8 -> 41.6, 50.5 -> 46.8 us; 8192 x 8192 with 1000 tokens 81.2 -> 79.7 us; 11008 x 4096 with
-  // 1280 tokens 92.5 -> 88.6 us; 4096 x 11008 and 8192 x 28672 the same either way (blocks of 14 column groups on the
-  // latter, which a count over the whole launch instead of the window would pick, measured 1.7 % slower).
-  // The sums do not depend on which workgroup takes which unit.
   const bool eight_waves = !a.tiles && ((tok == 32 && units <= knob_or(knobs().wide32_ksplit_max_units, kWide32KSplitMaxUnits)) ||
                                         (tok != 32 && units <= knob_or(knobs().wide64_ksplit_max_units, kWide64KSplitMaxUnits)));
-  if (!a.tiles && b.xcd_swizzle == 1 && knobs().xcd_cgs >= 0) {
-    const long rows = (long)a.n_groups * chunks;
-    const double w_cg = 512.0 * a.k * 0.375, x_tile = (double)tok * a.k * 2.0;
-    const long window = 32 * (eight_waves ? 1 : 2);                       // workgroups an XCD holds at a time
-    auto fetched = [&](long xc) {
-      const long tbs = 8 / (cg_pad / xc);
-      long slots = xc * ((rows + tbs - 1) / tbs);
-      if (slots > window) slots = window;
-      return (double)xc * w_cg + (double)((slots + xc - 1) / xc) * x_tile;
-    };
-    long best = cg_pad / 8;
-    double best_bytes = fetched(best);
-    for (long xc = 1; xc <= cg_pad; xc++) {
-      if (cg_pad % xc != 0 || cg_pad / xc > 8 || 8 % (cg_pad / xc) != 0) continue;
-      if (knobs().xcd_cgs > 0) {                                           // (forced, for measurements)
-        if (xc == knobs().xcd_cgs) best = xc;
-        continue;
-      }
-      if (fetched(xc) < 0.95 * best_bytes) { best = xc; best_bytes = fetched(xc); }
-    }
-    if (best != cg_pad / 8 || knobs().xcd_cgs > 0) {
+  if (!a.tiles)
+    if (const long xc = wide_uniform_blocks((long)a.n_groups * chunks, a.m, a.k, tok, 32 * (eight_waves ? 1 : 2))) {
       b.xcd_swizzle = 4;
-      b.xcd_cgs = (int)best;
-      grid = (unsigned)wide_block_grid_units(rows, a.m, best);
+      b.xcd_cgs = (int)xc;
+      grid = (unsigned)wide_block_grid_units((long)a.n_groups * chunks, a.m, xc);
     }
-  }
   if (tok == 32 && units <= knob_or(knobs().wide32_ksplit_max_units, kWide32KSplitMaxUnits))
     hipLaunchKernelGGL((sparse24_wide_kernel<2, 32, false, 2>), dim3(grid), dim3(512), 0, st, b);
   else if (tok == 32)
@@ -604,12 +614,15 @@ UniformPlan decide_uniform(int tokens, int stride, int n_groups, int m, int k, l
       (done > 0 ? rest >= kPlanWideMinRest
                 : ks64 || (long)n_groups * (rest / kWideTokens) * cgs >= knob_or(knobs().wide_min_units, kWideMinUnits))) {
     int t = rest / kWideTokens * kWideTokens;
-    // A rest above half a tile becomes a tile of its own; a smaller one too while the launch stays within one
-    // round of workgroups (two per CU), where its workgroups cost nothing and a launch of the narrow kernel for them
-    // would stream the weights once more (288 tokens on 8192 x 28672: 130.6 -> 111.5 us; 2056 on 4096 x 4096 69.3 ->
-    // 67.4 us).  Past one round the extra tile starts a round of its own (4104 tokens on 4096 x 4096: 88 -> 111 us).
+    // A rest above half a tile becomes a tile of its own; a smaller one too where that adds no workgroup to the busiest
+    // CU: its workgroups then cost next to nothing, while a launch of the narrow kernel for them streams the weights once
+    // more (4096 x 11008 with 2000 / 3016 / 3600 / 4000 tokens 130.4 -> 119.9, 182.0 -> 173.4, 212.0 -> 201.6, 218.7 -> 208.0 us;
+    // 8192 x 8192 with 4000 284.5 -> 273.0; 8192 x 28672 with 288 130.6 -> 111.5).  Where it does add one, that workgroup is a
+    // (half) round of its own (4096 x 4096 with 4104 tokens 83 against 109 us, 8192 x 8192 with 2056 151 against 199,
+    // 4096 x 11008 with 2056 123 against 132).  Within one round of two workgroups per CU it is even either way.
     const bool one_round = (long)n_groups * (rest / kWideTokens + 1) * cgs <= 512;
-    if (rest - t >= (one_round ? 1 : kPlanWideMinRest)) t = rest;
+    const bool no_longer = wide64_cu_rounds((long)n_groups * (rest / kWideTokens + 1), m, k) <= wide64_cu_rounds((long)n_groups * (rest / kWideTokens), m, k);
+    if (rest - t >= (one_round || no_longer ? 1 : kPlanWideMinRest)) t = rest;
     add(kUniWide64, done, t);
     done += t;
   }
