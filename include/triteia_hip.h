@@ -292,7 +292,8 @@ TRITEIA_HIP_API int triteia_hip_sgmv_routed_bf16(void* y, long y_stride, const v
  * int64), any order.  accumulate = 1 adds to y; 0 stores, and tokens without an adapter get zeros.  The shrink leaves the
  * routing and the intermediate in `scratch` for the expand, which takes the same sizes and the same `accumulate`.
  * triteia_hip_lora_scratch_bytes is 0 for what this pair does not take: more than 4096 tokens or 1024 adapters,
- * k % 32 != 0, r % 8 != 0, r > 128 or r > k (and the expand needs m % 8 == 0).
+ * k % 32 != 0, r % 8 != 0, r > 128 or r > k (and the expand needs m % 8 == 0).  Every tensor and the rows of x and y are
+ * read in 16-byte pieces and must be aligned to that.
  * Replaces lora_bgmv / lora_sgmv (triteia/python/ops/matmul/lora.py:22-105), which transpose every adapter respectively
  * build a segment table on the host on each call. */
 TRITEIA_HIP_API size_t triteia_hip_lora_scratch_bytes(int n_tokens, int n_adapters, int k, int r);

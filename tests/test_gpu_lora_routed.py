@@ -6,7 +6,8 @@ import torch
 
 from oracle import triteia_oracle as orc
 from triteia_amd.python import ops
-from triteia_amd.python.capi import lora_scratch
+from triteia_amd.python.capi import lora_scratch, lora_shrink
+from triteia_amd.python.capi._native import native
 
 pytestmark = pytest.mark.gpu
 
@@ -59,3 +60,35 @@ def test_lora_shapes_it_leaves_to_the_other_kernels():
     assert lora_scratch(4097, A) is None                                  # more tokens than indices fit in LDS
     assert lora_scratch(8, A[:, :4088]) is None                           # k no multiple of 32
     assert lora_scratch(8, A[:, :, :12]) is None                          # r no multiple of 8
+
+
+def test_lora_tensors_inside_a_16_byte_word():
+    """Views that start inside 16 bytes are left to the kernels of the other interfaces, with the same values."""
+    g = torch.Generator(device="cuda").manual_seed(3)
+    A, B, x = (torch.randn(s, generator=g, device="cuda").to(torch.float16) * 0.1 for s in ((3, 64, 16), (3, 16, 72), (20, 64)))
+    idx = torch.arange(20, device="cuda").remainder(4).sub(1).sort().values.to(torch.int32)
+    want = ops.lora_forloop(A, B, x, idx)
+
+    def shifted(t):
+        buf = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+        buf[1:].copy_(t.reshape(-1))
+        return buf[1:].view(t.shape)
+    for args in ((shifted(A), B, x), (A, shifted(B), x), (A, B, shifted(x))):
+        assert native().lora(*args, idx, None, 1.0) is None
+    y = ops.lora_bgmv(A, B, shifted(x), idx)
+    assert float((y - want).float().norm() / want.float().norm()) <= 2e-3     # as above
+    with pytest.raises(RuntimeError, match="16-byte aligned"):
+        lora_shrink(shifted(x), A, idx, lora_scratch(20, A), False)
+
+
+@pytest.mark.parametrize("r", [8, 24, 40, 72])
+def test_lora_infinite_weight_beside_the_padding_of_the_rank(r):
+    """The rank is padded to 16, 32, 64 or 128: an infinity in the last rank row stays one in its column alone."""
+    A = torch.ones((1, 32, r), dtype=torch.float16, device="cuda")
+    B = torch.ones((1, r, 16), dtype=torch.float16, device="cuda")
+    B[0, r - 1, 3] = float("inf")
+    x = torch.ones((5, 32), dtype=torch.float16, device="cuda")
+    y = ops.lora_bgmv(A, B, x, torch.zeros(5, dtype=torch.int32, device="cuda"))
+    want = torch.full((5, 16), 32.0 * r, dtype=torch.float16, device="cuda")
+    want[:, 3] = float("inf")
+    assert torch.equal(y, want)

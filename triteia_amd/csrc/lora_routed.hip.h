@@ -268,13 +268,15 @@ __global__ __launch_bounds__(256) void lora_expand_kernel(const LoraArgs<T> a) {
     }
     return;
   }
-  // the adapter's patch: a request covers two rank rows; rows past r and columns past m repeat the last ones (their
-  // products are with a zero intermediate, their columns are not stored)
+  // the adapter's patch: a request covers two rank rows; columns past m repeat the last ones (they are not stored).  Rows
+  // past r (r is a multiple of 8: both rows of a request) are cleared: a weight there that is not finite would turn the
+  // product with the zero intermediate into a NaN.
   const T* b = a.b + (long)d.x * a.r * a.m;
 #pragma unroll
   for (int i = 0; i < 2 * R16; i++) {
     const int piece = (wave + 4 * i) * 64 + lane, row = piece >> 5, c = (piece & 31) ^ (row & 31);
-    load_to_lds(b + (long)min(row, a.r - 1) * a.m + min(c0 + 8 * c, a.m - 8), patch + (wave + 4 * i) * 1024);
+    if (2 * (wave + 4 * i) < a.r) load_to_lds(b + (long)row * a.m + min(c0 + 8 * c, a.m - 8), patch + (wave + 4 * i) * 1024);
+    else *reinterpret_cast<lvec8<T>*>(patch + piece * 16) = lvec8<T>{0, 0, 0, 0, 0, 0, 0, 0};
   }
   const int j = lane & 15, q = lane >> 4;
   const int col = c0 + 64 * wave + 16 * q;           // this lane's 16 output columns

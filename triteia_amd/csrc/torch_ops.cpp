@@ -11,6 +11,7 @@
 #include <ATen/ATen.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include "../../include/triteia_hip.h"
@@ -22,6 +23,14 @@ using at::Tensor;
 struct Args {
   PyObject* const* v;
   Py_ssize_t n;
+  double number = 0;        // a last argument that is neither a tensor nor None
+  bool numeric = false;
+  Args(PyObject* const* values, Py_ssize_t count) : v(values), n(count) {
+    if (n == 0 || THPVariable_Check(v[n - 1]) || v[n - 1] == Py_None) return;
+    number = PyFloat_AsDouble(v[n - 1]);
+    numeric = !PyErr_Occurred();
+    PyErr_Clear();
+  }
   bool tensor(int i) const { return i < n && THPVariable_Check(v[i]); }
   const Tensor& operator[](int i) const { return THPVariable_Unpack(v[i]); }
   bool none(int i) const { return i < n && v[i] == Py_None; }
@@ -138,12 +147,16 @@ Tensor sbmm(const Args& a) {
   return routed(xc, q, meta, s, idx, y, 0, base, at_) ? y : Tensor();
 }
 
+// (a view that starts inside 16 bytes; a copy made by contiguous() does not)
+bool aligned(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
+
 bool lora_ok(const Tensor& A, const Tensor& B, const Tensor& x, const Tensor& indices) {
   return x.is_cuda() && x.dim() == 2 && (x.scalar_type() == at::kHalf || x.scalar_type() == at::kBFloat16) &&
          dense_on(A, x, x.scalar_type(), 3) && dense_on(B, x, x.scalar_type(), 3) && indices.device() == x.device() && indices.dim() == 1 &&
          indices.is_contiguous() && (indices.scalar_type() == at::kInt || indices.scalar_type() == at::kLong) &&
          sizes_ok({x.size(0), x.size(1), A.size(0), A.size(2), B.size(2)}) && indices.size(0) == x.size(0) && A.size(1) == x.size(1) &&
-         B.size(0) == A.size(0) && B.size(1) == A.size(2) && B.size(2) % 8 == 0;
+         B.size(0) == A.size(0) && B.size(1) == A.size(2) && B.size(2) % 8 == 0 && aligned(A) &&
+         aligned(B) && (!x.is_contiguous() || aligned(x));
 }
 size_t lora_bytes(const Tensor& A, const Tensor& x) { return triteia_hip_lora_scratch_bytes(x.size(0), A.size(0), A.size(1), A.size(2)); }
 bool lora_shrink(const Tensor& x, const Tensor& A, const Tensor& indices, const Tensor& scratch, bool accumulate, int dev, void* stream) {
@@ -160,9 +173,7 @@ bool lora_expand(const Tensor& y, const Tensor& A, const Tensor& B, const Tensor
 Tensor lora(const Args& a) {
   if (a.n != 6 || !a.tensor(0) || !a.tensor(1) || !a.tensor(2) || !a.tensor(3)) return {};
   const Tensor &A = a[0], &B = a[1], &x = a[2], &indices = a[3];
-  const double scale = PyFloat_AsDouble(a.v[5]);
-  if (PyErr_Occurred()) { PyErr_Clear(); return {}; }
-  if (!lora_ok(A, B, x, indices) || !base_ok(a, 4, x, x.size(1), B.size(2))) return {};
+  if (!a.numeric || !lora_ok(A, B, x, indices) || !base_ok(a, 4, x, x.size(1), B.size(2))) return {};
   const size_t bytes = lora_bytes(A, x);
   if (bytes == 0) return {};
   const Place at_(x);
@@ -172,7 +183,7 @@ Tensor lora(const Args& a) {
   if (!lora_shrink(xc, A, indices, scratch, base, at_.dev, at_.handle())) return {};
   // (without a base weight every row is written by the expand: tokens without an adapter get zeros)
   Tensor y = base ? at::matmul(xc, a[4].t()) : at::empty({x.size(0), B.size(2)}, x.options());
-  return lora_expand(y, A, B, scratch, scale, base, at_.dev, at_.handle()) ? y : Tensor();
+  return lora_expand(y, A, B, scratch, a.number, base, at_.dev, at_.handle()) ? y : Tensor();
 }
 
 // ldmm(indices, x, LwA, LwB, DeltaW, metas, ss, base or None): ops.ldmm.  One stream: with the LoRA pair at 10 us, a side
@@ -184,7 +195,7 @@ Tensor ldmm(const Args& a) {
   for (int i = 0; i < 7; i++)
     if (!a.tensor(i)) return {};
   const Tensor &indices = a[0], &x = a[1], &A = a[2], &B = a[3], &q = a[4], &meta = a[5], &s = a[6];
-  if (x.scalar_type() != at::kHalf || indices.scalar_type() != at::kInt || !lora_ok(A, B, x, indices) || s.dim() != 3) return {};
+  if (x.scalar_type() != at::kHalf || !lora_ok(A, B, x, indices) || s.dim() != 3) return {};
   const int64_t k = x.size(1), m = B.size(2);
   const size_t bytes = lora_bytes(A, x);
   if (bytes == 0 || !packed_ok(q, meta, s, x, q.size(0), k, m) || !base_ok(a, 7, x, k, m)) return {};
@@ -196,7 +207,8 @@ Tensor ldmm(const Args& a) {
   // (without a base weight the expand stores the adapters' rows and zeros in all others, the deltas' among them)
   Tensor y = base ? at::matmul(xc, a[7].t()) : at::empty({x.size(0), m}, x.options());
   if (!lora_expand(y, A, B, scratch, 1.0, base, at_.dev, at_.handle())) return {};
-  return routed(xc, q, meta, s, indices, y, A.size(0), true, at_) ? y : Tensor();
+  const Tensor idx = indices.scalar_type() == at::kInt ? indices : indices.to(at::kInt);
+  return routed(xc, q, meta, s, idx, y, A.size(0), true, at_) ? y : Tensor();
 }
 
 PyObject* wrap(Tensor&& t) {
@@ -204,42 +216,54 @@ PyObject* wrap(Tensor&& t) {
   return THPVariable_Wrap(std::move(t));
 }
 
+// Other Python threads run while an op allocates, calls torch and launches (the caller holds references to its arguments).
+struct WithoutGil {
+  PyThreadState* state = PyEval_SaveThread();
+  ~WithoutGil() { PyEval_RestoreThread(state); }
+};
+
+// torch's own translation of exceptions: an allocation that fails raises torch.OutOfMemoryError, as from Python
 template <Tensor (*F)(const Args&)>
 PyObject* call(PyObject*, PyObject* const* v, Py_ssize_t n) {
-  try {
-    return wrap(F(Args{v, n}));
-  } catch (const std::exception& e) {
-    PyErr_SetString(PyExc_RuntimeError, e.what());
-    return nullptr;
+  HANDLE_TH_ERRORS
+  const Args a(v, n);
+  Tensor y;
+  {
+    const WithoutGil released;
+    y = F(a);
   }
+  return wrap(std::move(y));
+  END_HANDLE_TH_ERRORS
 }
 
 // pack(weight, scales): (qweight, meta, meta_raw) of ops.utils.sparsity.prune_pack_2_4, or None
+bool packed(const Args& a, Tensor (&out)[3]) {
+  if (a.n != 2 || !a.tensor(0) || !a.tensor(1)) return false;
+  const Tensor &w = a[0], &s = a[1];
+  if (!w.is_cuda() || !dense_on(w, w, at::kHalf, 2) || !dense_on(s, w, at::kHalf, 2)) return false;
+  const int64_t k = w.size(0), m = w.size(1);
+  if (!sizes_ok({k, m}) || k % 32 != 0 || m % 64 != 0 || s.numel() != m ||
+      (reinterpret_cast<uintptr_t>(w.data_ptr()) | reinterpret_cast<uintptr_t>(s.data_ptr())) % 4 != 0)
+    return false;
+  const Place at_(w);
+  out[0] = at::empty({k / 32, 2 * m}, w.options().dtype(at::kInt));
+  out[1] = at::empty({m, k / 16}, w.options().dtype(at::kShort));
+  out[2] = at::empty({m, k / 16}, w.options().dtype(at::kShort));
+  return triteia_hip_pack_2_4(w.data_ptr(), s.data_ptr(), out[0].data_ptr(), out[1].data_ptr(), out[2].data_ptr(), k, m, at_.dev,
+                              at_.handle()) == 0;
+}
 PyObject* pack(PyObject*, PyObject* const* v, Py_ssize_t n) {
-  try {
-    const Args a{v, n};
-    if (n != 2 || !a.tensor(0) || !a.tensor(1)) Py_RETURN_NONE;
-    const Tensor &w = a[0], &s = a[1];
-    if (!w.is_cuda() || !dense_on(w, w, at::kHalf, 2) || !dense_on(s, w, at::kHalf, 2)) Py_RETURN_NONE;
-    const int64_t k = w.size(0), m = w.size(1);
-    if (!sizes_ok({k, m}) || k % 32 != 0 || m % 64 != 0 || s.numel() != m ||
-        (reinterpret_cast<uintptr_t>(w.data_ptr()) | reinterpret_cast<uintptr_t>(s.data_ptr())) % 4 != 0)
-      Py_RETURN_NONE;
-    const Place at_(w);
-    Tensor q = at::empty({k / 32, 2 * m}, w.options().dtype(at::kInt));
-    Tensor meta = at::empty({m, k / 16}, w.options().dtype(at::kShort)), raw = at::empty({m, k / 16}, w.options().dtype(at::kShort));
-    if (triteia_hip_pack_2_4(w.data_ptr(), s.data_ptr(), q.data_ptr(), meta.data_ptr(), raw.data_ptr(), k, m, at_.dev, at_.handle()))
-      Py_RETURN_NONE;
-    PyObject* out = PyTuple_New(3);
-    if (!out) return nullptr;
-    PyTuple_SET_ITEM(out, 0, THPVariable_Wrap(std::move(q)));
-    PyTuple_SET_ITEM(out, 1, THPVariable_Wrap(std::move(meta)));
-    PyTuple_SET_ITEM(out, 2, THPVariable_Wrap(std::move(raw)));
-    return out;
-  } catch (const std::exception& e) {
-    PyErr_SetString(PyExc_RuntimeError, e.what());
-    return nullptr;
+  HANDLE_TH_ERRORS
+  const Args a(v, n);
+  Tensor out[3];
+  bool done;
+  {
+    const WithoutGil released;
+    done = packed(a, out);
   }
+  if (!done) Py_RETURN_NONE;
+  return Py_BuildValue("(NNN)", THPVariable_Wrap(std::move(out[0])), THPVariable_Wrap(std::move(out[1])), THPVariable_Wrap(std::move(out[2])));
+  END_HANDLE_TH_ERRORS
 }
 
 #define METHOD(NAME_, FN_) {NAME_, reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(FN_)), METH_FASTCALL, nullptr}

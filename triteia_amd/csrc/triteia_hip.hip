@@ -1550,6 +1550,8 @@ int triteia_hip_lora_shrink(const void* x, long x_stride, const void* a, const v
   if (scratch_bytes < triteia_hip_lora_scratch_bytes(n_tokens, n_adapters, k, r) || reinterpret_cast<uintptr_t>(scratch) % 16 != 0)
     return fail(TRITEIA_HIP_ERR_ARGUMENT, "lora_shrink: the scratch must be 16-byte aligned and hold %zu bytes (got %zu)",
                 triteia_hip_lora_scratch_bytes(n_tokens, n_adapters, k, r), scratch_bytes);
+  if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(a)) % 16 != 0 || x_stride % 8 != 0)
+    return fail(TRITEIA_HIP_ERR_ARGUMENT, "lora_shrink: x, its rows and the adapters must be 16-byte aligned");
   DeviceGuard g(dev);
   if (!g.ok) return fail(TRITEIA_HIP_ERR_RUNTIME, "cannot select device %d", dev);
   hipStream_t st = static_cast<hipStream_t>(stream);
@@ -1563,6 +1565,8 @@ int triteia_hip_lora_expand(void* y, long y_stride, const void* b, const void* s
   if (!lora_routed_takes(n_tokens, n_adapters, k, r) || m < 0 || m % 8 != 0)
     return fail(TRITEIA_HIP_ERR_KERN_SHAPE, "lora_expand: tokens=%d adapters=%d k=%d r=%d m=%d", n_tokens, n_adapters, k, r, m);
   if (!y || !b || !scratch) return fail(TRITEIA_HIP_ERR_ARGUMENT, "lora_expand: null tensor pointer");
+  if ((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(scratch)) % 16 != 0 || y_stride % 8 != 0)
+    return fail(TRITEIA_HIP_ERR_ARGUMENT, "lora_expand: y, its rows, the adapters and the scratch must be 16-byte aligned");
   DeviceGuard g(dev);
   if (!g.ok) return fail(TRITEIA_HIP_ERR_RUNTIME, "cannot select device %d", dev);
   hipStream_t st = static_cast<hipStream_t>(stream);
