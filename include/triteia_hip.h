@@ -137,7 +137,7 @@ TRITEIA_HIP_API int triteia_hip_sbmm_2_4_bounded(const void* A, const void* B, c
  * kernel above plus the trailing `y += output`, sbmm.py:141):
  *   d = token_indices[t] - index_offset
  *   0 <= d < n_deltas :  C[t] = (accumulate ? C[t] : 0) + A[t] @ dequant(B[d])
- *   otherwise         :  C[t] untouched
+ *   otherwise         :  C[t] untouched; with accumulate = 2 (C[t] = A[t] @ dequant(B[d]) as with 0) zeros
  * token_indices: int32 [prob_n] on the device, any order.  The tokens are
  * grouped on the device, so each delta's weights are read once per launch.
  * workspace: >= triteia_hip_sbmm_routed_workspace_bytes(prob_n, n_deltas) bytes

@@ -33,7 +33,11 @@ __global__ __launch_bounds__(64 * KW, 2) void sparse24_share16_kernel(const Spar
   const int grp = unit / sh_pad;
   const int i = unit - grp * sh_pad;
   const int sh = p.xcd_swizzle ? (i & 7) * (sh_pad >> 3) + (i >> 3) : i;
-  if (sh >= shares || grp >= p.n_groups) return;
+  if (sh >= shares) return;
+  if (grp >= p.n_groups) {
+    if (ROUTED && p.clear_group) clear_unrouted(p, sh * kShareCols, kShareCols, threadIdx.x, 64 * KW);
+    return;
+  }
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
   const int rho = lane & 15;     // A: column rho of the share; B and D: token rho

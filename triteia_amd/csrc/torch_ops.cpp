@@ -113,9 +113,10 @@ Tensor bmm(const Args& a) {
              : y;
 }
 
-// y (+)= the routed product of x [tokens, k]; false: refused, nothing launched
+// The routed product of x [tokens, k], added to y (accumulate = 1) or stored with zeros in the rows without a delta
+// (2: y need not be initialised); false: refused, nothing launched
 bool routed(const Tensor& x, const Tensor& q, const Tensor& meta, const Tensor& s, const Tensor& indices, Tensor& y, int offset,
-            bool accumulate, const Place& at_) {
+            int accumulate, const Place& at_) {
   const int64_t tokens = x.size(0), k = x.size(1), m = y.size(1), n = q.size(0);
   Tensor ws;
   size_t bytes = 0;
@@ -143,8 +144,8 @@ Tensor sbmm(const Args& a) {
   const Tensor xc = x.is_contiguous() ? x : x.contiguous();
   const Tensor idx = indices.scalar_type() == at::kInt ? indices : indices.to(at::kInt);
   const bool base = !a.none(5);
-  Tensor y = base ? at::matmul(xc, a[5].t()) : at::zeros({tokens, m}, x.options());
-  return routed(xc, q, meta, s, idx, y, 0, base, at_) ? y : Tensor();
+  Tensor y = base ? at::matmul(xc, a[5].t()) : at::empty({tokens, m}, x.options());
+  return routed(xc, q, meta, s, idx, y, 0, base ? 1 : 2, at_) ? y : Tensor();
 }
 
 // (a view that starts inside 16 bytes; a copy made by contiguous() does not)
@@ -208,7 +209,7 @@ Tensor ldmm(const Args& a) {
   Tensor y = base ? at::matmul(xc, a[7].t()) : at::empty({x.size(0), m}, x.options());
   if (!lora_expand(y, A, B, scratch, 1.0, base, at_.dev, at_.handle())) return {};
   const Tensor idx = indices.scalar_type() == at::kInt ? indices : indices.to(at::kInt);
-  return routed(xc, q, meta, s, idx, y, A.size(0), true, at_) ? y : Tensor();
+  return routed(xc, q, meta, s, idx, y, A.size(0), 1, at_) ? y : Tensor();
 }
 
 PyObject* wrap(Tensor&& t) {

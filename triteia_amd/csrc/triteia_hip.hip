@@ -234,7 +234,7 @@ int launch_sparse24(Sparse24Args a, int nt, long tsplit, hipStream_t st, int zsp
   // most min(tokens, deltas) of them): on four wavefronts, like every routed launch.
   if (const int tiles = a.raw_indices && !a.raw_static && nt == 1 && tsplit == 1 && zsplit == 1 ? share16_tiles(a.n_groups, a.m, a.raw_count) : 0) {
     const long sh_pad = ((long)(a.m / (16 * tiles)) + 7) / 8 * 8;
-    const dim3 grid((unsigned)(a.n_groups * sh_pad));
+    const dim3 grid((unsigned)((a.n_groups + a.clear_group) * sh_pad));
     if (tiles == 1) hipLaunchKernelGGL((sparse24_share16_kernel<4, 8, 1, true>), grid, dim3(256), 0, st, a);
     else if (tiles == 2) hipLaunchKernelGGL((sparse24_share16_kernel<4, 4, 2, true>), grid, dim3(256), 0, st, a);
     else hipLaunchKernelGGL((sparse24_share16_kernel<4, 4, 4, true>), grid, dim3(256), 0, st, a);
@@ -254,7 +254,7 @@ int launch_sparse24(Sparse24Args a, int nt, long tsplit, hipStream_t st, int zsp
   // tokens 63.0 -> 64.8 us).
   if (a.xcd_swizzle == 1 && a.n_groups >= 8 && units * tsplit * zsplit <= 512 && (uniform || (a.raw_indices && a.raw_static))) a.xcd_swizzle = 5;
   else if (a.xcd_swizzle == 5) a.xcd_swizzle = 1;
-  const dim3 grid((unsigned)units, (unsigned)tsplit, (unsigned)zsplit);
+  const dim3 grid((unsigned)(units + a.clear_group * cb_pad), (unsigned)tsplit, (unsigned)zsplit);
 #define TRY(NT_, KW_, D_) if (nt == NT_ && kw == KW_ && depth == D_) { launch_one<NT_, KW_, D_>(a, grid, st); return check_launch("sparse24_grouped_kernel"); }
 #define TRY_EAGER(NT_, KW_, D_) if (nt == NT_ && kw == KW_ && depth == D_) { launch_one<NT_, KW_, D_, true>(a, grid, st); return check_launch("sparse24_grouped_kernel"); }
   if (a.raw_indices && a.raw_static) {
@@ -1002,8 +1002,9 @@ int triteia_hip_routed_in_kernel(int prob_n, int n_deltas, int prob_m, int prob_
   return shares ? 2 : 1;
 }
 
-int triteia_hip_route_plan(const void* token_indices, int index_offset, int n_deltas, int prob_n, void* workspace,
-                           size_t workspace_bytes, int dev, void* stream) {
+// `clear` (rows of m fp16): rows without a delta get zeros in the same launch; nullptr: none
+static int route_plan_impl(const void* token_indices, int index_offset, int n_deltas, int prob_n, void* workspace, size_t workspace_bytes,
+                           int dev, void* stream, void* clear, int m) {
   if (prob_n < 0 || n_deltas < 0) return fail(TRITEIA_HIP_ERR_PROB_SHAPE, "route_plan: tokens=%d deltas=%d", prob_n, n_deltas);
   if (n_deltas > kPlanMaxDeltas)
     return fail(TRITEIA_HIP_ERR_KERN_SHAPE, "route_plan: at most %d deltas per call (got %d)", kPlanMaxDeltas, n_deltas);
@@ -1015,11 +1016,16 @@ int triteia_hip_route_plan(const void* token_indices, int index_offset, int n_de
   if (prob_n > 0 && !token_indices) return fail(TRITEIA_HIP_ERR_ARGUMENT, "route_plan: null indices");
   DeviceGuard g(dev);
   if (!g.ok) return fail(TRITEIA_HIP_ERR_RUNTIME, "cannot select device %d", dev);
-  hipLaunchKernelGGL(route_plan_kernel, dim3(1), dim3(kPlanThreads), 0, static_cast<hipStream_t>(stream),
+  const int clear_blocks = clear ? (prob_n < 255 ? prob_n : 255) : 0;
+  hipLaunchKernelGGL(route_plan_kernel, dim3(1 + clear_blocks), dim3(kPlanThreads), 0, static_cast<hipStream_t>(stream),
                      static_cast<const int*>(token_indices), prob_n, n_deltas, index_offset,
                      triteia_hip_plan_tile_tokens(prob_n, n_deltas), plan_has_wide(prob_n, n_deltas), plan_has_big(prob_n, n_deltas),
-                     static_cast<int*>(workspace));
+                     static_cast<int*>(workspace), static_cast<uint16_t*>(clear), (long)m, m / 8);
   return check_launch("route_plan_kernel");
+}
+int triteia_hip_route_plan(const void* token_indices, int index_offset, int n_deltas, int prob_n, void* workspace,
+                           size_t workspace_bytes, int dev, void* stream) {
+  return route_plan_impl(token_indices, index_offset, n_deltas, prob_n, workspace, workspace_bytes, dev, stream, nullptr, 0);
 }
 
 int triteia_hip_sbmm_2_4_planned(const void* A, const void* B, const void* meta, void* C, const void* s,
@@ -1138,8 +1144,10 @@ int triteia_hip_sbmm_2_4_routed(const void* A, const void* B, const void* meta, 
                                 int prob_k, void* workspace, size_t workspace_bytes, int accumulate, int dev,
                                 void* stream) {
   if (int e = check_gemm_shape(prob_m, prob_n, prob_k, -1)) return e;
-  if (accumulate != 0 && accumulate != 1) return fail(TRITEIA_HIP_ERR_ARGUMENT, "sbmm_2_4_routed: accumulate=%d", accumulate);
+  if (accumulate < 0 || accumulate > 2) return fail(TRITEIA_HIP_ERR_ARGUMENT, "sbmm_2_4_routed: accumulate=%d", accumulate);
   if (n_deltas < 0) return fail(TRITEIA_HIP_ERR_PROB_SHAPE, "sbmm_2_4_routed: deltas=%d", n_deltas);
+  if (accumulate == 2 && prob_m != 0 && prob_n != 0 && (prob_k == 0 || n_deltas == 0))
+    return fail(TRITEIA_HIP_ERR_PROB_SHAPE, "sbmm_2_4_routed: accumulate=2 with k=%d and %d deltas", prob_k, n_deltas);
   if (prob_m == 0 || prob_n == 0 || prob_k == 0 || n_deltas == 0) return TRITEIA_HIP_OK;
   if (!A || !B || !meta || !C || !s) return fail(TRITEIA_HIP_ERR_ARGUMENT, "sbmm_2_4_routed: null tensor pointer");
   // (above 64 tokens only for at most 16 deltas, whose weights can be requested ahead of the routing: with 32 deltas of
@@ -1162,7 +1170,8 @@ int triteia_hip_sbmm_2_4_routed(const void* A, const void* B, const void* meta, 
     a.raw_count = prob_n;
     a.raw_offset = index_offset;
     a.n_groups = prob_n < n_deltas ? prob_n : n_deltas;
-    a.accumulate = accumulate;
+    a.accumulate = accumulate == 1;
+    a.clear_group = accumulate == 2;
     const int nt = pick_nt(prob_n, a.n_groups);
     // With at least two tokens per delta on average (four for batches above 64 tokens) nearly every
     // delta is in use: one group per delta, whose weights are requested before the indices have
@@ -1182,9 +1191,10 @@ int triteia_hip_sbmm_2_4_routed(const void* A, const void* B, const void* meta, 
     const long tsplit = prob_n <= (eager_ok ? 64 : 32) ? 1 : (prob_n <= 128 ? 2 : 4);
     return launch_sparse24(a, nt, tsplit, static_cast<hipStream_t>(stream));
   }
-  if (int e = triteia_hip_route_plan(token_indices, index_offset, n_deltas, prob_n, workspace, workspace_bytes, dev, stream))
+  if (int e = route_plan_impl(token_indices, index_offset, n_deltas, prob_n, workspace, workspace_bytes, dev, stream,
+                              accumulate == 2 ? C : nullptr, prob_m))
     return e;
-  return triteia_hip_sbmm_2_4_planned(A, B, meta, C, s, workspace, n_deltas, prob_m, prob_n, prob_k, accumulate, dev, stream);
+  return triteia_hip_sbmm_2_4_planned(A, B, meta, C, s, workspace, n_deltas, prob_m, prob_n, prob_k, accumulate == 1, dev, stream);
 }
 
 size_t triteia_hip_sbmm_routed_static_max_bytes(void) { return kStaticPlanBytes; }
