@@ -20,20 +20,29 @@ namespace {
 
 using at::Tensor;
 
+// A call's arguments, taken apart while the interpreter lock is held: what follows runs without it and sees no Python object.
+// Tensors are exactly torch.Tensor or Parameter; a subclass may give every operation another meaning, which the Python
+// path honours.
 struct Args {
-  PyObject* const* v;
-  Py_ssize_t n;
+  static constexpr int kMax = 8;
+  int n;
+  const Tensor* tensors[kMax] = {};
+  bool nones[kMax] = {};
   double number = 0;        // a last argument that is neither a tensor nor None
   bool numeric = false;
-  Args(PyObject* const* values, Py_ssize_t count) : v(values), n(count) {
-    if (n == 0 || THPVariable_Check(v[n - 1]) || v[n - 1] == Py_None) return;
-    number = PyFloat_AsDouble(v[n - 1]);
+  Args(PyObject* const* values, Py_ssize_t count) : n(count <= kMax ? (int)count : 0) {
+    for (int i = 0; i < n; i++) {
+      if (THPVariable_CheckExact(values[i])) tensors[i] = &THPVariable_Unpack(values[i]);
+      nones[i] = values[i] == Py_None;
+    }
+    if (n == 0 || nones[n - 1] || THPVariable_Check(values[n - 1])) return;
+    number = PyFloat_AsDouble(values[n - 1]);
     numeric = !PyErr_Occurred();
     PyErr_Clear();
   }
-  bool tensor(int i) const { return i < n && THPVariable_Check(v[i]); }
-  const Tensor& operator[](int i) const { return THPVariable_Unpack(v[i]); }
-  bool none(int i) const { return i < n && v[i] == Py_None; }
+  bool tensor(int i) const { return i < n && tensors[i] != nullptr; }
+  const Tensor& operator[](int i) const { return *tensors[i]; }
+  bool none(int i) const { return i < n && nones[i]; }
 };
 
 bool on(const Tensor& t, const Tensor& ref, at::ScalarType type, int64_t dim) {
