@@ -73,19 +73,22 @@ def ldmm(indices, x, LwA, LwB, DeltaW, metas, ss, base_weight=None, debug=False)
         # (the GEMM is enqueued ahead of the side stream's work: recorded into a HIP graph in the other order, the
         # step measured 30 us longer on 256 tokens x 4096 x 11008; launched eagerly the order makes no difference)
         y = torch.matmul(x_, base_weight.t())
-        with torch.cuda.stream(side):
-            plan = route_plan(idx32, M, workspace=ws)      # skips -1 and every index >= M (the delta tokens)
-            sgmv_routed(v, x_, A16, plan, accumulate=False)
-        if DeltaW.shape[0] > 0:
-            # LoRA tokens and delta tokens are different rows of y (disjoint index ranges): the expand stays
-            # on the side stream, beside the delta kernel, and joins at the end
-            side.wait_stream(cur)
+        try:
             with torch.cuda.stream(side):
-                sgmv_routed(y, v, B16, plan)
-            sbmm_2_4_routed(x_, DeltaW, metas, y, ss, idx32, index_offset=M, accumulate=True)
+                plan = route_plan(idx32, M, workspace=ws)      # skips -1 and every index >= M (the delta tokens)
+                sgmv_routed(v, x_, A16, plan, accumulate=False)
+            if DeltaW.shape[0] > 0:
+                # LoRA tokens and delta tokens are different rows of y (disjoint index ranges): the expand stays
+                # on the side stream, beside the delta kernel, and joins at the end
+                side.wait_stream(cur)
+                with torch.cuda.stream(side):
+                    sgmv_routed(y, v, B16, plan)
+                sbmm_2_4_routed(x_, DeltaW, metas, y, ss, idx32, index_offset=M, accumulate=True)
+        finally:
+            # (also where a step refuses its arguments: the buffers go back to the current stream's pool)
             cur.wait_stream(side)
+        if DeltaW.shape[0] > 0:
             return y.to(x.dtype)
-        cur.wait_stream(side)
         sgmv_routed(y, v, B16, plan)
     else:
         if base_weight is not None:
