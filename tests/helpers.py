@@ -55,3 +55,17 @@ def setknob(monkeypatch, name, value):
 def delknob(monkeypatch, name):
     monkeypatch.delenv(name, raising=False)
     reload_knobs()
+
+
+def without_native(monkeypatch):
+    """Every op takes its Python path: the native binding declines each call."""
+    import importlib
+
+    class Declines:
+        def __getattr__(self, name):
+            return lambda *args: None
+
+    for name in ("bmm", "ldmm", "lora", "sbmm", "sparse_low_precision"):
+        module = importlib.import_module("triteia_amd.python.ops.matmul." + name)
+        monkeypatch.setattr(module, "native", Declines)
+    monkeypatch.setattr(importlib.import_module("triteia_amd.python.nn.linear"), "native", Declines)

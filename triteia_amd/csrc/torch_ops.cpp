@@ -9,6 +9,7 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/autocast_mode.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <torch/csrc/Exceptions.h>
@@ -78,8 +79,17 @@ bool packed_ok(const Tensor& q, const Tensor& meta, const Tensor& s, const Tenso
          meta.size(2) == k / 16 && s.size(0) == n && s.size(1) == 1 && s.size(2) == m;
 }
 
+// (under autocast the base product has autocast's type, whatever its inputs': another one than x's is refused by the Python path)
 bool base_ok(const Args& a, int i, const Tensor& x, int64_t k, int64_t m) {
-  return a.none(i) || (a.tensor(i) && on(a[i], x, x.scalar_type(), 2) && a[i].size(0) == m && a[i].size(1) == k);
+  return a.none(i) || (a.tensor(i) && on(a[i], x, x.scalar_type(), 2) && a[i].size(0) == m && a[i].size(1) == k &&
+                       !(at::autocast::is_autocast_enabled(at::kCUDA) && at::autocast::get_autocast_dtype(at::kCUDA) != x.scalar_type()));
+}
+// x [tokens, k] times the layer's dense weight, which base_ok has let pass: what the kernels add to
+Tensor base_product(const Tensor& x, const Tensor& weight) {
+  Tensor y = at::matmul(x, weight.t());
+  TORCH_CHECK(y.scalar_type() == x.scalar_type() && y.is_contiguous(), "the base product is ", y.scalar_type(), ", expected a contiguous ",
+              x.scalar_type());
+  return y;
 }
 
 // matmul(qweight, x, meta, s): ops.matmul_4bit_2_4
@@ -153,7 +163,7 @@ Tensor sbmm(const Args& a) {
   const Tensor xc = x.is_contiguous() ? x : x.contiguous();
   const Tensor idx = indices.scalar_type() == at::kInt ? indices : indices.to(at::kInt);
   const bool base = !a.none(5);
-  Tensor y = base ? at::matmul(xc, a[5].t()) : at::empty({tokens, m}, x.options());
+  Tensor y = base ? base_product(xc, a[5]) : at::empty({tokens, m}, x.options());
   return routed(xc, q, meta, s, idx, y, 0, base ? 1 : 2, at_) ? y : Tensor();
 }
 
@@ -192,7 +202,7 @@ Tensor lora(const Args& a) {
   const bool base = !a.none(4);
   if (!lora_shrink(xc, A, indices, scratch, base, at_.dev, at_.handle())) return {};
   // (without a base weight every row is written by the expand: tokens without an adapter get zeros)
-  Tensor y = base ? at::matmul(xc, a[4].t()) : at::empty({x.size(0), B.size(2)}, x.options());
+  Tensor y = base ? base_product(xc, a[4]) : at::empty({x.size(0), B.size(2)}, x.options());
   return lora_expand(y, A, B, scratch, a.number, base, at_.dev, at_.handle()) ? y : Tensor();
 }
 
@@ -215,7 +225,7 @@ Tensor ldmm(const Args& a) {
   const bool base = !a.none(7);
   if (!lora_shrink(xc, A, indices, scratch, base, at_.dev, at_.handle())) return {};
   // (without a base weight the expand stores the adapters' rows and zeros in all others, the deltas' among them)
-  Tensor y = base ? at::matmul(xc, a[7].t()) : at::empty({x.size(0), m}, x.options());
+  Tensor y = base ? base_product(xc, a[7]) : at::empty({x.size(0), m}, x.options());
   if (!lora_expand(y, A, B, scratch, 1.0, base, at_.dev, at_.handle())) return {};
   const Tensor idx = indices.scalar_type() == at::kInt ? indices : indices.to(at::kInt);
   return routed(xc, q, meta, s, idx, y, A.size(0), 1, at_) ? y : Tensor();
