@@ -163,3 +163,14 @@ def test_bench_refuses_more_than_one_gpu():
     res = subprocess.run([sys.executable, os.path.join(ROOT, "bench.py"), "--gpus", "2"], capture_output=True, text=True)
     assert res.returncode == 2
     assert "ONE GPU" in res.stderr
+
+
+def test_sizes_past_a_grid_are_refused_before_the_launch():
+    lib = _ffi.lib()
+    null = ctypes.c_void_p(0)
+    expand = lambda m: lib.triteia_hip_lora_expand(null, m, null, null, 1, 1, 32, 8, m, 1.0, 0, 0, 0, null)
+    assert expand(65535 * 256) == _ffi.ERR_ARGUMENT             # (null pointers come after the sizes)
+    assert expand(65535 * 256 + 8) == _ffi.ERR_KERN_SHAPE
+    pack = lambda k, m: lib.triteia_hip_pack_2_4(null, null, null, null, null, k, m, 0, null)
+    assert pack(32, 2 ** 30 - 128) == _ffi.ERR_ARGUMENT
+    assert pack(32, 2 ** 30) == _ffi.ERR_PROB_SHAPE

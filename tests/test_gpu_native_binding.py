@@ -61,3 +61,36 @@ def test_module_with_a_base_under_autocast(layer):
     with torch.autocast("cuda", dtype=torch.bfloat16):
         with pytest.raises(RuntimeError, match="float16"):
             mod(layer["x"], layer["idx"])
+
+
+def test_failed_launch_raises(layer):
+    """An error that the HIP runtime reports for a launch (here one that the host has left behind: no such device) is
+    raised by the op; the call after it works."""
+    import ctypes
+
+    from triteia_amd.python.capi import _ffi
+    hip = ctypes.CDLL(_ffi.LIB_PATH)      # (symbols of the runtime that it is linked to)
+    t = layer
+    w = (torch.randn(64, 128, device="cuda") * 0.1).half()
+    scale = torch.full((1, 128), 0.02, dtype=torch.float16, device="cuda")
+    ops_ = dict(calls(t, None), matmul=lambda: ops.matmul_4bit_2_4(t["q"][0], t["x"], t["meta"][0], t["s"][0]),
+                bmm=lambda: ops.bmm_4bit_2_4(t["q"], t["x"][:N].unsqueeze(1), t["meta"], t["s"]),
+                pack=lambda: native().pack(w, scale)[0])
+    for name, op in ops_.items():
+        want = op()
+        torch.cuda.synchronize()
+        assert hip.hipSetDevice(1000) != 0
+        with pytest.raises(RuntimeError, match="triteia_hip error 4"):
+            op()
+        assert torch.equal(op(), want), name
+
+
+def test_more_deltas_than_a_plan_takes_are_refused_ahead_of_every_launch(layer):
+    n = 8193
+    q, meta, s = (torch.zeros(shape, dtype=dt, device="cuda") for shape, dt in
+                  (((n, K // 32, 2 * M_OUT), torch.int32), ((n, M_OUT, K // 16), torch.int16), ((n, 1, M_OUT), torch.float16)))
+    for base in (None, layer["base"]):
+        assert native().sbmm(q, layer["x"], meta, s, layer["idx"], base) is None
+        assert native().ldmm(layer["idx"], layer["x"], layer["A"], layer["B"], q, meta, s, base) is None
+        with pytest.raises(RuntimeError, match="8192"):
+            ops.sbmm_4bit_2_4_native(q, layer["x"], meta, s, layer["idx"], base_weight=base)

@@ -3,8 +3,9 @@
 // a call, more than most decode-size kernels take on the GPU; here 4 - 6 us.)
 //
 // Every function returns None for whatever is not the ordinary case -- another device, type, layout or shape, a pair
-// of sizes that the library refuses -- before it has launched anything; the Python op then takes its own path, which
-// checks the arguments one by one and raises the reference's error texts.  Nothing is kept between calls.
+// of sizes that the library refuses -- before any kernel of the library has been launched; the Python op then takes its
+// own path, which checks the arguments one by one and raises the reference's error texts.  A launch that fails raises.
+// Nothing is kept between calls.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -65,6 +66,14 @@ Tensor scratch_bytes(size_t bytes, const Tensor& like) {
   return at::empty({(int64_t)((bytes + 255) / 256 * 256)}, like.options().dtype(at::kByte));
 }
 
+// A library call that comes first: true if it was launched, false if it was refused.
+bool launched(int code) {
+  TORCH_CHECK(code != TRITEIA_HIP_ERR_RUNTIME, "triteia_hip error ", code, ": ", triteia_hip_last_error());
+  return code == TRITEIA_HIP_OK;
+}
+// A call behind others, whose arguments have been checked ahead of the first: there is no way back.
+void must_launch(int code) { TORCH_CHECK(code == TRITEIA_HIP_OK, "triteia_hip error ", code, ": ", triteia_hip_last_error()); }
+
 // sizes that fit the library's ints, on a GPU
 bool sizes_ok(std::initializer_list<int64_t> sizes) {
   for (int64_t s : sizes)
@@ -78,6 +87,8 @@ bool packed_ok(const Tensor& q, const Tensor& meta, const Tensor& s, const Tenso
          sizes_ok({n, k, m}) && q.size(0) == n && q.size(1) == k / 32 && q.size(2) == 2 * m && meta.size(0) == n && meta.size(1) == m &&
          meta.size(2) == k / 16 && s.size(0) == n && s.size(1) == 1 && s.size(2) == m;
 }
+// (what the routed product takes in one call, see triteia_hip_sbmm_2_4_routed)
+constexpr int64_t kMaxRoutedDeltas = 8192;
 
 // (under autocast the base product has autocast's type, whatever its inputs': another one than x's is refused by the Python path)
 bool base_ok(const Args& a, int i, const Tensor& x, int64_t k, int64_t m) {
@@ -108,10 +119,10 @@ Tensor matmul(const Args& a) {
   Tensor y = at::empty(shape, x.options());
   const size_t split = triteia_hip_bmm_scratch_bytes(m, 1, rows, k);
   const Tensor scratch = split ? scratch_bytes(split, x) : Tensor();
-  return triteia_hip_bmm_2_4_tokens_scratch(xc.data_ptr(), q.data_ptr(), meta.data_ptr(), y.data_ptr(), s.data_ptr(), m, 1, rows, k,
-                                            split ? scratch.data_ptr() : nullptr, split, at_.dev, at_.handle())
-             ? Tensor()
-             : y;
+  return launched(triteia_hip_bmm_2_4_tokens_scratch(xc.data_ptr(), q.data_ptr(), meta.data_ptr(), y.data_ptr(), s.data_ptr(), m, 1, rows, k,
+                                                     split ? scratch.data_ptr() : nullptr, split, at_.dev, at_.handle()))
+             ? y
+             : Tensor();
 }
 
 // bmm(qweights, xs, metas, ss): ops.bmm_4bit_2_4
@@ -126,15 +137,15 @@ Tensor bmm(const Args& a) {
   Tensor y = at::empty({n, tokens, m}, x.options());
   const size_t split = triteia_hip_bmm_scratch_bytes(m, n, tokens, k);
   const Tensor scratch = split ? scratch_bytes(split, x) : Tensor();
-  return triteia_hip_bmm_2_4_tokens_scratch(xc.data_ptr(), q.data_ptr(), meta.data_ptr(), y.data_ptr(), s.data_ptr(), m, n, tokens, k,
-                                            split ? scratch.data_ptr() : nullptr, split, at_.dev, at_.handle())
-             ? Tensor()
-             : y;
+  return launched(triteia_hip_bmm_2_4_tokens_scratch(xc.data_ptr(), q.data_ptr(), meta.data_ptr(), y.data_ptr(), s.data_ptr(), m, n, tokens, k,
+                                                     split ? scratch.data_ptr() : nullptr, split, at_.dev, at_.handle()))
+             ? y
+             : Tensor();
 }
 
 // The routed product of x [tokens, k], added to y (accumulate = 1) or stored with zeros in the rows without a delta
-// (2: y need not be initialised); false: refused, nothing launched
-bool routed(const Tensor& x, const Tensor& q, const Tensor& meta, const Tensor& s, const Tensor& indices, Tensor& y, int offset,
+// (2: y need not be initialised).  The library's answer.
+int routed(const Tensor& x, const Tensor& q, const Tensor& meta, const Tensor& s, const Tensor& indices, Tensor& y, int offset,
             int accumulate, const Place& at_) {
   const int64_t tokens = x.size(0), k = x.size(1), m = y.size(1), n = q.size(0);
   Tensor ws;
@@ -144,7 +155,7 @@ bool routed(const Tensor& x, const Tensor& q, const Tensor& meta, const Tensor& 
     ws = scratch_bytes(bytes, x);
   }
   return triteia_hip_sbmm_2_4_routed(x.data_ptr(), q.data_ptr(), meta.data_ptr(), y.data_ptr(), s.data_ptr(), indices.data_ptr(), offset, n,
-                                     m, tokens, k, bytes ? ws.data_ptr() : nullptr, bytes, accumulate, at_.dev, at_.handle()) == 0;
+                                     m, tokens, k, bytes ? ws.data_ptr() : nullptr, bytes, accumulate, at_.dev, at_.handle());
 }
 
 // sbmm(qweights, xs, metas, ss, indices, base or None): ops.sbmm_4bit_2_4_native
@@ -155,38 +166,45 @@ Tensor sbmm(const Args& a) {
   const Tensor &q = a[0], &x = a[1], &meta = a[2], &s = a[3], &indices = a[4];
   if (!x.is_cuda() || x.dim() != 2 || x.scalar_type() != at::kHalf || s.dim() != 3) return {};
   const int64_t tokens = x.size(0), k = x.size(1), m = s.size(2);
-  if (!sizes_ok({tokens}) || !packed_ok(q, meta, s, x, q.size(0), k, m) || !base_ok(a, 5, x, k, m)) return {};
+  if (!sizes_ok({tokens}) || q.size(0) > kMaxRoutedDeltas || !packed_ok(q, meta, s, x, q.size(0), k, m) || !base_ok(a, 5, x, k, m)) return {};
   if (indices.device() != x.device() || indices.dim() != 1 || indices.size(0) != tokens || !indices.is_contiguous() ||
       !at::isIntegralType(indices.scalar_type(), false))
     return {};
   const Place at_(x);
   const Tensor xc = x.is_contiguous() ? x : x.contiguous();
   const Tensor idx = indices.scalar_type() == at::kInt ? indices : indices.to(at::kInt);
-  const bool base = !a.none(5);
-  Tensor y = base ? base_product(xc, a[5]) : at::empty({tokens, m}, x.options());
-  return routed(xc, q, meta, s, idx, y, 0, base ? 1 : 2, at_) ? y : Tensor();
+  Tensor y;
+  if (a.none(5)) {
+    y = at::empty({tokens, m}, x.options());
+    return launched(routed(xc, q, meta, s, idx, y, 0, 2, at_)) ? y : Tensor();
+  }
+  y = base_product(xc, a[5]);
+  must_launch(routed(xc, q, meta, s, idx, y, 0, 1, at_));
+  return y;
 }
 
 // (a view that starts inside 16 bytes; a copy made by contiguous() does not)
 bool aligned(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
 
+// (the expand's grid has a row of workgroups per 256 columns)
+constexpr int64_t kMaxLoraColumns = 65535 * 256;
 bool lora_ok(const Tensor& A, const Tensor& B, const Tensor& x, const Tensor& indices) {
   return x.is_cuda() && x.dim() == 2 && (x.scalar_type() == at::kHalf || x.scalar_type() == at::kBFloat16) &&
          dense_on(A, x, x.scalar_type(), 3) && dense_on(B, x, x.scalar_type(), 3) && indices.device() == x.device() && indices.dim() == 1 &&
          indices.is_contiguous() && (indices.scalar_type() == at::kInt || indices.scalar_type() == at::kLong) &&
          sizes_ok({x.size(0), x.size(1), A.size(0), A.size(2), B.size(2)}) && indices.size(0) == x.size(0) && A.size(1) == x.size(1) &&
-         B.size(0) == A.size(0) && B.size(1) == A.size(2) && B.size(2) % 8 == 0 && aligned(A) &&
+         B.size(0) == A.size(0) && B.size(1) == A.size(2) && B.size(2) % 8 == 0 && B.size(2) <= kMaxLoraColumns && aligned(A) &&
          aligned(B) && (!x.is_contiguous() || aligned(x));
 }
 size_t lora_bytes(const Tensor& A, const Tensor& x) { return triteia_hip_lora_scratch_bytes(x.size(0), A.size(0), A.size(1), A.size(2)); }
-bool lora_shrink(const Tensor& x, const Tensor& A, const Tensor& indices, const Tensor& scratch, bool accumulate, int dev, void* stream) {
+int lora_shrink(const Tensor& x, const Tensor& A, const Tensor& indices, const Tensor& scratch, bool accumulate, int dev, void* stream) {
   return triteia_hip_lora_shrink(x.data_ptr(), x.size(1), A.data_ptr(), indices.data_ptr(), indices.scalar_type() == at::kLong, x.size(0), A.size(0),
                                  A.size(1), A.size(2), accumulate, scratch.data_ptr(), scratch.numel(), x.scalar_type() == at::kBFloat16, dev,
-                                 stream) == 0;
+                                 stream);
 }
-bool lora_expand(const Tensor& y, const Tensor& A, const Tensor& B, const Tensor& scratch, double scale, bool accumulate, int dev, void* stream) {
+int lora_expand(const Tensor& y, const Tensor& A, const Tensor& B, const Tensor& scratch, double scale, bool accumulate, int dev, void* stream) {
   return triteia_hip_lora_expand(y.data_ptr(), y.size(1), B.data_ptr(), scratch.data_ptr(), y.size(0), B.size(0), A.size(1), B.size(1), y.size(1),
-                                 (float)scale, accumulate, y.scalar_type() == at::kBFloat16, dev, stream) == 0;
+                                 (float)scale, accumulate, y.scalar_type() == at::kBFloat16, dev, stream);
 }
 
 // lora(weights_A, weights_B, x, indices, base or None, scale): ops.lora_bgmv / lora_sgmv / lora_sgmv_routed
@@ -200,10 +218,11 @@ Tensor lora(const Args& a) {
   const Tensor xc = x.is_contiguous() ? x : x.contiguous();
   const Tensor scratch = scratch_bytes(bytes, x);
   const bool base = !a.none(4);
-  if (!lora_shrink(xc, A, indices, scratch, base, at_.dev, at_.handle())) return {};
+  if (!launched(lora_shrink(xc, A, indices, scratch, base, at_.dev, at_.handle()))) return {};
   // (without a base weight every row is written by the expand: tokens without an adapter get zeros)
   Tensor y = base ? base_product(xc, a[4]) : at::empty({x.size(0), B.size(2)}, x.options());
-  return lora_expand(y, A, B, scratch, a.number, base, at_.dev, at_.handle()) ? y : Tensor();
+  must_launch(lora_expand(y, A, B, scratch, a.number, base, at_.dev, at_.handle()));
+  return y;
 }
 
 // ldmm(indices, x, LwA, LwB, DeltaW, metas, ss, base or None): ops.ldmm.  One stream: with the LoRA pair at 10 us, a side
@@ -218,17 +237,18 @@ Tensor ldmm(const Args& a) {
   if (x.scalar_type() != at::kHalf || !lora_ok(A, B, x, indices) || s.dim() != 3) return {};
   const int64_t k = x.size(1), m = B.size(2);
   const size_t bytes = lora_bytes(A, x);
-  if (bytes == 0 || !packed_ok(q, meta, s, x, q.size(0), k, m) || !base_ok(a, 7, x, k, m)) return {};
+  if (bytes == 0 || q.size(0) > kMaxRoutedDeltas || !packed_ok(q, meta, s, x, q.size(0), k, m) || !base_ok(a, 7, x, k, m)) return {};
   const Place at_(x);
   const Tensor xc = x.is_contiguous() ? x : x.contiguous();
   const Tensor scratch = scratch_bytes(bytes, x);
   const bool base = !a.none(7);
-  if (!lora_shrink(xc, A, indices, scratch, base, at_.dev, at_.handle())) return {};
+  if (!launched(lora_shrink(xc, A, indices, scratch, base, at_.dev, at_.handle()))) return {};
   // (without a base weight the expand stores the adapters' rows and zeros in all others, the deltas' among them)
   Tensor y = base ? base_product(xc, a[7]) : at::empty({x.size(0), m}, x.options());
-  if (!lora_expand(y, A, B, scratch, 1.0, base, at_.dev, at_.handle())) return {};
+  must_launch(lora_expand(y, A, B, scratch, 1.0, base, at_.dev, at_.handle()));
   const Tensor idx = indices.scalar_type() == at::kInt ? indices : indices.to(at::kInt);
-  return routed(xc, q, meta, s, idx, y, A.size(0), 1, at_) ? y : Tensor();
+  must_launch(routed(xc, q, meta, s, idx, y, A.size(0), 1, at_));
+  return y;
 }
 
 PyObject* wrap(Tensor&& t) {
@@ -269,8 +289,8 @@ bool packed(const Args& a, Tensor (&out)[3]) {
   out[0] = at::empty({k / 32, 2 * m}, w.options().dtype(at::kInt));
   out[1] = at::empty({m, k / 16}, w.options().dtype(at::kShort));
   out[2] = at::empty({m, k / 16}, w.options().dtype(at::kShort));
-  return triteia_hip_pack_2_4(w.data_ptr(), s.data_ptr(), out[0].data_ptr(), out[1].data_ptr(), out[2].data_ptr(), k, m, at_.dev,
-                              at_.handle()) == 0;
+  return launched(triteia_hip_pack_2_4(w.data_ptr(), s.data_ptr(), out[0].data_ptr(), out[1].data_ptr(), out[2].data_ptr(), k, m, at_.dev,
+                                       at_.handle()));
 }
 PyObject* pack(PyObject*, PyObject* const* v, Py_ssize_t n) {
   HANDLE_TH_ERRORS

@@ -1623,7 +1623,7 @@ int triteia_hip_lora_shrink(const void* x, long x_stride, const void* a, const v
 int triteia_hip_lora_expand(void* y, long y_stride, const void* b, const void* scratch, int n_tokens, int n_adapters, int k, int r, int m,
                             float scale, int accumulate, int bf16, int dev, void* stream) {
   if (n_tokens == 0 || m == 0) return TRITEIA_HIP_OK;
-  if (!lora_routed_takes(n_tokens, n_adapters, k, r) || m < 0 || m % 8 != 0)
+  if (!lora_routed_takes(n_tokens, n_adapters, k, r) || m < 0 || m % 8 != 0 || m > 65535 * kLoraExpandCols)   // (rows of the grid)
     return fail(TRITEIA_HIP_ERR_KERN_SHAPE, "lora_expand: tokens=%d adapters=%d k=%d r=%d m=%d", n_tokens, n_adapters, k, r, m);
   if (!y || !b || !scratch) return fail(TRITEIA_HIP_ERR_ARGUMENT, "lora_expand: null tensor pointer");
   if ((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(scratch)) % 16 != 0 || y_stride % 8 != 0)
@@ -1640,12 +1640,14 @@ int triteia_hip_pack_2_4(const void* weight, const void* scales, void* qweight, 
   if (prob_k < 0 || prob_m < 0 || prob_k % 32 != 0 || prob_m % 64 != 0)
     return fail(TRITEIA_HIP_ERR_PROB_SHAPE, "pack_2_4: k=%d, m=%d need k %% 32 == 0 and m %% 64 == 0", prob_k, prob_m);
   if (prob_k == 0 || prob_m == 0) return TRITEIA_HIP_OK;
+  const long row_blocks = (prob_k / 32 + kPackRows - 1) / kPackRows;
+  if (row_blocks > 65535) return fail(TRITEIA_HIP_ERR_PROB_SHAPE, "pack_2_4: k=%d is too long", prob_k);
+  if ((prob_m + (long)kPackCols - 1) / kPackCols * (64 * kPackRows) > 0xffffffffL)   // (threads along a dimension of the grid)
+    return fail(TRITEIA_HIP_ERR_PROB_SHAPE, "pack_2_4: m=%d is too wide", prob_m);
   if (!weight || !scales || !qweight || !meta || !meta_raw) return fail(TRITEIA_HIP_ERR_ARGUMENT, "pack_2_4: null tensor pointer");
   if ((reinterpret_cast<uintptr_t>(weight) | reinterpret_cast<uintptr_t>(scales)) % 4 != 0 ||
       (reinterpret_cast<uintptr_t>(qweight) | reinterpret_cast<uintptr_t>(meta)) % 8 != 0 || reinterpret_cast<uintptr_t>(meta_raw) % 4 != 0)
     return fail(TRITEIA_HIP_ERR_ARGUMENT, "pack_2_4: weight, scales and meta_raw need 4-byte, qweight and meta 8-byte alignment");
-  const long row_blocks = (prob_k / 32 + kPackRows - 1) / kPackRows;
-  if (row_blocks > 65535) return fail(TRITEIA_HIP_ERR_PROB_SHAPE, "pack_2_4: k=%d is too long", prob_k);
   DeviceGuard g(dev);
   if (!g.ok) return fail(TRITEIA_HIP_ERR_RUNTIME, "cannot select device %d", dev);
   hipLaunchKernelGGL(pack_2_4_kernel, dim3((prob_m + kPackCols - 1) / kPackCols, (unsigned)row_blocks), dim3(64 * kPackRows), 0,
