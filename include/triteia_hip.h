@@ -286,12 +286,6 @@ TRITEIA_HIP_API int triteia_hip_sgmv_routed_bf16(void* y, long y_stride, const v
                                  int n_adapters, int d_in, int d_out, float scale, const void* plan, int prob_n,
                                  int accumulate, int dev, void* stream);
 
-/* The dense base product of a small batch: y[t] = x[t] @ w^T.  x [tokens, k] and y [tokens, m] row-major, w [m, k] with rows
- * w_stride elements apart; fp16 (bf16 = 1: bf16), fp32 sums.  tokens <= 64, m % 16 == 0, k % 64 == 0, w_stride % 8 == 0,
- * every tensor 16-byte aligned. */
-TRITEIA_HIP_API int triteia_hip_base_gemm(const void* x, const void* w, long w_stride, void* y, int tokens, int m, int k, int bf16, int dev,
-                          void* stream);
-
 /* The LoRA pair on adapters as they are stored and on the batch's own indices, in two launches:
  *   y[t] (+)= scale * (x[t] @ A[i]) @ B[i],   i = indices[t] in [0, n_adapters)
  * A [n_adapters, k, r], B [n_adapters, r, m] row-major, fp16 (bf16 = 1: bf16) like x and y; indices int32 (index64 = 1:

@@ -174,3 +174,24 @@ def test_sizes_past_a_grid_are_refused_before_the_launch():
     pack = lambda k, m: lib.triteia_hip_pack_2_4(null, null, null, null, null, k, m, 0, null)
     assert pack(32, 2 ** 30 - 128) == _ffi.ERR_ARGUMENT
     assert pack(32, 2 ** 30) == _ffi.ERR_PROB_SHAPE
+
+
+def test_environment_is_read_in_one_place():
+    """The knobs' table is the only reader: no kernel is picked by a variable that it does not list."""
+    csrc = os.path.join(ROOT, "triteia_amd", "csrc")
+    calls = {f: len(re.findall(r"\bgetenv\s*\(", open(os.path.join(csrc, f)).read())) for f in sorted(os.listdir(csrc))}
+    assert {f: n for f, n in calls.items() if n} == {"triteia_hip.hip": 1}
+
+
+def test_every_entry_point_has_a_caller():
+    """What the library exports is called by the binding, the tests or the benchmark."""
+    text = ""
+    for folder in (os.path.join(ROOT, "triteia_amd"), os.path.join(ROOT, "tests"), ROOT):
+        for base, _, files in os.walk(folder):
+            if folder == ROOT and base != ROOT:
+                continue
+            for f in files:
+                if f.endswith((".py", ".cpp")) and f != "_ffi.py":
+                    text += open(os.path.join(base, f)).read()
+    unused = [n for n in _ffi.SIGNATURES if not re.search(n + r"\b", text) and not (n.endswith("_bf16") and n[:-5] in text)]
+    assert not unused

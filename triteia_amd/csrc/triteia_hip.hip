@@ -10,7 +10,6 @@
 #include <cstring>
 #include <mutex>
 
-#include "base_gemm.hip.h"
 #include "lora.hip.h"
 #include "lora_mfma.hip.h"
 #include "lora_routed.hip.h"
@@ -1546,57 +1545,7 @@ int lora_expand_impl(void* y, long y_stride, const void* w, const void* scratch,
 
 }  // namespace
 
-namespace {
-
-// PICK_COMMENT
-template <class T>
-int base_gemm_impl(const void* x, const void* w, long w_stride, void* y, int tokens, int m, int k, hipStream_t st) {
-  BaseArgs<T> a;
-  memset(&a, 0, sizeof(a));
-  a.x = static_cast<const T*>(x);
-  a.w = static_cast<const T*>(w);
-  a.w_stride = w_stride;
-  a.y = static_cast<T*>(y);
-  a.tokens = tokens;
-  a.m = m;
-  a.k = k;
-  const int variant = getenv("BV") ? atoi(getenv("BV")) : 0;
-  const dim3 g1((m + 15) / 16), g2((m + 31) / 32), g4((m + 63) / 64), b(64 * kBaseWaves);
-  if (tokens <= 16) {
-    if (variant == 0) hipLaunchKernelGGL((base_gemm_kernel<T, 1, 1, 4>), g1, b, 0, st, a);
-    else if (variant == 1) hipLaunchKernelGGL((base_gemm_kernel<T, 1, 1, 2>), g1, b, 0, st, a);
-    else if (variant == 2) hipLaunchKernelGGL((base_gemm_kernel<T, 2, 1, 2>), g2, b, 0, st, a);
-    else hipLaunchKernelGGL((base_gemm_kernel<T, 2, 1, 4>), g2, b, 0, st, a);
-  } else if (tokens <= 32) {
-    if (variant == 0) hipLaunchKernelGGL((base_gemm_kernel<T, 1, 2, 4>), g1, b, 0, st, a);
-    else if (variant == 1) hipLaunchKernelGGL((base_gemm_kernel<T, 1, 2, 2>), g1, b, 0, st, a);
-    else if (variant == 2) hipLaunchKernelGGL((base_gemm_kernel<T, 2, 2, 2>), g2, b, 0, st, a);
-    else hipLaunchKernelGGL((base_gemm_kernel<T, 2, 2, 3>), g2, b, 0, st, a);
-  } else {
-    if (variant == 0) hipLaunchKernelGGL((base_gemm_kernel<T, 1, 4, 2>), g1, b, 0, st, a);
-    else if (variant == 1) hipLaunchKernelGGL((base_gemm_kernel<T, 2, 4, 1>), g2, b, 0, st, a);
-    else if (variant == 2) hipLaunchKernelGGL((base_gemm_kernel<T, 2, 4, 2>), g2, b, 0, st, a);
-    else hipLaunchKernelGGL((base_gemm_kernel<T, 4, 4, 1>), g4, b, 0, st, a);
-  }
-  return check_launch("base_gemm_kernel");
-}
-
-}  // namespace
-
 extern "C" {
-
-int triteia_hip_base_gemm(const void* x, const void* w, long w_stride, void* y, int tokens, int m, int k, int bf16, int dev, void* stream) {
-  if (tokens < 0 || tokens > kBaseMaxTokens || m < 0 || m % 16 != 0 || k <= 0 || k % 64 != 0 || w_stride < k || w_stride % 8 != 0)
-    return fail(TRITEIA_HIP_ERR_PROB_SHAPE, "base_gemm: tokens=%d m=%d k=%d w_stride=%ld", tokens, m, k, w_stride);
-  if (tokens == 0 || m == 0) return TRITEIA_HIP_OK;
-  if (!x || !w || !y) return fail(TRITEIA_HIP_ERR_ARGUMENT, "base_gemm: null tensor pointer");
-  if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(y)) % 16 != 0)
-    return fail(TRITEIA_HIP_ERR_ARGUMENT, "base_gemm: x, w and y must be 16-byte aligned");
-  DeviceGuard g(dev);
-  if (!g.ok) return fail(TRITEIA_HIP_ERR_RUNTIME, "cannot select device %d", dev);
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  return bf16 ? base_gemm_impl<bf16_t>(x, w, w_stride, y, tokens, m, k, st) : base_gemm_impl<_Float16>(x, w, w_stride, y, tokens, m, k, st);
-}
 
 size_t triteia_hip_lora_scratch_bytes(int n_tokens, int n_adapters, int k, int r) {
   return lora_routed_takes(n_tokens, n_adapters, k, r) ? lora_cut(n_tokens, n_adapters, k, r).total : 0;

@@ -56,7 +56,6 @@ SIGNATURES = {
     "triteia_hip_bgmv_store_bf16": (_c_int, [_c_vp] * 4 + [_c_int] * 5 + [_c_float, _c_int, _c_vp]),
     "triteia_hip_sgmv_store": (_c_int, [_c_vp] * 4 + [_c_int] * 5 + [_c_vp]),
     "triteia_hip_sgmv_store_bf16": (_c_int, [_c_vp] * 4 + [_c_int] * 5 + [_c_vp]),
-    "triteia_hip_base_gemm": (_c_int, [_c_vp, _c_vp, _c_long, _c_vp] + [_c_int] * 5 + [_c_vp]),
     "triteia_hip_lora_scratch_bytes": (_c_sz, [_c_int] * 4),
     "triteia_hip_lora_shrink": (_c_int, [_c_vp, _c_long, _c_vp, _c_vp] + [_c_int] * 6 + [_c_vp, _c_sz, _c_int, _c_int, _c_vp]),
     "triteia_hip_lora_expand": (_c_int, [_c_vp, _c_long, _c_vp, _c_vp] + [_c_int] * 5 + [_c_float] + [_c_int] * 3 + [_c_vp]),
