@@ -94,3 +94,24 @@ def test_more_deltas_than_a_plan_takes_are_refused_ahead_of_every_launch(layer):
         assert native().ldmm(layer["idx"], layer["x"], layer["A"], layer["B"], q, meta, s, base) is None
         with pytest.raises(RuntimeError, match="8192"):
             ops.sbmm_4bit_2_4_native(q, layer["x"], meta, s, layer["idx"], base_weight=base)
+
+
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_capi_wrappers_of_the_lora_pair_and_the_packer(layer, accumulate):
+    """capi.lora_scratch / lora_shrink / lora_expand and capi.pack_2_4: the same launches as the ops, hence the same bits."""
+    from triteia_amd.python.capi import lora_expand, lora_scratch, lora_shrink, pack_2_4
+    t = layer
+    y = torch.matmul(t["x"], t["base"].t()) if accumulate else torch.empty((T, M_OUT), dtype=torch.float16, device="cuda")
+    scratch = lora_scratch(T, t["A"])
+    lora_shrink(t["x"], t["A"], t["idx"], scratch, accumulate)
+    lora_expand(y, t["B"], scratch, K, accumulate, scale=0.5)
+    assert torch.equal(y, ops.lora_bgmv(t["A"], t["B"], t["x"], t["idx"], base_weight=t["base"] if accumulate else None, scale=0.5))
+    with pytest.raises(RuntimeError, match="lora_shrink"):
+        lora_expand(y, t["B"], scratch, K, not accumulate)
+    w = (torch.randn(96, 192, device="cuda") * 0.1).half()
+    scale = torch.full((1, 192), 0.02, dtype=torch.float16, device="cuda")
+    for got, want in zip(pack_2_4(w, scale), native().pack(w, scale)):
+        assert torch.equal(got, want)
+    odd = torch.empty(96 * 192 + 1, dtype=torch.float16, device="cuda")[1:].view(96, 192)     # starts inside a pair: copied
+    odd.copy_(w)
+    assert all(torch.equal(got, want) for got, want in zip(pack_2_4(odd, scale), native().pack(w, scale)))

@@ -145,16 +145,21 @@ def lora_shrink(x, weights_A, indices, scratch, accumulate):
         _ffi.ptr(x), k, _ffi.ptr(weights_A), _ffi.ptr(indices), 1 if indices.dtype == torch.int64 else 0, n_tokens, n_adapters, k, r,
         1 if accumulate else 0, _ffi.ptr(scratch), scratch.numel(), 1 if dtype == torch.bfloat16 else 0, _ffi.device_index(x),
         _ffi.stream_of(x)))
+    scratch.lora_pair = (n_tokens, n_adapters, k, r, bool(accumulate))     # what `lora_expand` may read it as
 
 
 def lora_expand(y, weights_B, scratch, k, accumulate, scale=1.0):
     """The second launch: y [tokens, m] from the scratch of `lora_shrink` (whose A had k rows), weights_B
-    [n_adapters, r, m] contiguous."""
-    _ffi.require_gpu(y=y, weights_B=weights_B, scratch=scratch)
-    dtype = _lora_dtype(y, weights_B=weights_B)
+    [n_adapters, r, m] contiguous.  The scratch holds the shrink's tiles and token rows, which the kernel follows: it is
+    taken from a shrink of the same sizes only."""
     n_adapters, r, m = weights_B.shape
     if y.dim() != 2 or y.size(1) != m:
         raise RuntimeError("shape mismatch between y and weights_B")
+    want, have = (y.size(0), n_adapters, k, r, bool(accumulate)), getattr(scratch, "lora_pair", None)
+    if have != want:
+        raise RuntimeError(f"scratch must come from lora_shrink with (tokens, adapters, k, r, accumulate) = {want}, got {have}")
+    _ffi.require_gpu(y=y, weights_B=weights_B, scratch=scratch)
+    dtype = _lora_dtype(y, weights_B=weights_B)
     _check(_ffi.lib().triteia_hip_lora_expand(
         _ffi.ptr(y), m, _ffi.ptr(weights_B), _ffi.ptr(scratch), y.size(0), n_adapters, k, r, m, float(scale), 1 if accumulate else 0,
         1 if dtype == torch.bfloat16 else 0, _ffi.device_index(y), _ffi.stream_of(y)))
