@@ -2,6 +2,7 @@
 import pytest
 import torch
 
+from triteia_amd.python.capi._native import native
 from triteia_amd.python.ops.utils.sparsity import mask_creator, prune_pack_2_4
 
 pytestmark = pytest.mark.gpu
@@ -29,3 +30,16 @@ def test_pack_kernel_gives_the_codecs_bytes(k, m, values):
         assert a.dtype == b.dtype and a.shape == b.shape
         # (the scales are handed through: compared as bytes, for their NaNs)
         assert torch.equal(a.view(torch.uint8), b.view(torch.uint8)), name
+
+
+def test_packing_inside_a_trace():
+    """A trace follows torch's operations: it records the codec, and answers for other weights than those it was made with."""
+    g = torch.Generator(device="cuda").manual_seed(5)
+    # (whole multiples of the scale: torch's fuser may leave out the rounding of the quotient to fp16)
+    first, second = ((torch.randint(-8, 8, (64, 128), generator=g, device="cuda") * 0.5).half() for _ in range(2))
+    scale = torch.full((1, 128), 0.5, dtype=torch.float16, device="cuda")
+    traced = torch.jit.trace(prune_pack_2_4, (first, scale))
+    for w in (first, second):
+        for got, want in zip(traced(w, scale), prune_pack_2_4(w, scale)):
+            assert torch.equal(got, want)
+    assert native().pack(first, scale) is not None         # (the kernel, outside a trace)

@@ -10,6 +10,8 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/TensorSubclassLikeUtils.h>
+#include <ATen/TracerMode.h>
 #include <ATen/autocast_mode.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
@@ -24,7 +26,8 @@ using at::Tensor;
 
 // A call's arguments, taken apart while the interpreter lock is held: what follows runs without it and sees no Python object.
 // Tensors are exactly torch.Tensor or Parameter; a subclass may give every operation another meaning, which the Python
-// path honours.
+// path honours.  So may a transform's wrapper around a tensor, a dispatch mode and a trace: what they follow are torch's
+// operations, and a kernel launched from here would leave its result in them as a constant.
 struct Args {
   static constexpr int kMax = 8;
   int n;
@@ -33,8 +36,10 @@ struct Args {
   double number = 0;        // a last argument that is neither a tensor nor None
   bool numeric = false;
   Args(PyObject* const* values, Py_ssize_t count) : n(count <= kMax ? (int)count : 0) {
+    const bool traced = at::tracer::impl::is_dispatch_enabled();
     for (int i = 0; i < n; i++) {
-      if (THPVariable_CheckExact(values[i])) tensors[i] = &THPVariable_Unpack(values[i]);
+      if (!traced && THPVariable_CheckExact(values[i]) && !at::isTensorSubclassLike(THPVariable_Unpack(values[i])))
+        tensors[i] = &THPVariable_Unpack(values[i]);
       nones[i] = values[i] == Py_None;
     }
     if (n == 0 || nones[n - 1] || THPVariable_Check(values[n - 1])) return;
