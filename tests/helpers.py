@@ -57,15 +57,25 @@ def delknob(monkeypatch, name):
     reload_knobs()
 
 
-def without_native(monkeypatch):
-    """Every op takes its Python path: the native binding declines each call."""
+def watch_native(monkeypatch, decline=False):
+    """The names of the calls that the native binding answers from here on; with `decline` it answers none, so that
+    every op takes its Python path."""
     import importlib
 
-    class Declines:
+    from triteia_amd.python.capi._native import native
+    answered = []
+
+    class Watched:
         def __getattr__(self, name):
-            return lambda *args: None
+            def call(*args):
+                y = None if decline else getattr(native(), name)(*args)
+                if y is not None:
+                    answered.append(name)
+                return y
+            return call
 
     for name in ("bmm", "ldmm", "lora", "sbmm", "sparse_low_precision"):
         module = importlib.import_module("triteia_amd.python.ops.matmul." + name)
-        monkeypatch.setattr(module, "native", Declines)
-    monkeypatch.setattr(importlib.import_module("triteia_amd.python.nn.linear"), "native", Declines)
+        monkeypatch.setattr(module, "native", Watched)
+    monkeypatch.setattr(importlib.import_module("triteia_amd.python.nn.linear"), "native", Watched)
+    return answered

@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from oracle import triteia_oracle as orc
-from tests.helpers import activations, check_close, make_deltas, setknob, to_gpu
+from tests.helpers import activations, check_close, make_deltas, setknob, to_gpu, watch_native
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -71,9 +71,12 @@ def test_routed_sbmm_replays(monkeypatch, T, N, k, m, seed):
         assert bool((replayed[torch.from_numpy(hidx < 0).to(DEV)] == 0).all())
 
 
-def test_ldmm_replays():
-    """ldmm with a dense base: the routing and the LoRA shrink fork onto a second stream inside
-    the captured region and join before the expand."""
+@pytest.mark.parametrize("path", ["native binding", "python path"])
+def test_ldmm_replays(monkeypatch, path):
+    """ldmm with a dense base: on one stream as the native binding runs it; on the Python path (what the LoRA pair of the
+    binding does not take) the routing and the LoRA shrink fork onto a second stream inside the captured region and join
+    before the expand."""
+    answered = watch_native(monkeypatch, decline=path == "python path")
     from triteia_amd.python import ops
     T, M, N, k, m, r, seed = 96, 4, 5, 512, 768, 16, 211
     print(f"[case] graph replay of ldmm T={T} M={M} N={N} k={k} m={m} r={r}", flush=True)
@@ -107,6 +110,7 @@ def test_ldmm_replays():
         assert torch.equal(replayed, result), f"replay {rep} differs from the eager call"
         y0 = torch.matmul(x, gb.t()).float().cpu().numpy().astype(np.float64)
         check_close(replayed, y0 + orc.ldmm(hidx, hx, A, B, qw, meta, s), what=f"ldmm replay {rep}")
+    assert set(answered) == ({"ldmm"} if path == "native binding" else set())
 
 
 def test_matmul_and_bmm_replay():

@@ -13,7 +13,7 @@ import pytest
 import torch
 
 from oracle import triteia_oracle as orc
-from tests.helpers import activations, check_close, delknob, make_deltas, reload_knobs, setknob, to_gpu
+from tests.helpers import activations, check_close, delknob, make_deltas, reload_knobs, setknob, to_gpu, watch_native
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -909,6 +909,16 @@ def test_route_plan_is_a_stable_grouping(plan_rules):
 
 # ------------------------------------------------------------- lora / ldmm
 
+@pytest.fixture(params=["native binding", "python path"])
+def answered(request, monkeypatch):
+    """The LoRA and ldmm tests run twice: as the ops are called, where the native binding answers with the pair of kernels
+    that routes by itself, and on the ops' Python path with the kernels of the reference's own interfaces (which still
+    serves what that pair does not take).  The value is the list of calls that the binding answered."""
+    calls = watch_native(monkeypatch, decline=request.param == "python path")
+    yield calls
+    assert bool(calls) == (request.param == "native binding")
+
+
 def _lora_weights(M, k, r, m, seed, scale=1.0):
     rng = np.random.default_rng(seed)
     A = (rng.standard_normal((M, k, r)) * scale).astype(np.float16)
@@ -932,7 +942,7 @@ def _assert_allclose_scaled(got, ref, what):
     # segments longer than one pass of the row slots, ragged tails, a rank that is no power of two, the widest rank
     (301, 3, 1024, 2048, 16, 66), (71, 3, 512, 520, 24, 67), (41, 2, 1024, 512, 128, 68),
 ])
-def test_lora_ops(ops, T, M, k, m, r, seed):
+def test_lora_ops(ops, answered, T, M, k, m, r, seed):
     say(f"lora T={T} M={M} k={k} m={m} r={r} seed={seed}")
     A, B = _lora_weights(M, k, r, m, seed, scale=0.1)
     x = activations(T, k, seed + 1)
@@ -964,7 +974,9 @@ def test_lora_ops(ops, T, M, k, m, r, seed):
 def test_lora_on_the_matrix_cores(ops, monkeypatch, T, M, k, m, r, seed, dtype):
     """SGMV and routed SGMV with every launch the matrix-core kernels can take sent to them (by default: ranks 32 / 64 /
     128 with 16 rows per group and more), against the oracle; in bf16 with the oracle's bf16 intermediate.  The same
-    calls with those kernels switched off agree to the rounding of the intermediate."""
+    calls with those kernels switched off agree to the rounding of the intermediate.  On the ops' Python path: the native
+    binding answers with kernels of its own, which that switch does not reach."""
+    answered = watch_native(monkeypatch, decline=True)
     say(f"lora mfma T={T} M={M} k={k} m={m} r={r} seed={seed} {dtype}")
     rng = np.random.default_rng(seed)
     idx = np.sort(rng.integers(-1, M, size=T)).astype(np.int32)
@@ -1000,6 +1012,7 @@ def test_lora_on_the_matrix_cores(ops, monkeypatch, T, M, k, m, r, seed, dtype):
     gi2 = torch.from_numpy(idx[perm].copy()).to(DEV)
     gx2 = gx[torch.from_numpy(perm).to(DEV)].contiguous()
     check_close(ops.lora_sgmv_routed(gA, gB, gx2, gi2), ref[perm], tol=tol, what="lora_sgmv_routed unsorted (matrix cores)")
+    assert not answered
 
 
 @pytest.mark.parametrize("T,M,d_in,d_out,seed", [
@@ -1056,7 +1069,7 @@ def test_lora_kernels_store_instead_of_add(monkeypatch, T, M, d_in, d_out, seed,
 @pytest.mark.parametrize("T,M,k,m,r,seed", [
     (10, 5, 768, 256, 64, 161), (33, 4, 512, 1024, 16, 162), (71, 3, 512, 520, 24, 163), (41, 2, 1024, 512, 128, 164),
 ])
-def test_lora_ops_bf16(ops, T, M, k, m, r, seed):
+def test_lora_ops_bf16(ops, answered, T, M, k, m, r, seed):
     """The bfloat16 instantiation of BGMV / SGMV (the reference builds both element types: bgmv_all.cu:4-5,
     sgmv.cu:10).  bf16 keeps 8 significant bits: one rounding of an output is up to 2^-9 relative (1.1e-3 rms),
     and the rank-r intermediate, rounded to bf16 as well, can fall on the other side of a rounding boundary when
@@ -1084,7 +1097,7 @@ def test_lora_ops_bf16(ops, T, M, k, m, r, seed):
     (10, 5, 5, 768, 768, 8, 71), (10, 5, 5, 768, 768, 64, 72),          # tests/ops/test_ldmm.py:103
     (128, 2, 3, 4096, 2048, 16, 73), (128, 16, 16, 1024, 1024, 32, 74),
 ])
-def test_ldmm(ops, T, M, N, m, k, r, seed, plan_rules):
+def test_ldmm(ops, answered, T, M, N, m, k, r, seed, plan_rules):
     say(f"ldmm T={T} M={M} N={N} m={m} k={k} r={r} seed={seed}")
     qw, meta, s = make_deltas(N, k, m, seed)
     A, B = _lora_weights(M, k, r, m, seed + 1, scale=0.05)
@@ -1103,11 +1116,11 @@ def test_ldmm(ops, T, M, N, m, k, r, seed, plan_rules):
     only_delta = ops.sbmm_4bit_2_4_native(gq, gx, gm, gs, torch.where(gi >= M, gi - M, -1).int())
     rows = torch.from_numpy(idx >= M).to(DEV)
     assert torch.equal(out[rows], only_delta[rows])
-    # with a dense base weight (routing and the LoRA shrink then run on a side stream beside the base GEMM):
-    # the library GEMM's fp16 result is taken as given, the routed parts are added to it in place
+    # with a dense base weight (on the Python path routing and the LoRA shrink then run on a side stream beside the base
+    # GEMM): the library GEMM's fp16 result is taken as given, the routed parts are added to it in place
     base_w = (np.random.default_rng(seed + 4).standard_normal((m, k)) * 0.02).astype(np.float16)
     gb = torch.from_numpy(base_w).to(DEV)
-    for _ in range(3):                                   # several calls in a row share the side stream
+    for _ in range(3):                                   # (several calls in a row share the side stream)
         with_base = ops.ldmm(gi, gx, gA, gB, gq, gm, gs, base_weight=gb)
     torch.cuda.synchronize()
     y0 = torch.matmul(gx, gb.t())

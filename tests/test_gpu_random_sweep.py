@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 import torch
 
+from tests.helpers import watch_native
 from triteia_amd import workloads as W
 from triteia_amd.python import ops
 from triteia_amd.python.capi import routed_workspace, sbmm_2_4_routed
@@ -82,8 +83,10 @@ def test_sparse_entry_points_on_random_cases(seed):
             assert _rel(got[~none].float() + (3.0 if acc else 0.0), ref[~none]) < (4e-3 if acc else 2e-3), what
 
 
+@pytest.mark.parametrize("path", ["native binding", "python path"])
 @pytest.mark.parametrize("seed", [21, 22])
-def test_lora_and_ldmm_on_random_cases(seed):
+def test_lora_and_ldmm_on_random_cases(monkeypatch, seed, path):
+    answered = watch_native(monkeypatch, decline=path == "python path")
     rng = np.random.default_rng(seed)
     for case in range(100):
         kind = ["bgmv", "sgmv", "sgmv_routed", "ldmm", "ldmm"][int(rng.integers(0, 5))]
@@ -132,3 +135,4 @@ def test_lora_and_ldmm_on_random_cases(seed):
             assert bool((got[gi < 0] == 0).all()), what
         if float(ref.norm()) > 0:
             assert _rel(got, ref) < 2e-3, what
+    assert set(answered) == ({"lora", "ldmm"} if path == "native binding" else set())
