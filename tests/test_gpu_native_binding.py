@@ -115,3 +115,52 @@ def test_capi_wrappers_of_the_lora_pair_and_the_packer(layer, accumulate):
     odd = torch.empty(96 * 192 + 1, dtype=torch.float16, device="cuda")[1:].view(96, 192)     # starts inside a pair: copied
     odd.copy_(w)
     assert all(torch.equal(got, want) for got, want in zip(pack_2_4(odd, scale), native().pack(w, scale)))
+
+
+def test_ldmm_with_the_lora_pair_on_a_second_stream():
+    """A large batch with a base weight forks outside a capture and runs on one stream inside it: the same bits, call after
+    call on new inputs; a launch that fails between the fork and the join raises, and the calls after it are right."""
+    import ctypes
+
+    from triteia_amd.python.capi import _ffi
+    tokens, k, m, models, rank = 2049, 4096, 4096, 3, 16              # (the smallest batch of this layer, and one token)
+    g = torch.Generator(device="cuda").manual_seed(2)
+    rand = lambda *shape: (torch.randn(shape, generator=g, device="cuda") * 0.02).half()
+    q, meta, s = random_packed_deltas(models, k, m, 4, "cuda")
+    A, B, base = rand(models, k, rank), rand(models, rank, m), rand(m, k)
+    x = torch.empty((tokens, k), dtype=torch.float16, device="cuda")
+    idx = torch.empty(tokens, dtype=torch.int32, device="cuda")
+    inputs = [(random_activations(tokens, k, 10 + i, "cuda"),
+               torch.randint(-1, 2 * models, (tokens,), generator=g, device="cuda", dtype=torch.int32)) for i in range(4)]
+    call = lambda: native().ldmm(idx, x, A, B, q, meta, s, base)
+
+    def load(i):
+        x.copy_(inputs[i][0])
+        idx.copy_(inputs[i][1])
+
+    load(0)
+    call()
+    torch.cuda.synchronize()
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.stream(stream), torch.cuda.graph(graph, stream=stream):
+        captured = call()
+    want = []
+    for i in range(4):
+        load(i)
+        graph.replay()
+        want.append(captured.clone())
+    plain = torch.matmul(x, base.t())
+    assert torch.equal(want[3][idx < 0], plain[idx < 0]) and not torch.equal(want[3], plain)
+    for _ in range(3):                       # (nothing waits between the calls: each follows the copies and the call before it)
+        got = []
+        for i in range(4):
+            load(i)
+            got.append(call())
+        for i in range(4):
+            assert torch.equal(got[i], want[i]), i
+    hip = ctypes.CDLL(_ffi.LIB_PATH)
+    torch.cuda.synchronize()
+    assert hip.hipSetDevice(1000) != 0       # (an error that the host has left behind)
+    with pytest.raises(RuntimeError, match="triteia_hip error 4"):
+        call()
+    assert torch.equal(call(), want[3])

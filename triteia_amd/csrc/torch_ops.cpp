@@ -15,8 +15,12 @@
 #include <ATen/autocast_mode.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <c10/core/Event.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+
+#include <unordered_map>
 
 #include "../../include/triteia_hip.h"
 
@@ -230,10 +234,59 @@ Tensor lora(const Args& a) {
   return y;
 }
 
-// ldmm(indices, x, LwA, LwB, DeltaW, metas, ss, base or None): ops.ldmm.  One stream: with the LoRA pair at 10 us, a side
-// stream for it beside the base GEMM costs more in events than it hides (256 tokens over 32 adapters of rank 16 and 32
-// deltas of 4096 x 11008: 148 us on one stream, 149 with the shrink on a side stream, 153 with the expand there as well;
-// 38 against 75 and 84 us of host time).
+// A second stream beside the call's own (default priority, one per thread and device, made at first use).  The call's
+// stream waits for its work also where a later step throws: the buffers then go back to that stream's pool.
+class Beside {
+ public:
+  explicit Beside(const Place& at_) : own_(at_.stream.unwrap()), side_(stream(at_.dev).unwrap()), handle_(stream(at_.dev).stream()) { follow(); }
+  ~Beside() {
+    if (!joined_) {
+      try {
+        wait(side_, own_);
+      } catch (...) {           // (the exception on its way out is the one to report)
+      }
+    }
+  }
+  Beside(const Beside&) = delete;
+  Beside& operator=(const Beside&) = delete;
+  void follow() { wait(own_, side_); }      // what comes next on the second stream sees what the call's stream has so far
+  void join() {
+    wait(side_, own_);
+    joined_ = true;
+  }
+  void* handle() const { return handle_; }
+
+ private:
+  static void wait(const c10::Stream& first, const c10::Stream& second) {
+    c10::Event event(first.device_type());
+    event.record(first);
+    event.block(second);
+  }
+  static c10::hip::HIPStreamMasqueradingAsCUDA stream(c10::DeviceIndex dev) {
+    static thread_local std::unordered_map<int, c10::hip::HIPStreamMasqueradingAsCUDA> streams;
+    auto it = streams.find(dev);
+    if (it == streams.end()) it = streams.emplace(dev, c10::hip::getStreamFromPoolMasqueradingAsCUDA(false, dev)).first;
+    return it->second;
+  }
+  c10::Stream own_, side_;
+  void* handle_;
+  bool joined_ = false;
+};
+
+// Whether ldmm runs its LoRA pair on a second stream, the shrink beside the base product and the expand beside the deltas
+// (their rows of the output differ).  The fork and the joins hold a call up by about 60 us, which prompts hide and smaller
+// batches do not.  One stream -> two, a call among others, 4 - 32 deltas, 4 or 32 adapters of rank 16 or 64:
+//   4096 x 4096 with 2048 / 4096 tokens 126-175 -> 120-160 / 180-261 -> 172-247 us; 4096 x 11008 with 2048 / 4096
+//   247-386 -> 227-378 / 546-718 -> 515-704; 11008 x 4096 with 4096 400-587 -> 368-558; in 198 such shapes 5 % less on average,
+//   8 of them more than 2 % longer.
+// Below either bound: 4096 x 4096 with 768 tokens 66-114 -> 76-115, 1024 x 1024 with 4096 59-72 -> 99-129, 8192 x 13824 with
+// 1024 307-534 -> 302-541.  In a captured graph the fork costs more than it hides at every size (11008 x 4096, 32 + 32
+// models, 1024 / 4096 tokens of rank 16: 275 -> 300 / 546 -> 576).
+bool lora_beside(int64_t tokens, int64_t k, int64_t m) {
+  return tokens >= 2048 && tokens * k >= (int64_t(1) << 35) / m && c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None;
+}
+
+// ldmm(indices, x, LwA, LwB, DeltaW, metas, ss, base or None): ops.ldmm.
 Tensor ldmm(const Args& a) {
   if (a.n != 8) return {};
   for (int i = 0; i < 7; i++)
@@ -246,12 +299,23 @@ Tensor ldmm(const Args& a) {
   const Place at_(x);
   const Tensor xc = x.is_contiguous() ? x : x.contiguous();
   const Tensor scratch = scratch_bytes(bytes, x);
+  const Tensor idx = indices.scalar_type() == at::kInt ? indices : indices.to(at::kInt);
   const bool base = !a.none(7);
+  if (base && lora_beside(x.size(0), k, m)) {
+    Tensor y;                  // (like the other buffers ahead of the stream: freed only after it has been joined)
+    Beside side(at_);
+    if (!launched(lora_shrink(xc, A, indices, scratch, true, at_.dev, side.handle()))) return {};
+    y = base_product(xc, a[7]);
+    side.follow();
+    must_launch(lora_expand(y, A, B, scratch, 1.0, true, at_.dev, side.handle()));
+    must_launch(routed(xc, q, meta, s, idx, y, A.size(0), 1, at_));
+    side.join();
+    return y;
+  }
   if (!launched(lora_shrink(xc, A, indices, scratch, base, at_.dev, at_.handle()))) return {};
   // (without a base weight the expand stores the adapters' rows and zeros in all others, the deltas' among them)
   Tensor y = base ? base_product(xc, a[7]) : at::empty({x.size(0), m}, x.options());
   must_launch(lora_expand(y, A, B, scratch, 1.0, base, at_.dev, at_.handle()));
-  const Tensor idx = indices.scalar_type() == at::kInt ? indices : indices.to(at::kInt);
   must_launch(routed(xc, q, meta, s, idx, y, A.size(0), 1, at_));
   return y;
 }
