@@ -3,7 +3,7 @@ import pytest
 import torch
 
 from triteia_amd.python.capi._native import native
-from triteia_amd.python.ops.utils.sparsity import mask_creator, prune_pack_2_4
+from triteia_amd.python.ops.utils.sparsity import mask_creator, prune_pack_2_4, unpack_nibbles
 
 pytestmark = pytest.mark.gpu
 
@@ -43,3 +43,42 @@ def test_packing_inside_a_trace():
         for got, want in zip(traced(w, scale), prune_pack_2_4(w, scale)):
             assert torch.equal(got, want)
     assert native().pack(first, scale) is not None         # (the kernel, outside a trace)
+
+
+def _quantised(w, s):
+    """The codec's integers 0 .. 15 of weights [k, m] and scales [1, m]."""
+    return (torch.round(w / s).to(torch.int64) + 8).clamp(0, 15).to(torch.uint8)
+
+
+@pytest.mark.parametrize("scales", ["negative", "infinite", "nan", "subnormal", "zero"])
+def test_pack_kernel_on_unusual_scales(scales):
+    g = torch.Generator().manual_seed(9)
+    w = torch.randn((128, 192), generator=g).to(torch.float16)
+    w[::7] *= 6e-8                                                     # (subnormal weights among the others)
+    w[5::16] = float("inf")
+    w[6::16] = float("nan")
+    s = {"negative": -w.abs().nan_to_num(1.0, 1.0).amax(0, keepdim=True) * (2 / 15), "infinite": torch.full((1, 192), float("inf")),
+         "nan": torch.full((1, 192), float("nan")), "subnormal": torch.randint(1, 1024, (1, 192), generator=g) * 2.0 ** -24,
+         "zero": torch.zeros((1, 192))}[scales].to(torch.float16)
+    if scales in ("infinite", "zero"):
+        s[:, ::2] = -s[:, ::2]
+    w, s = w.cuda(), s.cuda()
+    got, want = prune_pack_2_4(w, s), prune_pack_2_4(w, s, mask=mask_creator(w.t().contiguous()))
+    for a, b in zip(got, want):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
+def test_pack_kernels_quotient_on_every_pair_of_fp16_values():
+    """Every weight with every scale, both all 2^16 bit patterns: two weights a group behind two zeros, so that the weights
+    are the two kept (a tie keeps the later)."""
+    every = torch.arange(65536, device="cuda", dtype=torch.int32).to(torch.int16).view(torch.float16)
+    s = every.reshape(1, -1)
+    rows = 1024                                                        # weights per pass: 2048 dense k x 65536 columns, 256 MB
+    for first in range(0, 65536, rows):
+        v = every[first:first + rows].reshape(rows // 2, 2)
+        w = torch.cat([torch.zeros_like(v), v], 1).reshape(-1, 1).expand(-1, 65536).contiguous()
+        qweight, _, _ = native().pack(w, s)
+        got = unpack_nibbles(qweight)
+        want = _quantised(every[first:first + rows].reshape(-1, 1), s)
+        assert torch.equal(got, want), f"weights {first} .. {first + rows - 1}"
+        print(f"[pairs] weights {first} .. {first + rows - 1}", flush=True)

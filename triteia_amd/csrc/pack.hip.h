@@ -32,10 +32,10 @@ struct PackedColumn {
 // fp16(fp32 v / s) rounded to an integer in [-8, 7], as half(1024 + 8 + integer).  The quotient is v * (1 / s) and one
 // correction by its remainder, within 2^-24 (1 + 2^-20) of the exact one: v and s have 11-bit mantissas, so an exact
 // quotient that is not itself a midpoint between two halves (12 bits) is at least 2^-23 away from every such midpoint,
-// and one that is a midpoint comes out exactly: the integer is that of a correctly rounded division (compared for all
-// 2^32 pairs of fp16 values, no difference), for 4 instructions instead of its 12.  The first estimate is bounded so that the remainder of an infinite quotient is not a
-// NaN; `s_rem` is s, or 0 for an infinite s (whose product with the estimate 0 would be one).  NaNs (0 / 0) count as zero.
-// The sum with 1032 in fp16 rounds to whole numbers, ties to even.
+// and one that is a midpoint comes out exactly: the integer is that of a correctly rounded division (the GPU test compares
+// all 2^32 pairs of fp16 values), for 4 instructions instead of its 12.  The first estimate is bounded so that the
+// remainder of an infinite quotient is not a NaN; `s_rem` is s, or 0 for an infinite s (whose product with the estimate 0
+// would be one).  NaNs (0 / 0) count as zero.  The sum with 1032 in fp16 rounds to whole numbers, ties to even.
 __device__ __forceinline__ _Float16 pack_quotient(_Float16 v, float s_rem, float inv) {
   const float x = (float)v;
   const float estimate = __builtin_amdgcn_fmed3f(x * inv, -16.f, 16.f);

@@ -79,7 +79,7 @@ __device__ __forceinline__ int wave_excl_scan(int v, int lane, int* total) {
 // One workgroup, the first; with `clear` the others store zeros in the rows of `clear` ([n_tokens][clear_stride] fp16,
 // clear_pieces 16-byte pieces each) whose token has no delta, beside the plan's chain of steps, which is the launch's length
 // (in place of a launch of its own that clears every row: 1000 tokens over 32 deltas of 4096 x 11008 161.3 -> 153.2 us a
-// call, 256 over 64 of 8192 x 28672 616.7 -> 607.4).
+// call; the launch saved is lost in the spread of calls of 600 us).
 // indices[t] - index_offset outside [0, n_deltas) means "no delta".
 //
 // The tokens are cut into `shares` of whole 64-token pieces, one per wavefront (as many as the 8192 LDS counters

@@ -494,8 +494,6 @@ __device__ __forceinline__ void tile_pass(const Sparse24Args& p, TileCtx& c, int
   }
 }
 
-// NT = widest token tile (16*NT tokens per pass) the instantiation supports; narrower passes
-// take the cheaper code path (fewer activation loads and MFMAs) at the same register budget.
 // Zeros in the columns [f0, f0 + columns) of every token without a delta (fused routing; columns a multiple of 8, 8-column
 // pieces over the threads).  By workgroups of their own behind those of the groups: the others' way to their first
 // request stays as it is, and the output needs no clearing launch (16 deltas of 4096 x 4096 with 64 tokens: 21.5 us a
@@ -509,6 +507,8 @@ __device__ __forceinline__ void clear_unrouted(const Sparse24Args& p, int f0, in
   }
 }
 
+// NT = widest token tile (16*NT tokens per pass) the instantiation supports; narrower passes
+// take the cheaper code path (fewer activation loads and MFMAs) at the same register budget.
 // EAGER: fused routing with group g = delta g (Sparse24Args::raw_static): the weights of the first
 // step are requested at once, together with the indices, instead of one memory round trip later.
 template <int NT, int KW, int DEPTH, bool EAGER = false, bool GS = false>
