@@ -94,11 +94,11 @@ class Problem:
             self.base = [(torch.randn((wl.m, wl.k), generator=g, device=dev) * 0.02).half() for _ in range(copies)]
             self.lora_a = (torch.randn((wl.n_lora, wl.k, wl.lora_rank), generator=g, device=dev) * 0.01).half()
             self.lora_b = (torch.randn((wl.n_lora, wl.lora_rank, wl.m), generator=g, device=dev) * 0.01).half()
-            self.v = torch.zeros((wl.tokens, wl.lora_rank), dtype=torch.float16, device=dev)
-            self.side = torch.cuda.Stream(device=dev)      # default priority
-            if wl.index_offset:
-                nb = self.lib.triteia_hip_sbmm_routed_workspace_bytes(wl.tokens, wl.n_lora)
-                self.ws_lora = torch.zeros((nb + 3) // 4, dtype=torch.int32, device=dev)
+            from triteia_amd.python import capi, ops
+            self.capi, self.ops = capi, ops
+            self.lora_scratch = capi.lora_scratch(wl.tokens, self.lora_a)
+            if self.lora_scratch is None:
+                raise SystemExit("bench.py: the ldmm workloads run on the LoRA pair that routes by itself: at most 4096 tokens")
 
     def _chk(self, rc):
         if rc != 0:
@@ -112,12 +112,6 @@ class Problem:
         for idx, ws in zip(self.idx_rot, self.ws_rot):
             self._chk(self.lib.triteia_hip_route_plan(P(idx), wl.index_offset, wl.n_deltas, wl.tokens, P(ws), self.ws_bytes, 0,
                                                       self.stream()))
-
-    def plan_lora(self):
-        """Split index space: the LoRA tokens (indices below index_offset) get a plan of their own."""
-        wl, P = self.wl, self.ffi.ptr
-        self._chk(self.lib.triteia_hip_route_plan(P(self.idx), 0, wl.n_lora, wl.tokens, P(self.ws_lora), self.ws_lora.numel() * 4, 0,
-                                                  self.stream()))
 
     def delta_kernel(self, i, accumulate=0):
         """Only the dominant kernel (on an existing plan for sbmm / ldmm)."""
@@ -160,46 +154,15 @@ class Problem:
             self._chk(self.lib.triteia_hip_sbmm_2_4_routed(P(self.x), P(q), P(me), P(self.out), P(s), P(self.idx_rot[r]), 0, wl.n_deltas,
                                                            wl.m, wl.tokens, wl.k, P(self.ws_rot[r]), self.ws_bytes, 0, 0, self.stream()))
         elif wl.index_offset:
-            # ldmm on a split index space, as triteia_amd.python.ops.ldmm runs it: LoRA plan, zero and shrink beside
-            # the base GEMM; then the expand (LoRA rows) beside the routed delta multiply (delta rows)
-            r = wl.lora_rank
-            cur, side = torch.cuda.current_stream(), self.side
+            # ldmm on a split index space (a token takes an adapter or a delta): the op as a program calls it
             q, me, s = self.weights[i % self.copies]
-            side.wait_stream(cur)
-            # (the GEMM is enqueued first: recorded into a graph the other way round, the step measured 30 us longer)
+            self.ops.ldmm(self.idx, self.x, self.lora_a, self.lora_b, q, me, s, base_weight=self.base[i % self.copies])
+        else:  # ldmm: dense base GEMM (library) + LoRA pair + routed delta on one routing plan, every routed token in both
             torch.matmul(self.x, self.base[i % self.copies].t(), out=self.out)
-            with torch.cuda.stream(side):
-                self.plan_lora()
-                self._chk(self.lib.triteia_hip_sgmv_routed(P(self.v), r, P(self.x), wl.k, P(self.lora_a), wl.k * r, wl.n_lora,
-                                                           wl.k, r, 1.0, P(self.ws_lora), wl.tokens, 0, 0, self.stream()))
-            side.wait_stream(cur)
-            with torch.cuda.stream(side):
-                self._chk(self.lib.triteia_hip_sgmv_routed(P(self.out), wl.m, P(self.v), r, P(self.lora_b), r * wl.m, wl.n_lora, r,
-                                                           wl.m, 1.0, P(self.ws_lora), wl.tokens, 1, 0, self.stream()))
-            self.delta_routed(i)
-            cur.wait_stream(side)
-        else:  # ldmm: dense base GEMM (library) + routed LoRA (SGMV) + routed delta, one routing plan for both
-            r = wl.lora_rank
-            cur = torch.cuda.current_stream()
-            side = self.side if os.environ.get("BENCH_LDMM_OVERLAP", "1") == "1" else None
-            if side is not None:
-                # routing and the LoRA shrink need only x: they run beside the base GEMM, which leaves CUs idle
-                side.wait_stream(cur)
-                # (the GEMM is enqueued first: recorded into a graph the other way round, the step measured 30 us longer)
-                torch.matmul(self.x, self.base[i % self.copies].t(), out=self.out)
-                with torch.cuda.stream(side):
-                    self.plan()
-                    self._chk(self.lib.triteia_hip_sgmv_routed(P(self.v), r, P(self.x), wl.k, P(self.lora_a), wl.k * r, wl.n_lora,
-                                                               wl.k, r, 1.0, P(self.ws), wl.tokens, 0, 0, self.stream()))
-                cur.wait_stream(side)
-            else:
-                torch.matmul(self.x, self.base[i % self.copies].t(), out=self.out)
-                self.plan()
-                self._chk(self.lib.triteia_hip_sgmv_routed(P(self.v), r, P(self.x), wl.k, P(self.lora_a), wl.k * r, wl.n_lora, wl.k, r,
-                                                           1.0, P(self.ws), wl.tokens, 0, 0, self.stream()))
-            st = self.stream()
-            self._chk(self.lib.triteia_hip_sgmv_routed(P(self.out), wl.m, P(self.v), r, P(self.lora_b), r * wl.m, wl.n_lora, r, wl.m,
-                                                       1.0, P(self.ws), wl.tokens, 1, 0, st))
+            capi = self.capi
+            capi.lora_shrink(self.x, self.lora_a, self.idx, self.lora_scratch, True)
+            capi.lora_expand(self.out, self.lora_b, self.lora_scratch, wl.k, True)
+            self.plan()
             self.delta_kernel(i, accumulate=1)
 
 
@@ -441,11 +404,13 @@ def run_sweep(torch, ffi):
 
 
 def measure_lora(torch, ffi, tokens=256, adapters=32, k=4096, m=11008, rank=16, calls=20):
-    """The LoRA companions at configuration 3's shape (rank-16 adapters on 4096 x 11008, the routing of cfg3): BGMV
-    (one adapter look-up per token) and routed SGMV (tokens grouped by a routing plan), each as shrink + expand, timed
-    as `calls` pairs in one captured HIP graph.  Bytes: every distinct adapter once, activations, the rank-r
-    intermediate written and read, the output read and written."""
+    """The LoRA companions at configuration 3's shape (rank-16 adapters on 4096 x 11008, the routing of cfg3), timed as
+    `calls` calls in one captured HIP graph: the op as a program calls it (the pair of kernels that routes by itself), and
+    the pairs behind the reference's own interfaces, BGMV (one adapter look-up per token) and routed SGMV (tokens grouped
+    by a routing plan that is there already).  Bytes: every distinct adapter once, activations, the rank-r intermediate
+    written and read, the output written (by the interfaces' pairs, which add, also read)."""
     from triteia_amd import workloads as W
+    from triteia_amd.python import ops
     from triteia_amd.python.capi import add_lora_bgmv, route_plan, sgmv_routed
     dev = "cuda:0"
     g = torch.Generator(device=dev).manual_seed(77)
@@ -462,7 +427,11 @@ def measure_lora(torch, ffi, tokens=256, adapters=32, k=4096, m=11008, rank=16, 
     plan = route_plan(idx32, adapters)
     used = len(set(int(i) for i in idx_np if i >= 0))
     routed = int((idx_np >= 0).sum())
-    nbytes = used * (k * rank + rank * m) * 2 + routed * (k * 2 + 4 * rank + 4 * m)
+    weights_and_x = used * (k * rank + rank * m) * 2 + routed * k * 2
+    stored, added = weights_and_x + routed * 8 * rank + tokens * 2 * m, weights_and_x + routed * (4 * rank + 4 * m)
+
+    def op():
+        ops.lora_bgmv(A, B, x, idx32)
 
     def bgmv():
         add_lora_bgmv(y, x, A_t, B_t, idx64, 0, 1.0)
@@ -472,8 +441,9 @@ def measure_lora(torch, ffi, tokens=256, adapters=32, k=4096, m=11008, rank=16, 
         sgmv_routed(y, v, B, plan)
 
     out = []
-    for name, fn, kernels in (("lora_bgmv", bgmv, "bgmv_shrink_kernel + bgmv_expand_kernel"),
-                              ("lora_sgmv_routed", sgmv, "sgmv_shrink_kernel + sgmv_expand_vec_kernel")):
+    for name, fn, kernels, nbytes in (("lora_bgmv", op, "lora_shrink_kernel + lora_expand_kernel", stored),
+                                      ("capi.add_lora_bgmv", bgmv, "bgmv_shrink_kernel + bgmv_expand_kernel", added),
+                                      ("capi.sgmv_routed pair", sgmv, "sgmv_shrink_kernel + sgmv_expand_vec_kernel", added)):
         for _ in range(3):
             fn()
         torch.cuda.synchronize()
@@ -500,7 +470,7 @@ def measure_lora(torch, ffi, tokens=256, adapters=32, k=4096, m=11008, rank=16, 
 
 
 def host_call_us(prob, wl, torch, n=300):
-    """Host time of one `ops.sbmm_4bit_2_4_native` call (Python mirror -> ctypes -> C ABI), launches left to queue up."""
+    """Host time of one `ops.sbmm_4bit_2_4_native` call (Python mirror -> native binding -> C ABI), launches left to queue up."""
     if wl.op != "sbmm":
         return None
     from triteia_amd.python import ops
