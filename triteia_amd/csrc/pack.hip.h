@@ -13,7 +13,7 @@
 // written by the wavefront that read it.  The workgroup's eight wavefronts are eight packed rows below each other,
 // which makes the pieces of the logical metadata (row = column, stride k / 8 B) 32 B long.
 // 4096 x 4096: 6442 us as some two hundred torch kernels (4.9 ms of them a segmented sort of groups of four) -> 11.8 us
-// (3.9 TB/s; the vector ALUs and memory are about even: with comparisons by rank and the compiler's divisions 22 us).
+// (3.5 TB/s; the vector ALUs and memory are about even: with comparisons by rank and the compiler's divisions 22 us).
 #pragma once
 #include "sparse24_gemm.hip.h"
 

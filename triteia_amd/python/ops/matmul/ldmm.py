@@ -46,12 +46,12 @@ def ldmm(indices, x, LwA, LwB, DeltaW, metas, ss, base_weight=None, debug=False)
     """One routed LoRA pass (shrink + expand) for the LoRA tokens plus one routed sparse pass for
     the delta tokens, both accumulating in place into the base output; no gathers, no host
     synchronisation.  The reference routes the LoRA tokens through BGMV, which wants every
-    adapter transposed on each call (ldmm.py:93-105); the routed SGMV kernels
-    read LwA / LwB as they are, one routing pass serving both of its stages.
+    adapter transposed on each call (ldmm.py:93-105); the kernels here read LwA / LwB as they are.
 
     indices int [B]; x [B, H1]; LwA [M, H1, R]; LwB [M, R, H2]; DeltaW / metas / ss the stacked
     packed deltas.  Returns [B, H2] in x.dtype."""
-    # fp16 batches of up to 4096 tokens: one stream, the LoRA pair that routes by itself; what follows is for the others
+    # fp16 batches of up to 4096 tokens: the LoRA pair that routes by itself; what follows, with a routing plan for the
+    # LoRA tokens, is for the others
     y = native().ldmm(indices, x, LwA, LwB, DeltaW, metas, ss, base_weight)
     if y is not None:
         return y
