@@ -303,6 +303,16 @@ TRITEIA_HIP_API int triteia_hip_lora_shrink(const void* x, long x_stride, const 
 TRITEIA_HIP_API int triteia_hip_lora_expand(void* y, long y_stride, const void* b, const void* scratch, int n_tokens, int n_adapters, int k,
                             int r, int m, float scale, int accumulate, int bf16, int dev, void* stream);
 
+/* out[n_tokens, prob_m] = x[n_tokens, prob_k] @ weight[prob_m, prob_k]^T, fp16 with fp32 sums: the dense base weight of a
+ * layer (F.linear's layout) for the tokens of a routed batch.  At most 256 tokens, prob_m % 8 == 0, prob_k % 64 == 0
+ * (triteia_hip_dense_ok says whether a shape is taken); rows x_stride / w_stride elements apart, everything aligned to 16
+ * bytes; out is contiguous.  triteia_hip_dense_scratch_bytes: what the call needs for shares of K (0: nothing).
+ * The reference leaves this product to torch.matmul (triteia/python/ops/matmul/sbmm.py, ldmm.py: base_weight). */
+TRITEIA_HIP_API int triteia_hip_dense_ok(int n_tokens, int prob_m, int prob_k);
+TRITEIA_HIP_API size_t triteia_hip_dense_scratch_bytes(int n_tokens, int prob_m, int prob_k);
+TRITEIA_HIP_API int triteia_hip_dense(const void* x, long x_stride, const void* weight, long w_stride, void* out, int n_tokens, int prob_m,
+                      int prob_k, void* scratch, size_t scratch_bytes, int dev, void* stream);
+
 /* Quantise, prune and pack a dense fp16 weight [prob_k, prob_m] (row-major) with one fp16 scale per column: of every
  * aligned group of 4 along k the two entries of largest magnitude are kept (of equal ones the later), as
  * clamp(round(w / scale) + 8, 0, 15) - 8.  Writes qweight and meta in the layouts above, and meta_raw int16

@@ -104,8 +104,24 @@ bool base_ok(const Args& a, int i, const Tensor& x, int64_t k, int64_t m) {
   return a.none(i) || (a.tensor(i) && on(a[i], x, x.scalar_type(), 2) && a[i].size(0) == m && a[i].size(1) == k &&
                        !(at::autocast::is_autocast_enabled(at::kCUDA) && at::autocast::get_autocast_dtype(at::kCUDA) != x.scalar_type()));
 }
-// x [tokens, k] times the layer's dense weight, which base_ok has let pass: what the kernels add to
-Tensor base_product(const Tensor& x, const Tensor& weight) {
+// (a view that starts inside 16 bytes; a copy made by contiguous() does not)
+bool aligned(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
+
+// x [tokens, k] times the layer's dense weight, which base_ok has let pass: what the kernels add to.  A few hundred fp16 rows
+// run on the library's own kernel, everything else -- more tokens, other types, rows that are not aligned, a product that
+// autograd records -- on torch's.
+Tensor base_product(const Tensor& x, const Tensor& weight, const Place& at_) {
+  const int64_t tokens = x.size(0), k = x.size(1), m = weight.size(0);
+  const bool recorded = (at::GradMode::is_enabled() && (x.requires_grad() || weight.requires_grad())) || x._fw_grad(0).defined() || weight._fw_grad(0).defined();
+  if (x.scalar_type() == at::kHalf && !recorded && sizes_ok({tokens, k, m}) && triteia_hip_dense_ok(tokens, m, k) && x.is_contiguous() &&
+      weight.stride(1) == 1 && weight.stride(0) >= k && weight.stride(0) % 8 == 0 && aligned(x) && aligned(weight) && !x.is_neg() && !weight.is_neg()) {
+    Tensor y = at::empty({tokens, m}, x.options());
+    const size_t bytes = triteia_hip_dense_scratch_bytes(tokens, m, k);
+    const Tensor scratch = bytes ? scratch_bytes(bytes, x) : Tensor();
+    must_launch(triteia_hip_dense(x.data_ptr(), k, weight.data_ptr(), weight.stride(0), y.data_ptr(), tokens, m, k, bytes ? scratch.data_ptr() : nullptr,
+                                  bytes, at_.dev, at_.handle()));
+    return y;
+  }
   Tensor y = at::matmul(x, weight.t());
   TORCH_CHECK(y.scalar_type() == x.scalar_type() && y.is_contiguous(), "the base product is ", y.scalar_type(), ", expected a contiguous ",
               x.scalar_type());
@@ -187,13 +203,10 @@ Tensor sbmm(const Args& a) {
     y = at::empty({tokens, m}, x.options());
     return launched(routed(xc, q, meta, s, idx, y, 0, 2, at_)) ? y : Tensor();
   }
-  y = base_product(xc, a[5]);
+  y = base_product(xc, a[5], at_);
   must_launch(routed(xc, q, meta, s, idx, y, 0, 1, at_));
   return y;
 }
-
-// (a view that starts inside 16 bytes; a copy made by contiguous() does not)
-bool aligned(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
 
 // (the expand's grid has a row of workgroups per 256 columns)
 constexpr int64_t kMaxLoraColumns = 65535 * 256;
@@ -229,7 +242,7 @@ Tensor lora(const Args& a) {
   const bool base = !a.none(4);
   if (!launched(lora_shrink(xc, A, indices, scratch, base, at_.dev, at_.handle()))) return {};
   // (without a base weight every row is written by the expand: tokens without an adapter get zeros)
-  Tensor y = base ? base_product(xc, a[4]) : at::empty({x.size(0), B.size(2)}, x.options());
+  Tensor y = base ? base_product(xc, a[4], at_) : at::empty({x.size(0), B.size(2)}, x.options());
   must_launch(lora_expand(y, A, B, scratch, a.number, base, at_.dev, at_.handle()));
   return y;
 }
@@ -305,7 +318,7 @@ Tensor ldmm(const Args& a) {
     Tensor y;                  // (like the other buffers ahead of the stream: freed only after it has been joined)
     Beside side(at_);
     if (!launched(lora_shrink(xc, A, indices, scratch, true, at_.dev, side.handle()))) return {};
-    y = base_product(xc, a[7]);
+    y = base_product(xc, a[7], at_);
     side.follow();
     must_launch(lora_expand(y, A, B, scratch, 1.0, true, at_.dev, side.handle()));
     must_launch(routed(xc, q, meta, s, idx, y, A.size(0), 1, at_));
@@ -314,7 +327,7 @@ Tensor ldmm(const Args& a) {
   }
   if (!launched(lora_shrink(xc, A, indices, scratch, base, at_.dev, at_.handle()))) return {};
   // (without a base weight the expand stores the adapters' rows and zeros in all others, the deltas' among them)
-  Tensor y = base ? base_product(xc, a[7]) : at::empty({x.size(0), m}, x.options());
+  Tensor y = base ? base_product(xc, a[7], at_) : at::empty({x.size(0), m}, x.options());
   must_launch(lora_expand(y, A, B, scratch, 1.0, base, at_.dev, at_.handle()));
   must_launch(routed(xc, q, meta, s, idx, y, A.size(0), 1, at_));
   return y;

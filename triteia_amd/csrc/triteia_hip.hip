@@ -10,6 +10,7 @@
 #include <cstring>
 #include <mutex>
 
+#include "dense_base.hip.h"
 #include "lora.hip.h"
 #include "lora_mfma.hip.h"
 #include "lora_routed.hip.h"
@@ -1582,6 +1583,127 @@ int triteia_hip_lora_expand(void* y, long y_stride, const void* b, const void* s
   hipStream_t st = static_cast<hipStream_t>(stream);
   return bf16 ? lora_expand_impl<bf16_t>(y, y_stride, b, scratch, n_tokens, n_adapters, k, r, m, scale, accumulate, st)
               : lora_expand_impl<_Float16>(y, y_stride, b, scratch, n_tokens, n_adapters, k, r, m, scale, accumulate, st);
+}
+
+}  // extern "C"
+
+namespace {
+// The dense base product: which tile and how many shares of K, for at most 256 tokens.
+// A launch is as long as its busiest CU's way through its units, or as the weights' way from HBM: a CU takes in about 77 GB/s of
+// tiles and needs 0.07 us more per chunk of K for a round of the units that fit it together (its LDS), the chip reads 8.7 TB/s
+// (weights partly from the Infinity Cache); a split costs 2.4 us for its second launch and its partial sums' way there and
+// back.  The constants were fitted to 5000 measured launches (23 layers of 512 x 512 .. 13824 x 13824, 1 .. 256 tokens, every tile below,
+// 1 .. 12 shares): the choice is 0.7 % behind the best of them on average, 13 % at most, and the product 15 % ahead of the library's
+// (hipBLASLt) on those 299 shapes: 13 tokens on 11008 x 4096 29.3 -> 19.3 us, 256 tokens on 4096 x 11008 48.4 -> 37.1, on
+// 13824 x 5120 137 -> 57; 11 % behind it at worst (4096 x 4096 with 200 tokens 17.9 -> 19.9).  From 300 tokens on the library's larger
+// tiles are level or ahead (4096 x 11008 with 384 49.7 against 67).
+constexpr int kDenseMaxTokens = 256;
+struct DensePick { int tokens, features, stages, splits; };
+constexpr DensePick kDenseTiles[] = {{16, 32, 12, 0}, {16, 64, 8, 0}, {32, 32, 8, 0}, {32, 64, 6, 0}, {64, 32, 6, 0},
+                                     {64, 64, 5, 0}, {64, 96, 5, 0}, {128, 64, 6, 0}, {128, 96, 5, 0}, {128, 128, 4, 0}};
+DensePick pick_dense(int tokens, int m, int k) {
+  DensePick best{};
+  double least = 1e300;
+  const int chunks = k / 64, smallest = tokens <= 16 ? 16 : tokens <= 32 ? 32 : 64;
+  for (DensePick t : kDenseTiles) {
+    if (t.tokens < smallest || (t.tokens == 128 ? tokens <= 64 : t.tokens > smallest)) continue;
+    const long tiles = (long)((m + t.features - 1) / t.features) * ((tokens + t.tokens - 1) / t.tokens);
+    const long ring = t.stages * 128L * (t.tokens + t.features), red = t.tokens * (t.features + 4L) * 4;
+    const long together = 163840 / (ring > red ? ring : red);
+    const double chunk = ((tokens < t.tokens ? tokens : t.tokens) + t.features) * 128 / 76700.0;   // us a chunk
+    const double hbm = (2.0 * k * m + 2.0 * tokens * k * (m < 8 * t.features ? (m + t.features - 1) / t.features : 8)) / 8.7e6;
+    for (int z : {1, 2, 3, 4, 6, 8, 12}) {
+      if (z > 1 && (4 * z > chunks || tiles * z > 600)) break;
+      const long per_cu = (tiles * z + 255) / 256;
+      const double cu = (double)chunks / z * (per_cu * chunk + (per_cu + together - 1) / together * 0.066);
+      double us = cu > hbm ? cu + 0.25 * hbm : hbm + 0.25 * cu;
+      if (z > 1) us += 2.36 + 8.0 * z * tokens * m / 2.7e6;
+      if (us < least) { least = us; best = t; best.splits = z; }
+    }
+  }
+  return best;
+}
+
+// more than 64 KB of LDS has to be granted once per device and kernel
+std::mutex g_dense_mutex;
+template <int NT, int TW, int F, int FW, int STAGES>
+int launch_dense_tile(const DenseArgs& a, hipStream_t st) {
+  using Tile = DenseTile<NT, TW, F, FW, STAGES>;
+  static bool ready[kMaxDevicesForAttr] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevicesForAttr) return fail(TRITEIA_HIP_ERR_RUNTIME, "dense_base_kernel: no current device");
+  if (Tile::kLdsBytes > 65536) {
+    std::lock_guard<std::mutex> lock(g_dense_mutex);
+    if (!ready[dev]) {
+      if (hipFuncSetAttribute(reinterpret_cast<const void*>(&dense_base_kernel<NT, TW, F, FW, STAGES>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              Tile::kLdsBytes) != hipSuccess)
+        return fail(TRITEIA_HIP_ERR_RUNTIME, "dense_base_kernel: cannot reserve %d bytes of LDS", Tile::kLdsBytes);
+      ready[dev] = true;
+    }
+  }
+  const long units = (long)((a.m + Tile::kFeatures - 1) / Tile::kFeatures) * ((a.tokens + Tile::kTokens - 1) / Tile::kTokens) * a.splits;
+  hipLaunchKernelGGL((dense_base_kernel<NT, TW, F, FW, STAGES>), dim3((unsigned)((units + 7) / 8 * 8)), dim3(Tile::kThreads), Tile::kLdsBytes, st, a);
+  return check_launch("dense_base_kernel");
+}
+int launch_dense(const DenseArgs& a, const DensePick& t, hipStream_t st) {
+  if (t.tokens == 16) return t.features == 32 ? launch_dense_tile<1, 1, 1, 2, 12>(a, st) : launch_dense_tile<1, 1, 1, 4, 8>(a, st);
+  if (t.tokens == 32) return t.features == 32 ? launch_dense_tile<1, 2, 1, 2, 8>(a, st) : launch_dense_tile<2, 1, 1, 4, 6>(a, st);
+  if (t.tokens == 64)
+    return t.features == 32 ? launch_dense_tile<2, 2, 1, 2, 6>(a, st) : t.features == 64 ? launch_dense_tile<4, 1, 1, 4, 5>(a, st)
+                                                                                         : launch_dense_tile<2, 2, 3, 2, 5>(a, st);
+  return t.features == 64 ? launch_dense_tile<4, 2, 2, 2, 6>(a, st) : t.features == 96 ? launch_dense_tile<4, 2, 3, 2, 5>(a, st)
+                                                                                       : launch_dense_tile<4, 2, 4, 2, 4>(a, st);
+}
+bool dense_shape_ok(int tokens, int m, int k) {
+  return tokens > 0 && tokens <= kDenseMaxTokens && m > 0 && k > 0 && m % 8 == 0 && k % 64 == 0 && m <= (1 << 24);
+}
+}  // namespace
+
+extern "C" {
+
+int triteia_hip_dense_ok(int n_tokens, int prob_m, int prob_k) { return dense_shape_ok(n_tokens, prob_m, prob_k); }
+
+size_t triteia_hip_dense_scratch_bytes(int n_tokens, int prob_m, int prob_k) {
+  if (!dense_shape_ok(n_tokens, prob_m, prob_k)) return 0;
+  const int splits = pick_dense(n_tokens, prob_m, prob_k).splits;
+  return splits > 1 ? sizeof(float) * (size_t)splits * n_tokens * prob_m : 0;
+}
+
+int triteia_hip_dense(const void* x, long x_stride, const void* weight, long w_stride, void* out, int n_tokens, int prob_m, int prob_k,
+                      void* scratch, size_t scratch_bytes, int dev, void* stream) {
+  if (n_tokens == 0 || prob_m == 0) return TRITEIA_HIP_OK;
+  if (!dense_shape_ok(n_tokens, prob_m, prob_k))
+    return fail(TRITEIA_HIP_ERR_KERN_SHAPE, "dense: %d tokens, m=%d, k=%d need 1 .. %d tokens, m %% 8 == 0 and k %% 64 == 0", n_tokens, prob_m, prob_k,
+                kDenseMaxTokens);
+  if (!x || !weight || !out) return fail(TRITEIA_HIP_ERR_ARGUMENT, "dense: null tensor pointer");
+  if (x_stride < prob_k || w_stride < prob_k || x_stride % 8 != 0 || w_stride % 8 != 0 ||
+      (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(weight) | reinterpret_cast<uintptr_t>(out)) % 16 != 0)
+    return fail(TRITEIA_HIP_ERR_ARGUMENT, "dense: rows of at least k elements, tensors and rows aligned to 16 bytes");
+  const DensePick t = pick_dense(n_tokens, prob_m, prob_k);
+  const size_t need = t.splits > 1 ? sizeof(float) * (size_t)t.splits * n_tokens * prob_m : 0;
+  if (need && (!scratch || scratch_bytes < need || reinterpret_cast<uintptr_t>(scratch) % 16 != 0))
+    return fail(TRITEIA_HIP_ERR_ARGUMENT, "dense: scratch must hold %zu bytes (got %zu), aligned to 16", need, scratch_bytes);
+  DeviceGuard g(dev);
+  if (!g.ok) return fail(TRITEIA_HIP_ERR_RUNTIME, "cannot select device %d", dev);
+  DenseArgs a{};
+  a.x = static_cast<const _Float16*>(x);
+  a.x_stride = x_stride;
+  a.w = static_cast<const _Float16*>(weight);
+  a.w_stride = w_stride;
+  a.out = static_cast<_Float16*>(out);
+  a.out_stride = prob_m;
+  a.tokens = n_tokens;
+  a.m = prob_m;
+  a.k = prob_k;
+  a.splits = t.splits;
+  a.partial = static_cast<float*>(scratch);
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  if (int e = launch_dense(a, t, st)) return e;
+  if (t.splits == 1) return TRITEIA_HIP_OK;
+  const long pieces = (long)n_tokens * (prob_m / 8);
+  hipLaunchKernelGGL(dense_reduce_kernel, dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, st, a.partial, t.splits, n_tokens, prob_m, a.out,
+                     a.out_stride);
+  return check_launch("dense_reduce_kernel");
 }
 
 int triteia_hip_pack_2_4(const void* weight, const void* scales, void* qweight, void* meta, void* meta_raw, int prob_k, int prob_m,
