@@ -101,9 +101,9 @@ TRITEIA_HIP_API int triteia_hip_bmm_2_4_tokens_scratch(const void* A, const void
                                        void* stream);
 TRITEIA_HIP_API size_t triteia_hip_bmm_scratch_bytes(int prob_m, int batch, int tokens, int prob_k);
 
-/* Which kernel the uniform-group entry points (mul_2_4: batch = 1; bmm_2_4*) run most of a launch's rows on: 0 = the
- * K-split streaming kernel (sparse24_grouped_kernel), 16 = shares of 16, 32 or 64 columns on sparse24_share16_kernel (at most 16 tokens per
- * matrix, launches of at most 32 / 64 / 128 column blocks of 128), 1000 + n = the same with K split over n workgroups (only
+/* Which kernel the uniform-group entry points (mul_2_4: batch = 1; bmm_2_4*) run most of a launch's rows on: 0 = a
+ * kernel whose wavefronts split K over a block of 128 columns (sparse24_grouped_kernel or sparse24_ktile_kernel), 16 = shares
+ * of 16, 32 or 64 columns on sparse24_share16_kernel (at most 16 tokens per matrix, launches of at most 32 / 64 / 128 column blocks of 128), 1000 + n = the same with K split over n workgroups (only
  * with_scratch != 0), 32 / 64 = 32- / 64-token tiles of sparse24_wide_kernel (+ 1: on eight wavefronts), 256 =
  * sparse24_tile256_kernel; -1 for a shape the entry points reject.  No counterpart in the reference; for benchmarks,
  * profiles and the test that guards the dispatch thresholds. */
@@ -304,8 +304,8 @@ TRITEIA_HIP_API int triteia_hip_lora_expand(void* y, long y_stride, const void* 
                             int r, int m, float scale, int accumulate, int bf16, int dev, void* stream);
 
 /* out[n_tokens, prob_m] = x[n_tokens, prob_k] @ weight[prob_m, prob_k]^T, fp16 with fp32 sums: the dense base weight of a
- * layer (F.linear's layout) for the tokens of a routed batch.  At most 256 tokens, prob_m % 8 == 0, prob_k % 64 == 0
- * (triteia_hip_dense_ok says whether a shape is taken); rows x_stride / w_stride elements apart, everything aligned to 16
+ * layer (F.linear's layout) for the tokens of a routed batch.  At most 256 tokens, prob_m % 8 == 0, prob_k % 64 == 0,
+ * and not up to 16 tokens on less than 2^20 weights (triteia_hip_dense_ok says whether a shape is taken); rows x_stride / w_stride elements apart, everything aligned to 16
  * bytes; out is contiguous.  triteia_hip_dense_scratch_bytes: what the call needs for shares of K (0: nothing).
  * The reference leaves this product to torch.matmul (triteia/python/ops/matmul/sbmm.py, ldmm.py: base_weight). */
 TRITEIA_HIP_API int triteia_hip_dense_ok(int n_tokens, int prob_m, int prob_k);

@@ -39,7 +39,7 @@ def _check(y, x, w):
 # leave the last feature group partly empty (96 features, m a multiple of 128), and the first batch that torch takes
 @pytest.mark.parametrize("tokens,k,m", [(1, 64, 128), (16, 128, 384), (17, 4096, 256), (32, 192, 128), (33, 2048, 128), (64, 4160, 384),
                                         (65, 512, 1408), (128, 8192, 128), (129, 64, 128), (200, 1088, 3200), (256, 2048, 11008),
-                                        (13, 11008, 4096), (256, 13824, 512), (257, 256, 128)])
+                                        (13, 11008, 4096), (256, 13824, 512), (257, 256, 128), (1, 1024, 1024)])
 def test_base_product(tokens, k, m):
     x, w = _operands(tokens, k, m)
     _check(_base_only(x, w, _packed(k, m)), x, w)

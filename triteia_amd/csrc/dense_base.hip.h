@@ -8,10 +8,10 @@
 //   * a ring of chunks of 64 k in LDS, all but one of them in flight.  One barrier a chunk, behind which the stage read in the
 //     chunk before is requested anew, request by request between the MFMAs (in one burst the wavefronts stand at the
 //     address unit's queue with their MFMAs behind it);
-//   * the two halves of a chunk belong to two sets of wavefronts with sums of their own: fewer operand reads per MFMA than
-//     with the tile cut in smaller pieces.  The halves meet in LDS at the end, from where whole rows go out;
-//   * feature groups start their walk over K spread around its chunks: rows of W lie a power of two apart, and in lockstep
-//     all workgroups would read the same few channels (13 tokens on 11008 x 4096 20.4 -> 19.1 us, on 8192 x 8192 28.2 -> 22.9);
+//   * one set of sums per result, added to in the order of K (where the walk starts at the first chunk): the bits of a plain MFMA
+//     product.  (Two sets of wavefronts on the halves of a chunk need fewer operand reads and measured the same.)
+//   * feature groups may start their walk over K spread around its chunks: rows of W lie a power of two apart, and in
+//     lockstep all workgroups read the same few channels (13 tokens on 8192 x 8192 31.6 -> 27.8 us);
 //   * K split over workgroups where a layer has too few tiles; a second launch adds the shares in order.
 #pragma once
 #include "sparse24_gemm.hip.h"
@@ -27,14 +27,15 @@ struct DenseArgs {
   long out_stride;
   int tokens, m, k;       // k a multiple of 64, m of 8
   int splits;             // shares of K over workgroups; 1: the result goes to `out`
+  int rotate;             // 1: feature groups start their walks over K spread around its chunks, 0: at the first
   float* partial;         // [splits][tokens][m] fp32 sums (splits > 1)
 };
 
-// NT x F: 16-token by 16-feature tiles of a wavefront; TW x FW wavefronts side by side in each half of a chunk.
+// NT x F: 16-token by 16-feature tiles of a wavefront; TW x FW wavefronts side by side.
 template <int NT, int TW, int F, int FW, int STAGES>
 struct DenseTile {
   static constexpr int kTokens = 16 * NT * TW, kFeatures = 16 * F * FW;
-  static constexpr int kWaves = 2 * TW * FW, kThreads = 64 * kWaves;
+  static constexpr int kWaves = TW * FW, kThreads = 64 * kWaves;
   static constexpr int kStageBytes = 128 * (kTokens + kFeatures);
   static constexpr int kRedStride = kFeatures + 4;
   static constexpr int kRedBytes = kTokens * kRedStride * 4;
@@ -42,7 +43,7 @@ struct DenseTile {
 };
 
 template <int NT, int TW, int F, int FW, int STAGES>
-__global__ __launch_bounds__(128 * TW * FW) void dense_base_kernel(const DenseArgs p) {
+__global__ __launch_bounds__(64 * TW * FW) void dense_base_kernel(const DenseArgs p) {
   using Tile = DenseTile<NT, TW, F, FW, STAGES>;
   constexpr int TT = Tile::kTokens, FF = Tile::kFeatures, WAVES = Tile::kWaves;
   constexpr int kXLoads = (TT / 8 + WAVES - 1) / WAVES, kWLoads = (FF / 8 + WAVES - 1) / WAVES;
@@ -52,7 +53,7 @@ __global__ __launch_bounds__(128 * TW * FW) void dense_base_kernel(const DenseAr
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, q = lane >> 4;
-  const int half = wave / (TW * FW), tw = (wave / FW) % TW, fw = wave % FW;
+  const int tw = wave / FW, fw = wave % FW;
 
   // Units in the order (feature group, share of K, token tile), token tiles fastest; an XCD (workgroup u runs on XCD u % 8)
   // takes a run of them: the token tiles of a feature group read its weights through one L2.
@@ -65,7 +66,7 @@ __global__ __launch_bounds__(128 * TW * FW) void dense_base_kernel(const DenseAr
   const int t0 = tt * TT, f0 = fg * FF;
   const int chunks = p.k >> 6;                   // (splits <= chunks: every share has one)
   const int c0 = (int)((long)z * chunks / p.splits), n = (int)((long)(z + 1) * chunks / p.splits) - c0;
-  const int rot = (int)((long)fg * n / groups);
+  const int rot = p.rotate ? (int)((long)fg * n / groups) : 0;
 
   // A request: 8 rows x 128 bytes; lane l takes 16 bytes of row l / 8, the piece (l % 8) ^ (l / 8) to position l % 8.
   // (rows past the end repeat the last one: their sums are not stored)
@@ -93,30 +94,33 @@ __global__ __launch_bounds__(128 * TW * FW) void dense_base_kernel(const DenseAr
   for (int f = 0; f < F; f++)
 #pragma unroll
     for (int t = 0; t < NT; t++) acc[f][t] = float4_t{0.f, 0.f, 0.f, 0.f};
-  const int piece = ((4 * half + q) ^ (r & 7)) * 16;
-  const uint32_t xrow = (16 * NT * tw + r) * 128 + piece;
-  const uint32_t wrow = 128 * TT + (16 * F * fw + r) * 128 + piece;
+  const int piece = (q ^ (r & 7)) * 16;                    // (of the chunk's second half: ^ 64)
+  const uint32_t xrow = (16 * NT * tw + r) * 128;
+  const uint32_t wrow = 128 * TT + (16 * F * fw + r) * 128;
   auto compute = [&](int stage, auto&& request) {
     const unsigned char* s = smem + stage * Tile::kStageBytes;
-    half8_t x[NT], w[F];
+    half8_t x[2][NT], w[2][F];
 #pragma unroll
-    for (int t = 0; t < NT; t++) x[t] = *reinterpret_cast<const half8_t*>(s + xrow + 2048 * t);
+    for (int h = 0; h < 2; h++) {
 #pragma unroll
-    for (int f = 0; f < F; f++) w[f] = *reinterpret_cast<const half8_t*>(s + wrow + 2048 * f);
+      for (int t = 0; t < NT; t++) x[h][t] = *reinterpret_cast<const half8_t*>(s + xrow + (piece ^ (64 * h)) + 2048 * t);
+#pragma unroll
+      for (int f = 0; f < F; f++) w[h][f] = *reinterpret_cast<const half8_t*>(s + wrow + (piece ^ (64 * h)) + 2048 * f);
+    }
     __builtin_amdgcn_sched_barrier(0);
-    constexpr int kGroup = (F * NT + kLoads - 1) / kLoads;
+    constexpr int kMfmas = 2 * F * NT, kGroup = (kMfmas + kLoads - 1) / kLoads;
 #pragma unroll
-    for (int e = 0; e < F * NT; e++) {
-      const int f = e / NT, t = e - f * NT;
-      acc[f][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[f], x[t], acc[f][t], 0, 0, 0);
-      if ((e + 1) % kGroup == 0 || e + 1 == F * NT) {
+    for (int e = 0; e < kMfmas; e++) {
+      const int h = e / (F * NT), f = e % (F * NT) / NT, t = e % NT;
+      acc[f][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[h][f], x[h][t], acc[f][t], 0, 0, 0);
+      if ((e + 1) % kGroup == 0 || e + 1 == kMfmas) {
         __builtin_amdgcn_sched_barrier(0);
         request(e / kGroup);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
 #pragma unroll
-    for (int i = (F * NT + kGroup - 1) / kGroup; i < kLoads; i++) request(i);
+    for (int i = (kMfmas + kGroup - 1) / kGroup; i < kLoads; i++) request(i);
   };
 
   for (int c = 0; c < AHEAD && c < n; c++)
@@ -141,31 +145,15 @@ __global__ __launch_bounds__(128 * TW * FW) void dense_base_kernel(const DenseAr
     stage = stage + 1 == STAGES ? 0 : stage + 1;
   }
 
-  // the halves' sums meet in LDS, from where whole rows go out
+  // through LDS, from where whole rows go out
   __syncthreads();
   float* red = reinterpret_cast<float*>(smem);
   // D: lane (token r, q) holds features 4q .. 4q + 3 of a tile
   float* mine = red + (16 * NT * tw + r) * Tile::kRedStride + 16 * F * fw + 4 * q;
-  if (half == 1) {
 #pragma unroll
-    for (int t = 0; t < NT; t++)
+  for (int t = 0; t < NT; t++)
 #pragma unroll
-      for (int f = 0; f < F; f++) *reinterpret_cast<float4_t*>(mine + 16 * t * Tile::kRedStride + 16 * f) = acc[f][t];
-  }
-  __syncthreads();
-  if (half == 0) {
-#pragma unroll
-    for (int t = 0; t < NT; t++)
-#pragma unroll
-      for (int f = 0; f < F; f++) {
-        float4_t* e = reinterpret_cast<float4_t*>(mine + 16 * t * Tile::kRedStride + 16 * f);
-        const float4_t o = *e;
-        float4_t s = acc[f][t];
-#pragma unroll
-        for (int i = 0; i < 4; i++) s[i] += o[i];
-        *e = s;
-      }
-  }
+    for (int f = 0; f < F; f++) *reinterpret_cast<float4_t*>(mine + 16 * t * Tile::kRedStride + 16 * f) = acc[f][t];
   __syncthreads();
   constexpr int kPieces = FF / 8;
   for (int e = tid; e < TT * kPieces; e += Tile::kThreads) {

@@ -17,6 +17,7 @@
 #include "pack.hip.h"
 #include "route_plan.hip.h"
 #include "sparse24_gemm.hip.h"
+#include "sparse24_ktile.hip.h"
 #include "sparse24_share.hip.h"
 #include "sparse24_tile256.hip.h"
 #include "sparse24_wide.hip.h"
@@ -64,7 +65,7 @@ struct Knobs {
   int wide32_min_units = kUnset, wide32_max_units = kUnset, wide32_ksplit_max_units = kUnset, wide64_ksplit_max_units = kUnset;
   int mid = 1, mid64_max_k = 0x7fffffff, mid_min_column_groups = 16, mid_min_units = kUnset, mid_min_half_tokens = 7, mid_narrow = 1, mid_depth = 0, plan_big = 1, plan_all64 = 1, lora_mfma = 1;
   int eager = 1, fused_route = 1;
-  int tile256 = 1, tile256_min_units = kUnset, tile256_max_units = kUnset, ksplit = 1, sub_shift = kUnset, share16 = 1, share16_max_blocks = kUnset;
+  int ktile = 1, tile256 = 1, tile256_min_units = kUnset, tile256_max_units = kUnset, ksplit = 1, sub_shift = kUnset, share16 = 1, share16_max_blocks = kUnset;
 };
 Knobs g_knobs;
 std::once_flag g_knobs_once;
@@ -79,7 +80,7 @@ void read_knobs() {
       {"WIDE32_KSPLIT_MAX_UNITS", &k.wide32_ksplit_max_units}, {"WIDE64_KSPLIT_MAX_UNITS", &k.wide64_ksplit_max_units},
       {"MID", &k.mid}, {"MID64_MAX_K", &k.mid64_max_k}, {"MID_MIN_COLUMN_GROUPS", &k.mid_min_column_groups},
       {"MID_MIN_UNITS", &k.mid_min_units}, {"MID_MIN_HALF_TOKENS", &k.mid_min_half_tokens}, {"MID_NARROW", &k.mid_narrow}, {"MID_DEPTH", &k.mid_depth}, {"PLAN_BIG", &k.plan_big}, {"PLAN_ALL64", &k.plan_all64}, {"LORA_MFMA", &k.lora_mfma}, {"EAGER", &k.eager}, {"FUSED_ROUTE", &k.fused_route},
-      {"TILE256", &k.tile256}, {"TILE256_MIN_UNITS", &k.tile256_min_units}, {"TILE256_MAX_UNITS", &k.tile256_max_units},
+      {"KTILE", &k.ktile}, {"TILE256", &k.tile256}, {"TILE256_MIN_UNITS", &k.tile256_min_units}, {"TILE256_MAX_UNITS", &k.tile256_max_units},
       {"KSPLIT", &k.ksplit}, {"SUB_SHIFT", &k.sub_shift}, {"SHARE16", &k.share16}, {"SHARE16_MAX_BLOCKS", &k.share16_max_blocks},
   };
   char name[64];
@@ -548,6 +549,104 @@ int pick_ksplit(long tokens, long n_groups, int m, int k) {
   return ks < 2 ? 1 : (int)ks;
 }
 
+// ---- tiles whose wavefronts split K (sparse24_ktile_kernel)
+struct KTilePick { int nt, kw, splits; };
+// Which uniform launches they take.
+//  * From 17 tokens on, while the 64-token x 128-column tiles are at most 768 (1.5 rounds of two workgroups per CU), 384 from 800
+//    tokens on: past that the wide kernels' shared activation tiles win (8192 x 8192 with 768 / 1024 tokens 75.9 -> 70.9 / 83.9 -> 96.2 us,
+//    4096 x 11008 with 512 / 1024 44.9 -> 38.5 / 71.1 -> 76.2; 4096 x 4096 and 11008 x 4096 with 1024 31.4 -> 30.8, 68.3 -> 70.1, 11008 x 4096
+//    with 900 61.0 -> 65.2; 4096 x 2048 with 1280 32.1 -> 27.4).  Small layers whose 16-token passes make the streaming kernel about
+//    a workgroup per CU stay with it (4096 x 4096 with 96 / 128 9.8 -> 10.0, 9.9 -> 10.1, 4096 x 2048 with 192 9.8 -> 10.1).  Launches of less than 4M weights and 600 tokens stay with the streaming kernel, whose
+//    eight wavefronts a column block start with less ahead of their first request (1024 x 1024 with 17 .. 512 tokens 5.5 - 6.0 -> 6.2 - 6.4
+//    us, with 640 8.1 -> 6.9).
+//  * Below, several matrices of up to 256 column blocks in all at a time: from 12 tokens on (4 of 2048 x 2048 with 16 8.4 -> 6.4, 4 of
+//    11008 x 4096 24.3 -> 17.3; 8 of 4096 x 11008, which stay, 32.5 -> 36.3 with 13), but for 33 .. 64 column blocks of k = 4096 .. 8191, the column shares' best ground (2 of 4096 x 4096 with 12 8.4 -> 9.2);
+//    with fewer where a long K leaves the column shares several rounds (2 of 13824 x 5120 with one 20.0 -> 15.1), elsewhere it is even
+//    or behind (8 of 4096 x 4096 with one 11.3 -> 11.5, 21 of 2048 x 2048 with three 9.5 -> 9.9).  A single matrix of 16 tokens and
+//    fewer stays with the column shares and the K split.
+bool ktile_takes(long tokens, long n_groups, int m, int k, bool x_aligned) {
+  const Knobs& kn = knobs();
+  // (a knob that asks for another kernel gets it)
+  if (!kn.ktile || kn.nt || kn.ksplit != 1 || kn.sub_shift != kUnset || kn.share16 != 1 || kn.wide != 1 || kn.wide_min_units != kUnset ||
+      kn.wide32_min_units != kUnset || kn.tile256 != 1 || kn.tile256_min_units != kUnset)
+    return false;
+  if (k % 128 != 0 || !x_aligned || tokens <= 0) return false;
+  const long blocks = n_groups * (m / 128);
+  if (tokens >= 17) {
+    if (tokens < 600 && n_groups * k * m < (1L << 22)) return false;
+    const long passes = blocks * ((tokens + 15) / 16);
+    if (k <= 4096 && m <= 4096 && passes > 128 && passes <= 256) return false;
+    // (several matrices of 25 .. 32 tokens that fill the wide kernel's 32-token tiles and about all CUs with eight wavefronts each: 8 of 4096 x
+    // 11008 with 32 36.1 -> 36.9, with 20 40.1 -> 34.4)
+    const long units32 = n_groups * ((m / 128 + 3) / 4);
+    if (n_groups > 1 && tokens > 24 && tokens <= 32 && units32 >= kWide32MinUnits && units32 <= kWide32KSplitMaxUnits) return false;
+    return blocks * ((tokens + 63) / 64) <= (tokens < 800 ? 768 : 384);
+  }
+  if (n_groups < 2 || blocks > 256) return false;
+  if (tokens >= 12) return !(blocks > 32 && blocks <= 64 && k >= 4096 && k < 8192);
+  return k >= 8192 && blocks > 64;
+}
+// Which tile and how many shares of K: the least of an estimate in us.  A step costs a wavefront's SIMD 0.12 for the weights' conversion
+// and 0.05 per 16 tokens for the products, and the CU 4 KB per 16 tokens and 7 for the weights at 75 GB/s; wavefronts of a tile hide
+// behind each other two to a SIMD; the sums' way through LDS takes 0.25 per wavefront and 16 tokens; a split costs 2.95 for its second launch and
+// its partial sums' way there and back.  Fitted to 4000 measured launches (28 layers and groups of them): 0.5 % behind the
+// best tile and split on average.
+KTilePick pick_ktile(long tokens, long n_groups, int m, int k, bool split) {
+  constexpr KTilePick kTiles[] = {{1, 8, 1}, {1, 4, 1}, {2, 4, 1}, {3, 4, 1}, {4, 4, 1}};
+  const long steps = k / 128;
+  KTilePick best{};
+  double least = 1e300;
+  for (KTilePick t : kTiles) {
+    if (t.nt > 1 && tokens <= 16 * (t.nt - (t.nt > 2 ? 2 : 1))) continue;
+    if (t.nt == 1 && tokens > 64) continue;
+    const long tiles = n_groups * (m / 128) * ((tokens + 16 * t.nt - 1) / (16 * t.nt));
+    for (int z : {1, 2, 3, 4, 6, 8, 11, 16}) {
+      if (z > 1 && (!split || tiles * z > 600 || steps < 4 * z)) break;
+      const double per_cu = (double)((tiles * z + 255) / 256), slots = 8 / t.kw, together = per_cu < slots ? per_cu : slots;
+      const long mine = ((steps + z - 1) / z + t.kw - 1) / t.kw;                 // steps of the longest wavefront
+      const double step = 0.052 * t.nt + 0.122, sharing = together * t.kw / 4;
+      const double rounds = (double)(((long)per_cu + (long)slots - 1) / (long)slots);
+      const double chain = rounds * (mine * (step * sharing > step + 0.1 ? step * sharing : step + 0.1) + 0.25 * t.nt * t.kw * together);
+      const double intake = per_cu * steps / z * (4 * t.nt + 7) / 75.0;
+      double us = 3.9 + (chain > intake ? chain : intake);
+      if (z > 1) us += 2.95 + 8.0 * z * tokens * n_groups * m / 2.3e6;
+      if (us < least) { least = us; best = t; best.splits = z; }
+    }
+  }
+  return best;
+}
+template <int NT, int KW>
+int launch_ktile_as(const Sparse24Args& a, int splits, hipStream_t st) {
+  using Tile = KTile<NT, KW>;
+  static_assert(Tile::kLdsBytes <= 65536 || KW == 8, "");
+  const long units = (long)a.n_groups * (a.m / 128) * splits * ((a.uniform_count + Tile::kTokens - 1) / Tile::kTokens);
+  if (units > 0x7ffffff0L) return fail(TRITEIA_HIP_ERR_PROB_SHAPE, "too many work units (%ld)", units);
+  if (Tile::kLdsBytes > 65536) {
+    // more than 64 KB of LDS has to be granted once per device
+    static bool ready[kMaxDevicesForAttr] = {};
+    static std::mutex mutex;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevicesForAttr)
+      return fail(TRITEIA_HIP_ERR_RUNTIME, "sparse24_ktile_kernel: no current device");
+    std::lock_guard<std::mutex> lock(mutex);
+    if (!ready[dev]) {
+      if (hipFuncSetAttribute(reinterpret_cast<const void*>(&sparse24_ktile_kernel<NT, KW>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              Tile::kLdsBytes) != hipSuccess)
+        return fail(TRITEIA_HIP_ERR_RUNTIME, "sparse24_ktile_kernel: cannot reserve %d bytes of LDS", Tile::kLdsBytes);
+      ready[dev] = true;
+    }
+  }
+  hipLaunchKernelGGL((sparse24_ktile_kernel<NT, KW>), dim3((unsigned)((units + 7) / 8 * 8)), dim3(64 * KW), Tile::kLdsBytes, st, a, splits);
+  return check_launch("sparse24_ktile_kernel");
+}
+int launch_ktile(const Sparse24Args& a, const KTilePick& t, hipStream_t st) {
+  if (t.kw == 8) return launch_ktile_as<1, 8>(a, t.splits, st);
+  if (t.nt == 1) return launch_ktile_as<1, 4>(a, t.splits, st);
+  if (t.nt == 2) return launch_ktile_as<2, 4>(a, t.splits, st);
+  if (t.nt == 3) return launch_ktile_as<3, 4>(a, t.splits, st);
+  return launch_ktile_as<4, 4>(a, t.splits, st);
+}
+
 UniformPlan decide_uniform(int tokens, int stride, int n_groups, int m, int k, long x_stride, bool have_scratch) {
   UniformPlan up;
   auto add = [&](int kind, int first, int count, int ksplit = 1) { up.seg[up.n++] = UniformSegment{kind, first, count, ksplit}; };
@@ -633,9 +732,12 @@ UniformPlan decide_uniform(int tokens, int stride, int n_groups, int m, int k, l
 }
 
 // bytes of fp32 partial sums that a K split of this launch writes (0: the launch is not split)
+size_t split_bytes(int splits, int tokens, int n_groups, int m) {
+  return splits > 1 ? sizeof(float) * (size_t)splits * (size_t)n_groups * (size_t)tokens * (size_t)m : 0;
+}
 size_t uniform_scratch_bytes(int tokens, int n_groups, int m, int k) {
-  const int ks = pick_ksplit(tokens, n_groups, m, k);
-  return ks > 1 ? sizeof(float) * (size_t)ks * (size_t)n_groups * (size_t)tokens * (size_t)m : 0;
+  return split_bytes(ktile_takes(tokens, n_groups, m, k, true) ? pick_ktile(tokens, n_groups, m, k, true).splits : pick_ksplit(tokens, n_groups, m, k),
+                     tokens, n_groups, m);
 }
 
 int launch_uniform(Sparse24Args a, int tokens, int stride, int delta_step, int n_groups, hipStream_t st,
@@ -643,9 +745,31 @@ int launch_uniform(Sparse24Args a, int tokens, int stride, int delta_step, int n
   a.n_groups = n_groups;
   a.uniform_stride = stride;
   a.delta_step = delta_step;
-  const bool have_scratch = scratch && stride == tokens && reinterpret_cast<uintptr_t>(scratch) % 16 == 0 &&
-                            scratch_bytes >= uniform_scratch_bytes(tokens, n_groups, a.m, a.k) &&
-                            uniform_scratch_bytes(tokens, n_groups, a.m, a.k) > 0;
+  // whether the caller's scratch takes the partial sums of so many shares of K
+  auto scratch_for = [&](int splits) {
+    return splits > 1 && scratch && stride == tokens && reinterpret_cast<uintptr_t>(scratch) % 16 == 0 &&
+           scratch_bytes >= split_bytes(splits, tokens, n_groups, a.m);
+  };
+  auto reduce = [&](const Sparse24Args& b, int splits) {
+    const long chunks = b.partial_rows * (a.m / 8);
+    hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st, b.partial, splits, b.partial_rows, a.m,
+                       a.scales, a.scales_stride, tokens, delta_step, a.out, a.out_stride);
+    return check_launch("splitk_reduce_kernel");
+  };
+  if (!a.accumulate && ktile_takes(tokens, n_groups, a.m, a.k, reinterpret_cast<uintptr_t>(a.x) % 16 == 0 && a.x_stride % 8 == 0)) {
+    KTilePick t = pick_ktile(tokens, n_groups, a.m, a.k, true);
+    if (t.splits > 1 && !scratch_for(t.splits)) t = pick_ktile(tokens, n_groups, a.m, a.k, false);
+    Sparse24Args b = a;
+    b.uniform_first = 0;
+    b.uniform_count = tokens;
+    if (t.splits > 1) {
+      b.partial = static_cast<float*>(scratch);
+      b.partial_rows = (long)n_groups * tokens;
+    }
+    if (int e = launch_ktile(b, t, st)) return e;
+    return t.splits > 1 ? reduce(b, t.splits) : TRITEIA_HIP_OK;
+  }
+  const bool have_scratch = scratch_for(pick_ksplit(tokens, n_groups, a.m, a.k));
   const UniformPlan up = decide_uniform(tokens, stride, n_groups, a.m, a.k, a.x_stride, have_scratch);
   for (int i = 0; i < up.n; i++) {
     const UniformSegment& sg = up.seg[i];
@@ -665,10 +789,7 @@ int launch_uniform(Sparse24Args a, int tokens, int stride, int delta_step, int n
       const int nt = sg.count <= 16 ? 1 : pick_nt_uniform(sg.count, n_groups, a.m / 128);
       e = launch_sparse24(b, nt, (sg.count + 16 * nt - 1) / (16 * nt), st, splits);
       if (e) return e;
-      const long chunks = b.partial_rows * (a.m / 8);
-      hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st, b.partial, splits,
-                         b.partial_rows, a.m, a.scales, a.scales_stride, tokens, delta_step, a.out, a.out_stride);
-      e = check_launch("splitk_reduce_kernel");
+      e = reduce(b, splits);
     } else {
       const int nt = pick_nt_uniform(sg.count, n_groups, a.m / 128);
       e = launch_sparse24(a, nt, (sg.count + 16 * nt - 1) / (16 * nt), st);
@@ -763,6 +884,10 @@ size_t triteia_hip_bmm_scratch_bytes(int prob_m, int batch, int tokens, int prob
 
 int triteia_hip_uniform_kernel(int prob_m, int batch, int tokens, int prob_k, int with_scratch) {
   if (prob_m <= 0 || batch <= 0 || tokens <= 0 || prob_k <= 0 || prob_m % 128 != 0 || prob_k % 64 != 0) return -1;
+  if (ktile_takes(tokens, batch, prob_m, prob_k, true)) {
+    const int splits = pick_ktile(tokens, batch, prob_m, prob_k, with_scratch != 0).splits;
+    return splits > 1 ? kUniSplitK + splits : 0;
+  }
   const bool sc = with_scratch && uniform_scratch_bytes(tokens, batch, prob_m, prob_k) > 0;
   const UniformPlan up = decide_uniform(tokens, tokens, batch, prob_m, prob_k, prob_k, sc);
   if (up.n == 0) return -1;
@@ -1647,14 +1772,17 @@ int launch_dense_tile(const DenseArgs& a, hipStream_t st) {
 }
 int launch_dense(const DenseArgs& a, const DensePick& t, hipStream_t st) {
   if (t.tokens == 16) return t.features == 32 ? launch_dense_tile<1, 1, 1, 2, 12>(a, st) : launch_dense_tile<1, 1, 1, 4, 8>(a, st);
-  if (t.tokens == 32) return t.features == 32 ? launch_dense_tile<1, 2, 1, 2, 8>(a, st) : launch_dense_tile<2, 1, 1, 4, 6>(a, st);
+  if (t.tokens == 32) return t.features == 32 ? launch_dense_tile<1, 2, 1, 2, 8>(a, st) : launch_dense_tile<1, 2, 1, 4, 6>(a, st);
   if (t.tokens == 64)
-    return t.features == 32 ? launch_dense_tile<2, 2, 1, 2, 6>(a, st) : t.features == 64 ? launch_dense_tile<4, 1, 1, 4, 5>(a, st)
-                                                                                         : launch_dense_tile<2, 2, 3, 2, 5>(a, st);
-  return t.features == 64 ? launch_dense_tile<4, 2, 2, 2, 6>(a, st) : t.features == 96 ? launch_dense_tile<4, 2, 3, 2, 5>(a, st)
-                                                                                       : launch_dense_tile<4, 2, 4, 2, 4>(a, st);
+    return t.features == 32 ? launch_dense_tile<1, 4, 1, 2, 6>(a, st) : t.features == 64 ? launch_dense_tile<2, 2, 1, 4, 5>(a, st)
+                                                                                         : launch_dense_tile<1, 4, 3, 2, 5>(a, st);
+  return t.features == 64 ? launch_dense_tile<2, 4, 2, 2, 6>(a, st) : t.features == 96 ? launch_dense_tile<2, 4, 3, 2, 5>(a, st)
+                                                                                       : launch_dense_tile<2, 4, 4, 2, 4>(a, st);
 }
+// (Up to 16 tokens on a layer of less than a million weights stay with the library: its kernel for them sums K in another order, and the
+// rows of a batch that have no delta keep its bits as they always have; there is a microsecond to win, 512 x 512 4.0 against 3.5.)
 bool dense_shape_ok(int tokens, int m, int k) {
+  if (tokens <= 16 && (long)m * k < (1L << 20)) return false;
   return tokens > 0 && tokens <= kDenseMaxTokens && m > 0 && k > 0 && m % 8 == 0 && k % 64 == 0 && m <= (1 << 24);
 }
 }  // namespace
@@ -1695,6 +1823,11 @@ int triteia_hip_dense(const void* x, long x_stride, const void* weight, long w_s
   a.tokens = n_tokens;
   a.m = prob_m;
   a.k = prob_k;
+  // Feature groups start their walks over K apart (DenseArgs::rotate) where the weight's way from HBM is what a launch takes, or where a
+  // split changes the order of the sums anyway (64 tokens on 4096 x 11008 27.0 -> 24.6 us, 128 on 8192 x 8192 43.4 -> 37.6, 13 31.6 -> 27.8).
+  // An unsplit launch of more tokens gains 0 - 6 % from it and walks K in order instead, as the library's own product does: the
+  // same bits on most layers, and the same for a row whatever batch it is in.
+  a.rotate = (t.splits > 1 || n_tokens <= 64) && (long)prob_k * prob_m >= (1L << 24);
   a.splits = t.splits;
   a.partial = static_cast<float*>(scratch);
   const hipStream_t st = static_cast<hipStream_t>(stream);
