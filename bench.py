@@ -228,6 +228,9 @@ def kernel_name(wl, lib, in_kernel):
         return "sparse24_grouped_kernel (routes in-kernel)"
     if wl.index_offset:
         return "sparse24_grouped_kernel"
+    kt = lib.triteia_hip_planned_ktile(wl.tokens, wl.n_deltas, wl.m, wl.k)
+    if kt:
+        return f"sparse24_ktile_plan_kernel<up to {kt} tokens a tile>"
     tk = lib.triteia_hip_planned_tile_kernel(wl.tokens, wl.n_deltas, wl.m, wl.k)
     if tk:
         return f"sparse24_wide_kernel<{tk}-token plan tiles>"

@@ -141,10 +141,10 @@ TRITEIA_HIP_API int triteia_hip_sbmm_2_4_bounded(const void* A, const void* B, c
  * token_indices: int32 [prob_n] on the device, any order.  The tokens are
  * grouped on the device, so each delta's weights are read once per launch.
  * workspace: >= triteia_hip_sbmm_routed_workspace_bytes(prob_n, n_deltas) bytes
- * of device memory, contents irrelevant on entry, overwritten (batches of at most 64
- * tokens over at most 64 deltas are always routed inside the multiply kernel and leave it
- * untouched; so are most batches of up to 256 tokens over at most 16 deltas, but not all:
- * pass the workspace for every batch above 64 tokens).
+ * of device memory, contents irrelevant on entry, overwritten (a batch that
+ * triteia_hip_routed_in_kernel answers 1 or 2 for is routed inside the multiply kernel and leaves it
+ * untouched; of the others, up to 256 tokens over at most 16 deltas and most batches of up to 64 tokens
+ * over at most 64 run without one too, more slowly).
  * n_deltas <= 8192. */
 TRITEIA_HIP_API int triteia_hip_sbmm_2_4_routed(const void* A, const void* B, const void* meta, void* C, const void* s,
                                 const void* token_indices, int index_offset, int n_deltas, int prob_m, int prob_n,
@@ -200,8 +200,11 @@ TRITEIA_HIP_API int triteia_hip_plan_tile_tokens(int prob_n, int n_deltas);
  * wide kernel taking the plan's narrow-only list, or its list of 64-token tiles where the narrow tiles are of 32
  * (wide layers; see the design notes).  No counterpart in
  * the reference; for benchmarks and profiles, and for tests that compare results bit for bit (the two
- * kernels add over K in different orders). */
+ * kernels add over K in different orders).  triteia_hip_planned_ktile, where it is not 0, comes first. */
 TRITEIA_HIP_API int triteia_hip_planned_tile_kernel(int prob_n, int n_deltas, int prob_m, int prob_k);
+/* 16, 32 or 64 if triteia_hip_sbmm_2_4_planned runs this batch and layer on sparse24_ktile_plan_kernel, in tiles of up to
+ * that many tokens (activations aligned to 16 bytes; its sums are sparse24_grouped_kernel's to the bit), 0 if not. */
+TRITEIA_HIP_API int triteia_hip_planned_ktile(int prob_n, int n_deltas, int prob_m, int prob_k);
 
 /* The order in which sparse24_wide_kernel numbers its units (token tile x group of 512 columns) on a layer of prob_m
  * columns (1: column groups padded to a multiple of 8, a contiguous run per XCD; 3: the same with the padding's idle
@@ -216,7 +219,8 @@ TRITEIA_HIP_API long triteia_hip_wide_block_grid_units(long rows, int prob_m, in
 
 /* 1 or 2 if triteia_hip_sbmm_2_4_routed handles this batch and layer in one launch, routing inside the multiply kernel
  * (the workspace stays untouched; 2: at most 16 tokens on the column-share kernel, sparse24_share16_kernel, 1: the
- * streaming kernel), 0 if it builds a routing plan first.  No counterpart in the reference; for
+ * streaming kernel), 0 if it builds a routing plan first (one that it could route in the kernel it still does when the
+ * workspace is null, too small or not aligned).  No counterpart in the reference; for
  * benchmarks and profiles. */
 TRITEIA_HIP_API int triteia_hip_routed_in_kernel(int prob_n, int n_deltas, int prob_m, int prob_k);
 

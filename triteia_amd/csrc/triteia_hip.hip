@@ -65,7 +65,7 @@ struct Knobs {
   int wide32_min_units = kUnset, wide32_max_units = kUnset, wide32_ksplit_max_units = kUnset, wide64_ksplit_max_units = kUnset;
   int mid = 1, mid64_max_k = 0x7fffffff, mid_min_column_groups = 16, mid_min_units = kUnset, mid_min_half_tokens = 7, mid_narrow = 1, mid_depth = 0, plan_big = 1, plan_all64 = 1, lora_mfma = 1;
   int eager = 1, fused_route = 1;
-  int ktile = 1, tile256 = 1, tile256_min_units = kUnset, tile256_max_units = kUnset, ksplit = 1, sub_shift = kUnset, share16 = 1, share16_max_blocks = kUnset;
+  int plan_ktile = 1, ktile = 1, tile256 = 1, tile256_min_units = kUnset, tile256_max_units = kUnset, ksplit = 1, sub_shift = kUnset, share16 = 1, share16_max_blocks = kUnset;
 };
 Knobs g_knobs;
 std::once_flag g_knobs_once;
@@ -80,7 +80,7 @@ void read_knobs() {
       {"WIDE32_KSPLIT_MAX_UNITS", &k.wide32_ksplit_max_units}, {"WIDE64_KSPLIT_MAX_UNITS", &k.wide64_ksplit_max_units},
       {"MID", &k.mid}, {"MID64_MAX_K", &k.mid64_max_k}, {"MID_MIN_COLUMN_GROUPS", &k.mid_min_column_groups},
       {"MID_MIN_UNITS", &k.mid_min_units}, {"MID_MIN_HALF_TOKENS", &k.mid_min_half_tokens}, {"MID_NARROW", &k.mid_narrow}, {"MID_DEPTH", &k.mid_depth}, {"PLAN_BIG", &k.plan_big}, {"PLAN_ALL64", &k.plan_all64}, {"LORA_MFMA", &k.lora_mfma}, {"EAGER", &k.eager}, {"FUSED_ROUTE", &k.fused_route},
-      {"KTILE", &k.ktile}, {"TILE256", &k.tile256}, {"TILE256_MIN_UNITS", &k.tile256_min_units}, {"TILE256_MAX_UNITS", &k.tile256_max_units},
+      {"KTILE", &k.ktile}, {"PLAN_KTILE", &k.plan_ktile}, {"TILE256", &k.tile256}, {"TILE256_MIN_UNITS", &k.tile256_min_units}, {"TILE256_MAX_UNITS", &k.tile256_max_units},
       {"KSPLIT", &k.ksplit}, {"SUB_SHIFT", &k.sub_shift}, {"SHARE16", &k.share16}, {"SHARE16_MAX_BLOCKS", &k.share16_max_blocks},
   };
   char name[64];
@@ -165,6 +165,16 @@ static int share16_tiles(long n_groups, int m, int tokens_per_group) {
   if (blocks > knob_or(knobs().share16_max_blocks, kShare16MaxBlocks)) return 0;
   return blocks <= 32 ? 1 : blocks <= 64 ? 2 : 4;
 }
+// About 512 workgroups run at a time.  When those belong to four or more deltas (narrow matrices),
+// the deltas start their walks over K spread evenly around the ring of steps; wide matrices are
+// streamed one or two at a time anyway and walk from step 0.
+// (counted in whole column blocks, whatever the share a workgroup takes: the start of a delta's walk fixes the order
+// of its fp32 sums, which must not depend on the share)
+static int rot_spread(int m, int k) {
+  const long side_by_side = 512 / (((long)(m / 128) + 7) / 8 * 8);
+  const int n_steps = (k / 32 + 3) / 4;
+  return side_by_side >= 4 ? n_steps / (int)(side_by_side < 16 ? side_by_side : 16) : 0;
+}
 int launch_sparse24(Sparse24Args a, int nt, long tsplit, hipStream_t st, int zsplit = 1) {
   if (a.n_groups <= 0 || a.m == 0 || a.k == 0) return TRITEIA_HIP_OK;
   if (tsplit < 1) tsplit = 1;
@@ -213,17 +223,7 @@ int launch_sparse24(Sparse24Args a, int nt, long tsplit, hipStream_t st, int zsp
   }
   const bool small = live_groups * cb_pad * tsplit * zsplit <= 256.5;
   const int depth = eager || kw == 8 ? 1 : (nt == 2 || (nt == 1 && small) ? 2 : 1);
-  // About 512 workgroups run at a time.  When those belong to four or more deltas (narrow matrices),
-  // the deltas start their walks over K spread evenly around the ring of steps; wide matrices are
-  // streamed one or two at a time anyway and walk from step 0.
-  // (counted in whole column blocks, whatever the share a workgroup takes: the start of a delta's walk fixes the order
-  // of its fp32 sums, which must not depend on the share)
-  {
-    const long side_by_side = 512 / (((long)(a.m / 128) + 7) / 8 * 8);
-    const int n_steps = (a.k / 32 + 3) / 4;
-    const long spread = side_by_side >= 4 ? n_steps / (side_by_side < 16 ? side_by_side : 16) : 0;
-    a.rot_spread = (int)spread;
-  }
+  a.rot_spread = rot_spread(a.m, a.k);
   if (const int tiles = uniform && nt == 1 && tsplit == 1 && zsplit == 1 && !a.ksplit_steps ? share16_tiles(a.n_groups, a.m, a.uniform_count) : 0) {
     const long sh_pad = ((long)(a.m / (16 * tiles)) + 7) / 8 * 8;
     const dim3 grid((unsigned)(a.n_groups * sh_pad));
@@ -615,27 +615,29 @@ KTilePick pick_ktile(long tokens, long n_groups, int m, int k, bool split) {
   }
   return best;
 }
+// More than 64 KB of LDS has to be granted to a kernel once per device.
+template <auto Kernel>
+int grant_lds(int bytes, const char* name) {
+  if (bytes <= 65536) return TRITEIA_HIP_OK;
+  static bool ready[kMaxDevicesForAttr] = {};
+  static std::mutex mutex;
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevicesForAttr) return fail(TRITEIA_HIP_ERR_RUNTIME, "%s: no current device", name);
+  std::lock_guard<std::mutex> lock(mutex);
+  if (!ready[dev]) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(Kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess)
+      return fail(TRITEIA_HIP_ERR_RUNTIME, "%s: cannot reserve %d bytes of LDS", name, bytes);
+    ready[dev] = true;
+  }
+  return TRITEIA_HIP_OK;
+}
 template <int NT, int KW>
 int launch_ktile_as(const Sparse24Args& a, int splits, hipStream_t st) {
   using Tile = KTile<NT, KW>;
   static_assert(Tile::kLdsBytes <= 65536 || KW == 8, "");
   const long units = (long)a.n_groups * (a.m / 128) * splits * ((a.uniform_count + Tile::kTokens - 1) / Tile::kTokens);
   if (units > 0x7ffffff0L) return fail(TRITEIA_HIP_ERR_PROB_SHAPE, "too many work units (%ld)", units);
-  if (Tile::kLdsBytes > 65536) {
-    // more than 64 KB of LDS has to be granted once per device
-    static bool ready[kMaxDevicesForAttr] = {};
-    static std::mutex mutex;
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevicesForAttr)
-      return fail(TRITEIA_HIP_ERR_RUNTIME, "sparse24_ktile_kernel: no current device");
-    std::lock_guard<std::mutex> lock(mutex);
-    if (!ready[dev]) {
-      if (hipFuncSetAttribute(reinterpret_cast<const void*>(&sparse24_ktile_kernel<NT, KW>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                              Tile::kLdsBytes) != hipSuccess)
-        return fail(TRITEIA_HIP_ERR_RUNTIME, "sparse24_ktile_kernel: cannot reserve %d bytes of LDS", Tile::kLdsBytes);
-      ready[dev] = true;
-    }
-  }
+  if (int e = grant_lds<sparse24_ktile_kernel<NT, KW>>(Tile::kLdsBytes, "sparse24_ktile_kernel")) return e;
   hipLaunchKernelGGL((sparse24_ktile_kernel<NT, KW>), dim3((unsigned)((units + 7) / 8 * 8)), dim3(64 * KW), Tile::kLdsBytes, st, a, splits);
   return check_launch("sparse24_ktile_kernel");
 }
@@ -645,6 +647,14 @@ int launch_ktile(const Sparse24Args& a, const KTilePick& t, hipStream_t st) {
   if (t.nt == 2) return launch_ktile_as<2, 4>(a, t.splits, st);
   if (t.nt == 3) return launch_ktile_as<3, 4>(a, t.splits, st);
   return launch_ktile_as<4, 4>(a, t.splits, st);
+}
+
+template <int MAXNT>
+int launch_ktile_plan_tile(const Sparse24Args& a, unsigned grid, hipStream_t st) {
+  static_assert(ktile_plan_lds<MAXNT>() <= 80 * 1024, "two workgroups per CU");
+  if (int e = grant_lds<sparse24_ktile_plan_kernel<MAXNT>>(ktile_plan_lds<MAXNT>(), "sparse24_ktile_plan_kernel")) return e;
+  hipLaunchKernelGGL((sparse24_ktile_plan_kernel<MAXNT>), dim3(grid), dim3(64 * kKTilePlanWaves), ktile_plan_lds<MAXNT>(), st, a);
+  return check_launch("sparse24_ktile_plan_kernel");
 }
 
 UniformPlan decide_uniform(int tokens, int stride, int n_groups, int m, int k, long x_stride, bool have_scratch) {
@@ -1103,6 +1113,57 @@ static bool mid_big(int prob_n, int n_deltas, int prob_m, int prob_k) {
          (knobs().plan_big > 1 || prob_n >= kMidBigMinTokensPerDelta * groups || mid_units32(prob_n, n_deltas, prob_m, 32) >= kMidBigManyUnits) &&
          mid_tiles(prob_n, n_deltas, prob_m, prob_k) && !mid_deep(prob_n, n_deltas, prob_m, 32);
 }
+// ---- a plan's tiles on the kernel whose wavefronts split K (sparse24_ktile_plan_kernel)
+// Its 64-token list where there is one and the 32-token tiles would be more than about one round of the 512 workgroups that run
+// together (measured list against list on 2700 random batches: up to 170 units of 64 tokens the 32-token tiles are 5 - 30 %
+// ahead, past 1650 units of 32 tokens the 64-token ones 4 - 19 %).
+constexpr long kKTileBigMinUnits32 = 600;
+static bool ktile_plan_big(int prob_n, int n_deltas, int prob_m) {
+  const long groups = n_deltas < prob_n ? n_deltas : prob_n;
+  return plan_has_big(prob_n, n_deltas) && (prob_n + 16 * groups) * (prob_m / 128) / 32 > kKTileBigMinUnits32;
+}
+// (a knob that asks for another kernel of a routed batch gets it; plan_ktile = 2: wherever the kernel can)
+static bool routed_knobs_unset() {
+  const Knobs& kn = knobs();
+  return !kn.nt && !kn.pass_nt && kn.wide == 1 && kn.wide_min_batch == 256 && kn.plan_wide_min_units == kUnset && kn.mid == 1 &&
+         kn.mid64_max_k == 0x7fffffff && kn.mid_min_column_groups == 16 && kn.mid_min_units == kUnset && kn.mid_min_half_tokens == 7 &&
+         kn.mid_narrow == 1 && !kn.mid_depth && kn.plan_big == 1 && kn.plan_all64 == 1 && kn.xcd_cgs == 0 && kn.xcd_swizzle == 1 &&
+         kn.wide_order_min_idle == kUnset && kn.eager == 1 && kn.fused_route == 1;
+}
+static bool ktile_plan_can(int prob_n, int prob_k) {
+  // (whole 128-deep K steps; 32-bit byte offsets of rows of activations)
+  return prob_k % 128 == 0 && (long)prob_n * prob_k * 2 < (1L << 32);
+}
+// Which planned batches it takes: all that would go to the streaming kernel (2164 random ones, k and m 512 .. 13824, 20 .. 4096 tokens over
+// 2 .. 64 deltas, evenly routed and Zipf: geometric mean 0.82 of its time, worst 1.10; 20 deltas of 3840 x 1152 with 1861 tokens
+// 73 -> 31 us, 5 of 11008 x 4096 with 279 63 -> 36, 32 of 4096 x 4096 with 513 53.5 -> 48), and of those for the wide kernels the ones of
+// few 64-token tiles, the deeper K the more (1027 random ones: 0.76 of the time, 17 of them more than 3 % slower, worst 1.23):
+// up to 256 units of 64 tokens x 128 columns any (0.42 - 0.80: half the CUs had no workgroup), up to one round of 512 from
+// k = 1280 on (0.71 - 0.91), two rounds from k = 2560 on (0.81 - 0.93), three from k = 4500 on (0.91).  Past that, with fewer
+// than 32 tokens a delta and on short K the wide kernels' shared activation tiles and fewer workgroups are ahead (the other 1626:
+// 1.03, up to 1.57; 4096 x 11008 with 2048 tokens over 4 deltas 134 -> 152 us).
+static bool ktile_plan_takes(int prob_n, int n_deltas, int prob_m, int prob_k) {
+  if (!knobs().plan_ktile || !ktile_plan_can(prob_n, prob_k)) return false;
+  if (knobs().plan_ktile == 2) return true;
+  if (!routed_knobs_unset()) return false;
+  if (!mid_tiles(prob_n, n_deltas, prob_m, prob_k)) return true;
+  const long groups = n_deltas < prob_n ? n_deltas : prob_n;
+  const long units = (prob_n + 32 * groups) * (prob_m / 128) / 64;   // tokens / 64 and half a tile per delta, as a randomly routed batch leaves them
+  if (units <= 256) return true;
+  if (prob_n < 32 * groups) return false;
+  return (units <= 512 && prob_k >= 1280) || (units <= 1024 && prob_k >= 2560) || (units <= 1536 && prob_k >= 4500 && prob_n >= 64 * groups);
+}
+// Batches that the multiply kernel could route by itself and that are better off with a plan on this kernel: the streaming kernel re-reads
+// activations in operand order, 16 rows x 64 bytes at a time, at 37 GB/s a CU, so a delta's tokens cost it time in proportion to
+// tokens x k; the plan is a launch of 4 - 5 us.  From 200K activations per delta on it pays whatever the layer (304 random
+// batches: 0.79 of the time, 7 more than 3 % slower, worst 1.13; 16 deltas of 13056 x 1408 with 219 tokens 63 -> 30 us, 5 of 13824 x 5120
+// with 80 51 -> 32), from 80K on where the launch is also more than a round of workgroups long (34: 0.85, worst 1.00);
+// below (16 deltas of 4096 x 4096 with 64 tokens, 16K) routing in the kernel stays ahead by the plan's launch.
+static bool ktile_plan_beats_in_kernel(int prob_n, int n_deltas, int prob_m, int prob_k) {
+  if (prob_k < 3500 || knobs().plan_ktile != 1 || !ktile_plan_takes(prob_n, n_deltas, prob_m, prob_k)) return false;
+  const long groups = n_deltas < prob_n ? n_deltas : prob_n, work = (long)prob_n * prob_k;
+  return work >= 200 * 1024 * groups || (work >= 80 * 1024 * groups && (prob_n + 16 * groups) * (prob_m / 128) / 32 >= kKTileBigMinUnits32);
+}
 int triteia_hip_wide_unit_order(int prob_m) { return prob_m >= 128 ? wide_unit_order(prob_m) : 0; }
 long triteia_hip_wide_grid_units(long rows, int prob_m, int order) {
   if (rows <= 0 || prob_m < 128) return 0;
@@ -1119,9 +1180,15 @@ int triteia_hip_planned_tile_kernel(int prob_n, int n_deltas, int prob_m, int pr
   return mid_tiles(prob_n, n_deltas, prob_m, prob_k) ? triteia_hip_plan_tile_tokens(prob_n, n_deltas) : 0;
 }
 
+int triteia_hip_planned_ktile(int prob_n, int n_deltas, int prob_m, int prob_k) {
+  if (prob_n <= 0 || n_deltas <= 0 || prob_m <= 0 || prob_k <= 0) return 0;
+  if (!ktile_plan_takes(prob_n, n_deltas, prob_m, prob_k)) return 0;
+  return ktile_plan_big(prob_n, n_deltas, prob_m) ? 64 : triteia_hip_plan_tile_tokens(prob_n, n_deltas);
+}
+
 int triteia_hip_routed_in_kernel(int prob_n, int n_deltas, int prob_m, int prob_k) {
   if (prob_n <= 0 || n_deltas <= 0 || prob_m <= 0 || prob_k <= 0) return 0;
-  if (!routed_in_kernel(prob_n, n_deltas, prob_m, prob_k)) return 0;
+  if (!routed_in_kernel(prob_n, n_deltas, prob_m, prob_k) || ktile_plan_beats_in_kernel(prob_n, n_deltas, prob_m, prob_k)) return 0;
   // (the launch that sbmm_2_4_routed makes of it: route first unless there are two tokens per delta; 16-token passes)
   const bool shares = prob_n <= 16 && !routed_eager_ok(prob_n, n_deltas) && pick_nt(prob_n, prob_n < n_deltas ? prob_n : n_deltas) == 1 &&
                       share16_tiles(prob_n < n_deltas ? prob_n : n_deltas, prob_m, prob_n);
@@ -1154,6 +1221,28 @@ int triteia_hip_route_plan(const void* token_indices, int index_offset, int n_de
   return route_plan_impl(token_indices, index_offset, n_deltas, prob_n, workspace, workspace_bytes, dev, stream, nullptr, 0);
 }
 
+static int launch_ktile_plan(Sparse24Args a, int prob_n, int n_deltas, const int* ws, const PlanLayout& L, hipStream_t st) {
+  const int tile = triteia_hip_plan_tile_tokens(prob_n, n_deltas);
+  const bool big = ktile_plan_big(prob_n, n_deltas, a.m);
+  if (big) {
+    a.tiles = reinterpret_cast<const int4*>(ws + L.big);
+    a.n_groups_dev = ws + L.header + 6;
+    a.n_groups = L.max_big;
+  } else if (plan_has_wide(prob_n, n_deltas)) {
+    a.tiles = reinterpret_cast<const int4*>(ws + L.all);
+    a.n_groups_dev = ws + L.header + 5;
+  }
+  a.rot_spread = rot_spread(a.m, a.k);
+  // Column blocks in 2, 4 or 8 parts over the XCDs.  More parts: every XCD the same tiles, whatever the routing left in them, but
+  // parts of few, uneven column blocks that each read all activations (of 8 against 4: up to 21 column blocks 0 - 20 % slower; from
+  // 44 on 1 - 4 % faster, under a skewed routing up to 25 %; of 2 against 4, below 29 column blocks 0 - 17 % faster).
+  const long blocks = a.m / 128;
+  a.xcd_cgs = blocks < 29 ? 2 : blocks < 45 ? 4 : 8;
+  const long runs = 8 / a.xcd_cgs, width = (blocks + a.xcd_cgs - 1) / a.xcd_cgs;
+  const long grid = 8 * ((width * a.n_groups + runs - 1) / runs);
+  if (grid * 256 > 0x7fffffffL) return fail(TRITEIA_HIP_ERR_PROB_SHAPE, "too many work units");
+  return big || tile == 64 ? launch_ktile_plan_tile<4>(a, (unsigned)grid, st) : launch_ktile_plan_tile<2>(a, (unsigned)grid, st);
+}
 int triteia_hip_sbmm_2_4_planned(const void* A, const void* B, const void* meta, void* C, const void* s,
                                  const void* plan, int n_deltas, int prob_m, int prob_n, int prob_k, int accumulate,
                                  int dev, void* stream) {
@@ -1213,6 +1302,8 @@ int triteia_hip_sbmm_2_4_planned(const void* A, const void* B, const void* meta,
   // re-read that way come from cache) until there is a workgroup per CU.  Measured on 4096 x 4096: one
   // delta with 64 / 128 tokens 24.4 -> 12.7 / 24.2 -> 18.8 us, two deltas with 256 tokens 24.6 -> 18.5 us;
   // launches of 250 workgroups and more lose 10 % that way and keep the plan's tile.
+  if (reinterpret_cast<uintptr_t>(B) % 16 == 0 && ktile_plan_takes(prob_n, n_deltas, prob_m, prob_k))
+    return launch_ktile_plan(a, prob_n, n_deltas, ws, L, static_cast<hipStream_t>(stream));
   int pass_nt = tile / 16;
   {
     const long cb_pad = (prob_m / 128 + 7) / 8 * 8;
@@ -1265,10 +1356,8 @@ int triteia_hip_sbmm_2_4_planned(const void* A, const void* B, const void* meta,
   return TRITEIA_HIP_OK;
 }
 
-int triteia_hip_sbmm_2_4_routed(const void* A, const void* B, const void* meta, void* C, const void* s,
-                                const void* token_indices, int index_offset, int n_deltas, int prob_m, int prob_n,
-                                int prob_k, void* workspace, size_t workspace_bytes, int accumulate, int dev,
-                                void* stream) {
+static int sbmm_routed(const void* A, const void* B, const void* meta, void* C, const void* s, const void* token_indices, int index_offset, int n_deltas, int prob_m, int prob_n,
+                                int prob_k, void* workspace, size_t workspace_bytes, int accumulate, int dev, void* stream, bool own_workspace) {
   if (int e = check_gemm_shape(prob_m, prob_n, prob_k, -1)) return e;
   if (accumulate < 0 || accumulate > 2) return fail(TRITEIA_HIP_ERR_ARGUMENT, "sbmm_2_4_routed: accumulate=%d", accumulate);
   if (n_deltas < 0) return fail(TRITEIA_HIP_ERR_PROB_SHAPE, "sbmm_2_4_routed: deltas=%d", n_deltas);
@@ -1284,8 +1373,13 @@ int triteia_hip_sbmm_2_4_routed(const void* A, const void* B, const void* meta, 
   // plan pays from 128 tokens on whatever the number of deltas, the plan launch being small against the kernel
   // and the wide kernels taking hot deltas: 8 / 4 deltas of 8192 x 28672 with 128 / 256 tokens 145 -> 130 /
   // 160 -> 122 us, while 8 or 16 deltas of 4096 x 11008 stay 8-12 % faster routed inside the kernel)
+  // (a batch of this size that comes without a workspace for the plan, or with activations that the plan's kernel for it cannot
+  // take, is routed in the kernel all the same, and so are all of them on the library's own scratch, whose plan is one for all streams)
   const bool eager_ok = routed_eager_ok(prob_n, n_deltas);
-  if (routed_in_kernel(prob_n, n_deltas, prob_m, prob_k)) {
+  const bool plan_better = own_workspace && workspace && workspace_bytes >= triteia_hip_sbmm_routed_workspace_bytes(prob_n, n_deltas) &&
+                           (reinterpret_cast<uintptr_t>(workspace) | reinterpret_cast<uintptr_t>(B)) % 16 == 0 &&
+                           ktile_plan_beats_in_kernel(prob_n, n_deltas, prob_m, prob_k);
+  if (routed_in_kernel(prob_n, n_deltas, prob_m, prob_k) && !plan_better) {
     // small batch: the multiply kernel routes by itself, no plan, no workspace traffic
     if (!token_indices) return fail(TRITEIA_HIP_ERR_ARGUMENT, "sbmm_2_4_routed: null indices");
     DeviceGuard g(dev);
@@ -1322,6 +1416,13 @@ int triteia_hip_sbmm_2_4_routed(const void* A, const void* B, const void* meta, 
     return e;
   return triteia_hip_sbmm_2_4_planned(A, B, meta, C, s, workspace, n_deltas, prob_m, prob_n, prob_k, accumulate == 1, dev, stream);
 }
+int triteia_hip_sbmm_2_4_routed(const void* A, const void* B, const void* meta, void* C, const void* s,
+                                const void* token_indices, int index_offset, int n_deltas, int prob_m, int prob_n,
+                                int prob_k, void* workspace, size_t workspace_bytes, int accumulate, int dev,
+                                void* stream) {
+  return sbmm_routed(A, B, meta, C, s, token_indices, index_offset, n_deltas, prob_m, prob_n, prob_k, workspace, workspace_bytes, accumulate, dev,
+                     stream, true);
+}
 
 size_t triteia_hip_sbmm_routed_static_max_bytes(void) { return kStaticPlanBytes; }
 
@@ -1341,8 +1442,8 @@ int triteia_hip_sbmm_2_4_routed_static(const void* A, const void* B, const void*
   void* plan = nullptr;
   if (int e = static_plan_address(&plan)) return e;
   // (the plan kernel writes every word of the plan that the multiply kernels read: nothing to clear)
-  return triteia_hip_sbmm_2_4_routed(A, B, meta, C, s, token_indices, index_offset, n_deltas, prob_m, prob_n, prob_k, plan,
-                                     kStaticPlanBytes, accumulate, -1, stream);
+  return sbmm_routed(A, B, meta, C, s, token_indices, index_offset, n_deltas, prob_m, prob_n, prob_k, plan, kStaticPlanBytes, accumulate, -1, stream,
+                     false);
 }
 
 }  // extern "C"

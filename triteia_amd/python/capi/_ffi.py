@@ -39,6 +39,7 @@ SIGNATURES = {
     "triteia_hip_plan_tile_tokens": (_c_int, [_c_int, _c_int]),
     "triteia_hip_routed_in_kernel": (_c_int, [_c_int, _c_int, _c_int, _c_int]),
     "triteia_hip_planned_tile_kernel": (_c_int, [_c_int, _c_int, _c_int, _c_int]),
+    "triteia_hip_planned_ktile": (_c_int, [_c_int, _c_int, _c_int, _c_int]),
     "triteia_hip_wide_unit_order": (_c_int, [_c_int]),
     "triteia_hip_wide_grid_units": (ctypes.c_long, [ctypes.c_long, _c_int, _c_int]),
     "triteia_hip_wide_block_grid_units": (ctypes.c_long, [ctypes.c_long, _c_int, _c_int]),
