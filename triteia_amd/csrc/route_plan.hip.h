@@ -122,81 +122,61 @@ __global__ __launch_bounds__(kPlanThreads) void route_plan_kernel(const int* __r
   }
   __syncthreads();
 
-  if (wave == 0) {
-    // exclusive scans over the deltas, 64 per iteration: token counts -> first slot in perm,
-    // tile counts -> first tile
-    int running = 0, tiles = 0, wides = 0, alls = 0, bigs = 0, groups = 0;
-    int4* tile_out = reinterpret_cast<int4*>(ws + L.tiles);
-    int4* wide_out = reinterpret_cast<int4*>(ws + L.wide);
-    int4* all_out = reinterpret_cast<int4*>(ws + L.all);
-    int4* big_out = reinterpret_cast<int4*>(ws + L.big);
-    for (int base = 0; base < n_deltas; base += 64) {
-      const int d = base + lane;
-      int c = 0;
-      if (d < n_deltas)
-        for (int w = 0; w < shares; w++) c += s_cursor[w * n_deltas + d];
-      int chunk_tokens, chunk_tiles, chunk_wides, chunk_alls;
-      const int offs = running + wave_excl_scan(c, lane, &chunk_tokens);
-      // split this delta's tokens: wide tiles first, the rest in narrow tiles
-      int nw = 0, c_wide = 0;
-      if (wide) {
-        nw = c / kPlanWideTile;
-        c_wide = nw * kPlanWideTile;
-        if (c - c_wide >= kPlanWideMinRest) { nw++; c_wide = c; }
-      }
-      const int c_rest = c - c_wide;
-      const int nt = (c_rest + tile - 1) / tile;
-      const int wpos = wides + wave_excl_scan(nw, lane, &chunk_wides);
-      const int tpos = tiles + wave_excl_scan(nt, lane, &chunk_tiles);
-      for (int i = 0; i < nw; i++) {
-        const int first = i * kPlanWideTile;
-        wide_out[wpos + i] = make_int4(d, offs + first, min(kPlanWideTile, c_wide - first), 0);
-      }
-      for (int i = 0; i < nt; i++) {
-        const int first = i * tile;
-        tile_out[tpos + i] = make_int4(d, offs + c_wide + first, min(tile, c_rest - first), 0);
-      }
-      if (wide) {
-        const int na = (c + tile - 1) / tile;
-        const int apos = alls + wave_excl_scan(na, lane, &chunk_alls);
-        for (int i = 0; i < na; i++) {
-          const int first = i * tile;
-          all_out[apos + i] = make_int4(d, offs + first, min(tile, c - first), 0);
-        }
-        alls += chunk_alls;
-      }
-      if (big) {
-        int chunk_bigs;
-        const int nb = (c + kPlanWideTile - 1) / kPlanWideTile;
-        const int bpos = bigs + wave_excl_scan(nb, lane, &chunk_bigs);
-        for (int i = 0; i < nb; i++) {
-          const int first = i * kPlanWideTile;
-          big_out[bpos + i] = make_int4(d, offs + first, min(kPlanWideTile, c - first), 0);
-        }
-        bigs += chunk_bigs;
-      }
+  // Exclusive scans over the deltas, 64 per iteration: token counts -> first slot in perm, tile counts -> first tile.  A chain of
+  // LDS reads and lane exchanges, so wavefronts 0 .. 3 each make one list of tiles and wavefront 4 the cursors, side by side
+  // (one wavefront doing all in turn: 1000 / 2048 / 4096 tokens over 32 / 8 / 500 deltas 5.3 -> 4.3, 5.5 -> 4.6, 19.3 -> 14.9 us in a
+  // graph, 256 tokens 3.9 -> 3.6; 72 and 128 tokens, with one or two shares, 3.2 -> 3.3).
+  int running = 0, entries = 0, groups = 0;
+  int4* const list = reinterpret_cast<int4*>(ws + (wave == 0 ? L.tiles : wave == 1 ? L.wide : wave == 2 ? L.all : L.big));
+  const int list_tile = wave == 1 || wave == 3 ? kPlanWideTile : tile;
+  const bool listed = wave == 0 || (wave <= 2 && wide) || (wave == 3 && big);
+  for (int base = 0; base < n_deltas; base += 64) {
+    const int d = base + lane;
+    int c = 0;
+    if (wave < 5 && d < n_deltas) {
+#pragma unroll 4
+      for (int w = 0; w < shares; w++) c += s_cursor[w * n_deltas + d];
+    }
+    __syncthreads();                           // (wavefront 4 overwrites the counts)
+    if (wave >= 5) continue;
+    int chunk_tokens;
+    const int offs = running + wave_excl_scan(c, lane, &chunk_tokens);
+    running += chunk_tokens;
+    if (wave == 4) {
+      // the shares' pieces of this delta's run of slots, in the order of the shares
+      int before = offs;
       if (d < n_deltas) {
-        // the shares' pieces of this delta's run of slots, in the order of the shares
-        int before = 0;
+#pragma unroll 4
         for (int w = 0; w < shares; w++) {
           const int mine = s_cursor[w * n_deltas + d];
-          s_cursor[w * n_deltas + d] = offs + before;
+          s_cursor[w * n_deltas + d] = before;
           before += mine;
         }
       }
-      running += chunk_tokens;
-      tiles += chunk_tiles;
-      wides += chunk_wides;
       groups += __popcll(__ballot(c > 0));
+    } else if (listed) {
+      // with wide tiles the narrow list has what they leave of a delta: a rest of up to 32 tokens
+      const int rest = c % kPlanWideTile, c_wide = !wide ? 0 : (rest >= kPlanWideMinRest ? c : c - rest);
+      const int skip = wave == 0 ? c_wide : 0, len = wave == 0 ? c - c_wide : wave == 1 ? c_wide : c;
+      const int n = (len + list_tile - 1) / list_tile;
+      int chunk;
+      const int pos = entries + wave_excl_scan(n, lane, &chunk);
+      for (int i = 0; i < n; i++) {
+        const int first = i * list_tile;
+        list[pos + i] = make_int4(d, offs + skip + first, min(list_tile, len - first), 0);
+      }
+      entries += chunk;
     }
-    if (lane == 0) {
-      ws[L.header + 0] = tiles;
+  }
+  if (lane == 0) {
+    if (wave == 0) ws[L.header + 0] = entries;
+    if (wave == 1) ws[L.header + 4] = entries;
+    if (wave == 2) ws[L.header + 5] = entries;
+    if (wave == 3) ws[L.header + 6] = entries;
+    if (wave == 4) {
       ws[L.header + 1] = running;
       ws[L.header + 2] = groups;
       ws[L.header + 3] = tile;
-      ws[L.header + 4] = wides;
-      ws[L.header + 5] = alls;
-      ws[L.header + 6] = bigs;
       ws[L.header + 7] = 0;
     }
   }
