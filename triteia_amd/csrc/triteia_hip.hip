@@ -565,6 +565,7 @@ struct KTilePick { int nt, kw, splits; };
 //    or behind (8 of 4096 x 4096 with one 11.3 -> 11.5, 21 of 2048 x 2048 with three 9.5 -> 9.9).  A single matrix of 16 tokens and
 //    fewer stays with the column shares and the K split.
 bool ktile_takes(long tokens, long n_groups, int m, int k, bool x_aligned) {
+  if (tokens < 12 && (n_groups < 2 || k < 8192)) return false;   // (the smallest calls are bound by the host)
   const Knobs& kn = knobs();
   // (a knob that asks for another kernel gets it)
   if (!kn.ktile || kn.nt || kn.ksplit != 1 || kn.sub_shift != kUnset || kn.share16 != 1 || kn.wide != 1 || kn.wide_min_units != kUnset ||
