@@ -218,8 +218,8 @@ def kernel_name(wl, lib, in_kernel):
         groups, per_group = (1, wl.tokens) if wl.op == "matmul" else (wl.n_deltas, max(1, wl.tokens // max(1, wl.n_deltas)))
         code = lib.triteia_hip_uniform_kernel(wl.m, groups, per_group, wl.k, 1)
         if code >= 1000:
-            return f"sparse24_grouped_kernel (K split over {code - 1000} workgroups) + splitk_reduce_kernel"
-        return {0: "sparse24_grouped_kernel", 16: "sparse24_share16_kernel", 32: "sparse24_wide_kernel<32 tokens>", 33: "sparse24_wide_kernel<32 tokens, 8 wavefronts>",
+            return f"sparse24_ktile_kernel or sparse24_grouped_kernel (K split over {code - 1000} workgroups) + splitk_reduce_kernel"
+        return {0: "sparse24_ktile_kernel or sparse24_grouped_kernel", 16: "sparse24_share16_kernel", 32: "sparse24_wide_kernel<32 tokens>", 33: "sparse24_wide_kernel<32 tokens, 8 wavefronts>",
                 64: "sparse24_wide_kernel<64 tokens>", 65: "sparse24_wide_kernel<64 tokens, 8 wavefronts>",
                 256: "sparse24_tile256_kernel"}.get(code, f"kernel code {code}")
     if in_kernel:
