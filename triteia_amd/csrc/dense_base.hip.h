@@ -86,7 +86,7 @@ __global__ __launch_bounds__(64 * TW * FW) void dense_base_kernel(const DenseArg
   auto issue = [&](int i, int c, int stage) {
     const uint32_t d = __builtin_amdgcn_readfirstlane(dst[i] + stage * Tile::kStageBytes);
     const _Float16* s = src[i] + (long)(c + rot < n ? c + rot : c + rot - n) * 64;
-    asm volatile("global_load_lds_dwordx4 %0, off" : : "v"(s), "{m0}"(d) : "memory");
+    direct_load(s, d);
   };
 
   float4_t acc[F][NT];

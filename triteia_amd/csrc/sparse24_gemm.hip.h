@@ -179,6 +179,18 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// 16 bytes per lane from global memory straight to LDS at `lds` (uniform) + 16 * lane: from `base` (uniform) + `off` bytes, or from
+// each lane's own `src`.  Written as inline assembly: the compiler counts a direct load as an LDS write and would drain every
+// outstanding request at the next barrier or LDS read, so the callers wait by hand.  M0, which holds the LDS address, is an input
+// operand, so the compiler writes it and knows it is live; the s_nop is the one wait state that a scalar write of M0 needs ahead of such a
+// request, which the compiler adds by itself only in front of instructions that it knows.
+__device__ __forceinline__ void direct_load(uint32_t off, const void* base, uint32_t lds) {
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "{m0}"(lds) : "memory");
+}
+__device__ __forceinline__ void direct_load(const void* src, uint32_t lds) {
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "{m0}"(lds) : "memory");
+}
+
 template <int NT>
 struct StepFrag {
   uint4_t wq[4];        // weights: groups a and a+4 (a = vector index) of 8 columns

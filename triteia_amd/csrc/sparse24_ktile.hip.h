@@ -85,7 +85,7 @@ __device__ __forceinline__ void ktile_run(const Sparse24Args& p, unsigned char* 
       const _Float16* base = PLAN ? x0 : x0 + (long)tile_start(j >> 2) * p.x_stride;
       const uint32_t off = PLAN ? rows[j & 3] + (x_lane ^ (64 * (j & 3))) : xoff[j & 3];
       const uint32_t d = __builtin_amdgcn_readfirstlane(lds_x + 1024 * j);
-      asm volatile("global_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "{m0}"(d) : "memory");
+      direct_load(off, base, d);
     }
   };
 

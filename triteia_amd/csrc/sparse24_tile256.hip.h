@@ -156,11 +156,11 @@ __global__ __launch_bounds__(512, 1) void sparse24_tile256_kernel(const Sparse24
     if (i < 4) {
       const _Float16* xb = p.x + phys(tx) * 64;
       const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_x + xst + 1024 * i);
-      asm volatile("global_load_lds_dwordx4 %0, %1" : : "v"(xoff[i]), "s"(xb), "{m0}"(dst) : "memory");
+      direct_load(xoff[i], xb, dst);
     } else if (stager) {
       const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_s + sst);
       const unsigned char* base = sbase + (long)phys(ts) * sstep;
-      asm volatile("global_load_lds_dwordx4 %0, %1" : : "v"(soff), "s"(base), "{m0}"(dst) : "memory");
+      direct_load(soff, base, dst);
     }
   };
   auto issue = [&](int tx, uint32_t xst, int ts, uint32_t sst) {
@@ -298,7 +298,7 @@ __global__ __launch_bounds__(512, 1) void sparse24_tile256_kernel(const Sparse24
   if (stager) {
     const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_s);
     const unsigned char* base = sbase + (long)phys(0) * sstep;
-    asm volatile("global_load_lds_dwordx4 %0, %1" : : "v"(soff), "s"(base), "{m0}"(dst) : "memory");
+    direct_load(soff, base, dst);
   }
   issue(0, 0, 1, kT256WStageBytes);
   issue(1, kT256XStageBytes, 2, 2 * kT256WStageBytes);

@@ -186,11 +186,10 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void sparse24_wide_kerne
     const int chunk = (lane & 15) ^ (row & 15);
     xoff[ii] = (uint32_t)(((long)s_rows[row] * p.x_stride + chunk * 8) * 2);
   }
-  // Direct-to-LDS loads and the waits for them are written as inline assembly: the compiler
+  // Direct-to-LDS loads (direct_load) and the waits for them are written as inline assembly: the compiler
   // counts a direct-to-LDS load as an LDS write, which the release fence of every barrier and
   // the first LDS read behind it must complete, i.e. it drains every outstanding request (the
-  // weights requested a moment ago included) once per K step.  The LDS address of a request is
-  // M0 + 16 * lane; M0 is an input operand of the statement, so the compiler writes it and knows it is live.
+  // weights requested a moment ago included) once per K step.
   const uint32_t lds_x_wave = (uint32_t)(uintptr_t)&xs[kh][0][4 * wave][0];
   // (`nta`: the 16-token tiles that hold tokens; the others are neither fetched nor multiplied)
   auto issue_x = [&](int st, int nta) {   // (nta: a constant where this is called)
@@ -201,7 +200,7 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void sparse24_wide_kerne
       if (ii >= nta) break;
       const uint32_t dst = __builtin_amdgcn_readfirstlane(lds_x_wave + (stage * TOK + 16 * ii) * 256);
       const _Float16* base = p.x + stc * 128;
-      asm volatile("global_load_lds_dwordx4 %0, %1" : : "v"(xoff[ii]), "s"(base), "{m0}"(dst) : "memory");
+      direct_load(xoff[ii], base, dst);
     }
   };
 
