@@ -28,6 +28,8 @@ ROUTED_ALTERNATIVES = {
     "plan, 32-token tiles on the wide kernel": {"TRITEIA_HIP_FUSED_ROUTE": "0", "TRITEIA_HIP_NT": "2", "TRITEIA_HIP_MID_MIN_UNITS": "1", "TRITEIA_HIP_MID_MIN_COLUMN_GROUPS": "1", "TRITEIA_HIP_MID_MIN_HALF_TOKENS": "0", "TRITEIA_HIP_MID_DEPTH": "1", "TRITEIA_HIP_PLAN_BIG": "0"},
     "plan, 32-token tiles on the wide kernel, two steps in flight": {"TRITEIA_HIP_FUSED_ROUTE": "0", "TRITEIA_HIP_NT": "2", "TRITEIA_HIP_MID_MIN_UNITS": "1", "TRITEIA_HIP_MID_MIN_COLUMN_GROUPS": "1", "TRITEIA_HIP_MID_MIN_HALF_TOKENS": "0", "TRITEIA_HIP_MID_DEPTH": "2", "TRITEIA_HIP_PLAN_BIG": "0"},
     "plan, 64-token tiles on the wide kernel": {"TRITEIA_HIP_FUSED_ROUTE": "0", "TRITEIA_HIP_NT": "4", "TRITEIA_HIP_MID_MIN_UNITS": "1", "TRITEIA_HIP_MID_MIN_COLUMN_GROUPS": "1", "TRITEIA_HIP_MID64_MAX_K": BIG, "TRITEIA_HIP_MID_MIN_HALF_TOKENS": "0", "TRITEIA_HIP_MID_DEPTH": "1"},
+    "plan, K-splitting tiles": {"TRITEIA_HIP_FUSED_ROUTE": "0", "TRITEIA_HIP_PLAN_KTILE": "2"},
+    "plan, no K-splitting tiles": {"TRITEIA_HIP_PLAN_KTILE": "0"},
 }
 # ... and for a single-matrix product
 UNIFORM_ALTERNATIVES = {
@@ -57,6 +59,10 @@ ROUTED_GRID = [
     (11008, 4096, 32, 64), (11008, 4096, 32, 256), (11008, 4096, 32, 1024), (11008, 4096, 8, 512),
     (4096, 4096, 16, 768), (4096, 11008, 4, 512), (4096, 11008, 8, 768), (8192, 8192, 8, 512), (8192, 8192, 8, 1536),
     (4096, 14336, 8, 1024), (4096, 14336, 16, 768), (8192, 8192, 16, 2048), (8192, 28672, 8, 512),
+    # thousands of tokens on layers of 4, 8, 12 and 15 column groups of 512, either side of where the wide kernel takes the hot deltas from the
+    # K-splitting tiles
+    (4096, 2048, 16, 16384), (4096, 4096, 4, 8192), (4096, 4096, 64, 4096), (4096, 4096, 64, 8192),
+    (11008, 4096, 16, 4096), (8192, 6144, 8, 2048), (8192, 6144, 8, 8192), (4096, 7680, 32, 4096),
 ]
 # Points where the host cannot know which alternative is ahead, with the tolerance allowed there.  The two-deep build of the
 # wide kernel holds two workgroups per CU, the one-deep build three; past the point where the plan's upper bound of tiles
@@ -68,7 +74,11 @@ ROUTED_GRID = [
 # 64-token tiles for the wide kernel and rests for the K-split kernel keeps the launch within one round and is 15-19 %
 # ahead here; a host rule for it was measured and is a coin flip (the same split is 15-20 % behind with 8 deltas randomly
 # routed and 4-9 % behind evenly routed, 15 % ahead Zipf-routed): only the device knows whether a batch spills.
-KNOWN_GAPS = {(4096, 11008, 32, 512): 1.15, (8192, 8192, 16, 2048): 1.30}
+# The last five: thousands of tokens on a narrow layer, where every token on the wide kernel, cut in 64-token (of 64 deltas with 4096 tokens in
+# 32-token) tiles, is 10 - 18 % ahead of the split between that kernel and the streaming kernel and of the K-splitting tiles alike: a rule for it
+# is still to be measured.
+KNOWN_GAPS = {(4096, 11008, 32, 512): 1.15, (8192, 8192, 16, 2048): 1.30, (4096, 2048, 16, 16384): 1.20, (4096, 4096, 4, 8192): 1.20,
+              (4096, 4096, 64, 4096): 1.25, (4096, 4096, 64, 8192): 1.25, (4096, 7680, 32, 4096): 1.25}
 # (k, m, tokens): single-matrix products around the windows of the wide kernels and of the K split
 UNIFORM_GRID = [
     (4096, 4096, 16), (4096, 4096, 128), (4096, 4096, 512), (4096, 4096, 640), (4096, 4096, 1024), (4096, 4096, 1536),

@@ -157,6 +157,24 @@ def test_dispatch_queries_at_the_documented_points():
     assert lib.triteia_hip_plan_tile_tokens(4096, 16) == 64
 
 
+def test_the_plans_k_splitting_tiles_have_an_upper_end():
+    """triteia_hip_planned_ktile (tokens, deltas, m, k): batches that the streaming kernel would take alone at any size; of those whose hot
+    deltas the wide kernel takes, by column groups of the layer, tokens per delta and units of 64 tokens x 128 columns."""
+    lib = _ffi.lib()
+    _ffi.reload_env()
+    ktile = lib.triteia_hip_planned_ktile
+    assert ktile(513, 32, 4096, 4096) == 32 and ktile(1536, 4, 4096, 4096) > 0
+    for tokens in (4096, 8192, 32768, 65536):            # eight and twelve column groups
+        assert ktile(tokens, 16, 4096, 4096) == 0 and ktile(tokens, 4, 4096, 4096) == 0 and ktile(tokens, 4, 6144, 8192) == 0
+    assert ktile(32768, 16, 1536, 4096) == 64            # three column groups: at any number of tokens
+    assert ktile(4096, 64, 4096, 4096) == 64             # 64 tokens per delta
+    assert ktile(6000, 64, 4096, 4096) == 64 and ktile(6200, 64, 4096, 4096) == 0   # either side of 96
+    # over 8 deltas, units of tokens and half a tile per delta x column blocks: up to 4096 on 28 blocks (seven groups), 3072 on 33 and 60
+    for blocks, units in ((28, 4096), (33, 3072), (60, 3072)):
+        most = units * 64 // blocks - 32 * 8
+        assert ktile(most, 8, 128 * blocks, 4096) == 64 and ktile(most + 64, 8, 128 * blocks, 4096) == 0, blocks
+
+
 def test_bench_refuses_more_than_one_gpu():
     import subprocess
     import sys

@@ -1135,9 +1135,25 @@ static bool ktile_plan_can(int prob_n, int prob_k) {
   // (whole 128-deep K steps; 32-bit byte offsets of rows of activations)
   return prob_k % 128 == 0 && (long)prob_n * prob_k * 2 < (1L << 32);
 }
-// Which planned batches it takes: all that would go to the streaming kernel (2164 random ones, k and m 512 .. 13824, 20 .. 4096 tokens over
+// Whether a planned batch's full 64-token tiles (or all of its tokens in such tiles) go to a launch of the wide kernel behind the streaming
+// kernel's.  That kernel needs whole 128-deep K steps and addresses activations with 32-bit byte offsets, and a batch that could not
+// reach the bar even with most of its tokens in wide tiles (one per 48 tokens) is not worth the empty launch.  Nor is one whose tiles
+// the 32-token wide kernel takes: that kernel on the narrow-only list is as fast or faster than a split between the two (cfg4 at
+// 512 / 768 tokens 955 -> 913 / 1075 -> 1032 us).
+static bool plan_wide_launch(int prob_n, int n_deltas, int prob_m, int prob_k) {
+  return plan_has_wide(prob_n, n_deltas) && !mid_tiles(prob_n, n_deltas, prob_m, prob_k) && prob_k % 128 == 0 && (long)prob_n * prob_k * 2 < (1L << 32) &&
+         (long)(prob_n / 48 + 1) * ((prob_m / 128 + 3) / 4) >= knob_or(knobs().plan_wide_min_units, kPlanWideMinUnits);
+}
+// Which planned batches it takes.  All that would go to the streaming kernel alone (2164 random ones, k and m 512 .. 13824, 20 .. 4096 tokens over
 // 2 .. 64 deltas, evenly routed and Zipf: geometric mean 0.82 of its time, worst 1.10; 20 deltas of 3840 x 1152 with 1861 tokens
-// 73 -> 31 us, 5 of 11008 x 4096 with 279 63 -> 36, 32 of 4096 x 4096 with 513 53.5 -> 48), and of those for the wide kernels the ones of
+// 73 -> 31 us, 5 of 11008 x 4096 with 279 63 -> 36, 32 of 4096 x 4096 with 513 53.5 -> 48).
+// Of those whose hot deltas go to the wide kernel on fewer than 16 column groups of 512 (7764 random ones, m 512 .. 7680, 512 .. 32768 tokens over 1 .. 64
+// deltas: 0.860 of the time, taking each one's better kernel 0.852, all of them 0.880): up to three groups any, which the wide
+// kernel pads to eight (0.45 - 0.85); below 96 tokens per delta any, whose 64-token tiles are half empty (0.67 - 0.98); else as
+// long as the wide kernel's shared activation tiles are not ahead, in units of 64 tokens x 128 columns up to 4096 below eight
+// groups (0.91 - 0.98 there, 0.98 - 1.06 above), 1536 with eight, which fill its order of units without an idle slot (1.01 -
+// 1.13 above; 16 deltas of 4096 x 4096 with 4096 tokens 100 against 114 us), 3072 with more (0.91 - 0.99, 1.02 - 1.14 above).
+// Of those for the wide kernels the ones of
 // few 64-token tiles, the deeper K the more (1027 random ones: 0.76 of the time, 17 of them more than 3 % slower, worst 1.23):
 // up to 256 units of 64 tokens x 128 columns any (0.42 - 0.80: half the CUs had no workgroup), up to one round of 512 from
 // k = 1280 on (0.71 - 0.91), two rounds from k = 2560 on (0.81 - 0.93), three from k = 4500 on (0.91).  Past that, with fewer
@@ -1147,9 +1163,12 @@ static bool ktile_plan_takes(int prob_n, int n_deltas, int prob_m, int prob_k) {
   if (!knobs().plan_ktile || !ktile_plan_can(prob_n, prob_k)) return false;
   if (knobs().plan_ktile == 2) return true;
   if (!routed_knobs_unset()) return false;
-  if (!mid_tiles(prob_n, n_deltas, prob_m, prob_k)) return true;
-  const long groups = n_deltas < prob_n ? n_deltas : prob_n;
+  const long groups = n_deltas < prob_n ? n_deltas : prob_n, cgs = (prob_m / 128 + 3) / 4;
   const long units = (prob_n + 32 * groups) * (prob_m / 128) / 64;   // tokens / 64 and half a tile per delta, as a randomly routed batch leaves them
+  if (!mid_tiles(prob_n, n_deltas, prob_m, prob_k)) {
+    if (!plan_wide_launch(prob_n, n_deltas, prob_m, prob_k) || cgs <= 3 || prob_n < 96 * groups) return true;
+    return cgs != 8 && units <= (cgs < 8 ? 4096 : 3072);
+  }
   if (units <= 256) return true;
   if (prob_n < 32 * groups) return false;
   return (units <= 512 && prob_k >= 1280) || (units <= 1024 && prob_k >= 2560) || (units <= 1536 && prob_k >= 4500 && prob_n >= 64 * groups);
@@ -1271,14 +1290,8 @@ int triteia_hip_sbmm_2_4_planned(const void* A, const void* B, const void* meta,
     a.tiles_alt = reinterpret_cast<const int4*>(ws + L.all);
     a.wide_gate = (prob_m / 128 + 3) / 4;
     a.wide_min_units = knob_or(knobs().plan_wide_min_units, kPlanWideMinUnits);
-    // The wide kernel needs whole 128-deep K steps, and a batch that could not reach the bar
-    // even with most of its tokens in wide tiles (one per 48 tokens) is not worth the empty
-    // launch: then the bar is out of reach on the device too and every tile list is the narrow-only one.
-    // (and it addresses activations with 32-bit byte offsets)
-    // Nor is it where the 32-token wide kernel takes the plan's tiles: that kernel on the narrow-only list is
-    // as fast or faster than a split between the two (cfg4 at 512 / 768 tokens 955 -> 913 / 1075 -> 1032 us).
-    wide_launch = !mid && prob_k % 128 == 0 && (long)prob_n * prob_k * 2 < (1L << 32) &&
-                  (long)(prob_n / 48 + 1) * a.wide_gate >= a.wide_min_units;
+    // (without that launch the bar is out of reach on the device too and every tile list is the narrow-only one)
+    wide_launch = plan_wide_launch(prob_n, n_deltas, prob_m, prob_k);
     if (!wide_launch) a.wide_min_units = 0x7fffffff;
     // One list of 64-token tiles over all tokens, for the device to take instead of {wide tiles, narrow rest} where that
     // costs no further round of workgroups (Sparse24Args::tiles_all64): the plan's narrow-only list when it is cut in
@@ -1297,14 +1310,14 @@ int triteia_hip_sbmm_2_4_planned(const void* A, const void* B, const void* meta,
       }
     }
   }
+  if (reinterpret_cast<uintptr_t>(B) % 16 == 0 && ktile_plan_takes(prob_n, n_deltas, prob_m, prob_k))
+    return launch_ktile_plan(a, prob_n, n_deltas, ws, L, static_cast<hipStream_t>(stream));
   // The plan's tiles are cut without knowledge of the layer.  Where they make a launch of very few
   // workgroups on this layer (one or two deltas, a narrow matrix: fewer than 200 even on the plan's
   // upper bound of tiles), the kernel takes them in narrower passes split over workgroups (the weights
   // re-read that way come from cache) until there is a workgroup per CU.  Measured on 4096 x 4096: one
   // delta with 64 / 128 tokens 24.4 -> 12.7 / 24.2 -> 18.8 us, two deltas with 256 tokens 24.6 -> 18.5 us;
   // launches of 250 workgroups and more lose 10 % that way and keep the plan's tile.
-  if (reinterpret_cast<uintptr_t>(B) % 16 == 0 && ktile_plan_takes(prob_n, n_deltas, prob_m, prob_k))
-    return launch_ktile_plan(a, prob_n, n_deltas, ws, L, static_cast<hipStream_t>(stream));
   int pass_nt = tile / 16;
   {
     const long cb_pad = (prob_m / 128 + 7) / 8 * 8;
