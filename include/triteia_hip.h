@@ -141,12 +141,21 @@ TRITEIA_HIP_API int triteia_hip_sbmm_2_4_bounded(const void* A, const void* B, c
  * token_indices: int32 [prob_n] on the device, any order.  The tokens are
  * grouped on the device, so each delta's weights are read once per launch.
  * workspace: >= triteia_hip_sbmm_routed_workspace_bytes(prob_n, n_deltas) bytes
- * of device memory, contents irrelevant on entry, overwritten (a batch that
- * triteia_hip_routed_in_kernel answers 1 or 2 for is routed inside the multiply kernel and leaves it
- * untouched; of the others, up to 256 tokens over at most 16 deltas and most batches of up to 64 tokens
- * over at most 64 run without one too, more slowly).
+ * of device memory, contents irrelevant on entry, overwritten.  A batch that
+ * triteia_hip_routed_leaves_workspace answers 1 for is routed inside the multiply kernel and leaves it
+ * untouched (it may be null, or shared with calls in flight on other streams): batches of at most 64 tokens
+ * over at most 64 deltas but for more than 32 tokens over more than 16 deltas of a layer of 2^25 weights and more, and
+ * most of up to 256 tokens over at most 16 deltas.
  * n_deltas <= 8192. */
 TRITEIA_HIP_API int triteia_hip_sbmm_2_4_routed(const void* A, const void* B, const void* meta, void* C, const void* s,
+                                const void* token_indices, int index_offset, int n_deltas, int prob_m, int prob_n,
+                                int prob_k, void* workspace, size_t workspace_bytes, int accumulate, int dev,
+                                void* stream);
+/* The same for a workspace that no other call in flight uses: small batches on a long K that a routing plan serves better
+ * are planned too (triteia_hip_routed_in_kernel says 0 for them; 57 tokens over 2 deltas of 11008 x 4096 47 -> 26 us).
+ * Without a workspace, or with one that is too small or not aligned to 16 bytes, they are routed in the kernel.  The results are
+ * triteia_hip_sbmm_2_4_routed's, bit for bit.  No counterpart in the reference. */
+TRITEIA_HIP_API int triteia_hip_sbmm_2_4_routed_own(const void* A, const void* B, const void* meta, void* C, const void* s,
                                 const void* token_indices, int index_offset, int n_deltas, int prob_m, int prob_n,
                                 int prob_k, void* workspace, size_t workspace_bytes, int accumulate, int dev,
                                 void* stream);
@@ -217,12 +226,13 @@ TRITEIA_HIP_API int triteia_hip_wide_unit_order(int prob_m);
 TRITEIA_HIP_API long triteia_hip_wide_grid_units(long rows, int prob_m, int order);
 TRITEIA_HIP_API long triteia_hip_wide_block_grid_units(long rows, int prob_m, int block_column_groups);
 
-/* 1 or 2 if triteia_hip_sbmm_2_4_routed handles this batch and layer in one launch, routing inside the multiply kernel
+/* 1 or 2 if triteia_hip_sbmm_2_4_routed_own handles this batch and layer in one launch, routing inside the multiply kernel
  * (the workspace stays untouched; 2: at most 16 tokens on the column-share kernel, sparse24_share16_kernel, 1: the
- * streaming kernel), 0 if it builds a routing plan first (one that it could route in the kernel it still does when the
- * workspace is null, too small or not aligned).  No counterpart in the reference; for
- * benchmarks and profiles. */
+ * streaming kernel), 0 if it builds a routing plan first.  triteia_hip_sbmm_2_4_routed does what it says too, but for the
+ * batches that only the former plans: 1 from triteia_hip_routed_leaves_workspace says that it routes in the kernel.  No
+ * counterpart in the reference; for callers that allocate, benchmarks and profiles. */
 TRITEIA_HIP_API int triteia_hip_routed_in_kernel(int prob_n, int n_deltas, int prob_m, int prob_k);
+TRITEIA_HIP_API int triteia_hip_routed_leaves_workspace(int prob_n, int n_deltas, int prob_m, int prob_k);
 
 
 /* The multiply step alone, on a plan made by triteia_hip_route_plan for the same

@@ -189,7 +189,7 @@ def test_default_rule_against_forced_alternatives_routed():
             def call(i):
                 q, me, s = weights[i % len(weights)]
                 stream = _ffi.stream_of(x)              # (torch's current stream: the capturing one while a graph is recorded)
-                rc = lib.triteia_hip_sbmm_2_4_routed(P(x), P(q), P(me), P(out), P(s), P(idx), 0, n, m, t, k, P(ws), ws.numel() * 4, 0, 0, stream)
+                rc = lib.triteia_hip_sbmm_2_4_routed_own(P(x), P(q), P(me), P(out), P(s), P(idx), 0, n, m, t, k, P(ws), ws.numel() * 4, 0, 0, stream)
                 assert rc == 0, _ffi.last_error()
             return call
 

@@ -175,6 +175,21 @@ def test_the_plans_k_splitting_tiles_have_an_upper_end():
         assert ktile(most, 8, 128 * blocks, 4096) == 64 and ktile(most + 64, 8, 128 * blocks, 4096) == 0, blocks
 
 
+def test_small_batches_leave_the_workspace():
+    """triteia_hip_routed_leaves_workspace (tokens, deltas, m, k): what callers that share a workspace over streams may rely on."""
+    lib = _ffi.lib()
+    _ffi.reload_env()
+    for k, m in ((4096, 4096), (11008, 4096), (13824, 13824)):
+        for tokens in (1, 16, 32, 33, 64):
+            for deltas in (1, 2, 16, 17, 64):
+                planned = tokens > 32 and deltas > 16 and k * m >= 1 << 25
+                assert lib.triteia_hip_routed_leaves_workspace(tokens, deltas, m, k) == (not planned), (tokens, deltas, m, k)
+    assert lib.triteia_hip_routed_leaves_workspace(256, 16, 4096, 4096) == 1 and lib.triteia_hip_routed_leaves_workspace(257, 16, 4096, 4096) == 0
+    assert lib.triteia_hip_routed_leaves_workspace(65, 17, 4096, 4096) == 0
+    # a plan that only a workspace of the call's own allows
+    assert lib.triteia_hip_routed_in_kernel(32, 1, 4096, 11008) == 0 and lib.triteia_hip_routed_in_kernel(64, 16, 4096, 4096) == 1
+
+
 def test_bench_refuses_more_than_one_gpu():
     import subprocess
     import sys

@@ -63,12 +63,13 @@ def test_a_batch_that_a_plan_serves_better_still_runs_without_a_workspace():
     out = torch.full((t, m), 9.0, dtype=torch.float16, device="cuda")
     args = lambda ws, size: (gx.data_ptr(), gq.data_ptr(), gm.data_ptr(), out.data_ptr(), gs.data_ptr(), gi.data_ptr(), 0, n, m, t, k, ws, size, 2, 0,
                              torch.cuda.current_stream().cuda_stream)
-    assert lib.triteia_hip_sbmm_2_4_routed(*args(None, 0)) == 0
-    assert torch.equal(out, want)
-    out.fill_(9.0)
     ws = torch.empty(lib.triteia_hip_sbmm_routed_workspace_bytes(t, n) + 16, dtype=torch.uint8, device="cuda")
-    assert lib.triteia_hip_sbmm_2_4_routed(*args(ws.data_ptr() + 4, ws.numel() - 16)) == 0      # (not aligned: routed in the kernel)
-    assert torch.equal(out, want)
+    for call in (lib.triteia_hip_sbmm_2_4_routed, lib.triteia_hip_sbmm_2_4_routed_own):
+        # (none, not aligned, too small: routed in the kernel)
+        for ptr, size in ((None, 0), (ws.data_ptr() + 4, ws.numel() - 16), (ws.data_ptr(), ws.numel() - 32)):
+            out.fill_(9.0)
+            assert call(*args(ptr, size)) == 0
+            assert torch.equal(out, want)
     graph = torch.cuda.CUDAGraph()
     torch.cuda.synchronize()
     with torch.cuda.graph(graph):
@@ -79,6 +80,27 @@ def test_a_batch_that_a_plan_serves_better_still_runs_without_a_workspace():
         torch.cuda.synchronize()
         assert torch.equal(y, want)
         assert torch.equal(ops.sbmm_4bit_2_4_native(gq, gx, gm, gs, gi), want)
+
+
+@pytest.mark.parametrize("n,t,k,m", [(2, 64, 8192, 256), (1, 32, 11008, 512), (4, 256, 4096, 256)])
+def test_a_workspace_that_other_calls_may_share_stays_untouched(n, t, k, m):
+    """triteia_hip_sbmm_2_4_routed routes such a batch in the kernel whatever workspace it is given; triteia_hip_sbmm_2_4_routed_own plans it."""
+    qw, meta, s = make_deltas(n, k, m, 3)
+    idx = (np.arange(t) % (n + 1) - 1).astype(np.int32)
+    x = activations(t, k, 5)
+    gq, gm, gs, gx, gi = to_gpu(qw, meta, s, x, idx)
+    lib = _ffi.lib()
+    assert lib.triteia_hip_routed_leaves_workspace(t, n, m, k) == 1 and lib.triteia_hip_routed_in_kernel(t, n, m, k) == 0
+    outs = []
+    for call, touched in ((lib.triteia_hip_sbmm_2_4_routed, False), (lib.triteia_hip_sbmm_2_4_routed_own, True)):
+        out = torch.full((t, m), 9.0, dtype=torch.float16, device="cuda")
+        ws = torch.full((lib.triteia_hip_sbmm_routed_workspace_bytes(t, n),), 0x5a, dtype=torch.uint8, device="cuda")
+        assert call(gx.data_ptr(), gq.data_ptr(), gm.data_ptr(), out.data_ptr(), gs.data_ptr(), gi.data_ptr(), 0, n, m, t, k, ws.data_ptr(), ws.numel(), 2, 0,
+                    torch.cuda.current_stream().cuda_stream) == 0
+        assert bool((ws != 0x5a).any()) is touched
+        outs.append(out)
+    assert torch.equal(*outs)
+    check_close(outs[0], orc.sbmm_4bit_2_4(qw, x, meta, s, idx), what=f"routed {n} deltas, {t} tokens, {k} x {m}")
 
 
 def test_activations_that_are_not_aligned_stay_with_the_kernels_before():

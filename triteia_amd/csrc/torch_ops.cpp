@@ -96,7 +96,7 @@ bool packed_ok(const Tensor& q, const Tensor& meta, const Tensor& s, const Tenso
          sizes_ok({n, k, m}) && q.size(0) == n && q.size(1) == k / 32 && q.size(2) == 2 * m && meta.size(0) == n && meta.size(1) == m &&
          meta.size(2) == k / 16 && s.size(0) == n && s.size(1) == 1 && s.size(2) == m;
 }
-// (what the routed product takes in one call, see triteia_hip_sbmm_2_4_routed)
+// (what the routed product takes in one call, see triteia_hip_sbmm_2_4_routed_own)
 constexpr int64_t kMaxRoutedDeltas = 8192;
 
 // (under autocast the base product has autocast's type, whatever its inputs': another one than x's is refused by the Python path)
@@ -179,8 +179,8 @@ int routed(const Tensor& x, const Tensor& q, const Tensor& meta, const Tensor& s
     bytes = triteia_hip_sbmm_routed_workspace_bytes(tokens, n);
     ws = scratch_bytes(bytes, x);
   }
-  return triteia_hip_sbmm_2_4_routed(x.data_ptr(), q.data_ptr(), meta.data_ptr(), y.data_ptr(), s.data_ptr(), indices.data_ptr(), offset, n,
-                                     m, tokens, k, bytes ? ws.data_ptr() : nullptr, bytes, accumulate, at_.dev, at_.handle());
+  return triteia_hip_sbmm_2_4_routed_own(x.data_ptr(), q.data_ptr(), meta.data_ptr(), y.data_ptr(), s.data_ptr(), indices.data_ptr(), offset, n,
+                                         m, tokens, k, bytes ? ws.data_ptr() : nullptr, bytes, accumulate, at_.dev, at_.handle());
 }
 
 // sbmm(qweights, xs, metas, ss, indices, base or None): ops.sbmm_4bit_2_4_native

@@ -1214,6 +1214,9 @@ int triteia_hip_routed_in_kernel(int prob_n, int n_deltas, int prob_m, int prob_
                       share16_tiles(prob_n < n_deltas ? prob_n : n_deltas, prob_m, prob_n);
   return shares ? 2 : 1;
 }
+int triteia_hip_routed_leaves_workspace(int prob_n, int n_deltas, int prob_m, int prob_k) {
+  return prob_n > 0 && n_deltas > 0 && prob_m > 0 && prob_k > 0 && routed_in_kernel(prob_n, n_deltas, prob_m, prob_k);
+}
 
 // `clear` (rows of m fp16): rows without a delta get zeros in the same launch; nullptr: none
 static int route_plan_impl(const void* token_indices, int index_offset, int n_deltas, int prob_n, void* workspace, size_t workspace_bytes,
@@ -1387,8 +1390,9 @@ static int sbmm_routed(const void* A, const void* B, const void* meta, void* C, 
   // plan pays from 128 tokens on whatever the number of deltas, the plan launch being small against the kernel
   // and the wide kernels taking hot deltas: 8 / 4 deltas of 8192 x 28672 with 128 / 256 tokens 145 -> 130 /
   // 160 -> 122 us, while 8 or 16 deltas of 4096 x 11008 stay 8-12 % faster routed inside the kernel)
-  // (a batch of this size that comes without a workspace for the plan, or with activations that the plan's kernel for it cannot
-  // take, is routed in the kernel all the same, and so are all of them on the library's own scratch, whose plan is one for all streams)
+  // (a batch of this size that a plan would serve better is planned only where the workspace is the call's own: calls that are
+  // routed in the kernel may share one over several streams.  Without a workspace for the plan, or with activations that the
+  // plan's kernel for it cannot take, it is routed in the kernel there too)
   const bool eager_ok = routed_eager_ok(prob_n, n_deltas);
   const bool plan_better = own_workspace && workspace && workspace_bytes >= triteia_hip_sbmm_routed_workspace_bytes(prob_n, n_deltas) &&
                            (reinterpret_cast<uintptr_t>(workspace) | reinterpret_cast<uintptr_t>(B)) % 16 == 0 &&
@@ -1434,6 +1438,13 @@ int triteia_hip_sbmm_2_4_routed(const void* A, const void* B, const void* meta, 
                                 const void* token_indices, int index_offset, int n_deltas, int prob_m, int prob_n,
                                 int prob_k, void* workspace, size_t workspace_bytes, int accumulate, int dev,
                                 void* stream) {
+  return sbmm_routed(A, B, meta, C, s, token_indices, index_offset, n_deltas, prob_m, prob_n, prob_k, workspace, workspace_bytes, accumulate, dev,
+                     stream, false);
+}
+int triteia_hip_sbmm_2_4_routed_own(const void* A, const void* B, const void* meta, void* C, const void* s,
+                                    const void* token_indices, int index_offset, int n_deltas, int prob_m, int prob_n,
+                                    int prob_k, void* workspace, size_t workspace_bytes, int accumulate, int dev,
+                                    void* stream) {
   return sbmm_routed(A, B, meta, C, s, token_indices, index_offset, n_deltas, prob_m, prob_n, prob_k, workspace, workspace_bytes, accumulate, dev,
                      stream, true);
 }

@@ -189,9 +189,12 @@ def sbmm_2_4_routed(A, B, meta, C, s, token_indices, index_offset=0, accumulate=
         raise RuntimeError("token_indices and C need one entry / row per row of A")
     if prob_m % 128 == 0 and prob_k % 64 == 0:
         _check_packed(B, meta, s, prob_m, prob_k, lead=(n_deltas,))
+    # (a workspace of the caller's may be in use on other streams, where this batch needs none)
+    routed = _ffi.lib().triteia_hip_sbmm_2_4_routed
     if workspace is None:
         workspace = routed_workspace(prob_n, n_deltas, A.device)
-    err = _ffi.lib().triteia_hip_sbmm_2_4_routed(
+        routed = _ffi.lib().triteia_hip_sbmm_2_4_routed_own
+    err = routed(
         _ffi.ptr(A), _ffi.ptr(B), _ffi.ptr(meta), _ffi.ptr(C), _ffi.ptr(s), _ffi.ptr(token_indices),
         int(index_offset), n_deltas, prob_m, prob_n, prob_k, _ffi.ptr(workspace),
         workspace.numel() * workspace.element_size(), 1 if accumulate else 0, _ffi.device_index(A), _ffi.stream_of(A))
