@@ -6,6 +6,7 @@ import re
 
 import pytest
 
+from tests.helpers import setknob
 from triteia_amd.python.capi import _ffi
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -188,6 +189,19 @@ def test_small_batches_leave_the_workspace():
     assert lib.triteia_hip_routed_leaves_workspace(65, 17, 4096, 4096) == 0
     # a plan that only a workspace of the call's own allows
     assert lib.triteia_hip_routed_in_kernel(32, 1, 4096, 11008) == 0 and lib.triteia_hip_routed_in_kernel(64, 16, 4096, 4096) == 1
+
+
+def test_the_scratch_of_uniform_launches_is_enough_for_either_kernel(monkeypatch):
+    """triteia_hip_bmm_scratch_bytes knows nothing of the activations' alignment, which decides between the K-splitting tiles and the kernels
+    before: it holds the shares of K of both."""
+    lib = _ffi.lib()
+    shapes = [(m, batch, tokens, k) for m in (128, 512, 768, 1536, 2560) for batch in (1, 2, 3, 8) for tokens in (1, 12, 17, 24, 31, 37, 64, 200)
+              for k in (4096, 8192, 11008, 14592, 17024, 23296)]
+    _ffi.reload_env()
+    both = [lib.triteia_hip_bmm_scratch_bytes(*shape) for shape in shapes]
+    setknob(monkeypatch, "TRITEIA_HIP_KTILE", 0)
+    before = [lib.triteia_hip_bmm_scratch_bytes(*shape) for shape in shapes]
+    assert all(a >= b for a, b in zip(both, before)) and sum(b > 0 for b in before) > 100
 
 
 def test_bench_refuses_more_than_one_gpu():

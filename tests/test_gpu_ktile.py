@@ -70,3 +70,15 @@ def test_rows_that_are_not_aligned():
     shifted.copy_(gx)
     a, b = ops.matmul_4bit_2_4(gq, shifted, gm, gs), ops.matmul_4bit_2_4(gq, gx, gm, gs)
     assert ((a.float() - b.float()).norm() / b.float().norm()).item() < 1e-4
+
+
+@pytest.mark.parametrize("b,t,k,m", [(1, 37, 17024, 1536), (3, 31, 23296, 768)])
+def test_rows_that_are_not_aligned_keep_their_split(monkeypatch, b, t, k, m):
+    """The scratch is for the shares of K of either kernel: more of them on the streaming kernel here than on the tiles."""
+    qw, meta, s, x = _case(b, t, k, m)
+    gq, gm, gs, gx = to_gpu(qw, meta, s, x)
+    shifted = torch.empty(b * t * k + 4, dtype=torch.float16, device="cuda")[4:].view(b, t, k)
+    shifted.copy_(gx)
+    out = ops.bmm_4bit_2_4(gq, shifted, gm, gs)
+    setknob(monkeypatch, "TRITEIA_HIP_KTILE", 0)
+    assert torch.equal(out, ops.bmm_4bit_2_4(gq, gx, gm, gs))

@@ -747,8 +747,12 @@ size_t split_bytes(int splits, int tokens, int n_groups, int m) {
   return splits > 1 ? sizeof(float) * (size_t)splits * (size_t)n_groups * (size_t)tokens * (size_t)m : 0;
 }
 size_t uniform_scratch_bytes(int tokens, int n_groups, int m, int k) {
-  return split_bytes(ktile_takes(tokens, n_groups, m, k, true) ? pick_ktile(tokens, n_groups, m, k, true).splits : pick_ksplit(tokens, n_groups, m, k),
-                     tokens, n_groups, m);
+  int splits = pick_ksplit(tokens, n_groups, m, k);       // (also of a launch for the K-splitting tiles: activations that are not aligned take this one)
+  if (ktile_takes(tokens, n_groups, m, k, true)) {
+    const int tiles = pick_ktile(tokens, n_groups, m, k, true).splits;
+    if (tiles > splits) splits = tiles;
+  }
+  return split_bytes(splits, tokens, n_groups, m);
 }
 
 int launch_uniform(Sparse24Args a, int tokens, int stride, int delta_step, int n_groups, hipStream_t st,
