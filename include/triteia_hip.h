@@ -319,8 +319,9 @@ TRITEIA_HIP_API int triteia_hip_lora_expand(void* y, long y_stride, const void* 
 
 /* out[n_tokens, prob_m] = x[n_tokens, prob_k] @ weight[prob_m, prob_k]^T, fp16 with fp32 sums: the dense base weight of a
  * layer (F.linear's layout) for the tokens of a routed batch.  At most 256 tokens, prob_m % 8 == 0, prob_k % 64 == 0,
- * and not up to 16 tokens on less than 2^20 weights (triteia_hip_dense_ok says whether a shape is taken); rows x_stride / w_stride elements apart, everything aligned to 16
- * bytes; out is contiguous.  triteia_hip_dense_scratch_bytes: what the call needs for shares of K (0: nothing).
+ * and not up to 16 tokens on less than 2^20 weights; rows x_stride / w_stride elements apart, everything aligned to 16
+ * bytes; out is contiguous.  triteia_hip_dense_ok: 1 where the ops take this product, 0 for the shapes it refuses and for those on which
+ * the library that torch calls is ahead (knob DENSE: 0 none, 2 every shape that can).  triteia_hip_dense_scratch_bytes: what the call needs for shares of K (0: nothing).
  * The reference leaves this product to torch.matmul (triteia/python/ops/matmul/sbmm.py, ldmm.py: base_weight). */
 TRITEIA_HIP_API int triteia_hip_dense_ok(int n_tokens, int prob_m, int prob_k);
 TRITEIA_HIP_API size_t triteia_hip_dense_scratch_bytes(int n_tokens, int prob_m, int prob_k);

@@ -204,6 +204,22 @@ def test_the_scratch_of_uniform_launches_is_enough_for_either_kernel(monkeypatch
     assert all(a >= b for a, b in zip(both, before)) and sum(b > 0 for b in before) > 100
 
 
+def test_which_base_products_the_library_takes(monkeypatch):
+    """triteia_hip_dense_ok (tokens, m, k): not where the library that torch calls measures ahead, and not at all under DENSE = 0."""
+    lib = _ffi.lib()
+    _ffi.reload_env()
+    ok = lib.triteia_hip_dense_ok
+    taken = [(13, 4096, 11008), (256, 11008, 4096), (256, 5120, 13824), (200, 4096, 4096), (128, 28672, 8192), (32, 2048, 2048), (17, 128, 64),
+             (128, 2048, 2048), (128, 9728, 5888), (193, 9728, 5888), (160, 4096, 11008), (256, 13824, 8192)]
+    left = [(129, 9728, 5888), (192, 9728, 5888), (160, 28672, 8192), (256, 28672, 8192), (129, 16384, 8192),       # the library is ahead
+            (257, 4096, 4096), (16, 512, 512), (13, 4096, 96)]                                                      # the kernel cannot or never did
+    assert all(ok(*shape) for shape in taken) and not any(ok(*shape) for shape in left)
+    setknob(monkeypatch, "TRITEIA_HIP_DENSE", 0)
+    assert not any(ok(*shape) for shape in taken)
+    setknob(monkeypatch, "TRITEIA_HIP_DENSE", 2)
+    assert [ok(*shape) for shape in left] == [1] * 5 + [0] * 3
+
+
 def test_bench_refuses_more_than_one_gpu():
     import subprocess
     import sys

@@ -65,7 +65,7 @@ struct Knobs {
   int wide32_min_units = kUnset, wide32_max_units = kUnset, wide32_ksplit_max_units = kUnset, wide64_ksplit_max_units = kUnset;
   int mid = 1, mid64_max_k = 0x7fffffff, mid_min_column_groups = 16, mid_min_units = kUnset, mid_min_half_tokens = 7, mid_narrow = 1, mid_depth = 0, plan_big = 1, plan_all64 = 1, lora_mfma = 1;
   int eager = 1, fused_route = 1;
-  int plan_ktile = 1, ktile = 1, tile256 = 1, tile256_min_units = kUnset, tile256_max_units = kUnset, ksplit = 1, sub_shift = kUnset, share16 = 1, share16_max_blocks = kUnset;
+  int dense = 1, plan_ktile = 1, ktile = 1, tile256 = 1, tile256_min_units = kUnset, tile256_max_units = kUnset, ksplit = 1, sub_shift = kUnset, share16 = 1, share16_max_blocks = kUnset;
 };
 Knobs g_knobs;
 std::once_flag g_knobs_once;
@@ -80,7 +80,7 @@ void read_knobs() {
       {"WIDE32_KSPLIT_MAX_UNITS", &k.wide32_ksplit_max_units}, {"WIDE64_KSPLIT_MAX_UNITS", &k.wide64_ksplit_max_units},
       {"MID", &k.mid}, {"MID64_MAX_K", &k.mid64_max_k}, {"MID_MIN_COLUMN_GROUPS", &k.mid_min_column_groups},
       {"MID_MIN_UNITS", &k.mid_min_units}, {"MID_MIN_HALF_TOKENS", &k.mid_min_half_tokens}, {"MID_NARROW", &k.mid_narrow}, {"MID_DEPTH", &k.mid_depth}, {"PLAN_BIG", &k.plan_big}, {"PLAN_ALL64", &k.plan_all64}, {"LORA_MFMA", &k.lora_mfma}, {"EAGER", &k.eager}, {"FUSED_ROUTE", &k.fused_route},
-      {"KTILE", &k.ktile}, {"PLAN_KTILE", &k.plan_ktile}, {"TILE256", &k.tile256}, {"TILE256_MIN_UNITS", &k.tile256_min_units}, {"TILE256_MAX_UNITS", &k.tile256_max_units},
+      {"DENSE", &k.dense}, {"KTILE", &k.ktile}, {"PLAN_KTILE", &k.plan_ktile}, {"TILE256", &k.tile256}, {"TILE256_MIN_UNITS", &k.tile256_min_units}, {"TILE256_MAX_UNITS", &k.tile256_max_units},
       {"KSPLIT", &k.ksplit}, {"SUB_SHIFT", &k.sub_shift}, {"SHARE16", &k.share16}, {"SHARE16_MAX_BLOCKS", &k.share16_max_blocks},
   };
   char name[64];
@@ -1848,12 +1848,9 @@ namespace {
 // tiles and needs 0.07 us more per chunk of K for a round of the units that fit it together (its LDS), the chip reads 8.7 TB/s
 // (weights partly from the Infinity Cache); a split costs 2.4 us for its second launch and its partial sums' way there and
 // back.  The constants were fitted to 5000 measured launches (23 layers of 512 x 512 .. 13824 x 13824, 1 .. 256 tokens, every tile below,
-// 1 .. 12 shares): the choice is 0.7 % behind the best of them on average, 13 % at most, and the product 15 % ahead of the library's
-// (hipBLASLt) on those 299 shapes: 13 tokens on 11008 x 4096 29.3 -> 19.3 us, 256 tokens on 4096 x 11008 48.4 -> 37.1, on
-// 13824 x 5120 137 -> 57; 11 % behind it at worst (4096 x 4096 with 200 tokens 17.9 -> 19.9).  From 300 tokens on the library's larger
-// tiles are level or ahead (4096 x 11008 with 384 49.7 against 67).
+// 1 .. 12 shares): the choice is 0.7 % behind the best of them on average, 13 % at most.
 constexpr int kDenseMaxTokens = 256;
-struct DensePick { int tokens, features, stages, splits; };
+struct DensePick { int tokens, features, stages, splits; double intake = 0, hbm = 0; };   // (the busiest CU's way through its tiles, the weights' from HBM, us)
 constexpr DensePick kDenseTiles[] = {{16, 32, 12, 0}, {16, 64, 8, 0}, {32, 32, 8, 0}, {32, 64, 6, 0}, {64, 32, 6, 0},
                                      {64, 64, 5, 0}, {64, 96, 5, 0}, {128, 64, 6, 0}, {128, 96, 5, 0}, {128, 128, 4, 0}};
 DensePick pick_dense(int tokens, int m, int k) {
@@ -1873,10 +1870,29 @@ DensePick pick_dense(int tokens, int m, int k) {
       const double cu = (double)chunks / z * (per_cu * chunk + (per_cu + together - 1) / together * 0.066);
       double us = cu > hbm ? cu + 0.25 * hbm : hbm + 0.25 * cu;
       if (z > 1) us += 2.36 + 8.0 * z * tokens * m / 2.7e6;
-      if (us < least) { least = us; best = t; best.splits = z; }
+      if (us < least) { least = us; best = t; best.splits = z; best.intake = cu; best.hbm = hbm; }
     }
   }
   return best;
+}
+// Which products it takes from the library (hipBLASLt).  Measured against it on 12652 random ones (k, m 512 .. 13824 and the layers of 7B - 70B
+// models, 1 .. 256 tokens; in a graph, the kernels alone), with a weight that the product before has read (warm) and with as many
+// weights in turn as the Infinity Cache does not hold (cold): 0.96 of the library's time warm, 0.83 cold.  Left to the library
+// are two regions in which its larger tiles are ahead:
+//   * 129 .. 192 tokens, which leave half of the second 128-token tile empty, where the way into the CUs is what the launch takes: 1.16 warm,
+//     1.01 cold (5888 x 9728 with 129 34.1 -> 48.9, 41.5 -> 47.7 us; the call with 8 deltas beside it 88.5 -> 93.4);
+//   * more than 128 tokens on 2^27 weights and more: 1.12, 1.09 (8192 x 28672 with 160 113 -> 172, 114 -> 169; the call 268 -> 321).
+// It is ahead warm, level cold, from 33 tokens on also on k = 1152 .. 3072 and less than 2^23 weights (2048 x 2048 with 100 6.7 -> 9.5 us warm,
+// 8.6 -> 10.0 cold), but its call on the host costs a small product more than that: with 8 deltas beside it 24.1 -> 17.8 us.
+// What stays is 13 tokens on 11008 x 4096 19.6 -> 18.5 warm, 29.3 -> 20.3 cold, 256 on 4096 x 11008 40.1 -> 35.5, 49.0 -> 38.4, on 13824 x
+// 5120 119 -> 57, 135 -> 57; at worst 1.40 and 1.19 (5632 x 768 with 69 tokens); 4096 x 4096 with 200, 17.2 -> 20.4 warm, is 22.1 -> 21.2
+// cold and in a call with 16 deltas 46.3 -> 45.3.  From 300 tokens on the library is level or ahead (4096 x 11008 with 384 49.7 against 67).
+bool dense_pays(int tokens, int m, int k) {
+  if (tokens <= 128) return true;
+  if ((long)m * k >= (1L << 27)) return false;
+  if (tokens > 192) return true;
+  const DensePick t = pick_dense(tokens, m, k);
+  return t.intake <= 15 || t.intake <= 2.15 * t.hbm;
 }
 
 // more than 64 KB of LDS has to be granted once per device and kernel
@@ -1919,7 +1935,9 @@ bool dense_shape_ok(int tokens, int m, int k) {
 
 extern "C" {
 
-int triteia_hip_dense_ok(int n_tokens, int prob_m, int prob_k) { return dense_shape_ok(n_tokens, prob_m, prob_k); }
+int triteia_hip_dense_ok(int n_tokens, int prob_m, int prob_k) {
+  return knobs().dense && dense_shape_ok(n_tokens, prob_m, prob_k) && (knobs().dense == 2 || dense_pays(n_tokens, prob_m, prob_k));
+}
 
 size_t triteia_hip_dense_scratch_bytes(int n_tokens, int prob_m, int prob_k) {
   if (!dense_shape_ok(n_tokens, prob_m, prob_k)) return 0;
