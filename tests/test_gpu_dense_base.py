@@ -94,3 +94,25 @@ def test_base_product_in_a_graph():
         torch.cuda.synchronize()
         assert torch.equal(y, want)
         assert torch.equal(_base_only(x, w, packed), want)
+
+
+def test_base_product_under_tunable_op(tmp_path):
+    """A process that has torch tune its products gets torch's, tuned or not."""
+    tokens, k, m = 13, 11008, 512                          # (K split over workgroups: other bits than torch's)
+    x, w = _operands(tokens, k, m)
+    packed = _packed(k, m)
+    tunable = torch.cuda.tunable
+    assert not tunable.is_enabled()
+    plain = _base_only(x, w, packed)
+    tuning = tunable.tuning_is_enabled()
+    tunable.set_filename(str(tmp_path / "results.csv"))    # (read when it is switched on; not the working folder's)
+    tunable.tuning_enable(False)
+    tunable.enable(True)
+    try:
+        y, want = _base_only(x, w, packed), torch.matmul(x, w.t())
+    finally:
+        tunable.enable(False)
+        tunable.tuning_enable(tuning)
+    assert torch.equal(y, want)
+    assert not torch.equal(plain, want)
+    assert torch.equal(_base_only(x, w, packed), plain)

@@ -19,6 +19,8 @@
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#define TORCH_CUDA_CPP_API TORCH_HIP_CPP_API   // (as the torch of this build names it, but for this header)
+#include <ATen/cuda/tunable/Tunable.h>
 
 #include <unordered_map>
 
@@ -109,11 +111,12 @@ bool aligned(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr())
 
 // x [tokens, k] times the layer's dense weight, which base_ok has let pass: what the kernels add to.  A few hundred fp16 rows
 // run on the library's own kernel, everything else -- more tokens, other types, rows that are not aligned, a product that
-// autograd records -- on torch's.
+// autograd records, a process that has torch tune its products (torch.cuda.tunable) -- on torch's.
 Tensor base_product(const Tensor& x, const Tensor& weight, const Place& at_) {
   const int64_t tokens = x.size(0), k = x.size(1), m = weight.size(0);
   const bool recorded = (at::GradMode::is_enabled() && (x.requires_grad() || weight.requires_grad())) || x._fw_grad(0).defined() || weight._fw_grad(0).defined();
-  if (x.scalar_type() == at::kHalf && !recorded && sizes_ok({tokens, k, m}) && triteia_hip_dense_ok(tokens, m, k) && x.is_contiguous() &&
+  if (x.scalar_type() == at::kHalf && !recorded && sizes_ok({tokens, k, m}) && triteia_hip_dense_ok(tokens, m, k) &&
+      !at::cuda::tunable::getTuningContext()->IsTunableOpEnabled() && x.is_contiguous() &&
       weight.stride(1) == 1 && weight.stride(0) >= k && weight.stride(0) % 8 == 0 && aligned(x) && aligned(weight) && !x.is_neg() && !weight.is_neg()) {
     Tensor y = at::empty({tokens, m}, x.options());
     const size_t bytes = triteia_hip_dense_scratch_bytes(tokens, m, k);
