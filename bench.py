@@ -216,10 +216,15 @@ def kernel_name(wl, lib, in_kernel):
     """The kernel that takes most of the workload's rows, as the library itself reports it."""
     if wl.op in ("matmul", "bmm"):
         groups, per_group = (1, wl.tokens) if wl.op == "matmul" else (wl.n_deltas, max(1, wl.tokens // max(1, wl.n_deltas)))
+        tiles = lib.triteia_hip_uniform_ktile(wl.m, groups, per_group, wl.k, 1)
+        if tiles:
+            shares, tile = divmod(tiles, 1000)
+            return (f"sparse24_ktile_kernel<{tile & ~1} tokens, {8 if tile & 1 else 4} wavefronts>"
+                    + (f" (K split over {shares} workgroups) + splitk_reduce_kernel" if shares > 1 else ""))
         code = lib.triteia_hip_uniform_kernel(wl.m, groups, per_group, wl.k, 1)
         if code >= 1000:
-            return f"sparse24_ktile_kernel or sparse24_grouped_kernel (K split over {code - 1000} workgroups) + splitk_reduce_kernel"
-        return {0: "sparse24_ktile_kernel or sparse24_grouped_kernel", 16: "sparse24_share16_kernel", 32: "sparse24_wide_kernel<32 tokens>", 33: "sparse24_wide_kernel<32 tokens, 8 wavefronts>",
+            return f"sparse24_grouped_kernel (K split over {code - 1000} workgroups) + splitk_reduce_kernel"
+        return {0: "sparse24_grouped_kernel", 16: "sparse24_share16_kernel", 32: "sparse24_wide_kernel<32 tokens>", 33: "sparse24_wide_kernel<32 tokens, 8 wavefronts>",
                 64: "sparse24_wide_kernel<64 tokens>", 65: "sparse24_wide_kernel<64 tokens, 8 wavefronts>",
                 256: "sparse24_tile256_kernel"}.get(code, f"kernel code {code}")
     if in_kernel:
@@ -270,7 +275,7 @@ def measure(prob, wl, torch, ffi, steps, warmup, use_graph=True, reps=None):
     # ---- dominant kernel alone: batches of back-to-back launches between two events
     # (a batch that the routed entry point routes inside the multiply kernel is one launch: the whole step; otherwise
     # the multiply runs on a routing plan made beforehand)
-    in_kernel = wl.op == "sbmm" and bool(lib.triteia_hip_routed_in_kernel(wl.tokens, wl.n_deltas, wl.m, wl.k))
+    in_kernel = wl.op == "sbmm" and bool(lib.triteia_hip_routed_leaves_workspace(wl.tokens, wl.n_deltas, wl.m, wl.k))
     kernel_call = prob.step if in_kernel else (prob.delta_routed if wl.index_offset else prob.delta_kernel)
     if wl.indices is not None and not in_kernel:
         prob.plan()

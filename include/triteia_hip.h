@@ -106,7 +106,10 @@ TRITEIA_HIP_API size_t triteia_hip_bmm_scratch_bytes(int prob_m, int batch, int 
  * of 16, 32 or 64 columns on sparse24_share16_kernel (at most 16 tokens per matrix, launches of at most 32 / 64 / 128 column blocks of 128), 1000 + n = the same with K split over n workgroups (only
  * with_scratch != 0), 32 / 64 = 32- / 64-token tiles of sparse24_wide_kernel (+ 1: on eight wavefronts), 256 =
  * sparse24_tile256_kernel; -1 for a shape the entry points reject.  No counterpart in the reference; for benchmarks,
- * profiles and the test that guards the dispatch thresholds. */
+ * profiles and the test that guards the dispatch thresholds.
+ * triteia_hip_uniform_ktile: the same of sparse24_ktile_kernel alone (activations aligned to 16 bytes): 1000 x shares of K + the tokens of
+ * its tile (16, 32, 48, 64; + 1 on eight wavefronts), 0 where another kernel runs. */
+TRITEIA_HIP_API int triteia_hip_uniform_ktile(int prob_m, int batch, int tokens, int prob_k, int with_scratch);
 TRITEIA_HIP_API int triteia_hip_uniform_kernel(int prob_m, int batch, int tokens, int prob_k, int with_scratch);
 
 /* Run-list form: for run r < prob_r, rows starts[r] .. starts[r]+counts[r]-1 of
@@ -324,6 +327,9 @@ TRITEIA_HIP_API int triteia_hip_lora_expand(void* y, long y_stride, const void* 
  * the library that torch calls is ahead (knob DENSE: 0 none, 2 every shape that can).  triteia_hip_dense_scratch_bytes: what the call needs for shares of K (0: nothing).
  * The reference leaves this product to torch.matmul (triteia/python/ops/matmul/sbmm.py, ldmm.py: base_weight). */
 TRITEIA_HIP_API int triteia_hip_dense_ok(int n_tokens, int prob_m, int prob_k);
+/* The tile of a shape that triteia_hip_dense takes: its tokens + 1000 x its features + 10^6 x (2 x shares of K + 1 if feature groups
+ * start their walks over K apart); 0 for others.  For benchmarks and tests. */
+TRITEIA_HIP_API int triteia_hip_dense_tile(int n_tokens, int prob_m, int prob_k);
 TRITEIA_HIP_API size_t triteia_hip_dense_scratch_bytes(int n_tokens, int prob_m, int prob_k);
 TRITEIA_HIP_API int triteia_hip_dense(const void* x, long x_stride, const void* weight, long w_stride, void* out, int n_tokens, int prob_m,
                       int prob_k, void* scratch, size_t scratch_bytes, int dev, void* stream);

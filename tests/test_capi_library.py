@@ -79,7 +79,9 @@ def test_other_argument_errors():
     assert lib.triteia_hip_plan_tile_tokens(256, 16) == 32
     assert lib.triteia_hip_plan_tile_tokens(4096, 4) == 64
     assert lib.triteia_hip_planned_tile_kernel(256, 32, 11008, 4096) == 32      # cfg3: wide layer, 32-token tiles
-    assert lib.triteia_hip_planned_tile_kernel(256, 16, 4096, 4096) == 0        # narrow layer: the K-split kernel
+    assert lib.triteia_hip_planned_tile_kernel(256, 16, 4096, 4096) == 0        # narrow layer: not on the wide kernel ...
+    assert lib.triteia_hip_planned_ktile(256, 16, 4096, 4096) == 32             # ... the K-splitting tiles
+    assert lib.triteia_hip_planned_ktile(256, 32, 11008, 4096) == 0
     assert lib.triteia_hip_planned_tile_kernel(2048, 32, 11008, 4096) == 64
     assert lib.triteia_hip_planned_tile_kernel(2048, 64, 28672, 8192) == 64     # 64-token tiles on a long K as well
     # 1024 tokens over 8 deltas: the plan is cut in 32-token tiles and lists 64-token tiles beside them for wide layers
@@ -122,11 +124,15 @@ def test_dispatch_queries_at_the_documented_points():
     lib = _ffi.lib()
     _ffi.reload_env()
     uniform = lib.triteia_hip_uniform_kernel          # (m, batch, tokens, k, with_scratch)
+    tiles = lib.triteia_hip_uniform_ktile
     assert uniform(4096, 1, 16, 4096, 1) == 16         # cfg0: K of 4096 is too short for a split across workgroups; 16-column shares
-    assert uniform(4096, 1, 17, 4096, 1) == 0          # more than one 16-token pass: the streaming kernel
+    assert uniform(4096, 1, 17, 4096, 1) == 0          # more than one 16-token pass: column blocks of 128 ...
+    assert tiles(4096, 1, 17, 4096, 1) == 1017         # ... on K-splitting tiles of 16 tokens, eight wavefronts
     assert uniform(11008, 1, 16, 4096, 1) == 16        # 86 column blocks: shares of 64 columns
     assert uniform(28672, 1, 16, 4096, 1) == 0         # 224 column blocks: the streaming kernel
+    assert tiles(28672, 1, 16, 4096, 1) == 0
     assert uniform(4096, 8, 1, 4096, 1) == 0           # cfg1: a workgroup per CU already
+    assert tiles(4096, 8, 1, 4096, 1) == 0
     assert uniform(8192, 1, 16, 8192, 1) == 1004       # long K, few workgroups: K split in 4 ...
     assert uniform(8192, 1, 16, 8192, 0) == 16         # ... only with a scratch buffer (without: shares of 32 columns)
     assert lib.triteia_hip_bmm_scratch_bytes(8192, 1, 16, 8192) == 4 * 16 * 8192 * 4
@@ -136,7 +142,16 @@ def test_dispatch_queries_at_the_documented_points():
     assert uniform(4096, 1, 4096, 4096, 1) == 64       # 64-token tiles, two workgroups per CU
     assert uniform(2048, 1, 8192, 4096, 1) == 256      # a narrow layer: one round of 256-token tiles
     assert uniform(28672, 1, 4096, 8192, 1) == 64      # several rounds: 64-token tiles, two workgroups per CU
-    assert uniform(4096, 1, 128, 4096, 1) == 0
+    assert uniform(4096, 1, 128, 4096, 1) == 0 and tiles(4096, 1, 128, 4096, 1) == 0   # 256 16-token passes: the streaming kernel
+    assert tiles(4096, 1, 129, 4096, 1) == 1032 and tiles(4096, 1, 768, 4096, 1) == 1048 and tiles(4096, 1, 1024, 4096, 1) == 0
+    assert uniform(4096, 1, 37, 11008, 1) == 1004 and tiles(4096, 1, 37, 11008, 1) == 4032   # long K, few workgroups: K split ...
+    assert uniform(4096, 1, 37, 11008, 0) == 0 and tiles(4096, 1, 37, 11008, 0) == 1017      # ... only with a scratch buffer
+    assert tiles(4096, 1, 11, 8192, 1) == 0 and tiles(4096, 1, 16, 4096, 1) == 0             # a single matrix of 16 tokens and fewer
+    assert tiles(2048, 4, 11, 2048, 1) == 0 and tiles(2048, 4, 12, 2048, 1) > 0              # several: from 12 on ...
+    assert tiles(2048, 4, 2, 8192, 1) == 0 and tiles(5120, 2, 1, 13824, 1) > 0               # ... with fewer on a long K past 64 column blocks
+    assert tiles(1024, 1, 599, 1024, 1) == 0 and tiles(1024, 1, 640, 1024, 1) > 0            # less than 2^22 weights: from 600 tokens on
+    assert tiles(11008, 1, 256, 4096, 1) > 0 and tiles(8192, 1, 769, 8192, 1) == 0           # 832 tiles of 64 tokens x 128 columns
+    assert tiles(4096, 1, 129, 4160, 1) == 0           # half a K step of 128 at the end
     assert uniform(100, 1, 16, 4096, 1) == -1          # not a legal shape
     routed = lib.triteia_hip_routed_in_kernel          # (tokens, deltas, m, k)
     assert routed(64, 16, 4096, 4096) == 1             # cfg2: one launch, no plan
@@ -152,8 +167,14 @@ def test_dispatch_queries_at_the_documented_points():
     assert routed(16, 4, 4096, 4096) == 1              # four tokens per delta: weights requested ahead of the routing
     assert routed(256, 32, 11008, 4096) == 0           # cfg3: planned ...
     assert lib.triteia_hip_planned_tile_kernel(256, 32, 11008, 4096) == 32   # ... and its 32-token tiles go to the wide kernel
-    assert lib.triteia_hip_planned_tile_kernel(256, 16, 4096, 4096) == 0     # a narrow layer keeps the streaming kernel
-    assert lib.triteia_hip_planned_tile_kernel(1024, 16, 4096, 4096) == 32   # except for a thousand tokens in full tiles
+    assert lib.triteia_hip_planned_tile_kernel(256, 16, 4096, 4096) == 0     # a narrow layer does not
+    assert lib.triteia_hip_planned_tile_kernel(1024, 16, 4096, 4096) == 32   # except for a thousand tokens in full tiles ...
+    planned = lib.triteia_hip_planned_ktile            # (tokens, deltas, m, k): first of all
+    assert planned(1024, 16, 4096, 4096) == 64         # ... which at 768 tiles of 64 tokens x 128 columns the K-splitting tiles have
+    assert planned(1024, 16, 4096, 2048) == 0 and planned(1024, 16, 8192, 4096) == 0 and planned(1024, 40, 4096, 4096) == 0
+    assert planned(1500, 16, 5120, 4480) == 0 and planned(1500, 16, 5120, 4608) == 64   # up to 1536 from k = 4500 on
+    assert planned(500, 22, 1024, 8192) == 32 and planned(279, 5, 4096, 11008) == 32
+    assert planned(256, 32, 11008, 4096) == 0 and planned(1000, 32, 11008, 4096) == 0   # the wide kernel
     assert lib.triteia_hip_plan_tile_tokens(64, 16) == 16
     assert lib.triteia_hip_plan_tile_tokens(4096, 16) == 64
 

@@ -103,6 +103,29 @@ def test_a_workspace_that_other_calls_may_share_stays_untouched(n, t, k, m):
     check_close(outs[0], orc.sbmm_4bit_2_4(qw, x, meta, s, idx), what=f"routed {n} deltas, {t} tokens, {k} x {m}")
 
 
+@pytest.mark.parametrize("k,m,counts", [(384, 1152, [63, 64, 65, 0, 47, 48, 49, 1]), (4096, 1024, [5] * 40)])
+def test_infinities_and_nan(monkeypatch, k, m, counts):
+    """They stay in their own rows (a tile's padding is its last token again) and meet the same weights as on the streaming kernel."""
+    qw, meta, s = make_deltas(len(counts), k, m, 3)
+    idx = _counts_to_indices(counts, 2, 4)
+    gq, gm, gs, gx, gi = to_gpu(qw, meta, s, activations(len(idx), k, 5), idx)
+    call = lambda: ops.sbmm_4bit_2_4_native(gq, gx, gm, gs, gi)
+    setknob(monkeypatch, "TRITEIA_HIP_PLAN_KTILE", 2)
+    setknob(monkeypatch, "TRITEIA_HIP_FUSED_ROUTE", 0)
+    assert _ffi.lib().triteia_hip_planned_ktile(len(idx), len(counts), m, k) > 0
+    clean = call()
+    rows = [int(np.flatnonzero(idx == d)[-1]) for d in (0, 2, 7)]
+    for row, column, value in zip(rows, (5, k // 2, k - 1), (float("inf"), float("-inf"), float("nan"))):
+        gx[row, column] = value
+    out = call()
+    kept = torch.ones(len(idx), dtype=torch.bool, device="cuda")
+    kept[rows] = False
+    assert torch.equal(out[kept], clean[kept])
+    other = _streaming(monkeypatch, call)
+    assert bool((~torch.isfinite(out[rows])).any(-1).all())
+    assert torch.equal(out.isnan(), other.isnan()) and torch.equal(out[~out.isnan()], other[~out.isnan()])
+
+
 def test_activations_that_are_not_aligned_stay_with_the_kernels_before():
     n, t, k, m = 3, 300, 1024, 512
     qw, meta, s = make_deltas(n, k, m, 3)

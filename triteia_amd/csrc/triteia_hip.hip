@@ -897,6 +897,12 @@ size_t triteia_hip_bmm_scratch_bytes(int prob_m, int batch, int tokens, int prob
   return uniform_scratch_bytes(tokens, batch, prob_m, prob_k);
 }
 
+int triteia_hip_uniform_ktile(int prob_m, int batch, int tokens, int prob_k, int with_scratch) {
+  if (prob_m <= 0 || batch <= 0 || tokens <= 0 || prob_k <= 0 || prob_m % 128 != 0 || !ktile_takes(tokens, batch, prob_m, prob_k, true)) return 0;
+  const KTilePick t = pick_ktile(tokens, batch, prob_m, prob_k, with_scratch != 0);
+  return 1000 * t.splits + 16 * t.nt + (t.kw == 8);
+}
+
 int triteia_hip_uniform_kernel(int prob_m, int batch, int tokens, int prob_k, int with_scratch) {
   if (prob_m <= 0 || batch <= 0 || tokens <= 0 || prob_k <= 0 || prob_m % 128 != 0 || prob_k % 64 != 0) return -1;
   if (ktile_takes(tokens, batch, prob_m, prob_k, true)) {
@@ -1875,6 +1881,12 @@ DensePick pick_dense(int tokens, int m, int k) {
   }
   return best;
 }
+// Feature groups start their walks over K apart (DenseArgs::rotate) where the weight's way from HBM is what a launch takes, or where a
+// split changes the order of the sums anyway (64 tokens on 4096 x 11008 27.0 -> 24.6 us, 128 on 8192 x 8192 43.4 -> 37.6, 13 31.6 -> 27.8).
+// An unsplit launch of more tokens gains 0 - 6 % from it and walks K in order instead.  So do unsplit ones of up to 64 on smaller
+// layers; rows of launches that are neither split nor rotated have the same bits whatever batch they are in, the bits of a plain MFMA
+// product (torch's, where its library adds in order too).  Others' depend on the number of tokens.
+bool dense_rotates(int tokens, int m, int k, int splits) { return (splits > 1 || tokens <= 64) && (long)k * m >= (1L << 24); }
 // Which products it takes from the library (hipBLASLt).  Measured against it on 12652 random ones (k, m 512 .. 13824 and the layers of 7B - 70B
 // models, 1 .. 256 tokens; in a graph, the kernels alone), with a weight that the product before has read (warm) and with as many
 // weights in turn as the Infinity Cache does not hold (cold): 0.96 of the library's time warm, 0.83 cold.  Left to the library
@@ -1939,6 +1951,12 @@ int triteia_hip_dense_ok(int n_tokens, int prob_m, int prob_k) {
   return knobs().dense && dense_shape_ok(n_tokens, prob_m, prob_k) && (knobs().dense == 2 || dense_pays(n_tokens, prob_m, prob_k));
 }
 
+int triteia_hip_dense_tile(int n_tokens, int prob_m, int prob_k) {
+  if (!dense_shape_ok(n_tokens, prob_m, prob_k)) return 0;
+  const DensePick t = pick_dense(n_tokens, prob_m, prob_k);
+  return ((2 * t.splits + dense_rotates(n_tokens, prob_m, prob_k, t.splits)) * 1000 + t.features) * 1000 + t.tokens;
+}
+
 size_t triteia_hip_dense_scratch_bytes(int n_tokens, int prob_m, int prob_k) {
   if (!dense_shape_ok(n_tokens, prob_m, prob_k)) return 0;
   const int splits = pick_dense(n_tokens, prob_m, prob_k).splits;
@@ -1971,11 +1989,7 @@ int triteia_hip_dense(const void* x, long x_stride, const void* weight, long w_s
   a.tokens = n_tokens;
   a.m = prob_m;
   a.k = prob_k;
-  // Feature groups start their walks over K apart (DenseArgs::rotate) where the weight's way from HBM is what a launch takes, or where a
-  // split changes the order of the sums anyway (64 tokens on 4096 x 11008 27.0 -> 24.6 us, 128 on 8192 x 8192 43.4 -> 37.6, 13 31.6 -> 27.8).
-  // An unsplit launch of more tokens gains 0 - 6 % from it and walks K in order instead, as the library's own product does: the
-  // same bits on most layers, and the same for a row whatever batch it is in.
-  a.rotate = (t.splits > 1 || n_tokens <= 64) && (long)prob_k * prob_m >= (1L << 24);
+  a.rotate = dense_rotates(n_tokens, prob_m, prob_k, t.splits);
   a.splits = t.splits;
   a.partial = static_cast<float*>(scratch);
   const hipStream_t st = static_cast<hipStream_t>(stream);

@@ -28,6 +28,7 @@ SIGNATURES = {
     "triteia_hip_reload_env": (None, []),
     "triteia_hip_bmm_2_4_tokens_scratch": (_c_int, [_c_vp] * 5 + [_c_int] * 4 + [_c_vp, _c_sz, _c_int, _c_vp]),
     "triteia_hip_bmm_scratch_bytes": (_c_sz, [_c_int] * 4),
+    "triteia_hip_uniform_ktile": (_c_int, [_c_int] * 5),
     "triteia_hip_uniform_kernel": (_c_int, [_c_int] * 5),
     "triteia_hip_sbmm_2_4": (_c_int, [_c_vp] * 8 + [_c_int] * 4 + [_c_vp, _c_int, _c_int, _c_vp] + [_c_int] * 4),
     "triteia_hip_sbmm_2_4_bounded": (_c_int, [_c_vp] * 8 + [_c_int] * 4 + [_c_vp, _c_int, _c_int, _c_vp] + [_c_int] * 5),
@@ -63,6 +64,7 @@ SIGNATURES = {
     "triteia_hip_lora_shrink": (_c_int, [_c_vp, _c_long, _c_vp, _c_vp] + [_c_int] * 6 + [_c_vp, _c_sz, _c_int, _c_int, _c_vp]),
     "triteia_hip_lora_expand": (_c_int, [_c_vp, _c_long, _c_vp, _c_vp] + [_c_int] * 5 + [_c_float] + [_c_int] * 3 + [_c_vp]),
     "triteia_hip_dense_ok": (_c_int, [_c_int] * 3),
+    "triteia_hip_dense_tile": (_c_int, [_c_int] * 3),
     "triteia_hip_dense_scratch_bytes": (_c_sz, [_c_int] * 3),
     "triteia_hip_dense": (_c_int, [_c_vp, _c_long, _c_vp, _c_long, _c_vp] + [_c_int] * 3 + [_c_vp, _c_sz, _c_int, _c_vp]),
     "triteia_hip_pack_2_4": (_c_int, [_c_vp] * 5 + [_c_int] * 3 + [_c_vp]),
