@@ -1907,23 +1907,10 @@ bool dense_pays(int tokens, int m, int k) {
   return t.intake <= 15 || t.intake <= 2.15 * t.hbm;
 }
 
-// more than 64 KB of LDS has to be granted once per device and kernel
-std::mutex g_dense_mutex;
 template <int NT, int TW, int F, int FW, int STAGES>
 int launch_dense_tile(const DenseArgs& a, hipStream_t st) {
   using Tile = DenseTile<NT, TW, F, FW, STAGES>;
-  static bool ready[kMaxDevicesForAttr] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevicesForAttr) return fail(TRITEIA_HIP_ERR_RUNTIME, "dense_base_kernel: no current device");
-  if (Tile::kLdsBytes > 65536) {
-    std::lock_guard<std::mutex> lock(g_dense_mutex);
-    if (!ready[dev]) {
-      if (hipFuncSetAttribute(reinterpret_cast<const void*>(&dense_base_kernel<NT, TW, F, FW, STAGES>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                              Tile::kLdsBytes) != hipSuccess)
-        return fail(TRITEIA_HIP_ERR_RUNTIME, "dense_base_kernel: cannot reserve %d bytes of LDS", Tile::kLdsBytes);
-      ready[dev] = true;
-    }
-  }
+  if (int e = grant_lds<dense_base_kernel<NT, TW, F, FW, STAGES>>(Tile::kLdsBytes, "dense_base_kernel")) return e;
   const long units = (long)((a.m + Tile::kFeatures - 1) / Tile::kFeatures) * ((a.tokens + Tile::kTokens - 1) / Tile::kTokens) * a.splits;
   hipLaunchKernelGGL((dense_base_kernel<NT, TW, F, FW, STAGES>), dim3((unsigned)((units + 7) / 8 * 8)), dim3(Tile::kThreads), Tile::kLdsBytes, st, a);
   return check_launch("dense_base_kernel");
