@@ -136,3 +136,25 @@ def test_activations_that_are_not_aligned_stay_with_the_kernels_before():
     a, b = (ops.sbmm_4bit_2_4_native(gq, v, gm, gs, gi) for v in (shifted, gx))
     # (the same exact products added up in another order, in fp32, and rounded once)
     assert ((a.float() - b.float()).norm() / b.float().norm()).item() < 1e-4
+
+
+def test_a_plan_for_small_batches_asks_for_aligned_activations():
+    """A batch that triteia_hip_sbmm_2_4_routed_own plans for the K-splitting tiles is routed in the kernel, the workspace untouched, if its
+    activations start inside 16 bytes: it is their address that counts, not the weights'."""
+    n, t, k, m = 2, 64, 8192, 256
+    qw, meta, s = make_deltas(n, k, m, 3)
+    idx = (np.arange(t) % (n + 1) - 1).astype(np.int32)
+    gq, gm, gs, gx, gi = to_gpu(qw, meta, s, activations(t, k, 5), idx)
+    shifted = torch.empty(t * k + 4, dtype=torch.float16, device="cuda")[4:].view(t, k)
+    shifted.copy_(gx)
+    lib = _ffi.lib()
+    assert lib.triteia_hip_planned_ktile(t, n, m, k) > 0 and gx.data_ptr() % 16 == 0 == gq.data_ptr() % 16
+    outs = []
+    for x in (gx, shifted):
+        out = torch.full((t, m), 9.0, dtype=torch.float16, device="cuda")
+        ws = torch.full((lib.triteia_hip_sbmm_routed_workspace_bytes(t, n),), 0x5a, dtype=torch.uint8, device="cuda")
+        assert lib.triteia_hip_sbmm_2_4_routed_own(x.data_ptr(), gq.data_ptr(), gm.data_ptr(), out.data_ptr(), gs.data_ptr(), gi.data_ptr(), 0, n, m, t, k,
+                                                   ws.data_ptr(), ws.numel(), 2, 0, torch.cuda.current_stream().cuda_stream) == 0
+        assert bool((ws != 0x5a).any()) is (x is gx)
+        outs.append(out)
+    assert torch.equal(*outs)

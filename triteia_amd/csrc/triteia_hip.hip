@@ -1145,6 +1145,8 @@ static bool ktile_plan_can(int prob_n, int prob_k) {
   // (whole 128-deep K steps; 32-bit byte offsets of rows of activations)
   return prob_k % 128 == 0 && (long)prob_n * prob_k * 2 < (1L << 32);
 }
+// (its direct loads of the activations are of 16 bytes; rows of a multiple of 128 elements start where the first does)
+static bool ktile_plan_reads(const void* activations) { return reinterpret_cast<uintptr_t>(activations) % 16 == 0; }
 // Whether a planned batch's full 64-token tiles (or all of its tokens in such tiles) go to a launch of the wide kernel behind the streaming
 // kernel's.  That kernel needs whole 128-deep K steps and addresses activations with 32-bit byte offsets, and a batch that could not
 // reach the bar even with most of its tokens in wide tiles (one per 48 tokens) is not worth the empty launch.  Nor is one whose tiles
@@ -1323,7 +1325,7 @@ int triteia_hip_sbmm_2_4_planned(const void* A, const void* B, const void* meta,
       }
     }
   }
-  if (reinterpret_cast<uintptr_t>(B) % 16 == 0 && ktile_plan_takes(prob_n, n_deltas, prob_m, prob_k))
+  if (ktile_plan_reads(A) && ktile_plan_takes(prob_n, n_deltas, prob_m, prob_k))
     return launch_ktile_plan(a, prob_n, n_deltas, ws, L, static_cast<hipStream_t>(stream));
   // The plan's tiles are cut without knowledge of the layer.  Where they make a launch of very few
   // workgroups on this layer (one or two deltas, a narrow matrix: fewer than 200 even on the plan's
@@ -1405,7 +1407,7 @@ static int sbmm_routed(const void* A, const void* B, const void* meta, void* C, 
   // plan's kernel for it cannot take, it is routed in the kernel there too)
   const bool eager_ok = routed_eager_ok(prob_n, n_deltas);
   const bool plan_better = own_workspace && workspace && workspace_bytes >= triteia_hip_sbmm_routed_workspace_bytes(prob_n, n_deltas) &&
-                           (reinterpret_cast<uintptr_t>(workspace) | reinterpret_cast<uintptr_t>(B)) % 16 == 0 &&
+                           reinterpret_cast<uintptr_t>(workspace) % 16 == 0 && ktile_plan_reads(A) &&
                            ktile_plan_beats_in_kernel(prob_n, n_deltas, prob_m, prob_k);
   if (routed_in_kernel(prob_n, n_deltas, prob_m, prob_k) && !plan_better) {
     // small batch: the multiply kernel routes by itself, no plan, no workspace traffic
