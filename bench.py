@@ -227,12 +227,10 @@ def kernel_name(wl, lib, in_kernel):
         return {0: "sparse24_grouped_kernel", 16: "sparse24_share16_kernel", 32: "sparse24_wide_kernel<32 tokens>", 33: "sparse24_wide_kernel<32 tokens, 8 wavefronts>",
                 64: "sparse24_wide_kernel<64 tokens>", 65: "sparse24_wide_kernel<64 tokens, 8 wavefronts>",
                 256: "sparse24_tile256_kernel"}.get(code, f"kernel code {code}")
-    if in_kernel:
+    if in_kernel or (wl.index_offset and lib.triteia_hip_routed_leaves_workspace(wl.tokens, wl.n_deltas, wl.m, wl.k)):
         if lib.triteia_hip_routed_in_kernel(wl.tokens, wl.n_deltas, wl.m, wl.k) == 2:
             return "sparse24_share16_kernel (routes in-kernel)"
         return "sparse24_grouped_kernel (routes in-kernel)"
-    if wl.index_offset:
-        return "sparse24_grouped_kernel"
     kt = lib.triteia_hip_planned_ktile(wl.tokens, wl.n_deltas, wl.m, wl.k)
     if kt:
         return f"sparse24_ktile_plan_kernel<up to {kt} tokens a tile>"
