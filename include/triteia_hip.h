@@ -320,6 +320,14 @@ TRITEIA_HIP_API int triteia_hip_lora_shrink(const void* x, long x_stride, const 
 TRITEIA_HIP_API int triteia_hip_lora_expand(void* y, long y_stride, const void* b, const void* scratch, int n_tokens, int n_adapters, int k,
                             int r, int m, float scale, int accumulate, int bf16, int dev, void* stream);
 
+/* The same product in one launch, without a scratch: every workgroup of a tile repeats x @ A for its own columns.  For what the
+ * pair takes with k % 64 == 0 and r <= 64 (and m % 8 == 0); triteia_hip_lora_ok is 1 where the ops take it, 0 where they take the pair (or
+ * neither takes the shape). */
+TRITEIA_HIP_API int triteia_hip_lora_ok(int n_tokens, int n_adapters, int k, int r, int m);
+TRITEIA_HIP_API int triteia_hip_lora(void* y, long y_stride, const void* x, long x_stride, const void* a, const void* b, const void* indices,
+                     int index64, int n_tokens, int n_adapters, int k, int r, int m, float scale, int accumulate, int bf16, int dev,
+                     void* stream);
+
 /* out[n_tokens, prob_m] = x[n_tokens, prob_k] @ weight[prob_m, prob_k]^T, fp16 with fp32 sums: the dense base weight of a
  * layer (F.linear's layout) for the tokens of a routed batch.  At most 256 tokens, prob_m % 8 == 0, prob_k % 64 == 0,
  * and not up to 16 tokens on less than 2^20 weights; rows x_stride / w_stride elements apart, everything aligned to 16

@@ -81,6 +81,120 @@ __device__ __forceinline__ void load_to_lds(const void* src, void* dst) {
 }
 __device__ __forceinline__ void wait_for_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
+// Inclusive sum over a wavefront's lanes (six additions on the vector ALU; through shuffles, which go by LDS, they took 0.3 us).
+__device__ __forceinline__ int lane_sums(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);     // row_shr:1, 2, 4, 8: inside rows of 16 lanes
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);     // row_bcast:15: a row's last lane to the row behind (rows 1 and 3)
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);     // row_bcast:31: the first half's sum to rows 2 and 3
+  return v;
+}
+
+// Every workgroup routes by itself: the tile (TT tokens of one adapter, in batch order) that is number `tile` of the batch, its
+// token rows in s_rows.  All of the workgroup's wavefronts call it; all wavefronts are past their last use of s.idx and s.hist when it
+// returns a tile.
+struct LoraTile {
+  int bin;        // adapter; n_adapters: tokens without one; -1: no such tile
+  int start;      // first list position: adapters in ascending order, their tokens in the batch's
+  int count;      // tokens
+};
+template <int THREADS, int TT>
+struct LoraRouteTables {
+  uint16_t* idx;      // [tokens]
+  int* hist;          // [adapters + 1]
+  int* wave_count;    // [THREADS / 64]
+  int* rows;          // [TT]
+};
+template <int THREADS, int TT, class T>
+__device__ __forceinline__ LoraTile lora_find_tile(const LoraArgs<T>& a, const int tile, const LoraRouteTables<THREADS, TT>& s) {
+  constexpr int WAVES = THREADS / 64;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int none = a.n_adapters;                               // bin of the tokens without an adapter
+
+  auto count = [&](int t, long v) {
+    const int d = v >= 0 && v < none ? (int)v : none;
+    s.idx[t] = (uint16_t)d;
+    atomicAdd(&s.hist[d], 1);                                  // (integer counts: the order does not matter)
+  };
+  auto count_all = [&](auto* indices) {
+    if (a.n_tokens <= THREADS) {
+      const long v = tid < a.n_tokens ? (long)indices[tid] : 0;   // (on its way while the bins are cleared)
+      for (int i = tid; i <= none; i += THREADS) s.hist[i] = 0;
+      __syncthreads();
+      if (tid < a.n_tokens) count(tid, v);
+      return;
+    }
+    for (int i = tid; i <= none; i += THREADS) s.hist[i] = 0;
+    __syncthreads();
+    // (four requests a lane in flight: the pair, 1000 tokens over 8 adapters of rank 64 19.25 -> 18.95 us, 2000 over 16 of rank 16 23.5 -> 22.5)
+    for (int t = tid; t < a.n_tokens; t += 4 * THREADS) {
+      long v[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) v[i] = indices[min(t + THREADS * i, a.n_tokens - 1)];
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        if (t + THREADS * i < a.n_tokens) count(t + THREADS * i, v[i]);
+    }
+  };
+  if (a.index64) count_all(static_cast<const long*>(a.indices));
+  else count_all(static_cast<const int*>(a.indices));
+  __syncthreads();
+
+  // the bin that the tile belongs to, its tokens' first list position and the tile's number inside the bin
+  int bin = -1, bin_tokens = 0, start = 0, in_bin = 0;
+  for (int base = 0, before = 0; base <= none; base += 64) {   // (before: tiles << 16 | tokens of the bins so far)
+    const int b = base + lane;
+    const int c = b > none || (b == none && a.accumulate) ? 0 : s.hist[b];
+    const int own = ((c + TT - 1) / TT) << 16 | c;
+    const int incl = lane_sums(own) + before, excl = incl - own;
+    const unsigned long long hit = __ballot(tile >= (excl >> 16) && tile < (incl >> 16));
+    if (hit) {
+      const int src = __ffsll((long long)hit) - 1;
+      bin = base + src;
+      bin_tokens = __builtin_amdgcn_readlane(c, src);
+      const int e = __builtin_amdgcn_readlane(excl, src);
+      start = e & 0xffff;
+      in_bin = tile - (e >> 16);
+      break;
+    }
+    before = __builtin_amdgcn_readlane(incl, 63);
+  }
+  if (bin < 0) return {-1, 0, 0};
+  const int rank0 = in_bin * TT;
+  const int cnt = min(TT, bin_tokens - rank0);
+  const int pieces = (a.n_tokens + 63) >> 6, per_wave = (pieces + WAVES - 1) / WAVES;
+  const int first = wave * per_wave, last = min(pieces, first + per_wave);
+  int rank = -rank0;
+  if (per_wave == 1) {
+    // one piece a wavefront: each counts the pieces before its own itself
+#pragma unroll
+    for (int w = 0; w < WAVES - 1; w++)
+      if (w < wave) rank += __popcll(__ballot(64 * w + lane < a.n_tokens && s.idx[64 * w + lane] == bin));
+  } else {
+    int mine = 0;
+    for (int ch = first; ch < last; ch++) {
+      const int t = ch * 64 + lane;
+      mine += __popcll(__ballot(t < a.n_tokens && s.idx[t] == bin));
+    }
+    if (lane == 0) s.wave_count[wave] = mine;
+    __syncthreads();
+    for (int w = 0; w < wave; w++) rank += s.wave_count[w];
+  }
+  for (int ch = first; ch < last; ch++) {
+    const int t = ch * 64 + lane;
+    const bool member = t < a.n_tokens && s.idx[t] == bin;
+    const unsigned long long members = __ballot(member);
+    const int at = rank + __popcll(members & ((1ull << lane) - 1ull));
+    if (member && at >= 0 && at < cnt) s.rows[at] = t;
+    rank += __popcll(members);
+  }
+  __syncthreads();
+  return {bin, start + rank0, cnt};
+}
+
 // R16: 16-rank tiles (r <= 16 R16); NT: 16-token tiles.  grid (tiles, shares of K), block 256.
 template <class T, int R16, int NT>
 __global__ __launch_bounds__(256) void lora_shrink_kernel(const LoraArgs<T> a) {
@@ -96,90 +210,13 @@ __global__ __launch_bounds__(256) void lora_shrink_kernel(const LoraArgs<T> a) {
   __shared__ int s_rows[TT];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int none = a.n_adapters;                               // bin of the tokens without an adapter
-
-  for (int i = tid; i <= none; i += 256) s_hist[i] = 0;
-  __syncthreads();
-  auto count = [&](int t, long v) {
-    const int d = v >= 0 && v < none ? (int)v : none;
-    s_idx[t] = (uint16_t)d;
-    atomicAdd(&s_hist[d], 1);                                  // (integer counts: the order does not matter)
-  };
-  auto count_all = [&](auto* indices) {
-    int t = tid;
-    // from three requests a lane on: four in flight (the pair, 1000 tokens over 8 adapters of rank 64 19.25 -> 18.95 us, 2000 over 16 of
-    // rank 16 23.5 -> 22.5; on 100 tokens the longer code costs more than it gives, 8.6 -> 9.4 with eight shares in flight in
-    // the expand as well)
-    for (; a.n_tokens > 512 && t < a.n_tokens; t += 4 * 256) {
-      long v[4];
-#pragma unroll
-      for (int i = 0; i < 4; i++) v[i] = indices[min(t + 256 * i, a.n_tokens - 1)];
-#pragma unroll
-      for (int i = 0; i < 4; i++)
-        if (t + 256 * i < a.n_tokens) count(t + 256 * i, v[i]);
-    }
-    for (; t < a.n_tokens; t += 256) count(t, indices[t]);
-  };
-  if (a.index64) count_all(static_cast<const long*>(a.indices));
-  else count_all(static_cast<const int*>(a.indices));
-  __syncthreads();
-
-  // the bin that this tile belongs to, its tokens' first list position and its number inside the bin
-  const int tile = blockIdx.x;
-  int bin = -1, bin_tokens = 0, start = 0, in_bin = 0;
-  for (int base = 0, before = 0; base <= none; base += 64) {   // (before: tiles << 16 | tokens of the bins so far)
-    const int b = base + lane;
-    const int c = b > none || (b == none && a.accumulate) ? 0 : s_hist[b];
-    const int own = ((c + TT - 1) / TT) << 16 | c;
-    int incl = own;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int up = __shfl_up(incl, off, 64);
-      if (lane >= off) incl += up;
-    }
-    incl += before;
-    const int excl = incl - own;
-    const unsigned long long hit = __ballot(tile >= (excl >> 16) && tile < (incl >> 16));
-    if (hit) {
-      const int src = __ffsll((long long)hit) - 1;
-      const int e = __shfl(excl, src, 64);
-      bin = base + src;
-      bin_tokens = __shfl(c, src, 64);
-      start = e & 0xffff;
-      in_bin = tile - (e >> 16);
-      break;
-    }
-    before = __shfl(incl, 63, 64);
-  }
+  const int none = a.n_adapters, tile = blockIdx.x;
+  const LoraTile found = lora_find_tile<256, TT>(a, tile, {s_idx, s_hist, s_wave_count, s_rows});
+  const int bin = found.bin, start = found.start, cnt = found.count;
   if (bin < 0) {
     if (blockIdx.y == 0 && tid == 0) a.tiles[tile] = make_int4(0, 0, 0, 0);
     return;
   }
-  const int rank0 = in_bin * TT;
-  const int cnt = min(TT, bin_tokens - rank0);
-  {
-    const int chunks = (a.n_tokens + 63) >> 6, per_wave = (chunks + 3) >> 2;
-    const int first = wave * per_wave, last = min(chunks, first + per_wave);
-    int mine = 0;
-    for (int ch = first; ch < last; ch++) {
-      const int t = ch * 64 + lane;
-      mine += __popcll(__ballot(t < a.n_tokens && s_idx[t] == bin));
-    }
-    if (lane == 0) s_wave_count[wave] = mine;
-    __syncthreads();
-    int rank = -rank0;
-    for (int w = 0; w < wave; w++) rank += s_wave_count[w];
-    for (int ch = first; ch < last; ch++) {
-      const int t = ch * 64 + lane;
-      const bool member = t < a.n_tokens && s_idx[t] == bin;
-      const unsigned long long members = __ballot(member);
-      const int at = rank + __popcll(members & ((1ull << lane) - 1ull));
-      if (member && at >= 0 && at < cnt) s_rows[at] = t;
-      rank += __popcll(members);
-    }
-    __syncthreads();
-  }
-  start += rank0;
   if (blockIdx.y == 0) {
     if (tid == 0) a.tiles[tile] = make_int4(bin == none ? -1 : bin, start, cnt, 0);
     if (tid < cnt) a.perm[start + tid] = s_rows[tid];

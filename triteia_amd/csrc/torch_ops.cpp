@@ -232,6 +232,16 @@ int lora_expand(const Tensor& y, const Tensor& A, const Tensor& B, const Tensor&
                                  (float)scale, accumulate, y.scalar_type() == at::kBFloat16, dev, stream);
 }
 
+// (one launch, where triteia_hip_lora_ok says that it pays)
+bool lora_at_once(const Tensor& A, const Tensor& B, const Tensor& x) {
+  return triteia_hip_lora_ok(x.size(0), A.size(0), A.size(1), A.size(2), B.size(2));
+}
+int lora_fused(const Tensor& y, const Tensor& x, const Tensor& A, const Tensor& B, const Tensor& indices, double scale, bool accumulate, int dev, void* stream) {
+  return triteia_hip_lora(y.data_ptr(), y.size(1), x.data_ptr(), x.size(1), A.data_ptr(), B.data_ptr(), indices.data_ptr(),
+                          indices.scalar_type() == at::kLong, x.size(0), A.size(0), A.size(1), A.size(2), B.size(2), (float)scale, accumulate,
+                          x.scalar_type() == at::kBFloat16, dev, stream);
+}
+
 // lora(weights_A, weights_B, x, indices, base or None, scale): ops.lora_bgmv / lora_sgmv / lora_sgmv_routed
 Tensor lora(const Args& a) {
   if (a.n != 6 || !a.tensor(0) || !a.tensor(1) || !a.tensor(2) || !a.tensor(3)) return {};
@@ -241,8 +251,13 @@ Tensor lora(const Args& a) {
   if (bytes == 0) return {};
   const Place at_(x);
   const Tensor xc = x.is_contiguous() ? x : x.contiguous();
-  const Tensor scratch = scratch_bytes(bytes, x);
   const bool base = !a.none(4);
+  if (lora_at_once(A, B, x)) {
+    Tensor y = base ? base_product(xc, a[4], at_) : at::empty({x.size(0), B.size(2)}, x.options());
+    must_launch(lora_fused(y, xc, A, B, indices, a.number, base, at_.dev, at_.handle()));
+    return y;
+  }
+  const Tensor scratch = scratch_bytes(bytes, x);
   if (!launched(lora_shrink(xc, A, indices, scratch, base, at_.dev, at_.handle()))) return {};
   // (without a base weight every row is written by the expand: tokens without an adapter get zeros)
   Tensor y = base ? base_product(xc, a[4], at_) : at::empty({x.size(0), B.size(2)}, x.options());
@@ -298,9 +313,8 @@ class Beside {
 // Below either bound: 4096 x 4096 with 768 tokens 66-114 -> 76-115, 1024 x 1024 with 4096 59-72 -> 99-129, 8192 x 13824 with
 // 1024 307-534 -> 302-541.  In a captured graph the fork costs more than it hides at every size (11008 x 4096, 32 + 32
 // models, 1024 / 4096 tokens of rank 16: 275 -> 300 / 546 -> 576).
-bool lora_beside(int64_t tokens, int64_t k, int64_t m) {
-  return tokens >= 2048 && tokens * k >= (int64_t(1) << 35) / m && c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None;
-}
+bool lora_hides(int64_t tokens, int64_t k, int64_t m) { return tokens >= 2048 && tokens * k >= (int64_t(1) << 35) / m; }
+bool captured() { return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None; }
 
 // ldmm(indices, x, LwA, LwB, DeltaW, metas, ss, base or None): ops.ldmm.
 Tensor ldmm(const Args& a) {
@@ -314,10 +328,18 @@ Tensor ldmm(const Args& a) {
   if (bytes == 0 || q.size(0) > kMaxRoutedDeltas || !packed_ok(q, meta, s, x, q.size(0), k, m) || !base_ok(a, 7, x, k, m)) return {};
   const Place at_(x);
   const Tensor xc = x.is_contiguous() ? x : x.contiguous();
-  const Tensor scratch = scratch_bytes(bytes, x);
   const Tensor idx = indices.scalar_type() == at::kInt ? indices : indices.to(at::kInt);
   const bool base = !a.none(7);
-  if (base && lora_beside(x.size(0), k, m)) {
+  const bool large = base && lora_hides(x.size(0), k, m);      // (the pair on either one stream or two: the same bits in a graph)
+  if (!large && lora_at_once(A, B, x)) {
+    // (without a base weight the LoRA launch stores the adapters' rows and zeros in all others, the deltas' among them)
+    Tensor y = base ? base_product(xc, a[7], at_) : at::empty({x.size(0), m}, x.options());
+    must_launch(lora_fused(y, xc, A, B, indices, 1.0, base, at_.dev, at_.handle()));
+    must_launch(routed(xc, q, meta, s, idx, y, A.size(0), 1, at_));
+    return y;
+  }
+  const Tensor scratch = scratch_bytes(bytes, x);
+  if (large && !captured()) {
     Tensor y;                  // (like the other buffers ahead of the stream: freed only after it has been joined)
     Beside side(at_);
     if (!launched(lora_shrink(xc, A, indices, scratch, true, at_.dev, side.handle()))) return {};

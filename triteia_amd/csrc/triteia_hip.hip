@@ -12,6 +12,7 @@
 
 #include "dense_base.hip.h"
 #include "lora.hip.h"
+#include "lora_fused.hip.h"
 #include "lora_mfma.hip.h"
 #include "lora_routed.hip.h"
 #include "pack.hip.h"
@@ -63,7 +64,7 @@ struct Knobs {
   int nt = 0, xcd_swizzle = 1, xcd_cgs = 0 /* 0: the rule, n > 0: blocks of n column groups, -1: never */, wide_order_min_idle = kUnset, pass_nt = 0;
   int wide = 1, wide_min_units = kUnset, wide_min_batch = 256, plan_wide_min_units = kUnset;
   int wide32_min_units = kUnset, wide32_max_units = kUnset, wide32_ksplit_max_units = kUnset, wide64_ksplit_max_units = kUnset;
-  int mid = 1, mid64_max_k = 0x7fffffff, mid_min_column_groups = 16, mid_min_units = kUnset, mid_min_half_tokens = 7, mid_narrow = 1, mid_depth = 0, plan_big = 1, plan_all64 = 1, lora_mfma = 1;
+  int mid = 1, mid64_max_k = 0x7fffffff, mid_min_column_groups = 16, mid_min_units = kUnset, mid_min_half_tokens = 7, mid_narrow = 1, mid_depth = 0, plan_big = 1, plan_all64 = 1, lora_mfma = 1, lora_fused = 1;
   int eager = 1, fused_route = 1;
   int dense = 1, plan_ktile = 1, ktile = 1, tile256 = 1, tile256_min_units = kUnset, tile256_max_units = kUnset, ksplit = 1, sub_shift = kUnset, share16 = 1, share16_max_blocks = kUnset;
 };
@@ -79,7 +80,7 @@ void read_knobs() {
       {"WIDE32_MIN_UNITS", &k.wide32_min_units}, {"WIDE32_MAX_UNITS", &k.wide32_max_units},
       {"WIDE32_KSPLIT_MAX_UNITS", &k.wide32_ksplit_max_units}, {"WIDE64_KSPLIT_MAX_UNITS", &k.wide64_ksplit_max_units},
       {"MID", &k.mid}, {"MID64_MAX_K", &k.mid64_max_k}, {"MID_MIN_COLUMN_GROUPS", &k.mid_min_column_groups},
-      {"MID_MIN_UNITS", &k.mid_min_units}, {"MID_MIN_HALF_TOKENS", &k.mid_min_half_tokens}, {"MID_NARROW", &k.mid_narrow}, {"MID_DEPTH", &k.mid_depth}, {"PLAN_BIG", &k.plan_big}, {"PLAN_ALL64", &k.plan_all64}, {"LORA_MFMA", &k.lora_mfma}, {"EAGER", &k.eager}, {"FUSED_ROUTE", &k.fused_route},
+      {"MID_MIN_UNITS", &k.mid_min_units}, {"MID_MIN_HALF_TOKENS", &k.mid_min_half_tokens}, {"MID_NARROW", &k.mid_narrow}, {"MID_DEPTH", &k.mid_depth}, {"PLAN_BIG", &k.plan_big}, {"PLAN_ALL64", &k.plan_all64}, {"LORA_MFMA", &k.lora_mfma}, {"LORA_FUSED", &k.lora_fused}, {"EAGER", &k.eager}, {"FUSED_ROUTE", &k.fused_route},
       {"DENSE", &k.dense}, {"KTILE", &k.ktile}, {"PLAN_KTILE", &k.plan_ktile}, {"TILE256", &k.tile256}, {"TILE256_MIN_UNITS", &k.tile256_min_units}, {"TILE256_MAX_UNITS", &k.tile256_max_units},
       {"KSPLIT", &k.ksplit}, {"SUB_SHIFT", &k.sub_shift}, {"SHARE16", &k.share16}, {"SHARE16_MAX_BLOCKS", &k.share16_max_blocks},
   };
@@ -1807,6 +1808,89 @@ int lora_expand_impl(void* y, long y_stride, const void* w, const void* scratch,
 }
 #undef LORA_PICK
 
+// The product in one launch (lora_fused_kernel): tiles of 16 tokens, of 32 from 32 tokens an adapter on; as many chunks of columns as make
+// about a workgroup per CU on the bound on the tiles, at most one per eight pieces of 64 (one a wavefront).  A tile's chunks run on one XCD, whose
+// 32 CUs hold a workgroup each: one more of them there than that is a second round (11 adapters of rank 8 on 1152 x 12032 11.5 us with
+// 23 chunks, 6.4 with 16).
+struct LoraFusedCut {
+  int r16, nt, tiles, chunks, columns;
+};
+LoraFusedCut lora_fused_cut(int n_tokens, int n_adapters, int r, int m) {
+  LoraFusedCut c;
+  c.r16 = r <= 16 ? 1 : r <= 32 ? 2 : 4;
+  const int groups = n_adapters < n_tokens ? n_adapters : n_tokens;
+  c.nt = n_tokens < 32 * groups ? 1 : 2;
+  c.tiles = lora_max_tiles(n_tokens, n_adapters, 16 * c.nt);
+  const int pieces = (m + 63) / 64;
+  int chunks = c.tiles < 8 ? 256 / c.tiles : 32 / ((c.tiles + 7) / 8);
+  if (chunks > (pieces + 7) / 8) chunks = (pieces + 7) / 8;
+  if (chunks < 1) chunks = 1;
+  c.columns = 64 * ((pieces + chunks - 1) / chunks);
+  c.chunks = (m + c.columns - 1) / c.columns;
+  return c;
+}
+bool lora_fused_can(int n_tokens, int n_adapters, int k, int r, int m) {
+  return lora_routed_takes(n_tokens, n_adapters, k, r) && k % 64 == 0 && r <= 64 && m >= 0 && m % 8 == 0;
+}
+// Where it takes the place of the pair: as long as what a workgroup reads for its first product, (rank + tokens of a tile) x k halves, is little
+// enough: about 40 KB are in flight on a CU at a time, so it costs a microsecond per 40 - 90 KB, where the pair spreads the same over
+// all CUs.  The lines were drawn on 1500 random calls (1 .. 2048 tokens over 2 .. 64 adapters of rank 8 .. 64, k and m 512 .. 13824, evenly routed
+// and Zipf, fp16 and bf16): one launch against the pair in a graph / called one by one, where up to 64 tokens the pair's two launches
+// are the host's 8 us:
+//   up to 64 tokens   up to 96 KB 0.92 / 0.78, to 128 KB 1.02 / 0.89, to 256 KB 1.13 / 0.97;
+//   up to 256         up to 128 KB 0.90 / 0.83, to 256 KB 1.00 / 0.95;
+//   more              up to 400 KB 0.86 / 0.85, to 512 KB 0.96 / 0.95, past that 1.03 / 1.01
+// (worst 1.27 in a graph: 63 tokens over 62 adapters, half of whose tiles the routing leaves empty).  Rank 128 never (1.1 - 2.5); below k = 512
+// some wavefronts have no step.
+bool lora_fused_takes(int n_tokens, int n_adapters, int k, int r, int m) {
+  if (!knobs().lora_fused || m == 0 || !lora_fused_can(n_tokens, n_adapters, k, r, m)) return false;
+  if (knobs().lora_fused == 2) return true;
+  const LoraFusedCut c = lora_fused_cut(n_tokens, n_adapters, r, m);
+  const long read = (long)((r < 16 ? 16 : r) + 16 * c.nt) * k * 2;
+  return k >= 512 && read <= 1024L * (n_tokens <= 64 ? 96 : n_tokens <= 256 ? 128 : 400);
+}
+template <class T, int R16, int NT>
+int launch_lora_fused(const LoraFusedArgs<T>& a, hipStream_t st) {
+  using Tile = LoraFusedTile<R16, NT>;
+  if (int e = grant_lds<lora_fused_kernel<T, R16, NT>>(Tile::kLdsBytes, "lora_fused_kernel")) return e;
+  const unsigned grid = (unsigned)(a.tiles >= 8 ? (a.tiles + 7) / 8 * 8 : a.tiles) * a.chunks;
+  hipLaunchKernelGGL((lora_fused_kernel<T, R16, NT>), dim3(grid), dim3(Tile::kThreads), Tile::kLdsBytes, st, a);
+  return check_launch("lora_fused_kernel");
+}
+template <class T>
+int lora_fused_impl(void* y, long y_stride, const void* x, long x_stride, const void* wa, const void* wb, const void* indices, int index64, int n_tokens,
+                    int n_adapters, int k, int r, int m, float scale, int accumulate, hipStream_t st) {
+  const LoraFusedCut c = lora_fused_cut(n_tokens, n_adapters, r, m);
+  LoraFusedArgs<T> a;
+  memset(&a, 0, sizeof(a));
+  a.l.x = static_cast<const T*>(x);
+  a.l.x_stride = x_stride;
+  a.l.a = static_cast<const T*>(wa);
+  a.l.b = static_cast<const T*>(wb);
+  a.l.y = static_cast<T*>(y);
+  a.l.y_stride = y_stride;
+  a.l.indices = indices;
+  a.l.index64 = index64;
+  a.l.n_tokens = n_tokens;
+  a.l.n_adapters = n_adapters;
+  a.l.k = k;
+  a.l.r = r;
+  a.l.m = m;
+  a.l.scale = scale;
+  a.l.accumulate = accumulate;
+  a.tiles = c.tiles;
+  a.chunks = c.chunks;
+  a.columns = c.columns;
+  switch (c.r16 * 10 + c.nt) {
+    case 11: return launch_lora_fused<T, 1, 1>(a, st);
+    case 12: return launch_lora_fused<T, 1, 2>(a, st);
+    case 21: return launch_lora_fused<T, 2, 1>(a, st);
+    case 22: return launch_lora_fused<T, 2, 2>(a, st);
+    case 41: return launch_lora_fused<T, 4, 1>(a, st);
+    default: return launch_lora_fused<T, 4, 2>(a, st);
+  }
+}
+
 }  // namespace
 
 extern "C" {
@@ -1831,6 +1915,24 @@ int triteia_hip_lora_shrink(const void* x, long x_stride, const void* a, const v
   hipStream_t st = static_cast<hipStream_t>(stream);
   return bf16 ? lora_shrink_impl<bf16_t>(x, x_stride, a, indices, index64, n_tokens, n_adapters, k, r, accumulate, scratch, st)
               : lora_shrink_impl<_Float16>(x, x_stride, a, indices, index64, n_tokens, n_adapters, k, r, accumulate, scratch, st);
+}
+
+int triteia_hip_lora_ok(int n_tokens, int n_adapters, int k, int r, int m) { return lora_fused_takes(n_tokens, n_adapters, k, r, m); }
+
+int triteia_hip_lora(void* y, long y_stride, const void* x, long x_stride, const void* a, const void* b, const void* indices, int index64, int n_tokens,
+                     int n_adapters, int k, int r, int m, float scale, int accumulate, int bf16, int dev, void* stream) {
+  if (n_tokens == 0 || m == 0) return TRITEIA_HIP_OK;
+  if (!lora_fused_can(n_tokens, n_adapters, k, r, m))
+    return fail(TRITEIA_HIP_ERR_KERN_SHAPE, "lora: tokens=%d adapters=%d k=%d r=%d m=%d", n_tokens, n_adapters, k, r, m);
+  if (!y || !x || !a || !b || !indices) return fail(TRITEIA_HIP_ERR_ARGUMENT, "lora: null tensor pointer");
+  if ((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) % 16 != 0 ||
+      x_stride % 8 != 0 || y_stride % 8 != 0)
+    return fail(TRITEIA_HIP_ERR_ARGUMENT, "lora: x, y, their rows and the adapters must be 16-byte aligned");
+  DeviceGuard g(dev);
+  if (!g.ok) return fail(TRITEIA_HIP_ERR_RUNTIME, "cannot select device %d", dev);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  return bf16 ? lora_fused_impl<bf16_t>(y, y_stride, x, x_stride, a, b, indices, index64, n_tokens, n_adapters, k, r, m, scale, accumulate, st)
+              : lora_fused_impl<_Float16>(y, y_stride, x, x_stride, a, b, indices, index64, n_tokens, n_adapters, k, r, m, scale, accumulate, st);
 }
 
 int triteia_hip_lora_expand(void* y, long y_stride, const void* b, const void* scratch, int n_tokens, int n_adapters, int k, int r, int m,

@@ -63,6 +63,8 @@ SIGNATURES = {
     "triteia_hip_lora_scratch_bytes": (_c_sz, [_c_int] * 4),
     "triteia_hip_lora_shrink": (_c_int, [_c_vp, _c_long, _c_vp, _c_vp] + [_c_int] * 6 + [_c_vp, _c_sz, _c_int, _c_int, _c_vp]),
     "triteia_hip_lora_expand": (_c_int, [_c_vp, _c_long, _c_vp, _c_vp] + [_c_int] * 5 + [_c_float] + [_c_int] * 3 + [_c_vp]),
+    "triteia_hip_lora_ok": (_c_int, [_c_int] * 5),
+    "triteia_hip_lora": (_c_int, [_c_vp, _c_long, _c_vp, _c_long, _c_vp, _c_vp, _c_vp] + [_c_int] * 6 + [_c_float] + [_c_int] * 3 + [_c_vp]),
     "triteia_hip_dense_ok": (_c_int, [_c_int] * 3),
     "triteia_hip_dense_tile": (_c_int, [_c_int] * 3),
     "triteia_hip_dense_scratch_bytes": (_c_sz, [_c_int] * 3),
