@@ -171,6 +171,32 @@ __device__ __forceinline__ _Float16 scaled_sum_f16(_Float16 old, float acc, _Flo
   return (_Float16)sum;
 }
 
+// Sixteen tokens x 128 columns of fp16 results in a wavefront's registers, from the order of the accumulators of the wide tiles -- v[j] of
+// lane (token r, q) is columns 32 q + 8 j .. + 7 -- to the order in which whole rows leave -- v[i] is columns 8 r .. + 7 of token 4 i + q --
+// and back, through 4 KB of LDS that only this wavefront uses (16-byte pieces swizzled by row: no bank conflicts).  Stored in the order
+// of the accumulators a request writes 64 pieces of 16 bytes in as many cache lines, in the other four rows of 256 bytes.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+__device__ __forceinline__ void to_rows(half8_t (&v)[4], unsigned char* place, int r, int q) {
+#pragma unroll
+  for (int j = 0; j < 4; j++) *reinterpret_cast<half8_t*>(place + r * 256 + ((4 * q + j) ^ r) * 16) = v[j];
+  wave_lds_fence();
+#pragma unroll
+  for (int i = 0; i < 4; i++) v[i] = *reinterpret_cast<const half8_t*>(place + (4 * i + q) * 256 + (r ^ (4 * i + q)) * 16);
+  wave_lds_fence();
+}
+__device__ __forceinline__ void from_rows(half8_t (&v)[4], unsigned char* place, int r, int q) {
+#pragma unroll
+  for (int i = 0; i < 4; i++) *reinterpret_cast<half8_t*>(place + (4 * i + q) * 256 + (r ^ (4 * i + q)) * 16) = v[i];
+  wave_lds_fence();
+#pragma unroll
+  for (int j = 0; j < 4; j++) v[j] = *reinterpret_cast<const half8_t*>(place + r * 256 + ((4 * q + j) ^ r) * 16);
+  wave_lds_fence();
+}
+
 // Workgroup barrier that orders LDS traffic only: outstanding global loads (the prefetch
 // ring) are not waited for.
 __device__ __forceinline__ void lds_barrier() {

@@ -333,32 +333,39 @@ __global__ __launch_bounds__(512, 1) void sparse24_tile256_kernel(const Sparse24
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no direct load may outlive the block's LDS
 
+  __syncthreads();                                     // every wavefront has read its last tile: the memory of the x tiles is free
   if (!active) return;
-  // epilogue: lane (n = r, qq = q) holds features 32q + 8j + c of token tq*64 + 16nt + r
+  // epilogue: lane (n = r, qq = q) holds features 32q + 8j + c of token tq*64 + 16nt + r; whole rows leave (to_rows)
   const _Float16* sc = p.scales + (long)delta * p.scales_stride + cb * 128 + 32 * q;
   half8_t sv[4];
 #pragma unroll
   for (int j = 0; j < 4; j++) sv[j] = *reinterpret_cast<const half8_t*>(sc + 8 * j);
+  static_assert(kT256XStages * kT256XStageBytes >= 8 * 4096, "");
+  unsigned char* place = xs + 4096 * wave;
 #pragma unroll
   for (int nt = 0; nt < 4; nt++) {
-    const int slot = tq * 64 + nt * 16 + r;
-    if (slot >= cnt) continue;
-    _Float16* op = p.out + (long)s_rows[slot] * p.out_stride + cb * 128 + 32 * q;
-    // (when the sums are added to what is there: a token's four pieces are requested together, ahead of the arithmetic)
-    half8_t olds[4];
+    const int slot0 = tq * 64 + nt * 16;
+    if (slot0 >= cnt) break;
+    _Float16* op[4];
 #pragma unroll
-    for (int j = 0; j < 4; j++) olds[j] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+    for (int i = 0; i < 4; i++) op[i] = p.out + (long)s_rows[slot0 + 4 * i + q] * p.out_stride + cb * 128 + 8 * r;
+    // (when the sums are added to what is there: a tile's rows are requested together, ahead of the arithmetic)
+    half8_t o[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) o[i] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
     if (p.accumulate) {
 #pragma unroll
-      for (int j = 0; j < 4; j++) olds[j] = *reinterpret_cast<const half8_t*>(op + 8 * j);
+      for (int i = 0; i < 4; i++) o[i] = *reinterpret_cast<const half8_t*>(op[i]);
+      from_rows(o, place, r, q);
     }
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      half8_t o;
+    for (int j = 0; j < 4; j++)
 #pragma unroll
-      for (int c = 0; c < 8; c++) o[c] = scaled_sum_f16(olds[j][c], acc[c][nt][j], sv[j][c]);
-      *reinterpret_cast<half8_t*>(op + 8 * j) = o;
-    }
+      for (int c = 0; c < 8; c++) o[j][c] = scaled_sum_f16(o[j][c], acc[c][nt][j], sv[j][c]);
+    to_rows(o, place, r, q);
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      if (slot0 + 4 * i + q < cnt) *reinterpret_cast<half8_t*>(op[i]) = o[i];
   }
 }
 
