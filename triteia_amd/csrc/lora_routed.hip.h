@@ -27,6 +27,7 @@ namespace triteia_hip {
 
 constexpr int kLoraMaxTokens = 4096;      // indices in LDS
 constexpr int kLoraMaxAdapters = 1024;    // histogram in LDS
+constexpr int kLoraMaxSplits = 8;         // shares of K
 constexpr int kLoraExpandCols = 256;      // output columns of an expand workgroup
 
 template <class T>
@@ -332,23 +333,30 @@ __global__ __launch_bounds__(256) void lora_expand_kernel(const LoraArgs<T> a) {
     else *reinterpret_cast<lvec8<T>*>(patch + piece * 16) = lvec8<T>{0, 0, 0, 0, 0, 0, 0, 0};
   }
   const int j = lane & 15, q = lane >> 4;
-  const int col = c0 + 64 * wave + 16 * q;           // this lane's 16 output columns
+  const int col = c0 + 64 * wave + 8 * q;            // this lane's output columns: col .. + 7 and col + 32 .. + 39
   int rows[NT];
 #pragma unroll
   for (int nt = 0; nt < NT; nt++) rows[nt] = a.perm[d.y + min(16 * nt + j, cnt - 1)];
-  // the intermediate: the shares of K in order, rounded once
+  // the intermediate: the shares of K in order, rounded once (eight ranks of a token at a time, all shares requested together)
   for (int e = tid; e < TT * 2 * R16; e += 256) {
     const int tok = e / (2 * R16), f = (e - tok * (2 * R16)) * 8;
     lvec8<T> o = {0, 0, 0, 0, 0, 0, 0, 0};
     if (tok < cnt && f < a.r) {
-      lm_float4 lo = {0.f, 0.f, 0.f, 0.f}, hi = {0.f, 0.f, 0.f, 0.f};
       const float* p = a.partial + (long)(d.y + tok) * a.r + f;
-#pragma unroll 4
-      for (int z = 0; z < a.splits; z++) {
-        const lm_float4 l = *reinterpret_cast<const lm_float4*>(p), h = *reinterpret_cast<const lm_float4*>(p + 4);
+      lm_float4 part[kLoraMaxSplits][2];
 #pragma unroll
-        for (int i = 0; i < 4; i++) { lo[i] += l[i]; hi[i] += h[i]; }
+      for (int z = 0; z < kLoraMaxSplits; z++) {
+        if (z >= a.splits) break;
+        part[z][0] = *reinterpret_cast<const lm_float4*>(p);
+        part[z][1] = *reinterpret_cast<const lm_float4*>(p + 4);
         p += (long)a.n_tokens * a.r;
+      }
+      lm_float4 lo = {0.f, 0.f, 0.f, 0.f}, hi = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int z = 0; z < kLoraMaxSplits; z++) {
+        if (z >= a.splits) break;
+#pragma unroll
+        for (int i = 0; i < 4; i++) { lo[i] += part[z][0][i]; hi[i] += part[z][1][i]; }
       }
 #pragma unroll
       for (int i = 0; i < 4; i++) { o[i] = (T)lo[i]; o[4 + i] = (T)hi[i]; }
@@ -361,7 +369,7 @@ __global__ __launch_bounds__(256) void lora_expand_kernel(const LoraArgs<T> a) {
 #pragma unroll
     for (int h = 0; h < 2; h++) {
       old[nt][h] = lvec8<T>{0, 0, 0, 0, 0, 0, 0, 0};
-      if (a.accumulate) old[nt][h] = *reinterpret_cast<const lvec8<T>*>(a.y + (long)rows[nt] * a.y_stride + min(col + 8 * h, a.m - 8));
+      if (a.accumulate) old[nt][h] = *reinterpret_cast<const lvec8<T>*>(a.y + (long)rows[nt] * a.y_stride + min(col + 32 * h, a.m - 8));
     }
   wait_for_loads();
   __syncthreads();
@@ -379,8 +387,9 @@ __global__ __launch_bounds__(256) void lora_expand_kernel(const LoraArgs<T> a) {
     const int row = 16 * rt + 4 * q + (j >> 2);
 #pragma unroll
     for (int cc = 0; cc < 4; cc++) {
-      // A row 4 q' + i of MFMA cc = column 16 q' + 4 cc + i of the wavefront's 64: a lane of D ends up with 16 adjacent columns
-      const int c = 8 * wave + 2 * (j & 3) + (cc >> 1);
+      // A row 4 q' + i of MFMA cc = column 32 (cc / 2) + 8 q' + 4 (cc % 2) + i of the wavefront's 64: a lane of D ends up with two runs of
+      // 8 columns, and a store of four lanes with 64 consecutive bytes of a token
+      const int c = 8 * wave + 4 * (cc >> 1) + (j & 3);
       const lvec4<T> A = lds_read_transposed<T>(patch + row * 512 + ((c ^ (row & 31)) * 16) + 8 * (cc & 1));
 #pragma unroll
       for (int nt = 0; nt < NT; nt++) acc[cc][nt] = LoraMfma16<T>::run(A, B[nt], acc[cc][nt]);
@@ -392,11 +401,11 @@ __global__ __launch_bounds__(256) void lora_expand_kernel(const LoraArgs<T> a) {
     T* yp = a.y + (long)rows[nt] * a.y_stride + col;
 #pragma unroll
     for (int h = 0; h < 2; h++) {
-      if (col + 8 * h >= a.m) continue;
+      if (col + 32 * h >= a.m) continue;
       lvec8<T> o;
 #pragma unroll
       for (int i = 0; i < 8; i++) o[i] = (T)__builtin_fmaf(acc[2 * h + (i >> 2)][nt][i & 3], a.scale, (float)old[nt][h][i]);
-      *reinterpret_cast<lvec8<T>*>(yp + 8 * h) = o;
+      *reinterpret_cast<lvec8<T>*>(yp + 32 * h) = o;
     }
   }
 }

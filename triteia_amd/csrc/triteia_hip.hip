@@ -1737,7 +1737,7 @@ LoraCut lora_cut(int n_tokens, int n_adapters, int k, int r) {
   c.max_tiles = lora_max_tiles(n_tokens, n_adapters, 16 * c.nt);
   const int steps = k / 32;
   int splits = 192 / c.max_tiles;
-  splits = splits < 1 ? 1 : splits > 8 ? 8 : splits;
+  splits = splits < 1 ? 1 : splits > kLoraMaxSplits ? kLoraMaxSplits : splits;
   int per = (steps + splits - 1) / splits;
   if (per < 4) per = 4;
   c.splits = (steps + per - 1) / per;
