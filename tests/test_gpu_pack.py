@@ -3,6 +3,7 @@ import pytest
 import torch
 
 from triteia_amd.python.capi._native import native
+from triteia_amd.python.ops.utils.generator import fp16_to_sparse
 from triteia_amd.python.ops.utils.sparsity import mask_creator, prune_pack_2_4, unpack_nibbles
 
 pytestmark = pytest.mark.gpu
@@ -82,3 +83,43 @@ def test_pack_kernels_quotient_on_every_pair_of_fp16_values():
         want = _quantised(every[first:first + rows].reshape(-1, 1), s)
         assert torch.equal(got, want), f"weights {first} .. {first + rows - 1}"
         print(f"[pairs] weights {first} .. {first + rows - 1}", flush=True)
+
+
+@pytest.mark.parametrize("shape", [(96,), (1, 192), (192, 1)])
+def test_fp16_to_sparse_in_one_call_and_step_by_step(shape):
+    """What the one native call answers is what the moves, views and the packing give one by one, and it answers for plain tensors on
+    the current GPU only."""
+    g = torch.Generator(device="cuda").manual_seed(9)
+    m = max(shape) // 64 * 64
+    w = (torch.randn((160, m), generator=g, device="cuda") * 0.02).half()
+    s = (w.abs().amax(0) * (2 / 15)).reshape([m if d > 1 else 1 for d in shape])
+    got = fp16_to_sparse(w, s)
+    packed = prune_pack_2_4(w, s.reshape(1, -1))
+    assert got[0] is w and got[2].data_ptr() == s.data_ptr()
+    for a, b in zip(got, (w, packed[0], packed[2], packed[1], packed[3])):
+        assert a.shape == b.shape and a.dtype == b.dtype and torch.equal(a, b)
+    assert native().sparse(w, s) is not None
+    wide = torch.zeros((160, 2 * m), dtype=torch.float16, device="cuda")
+    wide[:, :m] = w
+    for args in ((wide[:, :m], s), (w.float(), s), (w, s.float()), (w.cpu(), s), (w, s.cpu()), (w, s[:-1] if s.dim() == 1 else s.flatten()[:-1]),
+                 (w[:-1], s), (w, s.clone().requires_grad_())):
+        assert native().sparse(*args) is None
+    for a, b in zip(fp16_to_sparse(wide[:, :m], s.cpu()), got):
+        assert torch.equal(a, b)
+
+
+def test_fp16_to_sparse_follows_function_modes():
+    class Seen(torch.overrides.TorchFunctionMode):
+        calls = 0
+
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            Seen.calls += 1
+            return func(*args, **(kwargs or {}))
+
+    w, s = torch.ones((64, 128), dtype=torch.float16, device="cuda"), torch.ones((1, 128), dtype=torch.float16, device="cuda")
+    want = fp16_to_sparse(w, s)
+    with Seen():
+        got = fp16_to_sparse(w, s)
+    assert Seen.calls > 0
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)

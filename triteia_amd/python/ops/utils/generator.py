@@ -32,6 +32,11 @@ def fp16_to_sparse(weights, scale, device="cuda", mask=None):
 
     Returns (weights, qweight, scales, meta, meta_raw), the reference's five values (generator.py:105-123);
     `meta_raw` is the metadata before the kernel's re-layout: int16 [m, k/16], row = output column."""
+    if mask is None and device == "cuda" and weights.is_cuda:
+        from triteia_amd.python.capi._native import native
+        packed = native().sparse(weights, scale)
+        if packed is not None:
+            return packed
     weights = weights.to(device)
     scale = scale.to(device).reshape(1, -1)
     qweight, meta, s, raw = prune_pack_2_4(weights, scale, mask)
