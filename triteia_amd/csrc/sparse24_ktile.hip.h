@@ -149,6 +149,13 @@ __device__ __forceinline__ void ktile_run(const Sparse24Args& p, unsigned char* 
     __builtin_amdgcn_sched_barrier(0);
   };
 
+  // The scales of this thread's 8 columns (the same ones for every 16 tokens), for the epilogue of an unsplit uniform launch, ahead of the
+  // loop: among the sums they are a round trip to memory for every 16 tokens (loads are not moved across a barrier).  100 tokens on
+  // 4096 x 11008 14.3 -> 13.3 us, 1315 on 3328 x 640 12.5 -> 12.3.  Tiles of 64 tokens have no registers to keep them in: behind the loop, once.
+  // (a plan's tiles, mostly of 16 or 32 tokens, lost 0.7 - 1.3 % by either)
+  const _Float16* sc = p.scales + (long)delta * p.scales_stride + cb * 128;
+  half8_t scales = {0, 0, 0, 0, 0, 0, 0, 0};
+  if (!PLAN && NT < 4 && splits == 1) scales = *reinterpret_cast<const half8_t*>(sc + (tid & 15) * 8);
   WFrag ring[2];
   if (n > 0) issue_x(0);
   __builtin_amdgcn_sched_barrier(0);
@@ -164,13 +171,18 @@ __device__ __forceinline__ void ktile_run(const Sparse24Args& p, unsigned char* 
     __builtin_amdgcn_sched_barrier(0);
   }
   asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+  if (!PLAN && NT == 4 && splits == 1) scales = *reinterpret_cast<const half8_t*>(sc + (tid & 15) * 8);
 
-  // the wavefronts' sums, added in order, 16 tokens at a time
-  const _Float16* sc = p.scales + (long)delta * p.scales_stride + cb * 128;
+  // the wavefronts' sums, added in order, 16 tokens at a time, each of the first 256 threads 8 columns of one (as a loop over such pieces,
+  // which ran once, 2436 tokens over 8 plan deltas of 1280 x 1536 took 21.3 us instead of 20.8)
   float(*red)[16][kRedStride] = reinterpret_cast<float(*)[16][kRedStride]>(smem);
+  static_assert(64 * KW >= 256, "a thread for every 8 columns of 16 tokens");
+  const int tok = tid >> 4, f0 = (tid & 15) * 8;
 #pragma unroll
   for (int nt = 0; nt < NT; nt++) {
     if (first + 16 * nt >= count) break;
+    const int t = PLAN ? 16 * nt + tok : tile_start(nt) + tok;
+    const bool live = tid < 256 && t < count && (PLAN || t >= first + 16 * nt);
     lds_barrier();
     float* dst = &red[wave][r][32 * q];
 #pragma unroll
@@ -179,42 +191,32 @@ __device__ __forceinline__ void ktile_run(const Sparse24Args& p, unsigned char* 
       *reinterpret_cast<float4_t*>(dst + 8 * j + 4) = float4_t{acc[4][nt][j], acc[5][nt][j], acc[6][nt][j], acc[7][nt][j]};
     }
     lds_barrier();
-    for (int e = tid; e < 256; e += 64 * KW) {
-      const int tok = e >> 4, f0 = (e & 15) * 8;
-      long row;
-      if (PLAN) {
-        if (16 * nt + tok >= count) continue;
-        row = s_rows[16 * nt + tok];
-      } else {
-        const int t = tile_start(nt) + tok;
-        if (t < first + 16 * nt || t >= count) continue;
-        row = row0 + t;
-      }
-      float v[8];
+    if (!live) continue;
+    const long row = PLAN ? s_rows[t] : row0 + t;
+    float v[8];
 #pragma unroll
-      for (int i = 0; i < 8; i++) v[i] = 0.f;
+    for (int i = 0; i < 8; i++) v[i] = 0.f;
 #pragma unroll
-      for (int w = 0; w < KW; w++) {
-        const float4_t a0 = *reinterpret_cast<const float4_t*>(&red[w][tok][f0]);
-        const float4_t a1 = *reinterpret_cast<const float4_t*>(&red[w][tok][f0 + 4]);
+    for (int w = 0; w < KW; w++) {
+      const float4_t a0 = *reinterpret_cast<const float4_t*>(&red[w][tok][f0]);
+      const float4_t a1 = *reinterpret_cast<const float4_t*>(&red[w][tok][f0 + 4]);
 #pragma unroll
-        for (int i = 0; i < 4; i++) { v[i] += a0[i]; v[4 + i] += a1[i]; }
-      }
-      if (!PLAN && splits > 1) {
-        float* pp = p.partial + ((long)z * p.partial_rows + row) * p.m + cb * 128 + f0;
-        *reinterpret_cast<float4_t*>(pp) = float4_t{v[0], v[1], v[2], v[3]};
-        *reinterpret_cast<float4_t*>(pp + 4) = float4_t{v[4], v[5], v[6], v[7]};
-        continue;
-      }
-      const half8_t sv = *reinterpret_cast<const half8_t*>(sc + f0);
-      _Float16* op = p.out + row * p.out_stride + cb * 128 + f0;
-      half8_t old = {0, 0, 0, 0, 0, 0, 0, 0};
-      if (PLAN && p.accumulate) old = *reinterpret_cast<const half8_t*>(op);
-      half8_t o;
-#pragma unroll
-      for (int i = 0; i < 8; i++) o[i] = scaled_sum_f16(old[i], v[i], sv[i]);
-      *reinterpret_cast<half8_t*>(op) = o;
+      for (int i = 0; i < 4; i++) { v[i] += a0[i]; v[4 + i] += a1[i]; }
     }
+    if (!PLAN && splits > 1) {
+      float* pp = p.partial + ((long)z * p.partial_rows + row) * p.m + cb * 128 + f0;
+      *reinterpret_cast<float4_t*>(pp) = float4_t{v[0], v[1], v[2], v[3]};
+      *reinterpret_cast<float4_t*>(pp + 4) = float4_t{v[4], v[5], v[6], v[7]};
+      continue;
+    }
+    const half8_t sv = PLAN ? *reinterpret_cast<const half8_t*>(sc + f0) : scales;
+    _Float16* op = p.out + row * p.out_stride + cb * 128 + f0;
+    half8_t old = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (PLAN && p.accumulate) old = *reinterpret_cast<const half8_t*>(op);
+    half8_t o;
+#pragma unroll
+    for (int i = 0; i < 8; i++) o[i] = scaled_sum_f16(old[i], v[i], sv[i]);
+    *reinterpret_cast<half8_t*>(op) = o;
   }
 }
 
