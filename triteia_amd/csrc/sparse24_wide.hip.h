@@ -368,27 +368,21 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void sparse24_wide_kerne
   else
     k_loop(std::integral_constant<int, NT>{});
 
+  float* red = reinterpret_cast<float*>(&xs[0][0][0][0]) + wave * (32 * NT * 64) + lane;   // (KS = 2)
   if (KS == 2) {
     // the second half's sums go to the first half through the memory of the activation rings (same size:
-    // 2048 * TOK bytes), register by register with consecutive lanes side by side
+    // 2048 * TOK bytes), register by register with consecutive lanes side by side, 8 KB for every 16 tokens
     __syncthreads();   // every wavefront has read its last tile
-    float* red = reinterpret_cast<float*>(&xs[0][0][0][0]) + wave * (32 * NT * 64) + lane;
     if (kh == 1) {
-#pragma unroll
-      for (int cc = 0; cc < 8; cc++)
-#pragma unroll
-        for (int nt = 0; nt < NT; nt++)
-#pragma unroll
-          for (int j = 0; j < 4; j++) red[((cc * NT + nt) * 4 + j) * 64] = acc[cc][nt][j];
-    }
-    __syncthreads();
-    if (kh == 1) return;
-#pragma unroll
-    for (int cc = 0; cc < 8; cc++)
 #pragma unroll
       for (int nt = 0; nt < NT; nt++)
 #pragma unroll
-        for (int j = 0; j < 4; j++) acc[cc][nt][j] += red[((cc * NT + nt) * 4 + j) * 64];
+        for (int cc = 0; cc < 8; cc++)
+#pragma unroll
+          for (int j = 0; j < 4; j++) red[((nt * 8 + cc) * 4 + j) * 64] = acc[cc][nt][j];
+    }
+    __syncthreads();
+    if (kh == 1) return;
   }
   if (KS == 1) __syncthreads();                   // every wavefront has read its last tile: the rings' memory is free
   if (!active) return;
@@ -398,14 +392,20 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void sparse24_wide_kerne
   half8_t sv[4];
 #pragma unroll
   for (int j = 0; j < 4; j++) sv[j] = *reinterpret_cast<const half8_t*>(sc + 8 * j);
-  // (this wavefront's part of the rings: with K halved inside the workgroup it is where it has just read the second half's sums)
-  unsigned char* place = reinterpret_cast<unsigned char*>(&xs[0][0][0][0]) + wave * (256 * KS * TOK);
+  // (this wavefront's part of the rings: with K halved inside the workgroup each 16 tokens' results turn where their second half's sums
+  // were, which are added 16 tokens at a time: all at once they do not fit the registers of the 64-token build)
 #pragma unroll
   for (int nt = 0; nt < NT; nt++) {
     if (16 * nt >= cnt) break;
-    _Float16* op[4];
+    unsigned char* place = reinterpret_cast<unsigned char*>(&xs[0][0][0][0]) + wave * (256 * KS * TOK) + nt * (4096 * KS);
+    if (KS == 2) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) op[i] = p.out + (long)s_rows[16 * nt + 4 * i + q] * p.out_stride + cb * 128 + 8 * r;
+      for (int cc = 0; cc < 8; cc++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc[cc][nt][j] += red[((nt * 8 + cc) * 4 + j) * 64];
+      wave_lds_fence();
+    }
+    auto at = [&](int i) { return p.out + (long)s_rows[16 * nt + 4 * i + q] * p.out_stride + cb * 128 + 8 * r; };
     // (when the sums are added to what is there: a tile's rows are requested together, ahead of the arithmetic.  All tiles at once would
     // be one round trip in all, but holds 16 registers per tile, which the 64-token builds do not have.)
     half8_t o[4];
@@ -413,7 +413,7 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void sparse24_wide_kerne
     for (int i = 0; i < 4; i++) o[i] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
     if (p.accumulate) {
 #pragma unroll
-      for (int i = 0; i < 4; i++) o[i] = *reinterpret_cast<const half8_t*>(op[i]);
+      for (int i = 0; i < 4; i++) o[i] = *reinterpret_cast<const half8_t*>(at(i));
       from_rows(o, place, r, q);
     }
 #pragma unroll
@@ -423,7 +423,7 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void sparse24_wide_kerne
     to_rows(o, place, r, q);
 #pragma unroll
     for (int i = 0; i < 4; i++)
-      if (16 * nt + 4 * i + q < cnt) *reinterpret_cast<half8_t*>(op[i]) = o[i];
+      if (16 * nt + 4 * i + q < cnt) *reinterpret_cast<half8_t*>(at(i)) = o[i];
   }
 }
 
