@@ -241,6 +241,17 @@ def test_which_base_products_the_library_takes(monkeypatch):
     assert [ok(*shape) for shape in left] == [1] * 5 + [0] * 3
 
 
+def test_which_lora_calls_take_one_launch():
+    """triteia_hip_lora_ok (tokens, adapters, k, r, m): not where a workgroup's columns are many, however little it reads for the first product."""
+    ok = _ffi.lib().triteia_hip_lora_ok
+    _ffi.reload_env()
+    taken = [(16, 16, 1024, 16, 2048), (600, 8, 2048, 32, 2048), (100, 32, 1536, 16, 11008), (16, 16, 1024, 16, 12928), (1375, 46, 1280, 64, 4096),
+             (4, 64, 512, 8, 13824), (600, 8, 2048, 32, 13824)]
+    left = [(62, 62, 1024, 16, 12928), (63, 62, 1024, 16, 12928), (60, 54, 768, 8, 10496), (101, 58, 896, 8, 13824),     # few tokens an adapter
+            (1375, 46, 1280, 64, 13312), (1334, 45, 2432, 8, 13056), (307, 62, 1536, 64, 13440), (1603, 60, 1152, 8, 11648)]
+    assert [c for c in taken if not ok(*c)] == [] and [c for c in left if ok(*c)] == []
+
+
 def test_bench_refuses_more_than_one_gpu():
     import subprocess
     import sys

@@ -1832,22 +1832,30 @@ LoraFusedCut lora_fused_cut(int n_tokens, int n_adapters, int r, int m) {
 bool lora_fused_can(int n_tokens, int n_adapters, int k, int r, int m) {
   return lora_routed_takes(n_tokens, n_adapters, k, r) && k % 64 == 0 && r <= 64 && m >= 0 && m % 8 == 0;
 }
-// Where it takes the place of the pair: as long as what a workgroup reads for its first product, (rank + tokens of a tile) x k halves, is little
-// enough: about 40 KB are in flight on a CU at a time, so it costs a microsecond per 40 - 90 KB, where the pair spreads the same over
-// all CUs.  The lines were drawn on 1500 random calls (1 .. 2048 tokens over 2 .. 64 adapters of rank 8 .. 64, k and m 512 .. 13824, evenly routed
-// and Zipf, fp16 and bf16): one launch against the pair in a graph / called one by one, where up to 64 tokens the pair's two launches
-// are the host's 8 us:
-//   up to 64 tokens   up to 96 KB 0.92 / 0.78, to 128 KB 1.02 / 0.89, to 256 KB 1.13 / 0.97;
-//   up to 256         up to 128 KB 0.90 / 0.83, to 256 KB 1.00 / 0.95;
-//   more              up to 400 KB 0.86 / 0.85, to 512 KB 0.96 / 0.95, past that 1.03 / 1.01
-// (worst 1.27 in a graph: 63 tokens over 62 adapters, half of whose tiles the routing leaves empty).  Rank 128 never (1.1 - 2.5); below k = 512
-// some wavefronts have no step.
+// Where it takes the place of the pair.  A workgroup walks all of K for its first product and all of its columns for the second, where the pair
+// spreads both over all CUs, so both are limited:
+//   * what it reads for the first product, (rank + tokens of a tile) x k halves.  One launch against the pair on 34754 random calls (1 .. 2048
+//     tokens over 2 .. 64 adapters of rank 8 .. 64, k and m 512 .. 13824, evenly routed and Zipf, fp16 and bf16), in a graph / called one by
+//     one, where up to 64 tokens the pair's two launches are the host's 8 us:
+//       up to 64 tokens   up to 96 KB 0.88 / 0.68, to 128 KB 0.92 / 0.74, to 256 KB 0.99 / 0.81, past that 1.16 / 1.00;
+//       up to 256         up to 128 KB 0.87 / 0.76, to 256 KB 0.93 / 0.85, to 400 KB 0.99 / 0.94, past that 1.09 / 1.06;
+//       more              up to 400 KB 0.81 / 0.79, to 512 KB 0.86 / 0.86, past that 0.90 / 0.90.
+//   * its columns.  There are as many chunks of them as fit one round on the bound on the tiles: many tiles on a wide layer leave each workgroup
+//     a long way to go, and a bound far above the live tiles leaves CUs without one.  Inside the lines above, in a graph:
+//       fewer than 3 tokens an adapter   up to 1536 columns 0.87, to 2048 0.99 (worst 1.12), past that 1.03 (1.40);
+//       up to 8                          up to 2048 0.88, to 3072 0.95 (1.08), past that 1.02 (1.26);
+//       more                             up to 4096 0.82, past that 1.01 (1.37: 1375 tokens over 46 adapters, one chunk of 13312 columns).
+// Of what it takes, one call in 1400 is more than 5 % behind the pair, none more than 7 %.  ldmm, whose other launches hide the host's share, has
+// the same rule: there the whole call takes 0.94 of its time with the pair in a graph, and none of 4374 more than 1.05.
+// Rank 128 never (1.1 - 2.5); below k = 512 some wavefronts have no step.
 bool lora_fused_takes(int n_tokens, int n_adapters, int k, int r, int m) {
   if (!knobs().lora_fused || m == 0 || !lora_fused_can(n_tokens, n_adapters, k, r, m)) return false;
   if (knobs().lora_fused == 2) return true;
   const LoraFusedCut c = lora_fused_cut(n_tokens, n_adapters, r, m);
   const long read = (long)((r < 16 ? 16 : r) + 16 * c.nt) * k * 2;
-  return k >= 512 && read <= 1024L * (n_tokens <= 64 ? 96 : n_tokens <= 256 ? 128 : 400);
+  const int groups = n_adapters < n_tokens ? n_adapters : n_tokens;
+  const int most = n_tokens < 3 * groups ? 1536 : n_tokens < 8 * groups ? 2048 : 4096;
+  return k >= 512 && c.columns <= most && read <= 1024L * (n_tokens <= 64 ? 96 : n_tokens <= 256 ? 128 : 400);
 }
 template <class T, int R16, int NT>
 int launch_lora_fused(const LoraFusedArgs<T>& a, hipStream_t st) {
