@@ -44,13 +44,12 @@ struct LoraFusedTile {
   static constexpr int kVStride = kRanks + 8, kVBytes = kTokens * kVStride * 2;
   static constexpr int kRingBytes = kWaves * kWaveBytes;
   static constexpr int kLdsBytes = kRingBytes + kRedBytes + kVBytes + 4 * kTokens + 4 * kWaves;
-  static constexpr int kTogether = kLdsBytes <= 81920 ? 2 : 1;       // workgroups on a CU
-  static_assert(kLdsBytes <= 163840, "");
+  static_assert(kLdsBytes > 81920 && kLdsBytes <= 163840, "one workgroup on a CU");
   static_assert(kRingBytes >= 2 * kLoraMaxTokens + 4 * (kLoraMaxAdapters + 1), "the routing's tables lie in the ring");
 };
 
 template <class T, int R16, int NT>
-__global__ __launch_bounds__((LoraFusedTile<R16, NT>::kThreads), (LoraFusedTile<R16, NT>::kTogether * LoraFusedTile<R16, NT>::kWaves / 4)) void lora_fused_kernel(const LoraFusedArgs<T> p) {
+__global__ __launch_bounds__((LoraFusedTile<R16, NT>::kThreads), (LoraFusedTile<R16, NT>::kWaves / 4)) void lora_fused_kernel(const LoraFusedArgs<T> p) {
   using Tile = LoraFusedTile<R16, NT>;
   constexpr int TT = Tile::kTokens, WAVES = Tile::kWaves, DEPTH = Tile::kDepth, STRIPS = Tile::kStrips;
   constexpr int kLoads = 2 * R16 + 2 * NT;                           // requests of a step

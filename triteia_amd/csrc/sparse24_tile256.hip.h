@@ -349,19 +349,11 @@ __global__ __launch_bounds__(512, 1) void sparse24_tile256_kernel(const Sparse24
     _Float16* op[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) op[i] = p.out + (long)s_rows[slot0 + 4 * i + q] * p.out_stride + cb * 128 + 8 * r;
-    // (when the sums are added to what is there: a tile's rows are requested together, ahead of the arithmetic)
     half8_t o[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) o[i] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
-    if (p.accumulate) {
-#pragma unroll
-      for (int i = 0; i < 4; i++) o[i] = *reinterpret_cast<const half8_t*>(op[i]);
-      from_rows(o, place, r, q);
-    }
 #pragma unroll
     for (int j = 0; j < 4; j++)
 #pragma unroll
-      for (int c = 0; c < 8; c++) o[j][c] = scaled_sum_f16(o[j][c], acc[c][nt][j], sv[j][c]);
+      for (int c = 0; c < 8; c++) o[j][c] = scaled_sum_f16((_Float16)0.f, acc[c][nt][j], sv[j][c]);
     to_rows(o, place, r, q);
 #pragma unroll
     for (int i = 0; i < 4; i++)

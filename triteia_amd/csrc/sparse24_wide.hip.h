@@ -36,6 +36,7 @@ constexpr int kWideStages = 4;        // activation tiles in flight (LDS ring)
 template <int DEPTH, int TOK = kWideTokens, bool PLAN_ALL = false, int KS = 1>
 __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void sparse24_wide_kernel(const Sparse24Args p) {
   constexpr int NT = TOK / 16;
+  constexpr bool ADDS = PLAN_ALL || (TOK == kWideTokens && KS == 1);   // a build that a plan launches (uniform launches store)
   __shared__ __attribute__((aligned(1024))) _Float16 xs[KS][kWideStages][TOK][128];
   __shared__ int s_rows[TOK];
 
@@ -411,7 +412,7 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 2 : 1) void sparse24_wide_kerne
     half8_t o[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) o[i] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
-    if (p.accumulate) {
+    if (ADDS && p.accumulate) {
 #pragma unroll
       for (int i = 0; i < 4; i++) o[i] = *reinterpret_cast<const half8_t*>(at(i));
       from_rows(o, place, r, q);

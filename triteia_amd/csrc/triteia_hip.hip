@@ -756,6 +756,7 @@ size_t uniform_scratch_bytes(int tokens, int n_groups, int m, int k) {
   return split_bytes(splits, tokens, n_groups, m);
 }
 
+// (stores its results; a.accumulate is for launches on a plan or on raw indices)
 int launch_uniform(Sparse24Args a, int tokens, int stride, int delta_step, int n_groups, hipStream_t st,
                    void* scratch = nullptr, size_t scratch_bytes = 0) {
   a.n_groups = n_groups;
@@ -772,7 +773,7 @@ int launch_uniform(Sparse24Args a, int tokens, int stride, int delta_step, int n
                        a.scales, a.scales_stride, tokens, delta_step, a.out, a.out_stride);
     return check_launch("splitk_reduce_kernel");
   };
-  if (!a.accumulate && ktile_takes(tokens, n_groups, a.m, a.k, reinterpret_cast<uintptr_t>(a.x) % 16 == 0 && a.x_stride % 8 == 0)) {
+  if (ktile_takes(tokens, n_groups, a.m, a.k, reinterpret_cast<uintptr_t>(a.x) % 16 == 0 && a.x_stride % 8 == 0)) {
     KTilePick t = pick_ktile(tokens, n_groups, a.m, a.k, true);
     if (t.splits > 1 && !scratch_for(t.splits)) t = pick_ktile(tokens, n_groups, a.m, a.k, false);
     Sparse24Args b = a;
