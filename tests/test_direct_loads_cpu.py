@@ -48,5 +48,6 @@ def test_wait_states_ahead_of_direct_loads(tmp_path):
     assert not early, f"{len(early)} loads right behind their write of M0: {early[0]}"
     assert not base, f"{len(base)} loads within five instructions of their base: {base[0]}"
     # (the kernels that bring their tiles this way are all in there)
-    for part in ("sparse24_wide_kernel", "sparse24_tile256_kernel", "sparse24_ktile_kernel", "sparse24_ktile_plan_kernel", "dense_base_kernel", "lora_shrink_kernel"):
+    for part in ("sparse24_wide_kernel", "sparse24_tile256_kernel", "sparse24_ktile_kernel", "sparse24_ktile_plan_kernel", "dense_base_kernel", "lora_shrink_kernel",
+                 "lora_fused_kernel"):
         assert any(part in kernel for kernel in seen), part

@@ -7,6 +7,7 @@ import torch
 
 from oracle import triteia_oracle as orc
 from tests.helpers import activations, check_close, make_deltas, setknob, to_gpu, watch_native
+from triteia_amd.python.capi import _ffi
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -71,14 +72,16 @@ def test_routed_sbmm_replays(monkeypatch, T, N, k, m, seed):
         assert bool((replayed[torch.from_numpy(hidx < 0).to(DEV)] == 0).all())
 
 
-@pytest.mark.parametrize("path", ["native binding", "python path"])
+@pytest.mark.parametrize("path", ["native binding, pair", "native binding, one launch", "python path"])
 def test_ldmm_replays(monkeypatch, path):
-    """ldmm with a dense base: on one stream as the native binding runs it; on the Python path (what the LoRA pair of the
+    """ldmm with a dense base: on one stream as the native binding runs it, with the LoRA pair and with its product in one launch; on the Python path (what the LoRA pair of the
     binding does not take) the routing and the LoRA shrink fork onto a second stream inside the captured region and join
     before the expand."""
     answered = watch_native(monkeypatch, decline=path == "python path")
     from triteia_amd.python import ops
     T, M, N, k, m, r, seed = 96, 4, 5, 512, 768, 16, 211
+    setknob(monkeypatch, "TRITEIA_HIP_LORA_FUSED", 2 if path == "native binding, one launch" else 0)
+    assert bool(_ffi.lib().triteia_hip_lora_ok(T, M, k, r, m)) == (path == "native binding, one launch")
     print(f"[case] graph replay of ldmm T={T} M={M} N={N} k={k} m={m} r={r}", flush=True)
     qw, meta, s = make_deltas(N, k, m, seed)
     rng = np.random.default_rng(seed + 1)
@@ -110,7 +113,7 @@ def test_ldmm_replays(monkeypatch, path):
         assert torch.equal(replayed, result), f"replay {rep} differs from the eager call"
         y0 = torch.matmul(x, gb.t()).float().cpu().numpy().astype(np.float64)
         check_close(replayed, y0 + orc.ldmm(hidx, hx, A, B, qw, meta, s), what=f"ldmm replay {rep}")
-    assert set(answered) == ({"ldmm"} if path == "native binding" else set())
+    assert set(answered) == ({"ldmm"} if path != "python path" else set())
 
 
 def test_matmul_and_bmm_replay():

@@ -1,15 +1,21 @@
 """The LoRA pair that routes by itself (lora_shrink / lora_expand) against the oracle, at the edges of its tiles, splits
-and layouts."""
+and layouts.  (Its product in one launch, which takes small calls otherwise, is off.)"""
 import numpy as np
 import pytest
 import torch
 
 from oracle import triteia_oracle as orc
+from tests.helpers import setknob
 from triteia_amd.python import ops
-from triteia_amd.python.capi import lora_scratch, lora_shrink
+from triteia_amd.python.capi import _ffi, lora_scratch, lora_shrink
 from triteia_amd.python.capi._native import native
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def pair(monkeypatch):
+    setknob(monkeypatch, "TRITEIA_HIP_LORA_FUSED", 0)
 
 
 @pytest.mark.parametrize("T,M,k,r,m", [
@@ -35,7 +41,7 @@ def test_lora_pair_against_the_oracle(T, M, k, r, m, dtype):
     ref = orc.lora(A, B, x, idx, intermediate=dtype) if dtype == "bf16" else orc.lora(A, B, x, idx)
     tdt = torch.bfloat16 if dtype == "bf16" else torch.float16
     gA, gB, gx = (torch.from_numpy(np.ascontiguousarray(v)).cuda().to(tdt) for v in (A, B, x))
-    assert lora_scratch(T, gA) is not None
+    assert lora_scratch(T, gA) is not None and not _ffi.lib().triteia_hip_lora_ok(T, M, k, r, m)
     # one rounding of the intermediate and one of the result: 2^-11 (2^-8) relative each, and the oracle's own
     tol = 2e-2 if dtype == "bf16" else 2e-3
     scale = max(1e-6, float(np.sqrt(np.mean(np.square(ref.astype(np.float64))))))

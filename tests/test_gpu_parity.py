@@ -6,6 +6,7 @@ mean|d|/mean|ref| < 2e-3 (tests/ops/test_matmul.py:18-22, test_sbmm.py:47-61); L
 additionally allclose(rtol=atol=5e-3) scaled to the output magnitude (tests/ops/test_ldmm.py:73).
 Routing and -1 handling are checked bit-exactly.
 """
+import os
 import sys
 
 import numpy as np
@@ -909,14 +910,24 @@ def test_route_plan_is_a_stable_grouping(plan_rules):
 
 # ------------------------------------------------------------- lora / ldmm
 
-@pytest.fixture(params=["native binding", "python path"])
+@pytest.fixture(params=["native binding, pair", "native binding, one launch", "python path"])
 def answered(request, monkeypatch):
-    """The LoRA and ldmm tests run twice: as the ops are called, where the native binding answers with the pair of kernels
-    that routes by itself, and on the ops' Python path with the kernels of the reference's own interfaces (which still
-    serves what that pair does not take).  The value is the list of calls that the binding answered."""
+    """The LoRA and ldmm tests run as the ops are called, where the native binding answers with the pair of kernels that
+    routes by itself or with its product in one launch (each forced where it can run), and on the ops' Python path with the
+    kernels of the reference's own interfaces (which still serves what that pair does not take).  The value is the list of calls
+    that the binding answered."""
+    setknob(monkeypatch, "TRITEIA_HIP_LORA_FUSED", 2 if request.param == "native binding, one launch" else 0)
     calls = watch_native(monkeypatch, decline=request.param == "python path")
     yield calls
-    assert bool(calls) == (request.param == "native binding")
+    assert bool(calls) == (request.param != "python path")
+
+
+def _say_lora_kernel(T, M, k, r, m):
+    """Under the fixture's knob: the one launch wherever it can run, or nowhere."""
+    from triteia_amd.python.capi import _ffi
+    can = os.environ["TRITEIA_HIP_LORA_FUSED"] == "2" and k % 64 == 0 and r <= 64 and m % 8 == 0
+    assert bool(_ffi.lib().triteia_hip_lora_ok(T, M, k, r, m)) == can
+    say("LoRA in one launch" if can else "LoRA pair")
 
 
 def _lora_weights(M, k, r, m, seed, scale=1.0):
@@ -944,6 +955,7 @@ def _assert_allclose_scaled(got, ref, what):
 ])
 def test_lora_ops(ops, answered, T, M, k, m, r, seed):
     say(f"lora T={T} M={M} k={k} m={m} r={r} seed={seed}")
+    _say_lora_kernel(T, M, k, r, m)
     A, B = _lora_weights(M, k, r, m, seed, scale=0.1)
     x = activations(T, k, seed + 1)
     idx = np.sort(np.random.default_rng(seed + 2).integers(-1, M, size=T)).astype(np.int32)
@@ -1075,6 +1087,7 @@ def test_lora_ops_bf16(ops, answered, T, M, k, m, r, seed):
     and the rank-r intermediate, rounded to bf16 as well, can fall on the other side of a rounding boundary when
     the fp32 sums are taken in another order; the bound here is 1e-2 relative Frobenius error."""
     say(f"lora bf16 T={T} M={M} k={k} m={m} r={r} seed={seed}")
+    _say_lora_kernel(T, M, k, r, m)
     rng = np.random.default_rng(seed)
     A = orc.round_bf16(rng.standard_normal((M, k, r)) * 0.1).astype(np.float32)
     B = orc.round_bf16(rng.standard_normal((M, r, m)) * 0.1).astype(np.float32)
@@ -1099,6 +1112,7 @@ def test_lora_ops_bf16(ops, answered, T, M, k, m, r, seed):
 ])
 def test_ldmm(ops, answered, T, M, N, m, k, r, seed, plan_rules):
     say(f"ldmm T={T} M={M} N={N} m={m} k={k} r={r} seed={seed}")
+    _say_lora_kernel(T, M, k, r, m)
     qw, meta, s = make_deltas(N, k, m, seed)
     A, B = _lora_weights(M, k, r, m, seed + 1, scale=0.05)
     x = activations(T, k, seed + 2)

@@ -13,7 +13,8 @@ class Subclass(torch.Tensor):
 
 
 # function -> its tensor arguments, and what follows them
-FUNCTIONS = {"matmul": (4, ()), "bmm": (4, ()), "sbmm": (5, (None,)), "lora": (4, (None, 1.0)), "ldmm": (7, (None,)), "pack": (2, ())}
+FUNCTIONS = {"matmul": (4, ()), "bmm": (4, ()), "sbmm": (5, (None,)), "lora": (4, (None, 1.0)), "ldmm": (7, (None,)), "pack": (2, ()),
+             "sparse": (2, ())}
 STRANGE = {"none": None, "list": [0, 1], "array": np.zeros(3, dtype=np.int32), "number": 3, "text": "x", "object": object(),
            "subclass": torch.zeros(2, 2).as_subclass(Subclass)}
 
