@@ -9,7 +9,7 @@
 // over a few MB that mostly come from cache.  So
 //   * every workgroup of the shrink routes by itself: the batch's indices (at most 4096) go to LDS with a histogram of
 //     the adapters, a scan over that finds the workgroup's tile (16 NT tokens of one adapter), ballots list its tokens in
-//     batch order.  About a microsecond, against a launch of its own (5 - 7 us with its gap).  The workgroups of a tile's
+//     batch order.  About 2 us, against a launch of its own (5 - 7 us with its gap).  The workgroups of a tile's
 //     first share of K leave the tile and its token rows behind for the expand;
 //   * K is split over gridDim.y so that a few tiles still fill the chip and a wavefront has all of its operands in flight at
 //     once: the adapter's rows by direct-to-LDS loads (a step of 32 k is 64 r consecutive bytes), activations straight into
@@ -18,8 +18,8 @@
 //     k fastest: ds_read_b64_tr_b16 transposes on the way out of LDS (lane i of 16 gives the address of row i / 4, columns
 //     4 (i % 4) ..; it receives column i of the four rows: measured on the device).  16-byte chunks are XOR-swizzled by row.
 // Measured: 100 Zipf-routed tokens over 32 adapters of rank 16 on 4096 x 11008, two transposing copies and the BGMV pair
-// 48 us -> 8.5 us; 1000 tokens over 8 of rank 64 on 4096 x 4096 in bf16, 31 + 9 us of kernels behind 250 us of host round
-// trips -> 19.5 us, of which 8 MB each in and out take 4.
+// 48 us -> 9.2 us a call, 8.4 in a graph; 1000 tokens over 8 of rank 64 on 4096 x 4096 in bf16, 31 + 9 us of kernels behind 250 us of
+// host round trips -> 19.2 us a call, 17.9 in a graph, of which 8 MB each in and out take 4.
 #pragma once
 #include "lora_mfma.hip.h"
 
@@ -130,7 +130,8 @@ __device__ __forceinline__ LoraTile lora_find_tile(const LoraArgs<T>& a, const i
     }
     for (int i = tid; i <= none; i += THREADS) s.hist[i] = 0;
     __syncthreads();
-    // (four requests a lane in flight: the pair, 1000 tokens over 8 adapters of rank 64 19.25 -> 18.95 us, 2000 over 16 of rank 16 23.5 -> 22.5)
+    // (four requests a lane in flight: the pair, 1000 tokens over 8 adapters of rank 64 19.25 -> 18.95 us, 2000 over 16 of rank 16 23.5 -> 22.5;
+    // level at 257 .. 512 tokens, which have two)
     for (int t = tid; t < a.n_tokens; t += 4 * THREADS) {
       long v[4];
 #pragma unroll
@@ -337,7 +338,9 @@ __global__ __launch_bounds__(256) void lora_expand_kernel(const LoraArgs<T> a) {
   int rows[NT];
 #pragma unroll
   for (int nt = 0; nt < NT; nt++) rows[nt] = a.perm[d.y + min(16 * nt + j, cnt - 1)];
-  // the intermediate: the shares of K in order, rounded once (eight ranks of a token at a time, all shares requested together)
+  // the intermediate: the shares of K in order, rounded once (eight ranks of a token at a time, all shares requested together:
+  // against four at a time the pair with eight shares, 400 tokens over 32 adapters of rank 16 on 4096 x 4096 10.0 -> 9.6 us, 512 over 8 of rank 64
+  // in bf16 18.0 -> 17.7, 1000 18.1 -> 17.9; launches of up to four, 100 over 32 of rank 16 on 4096 x 11008 among them, are level)
   for (int e = tid; e < TT * 2 * R16; e += 256) {
     const int tok = e / (2 * R16), f = (e - tok * (2 * R16)) * 8;
     lvec8<T> o = {0, 0, 0, 0, 0, 0, 0, 0};

@@ -149,10 +149,10 @@ __device__ __forceinline__ void ktile_run(const Sparse24Args& p, unsigned char* 
     __builtin_amdgcn_sched_barrier(0);
   };
 
-  // The scales of this thread's 8 columns (the same ones for every 16 tokens), for the epilogue of an unsplit uniform launch, ahead of the
-  // loop: among the sums they are a round trip to memory for every 16 tokens (loads are not moved across a barrier).  100 tokens on
-  // 4096 x 11008 14.3 -> 13.3 us, 1315 on 3328 x 640 12.5 -> 12.3.  Tiles of 64 tokens have no registers to keep them in: behind the loop, once.
-  // (a plan's tiles, mostly of 16 or 32 tokens, lost 0.7 - 1.3 % by either)
+  // The scales of this thread's 8 columns (the same ones for every 16 tokens), for the epilogue of an unsplit uniform launch: among the sums
+  // they are a round trip to memory for every 16 tokens (loads are not moved across a barrier).  Tiles of up to 48 tokens request them
+  // ahead of the loop (1315 tokens on 3328 x 640, in tiles of 32, 12.5 -> 12.3 us); tiles of 64 have no registers to keep them in and request them once,
+  // behind it (100 tokens on 4096 x 11008 14.3 -> 13.4).  A plan's tiles, mostly of 16 or 32 tokens, lost 0.7 - 1.3 % by either.
   const _Float16* sc = p.scales + (long)delta * p.scales_stride + cb * 128;
   half8_t scales = {0, 0, 0, 0, 0, 0, 0, 0};
   if (!PLAN && NT < 4 && splits == 1) scales = *reinterpret_cast<const half8_t*>(sc + (tid & 15) * 8);

@@ -310,10 +310,12 @@ void fill_weights(Sparse24Args& a, const void* A, const void* B, const void* met
 
 
 // 32-token launches of at most one workgroup per CU run with eight wavefronts per workgroup (K split in two inside the
-// workgroup): 20-27 % faster from 160 to 256 units, slower beyond (two rounds of workgroups that fill a CU each).
+// workgroup): 12-20 % faster up to 256 units (4096 x 4096 with 640 / 1024 tokens 31.8 -> 26.8, 33.9 -> 29.8 us, 8192 x 8192 with 320 / 512 56.9 -> 46.4,
+// 60.3 -> 50.9), slower beyond (two rounds of workgroups that fill a CU each; 4096 x 4096 with 1280 44.6 -> 51.3).
 constexpr long kWide32KSplitMaxUnits = 256;
-// The same for 64-token tiles (256 registers, 128 KiB of LDS): 9-20 % faster than the 32-token build with four wavefronts
-// at 257-448 of its units and than the 64-token build with four wavefronts up to 256 units (one workgroup per CU).
+// The same for 64-token tiles (256 registers, 128 KiB of LDS) up to 256 units, one workgroup per CU: 15-20 % faster than the 32-token build with
+// four wavefronts at 257-512 of its units (4096 x 4096 with 1280 / 2048 tokens 44.6 -> 37.6, 51.7 -> 44.1 us, 8192 x 28672 with 192 81.7 -> 65.7) and than the
+// 64-token build with four (46.5 -> 37.6, 52.7 -> 44.1, 84.7 -> 65.7); beyond, 4096 x 4096 with 2100 / 2304 tokens 64.0 -> 74.4, 67.0 -> 76.7.
 constexpr long kWide64KSplitMaxUnits = 256;
 // Wide (64-token x 512-column) tiles: groups from a plan's wide list or uniform groups.  `tok` = 32: uniform groups
 // in 32-token tiles on the 32-token build with two steps of weights in flight (launches that do not fill the chip).
@@ -329,7 +331,8 @@ constexpr long kWide64KSplitMaxUnits = 256;
 // a column group through another L2: the same on most of these, 4-7 % behind on 5120 x 13824 and 5120 x 5120 (4096 tokens
 // on one matrix 333 against 310 us, 143 against 138 us).  With two idle slots in 24 (m = 11008) neither order gains (cfg3's
 // delta kernel 86.3 -> 87.6-92.7 us with order 3, 85.4 -> 89.2 us with order 2; one matrix with 4096 tokens 218 -> 215 us): its
-// launches fit the three workgroups per CU either way, and the busiest CU decides.
+// launches fit the three workgroups per CU either way, and the busiest CU decides.  (With results stored as whole rows, one matrix, padded -> order
+// 3: 4096 x 14336 and 13824 with 1024 tokens 77.8 -> 73.1, 76.0 -> 72.6 us, 4096 x 2048 with 2048 43.9 -> 33.7, 4096 x 5120 with 2048 64.3 -> 65.2.)
 constexpr int kWideOrderMinIdleSlots = 3;
 static int wide_unit_order(int m) {
   const int cgs = (m / 128 + 3) / 4, cg_pad = (cgs + 7) / 8 * 8;
@@ -407,8 +410,8 @@ static unsigned plan_wide_grid(Sparse24Args& b, long rows, int m, int tok, int p
 // activations of their distinct tiles once each: with units numbered column group first, a window of W units over
 // blocks of c column groups fetches c x (weights of a column group) + W / c x (activations of a tile), least near
 // c = sqrt(W x tile / column group).  Measured (order 1 -> the rule): 4096 x 4096 with 640 / 1024 / 1536 / 2048 tokens
-// 28.3 -> 27.1, 32.1 -> 30.6, 43.8 -> 41.6, 50.5 -> 46.8 us; 8192 x 8192 with 1000 tokens 81.2 -> 79.7 us; 11008 x 4096 with
-// 1280 tokens 92.5 -> 88.6 us; 4096 x 11008 and 8192 x 28672 the same either way (blocks of 14 column groups on the
+// 28.7 -> 28.8, 32.8 -> 33.4, 41.9 -> 40.5, 47.4 -> 45.4 us; 8192 x 8192 with 1000 tokens 81.4 -> 81.5 us; 11008 x 4096 with
+// 1280 tokens 86.9 -> 83.6 us; 4096 x 11008 and 8192 x 28672 the same either way (blocks of 14 column groups on the
 // latter, which a count over the whole launch instead of the window would pick, measured 1.7 % slower).
 // The sums do not depend on which workgroup takes which unit.  Returns the c of order 4, 0 = the layer's own order.
 static long wide_uniform_blocks(long rows, int m, int k, int tok, long window) {
@@ -501,16 +504,17 @@ int launch_tile256(const Sparse24Args& a, hipStream_t st) {
   return check_launch("sparse24_tile256_kernel");
 }
 // (token tile, column pair) units for which a uniform launch takes this kernel: launches of one round of workgroups
-// (one per CU) that fill most of the chip.  Measured against 64-token tiles: 4096 tokens on 4096 x 4096 (256 units) 89.1
-// against 95.8 us (82.8 against 83.4 on another box), on 8192 x 8192 (512 units) 290 against 294 us; 4096 x 11008
-// (688 units) 228 against 227 us; 8192 x 28672 (1792 units) 994 against 950 us; 2048 tokens on 4096 x 11008 (344 units:
-// a second round of a third of the chip) 139 against 116 us; on 4096 x 4096 (128 units: half the CUs idle) 72 against 55 us.
+// (one per CU) that fill most of the chip, on the narrow layers that decide_uniform leaves to it.  64-token tiles -> this: 4096 x 2048 with
+// 4096 / 5632 / 6144 / 8192 tokens (128 / 176 / 192 / 256 units) 51.6 -> 62.6, 67.5 -> 65.0, 71.1 -> 67.0, 81.1 -> 77.5 us, with 9216 / 12288 /
+// 16384 (a second round) 113 -> 131, 122 -> 137, 161 -> 160; 4096 x 3072 with 2048 / 3840 / 5376 39.9 -> 61.1, 66.4 -> 66.6, 108 -> 130.
 constexpr long kTile256MinUnits = 192, kTile256MaxUnits = 256;
 
 // The wide kernel pays off when there are enough tiles to occupy the GPU; below that the narrow
 // kernel's smaller units win.  Knob `wide` = 0 disables it; `wide_min_units` moves the threshold.
 bool wide_enabled() { return knobs().wide != 0; }
-constexpr long kWideMinUnits = 160;   // 4096 x 4096: 1024 tokens (128 tiles) 54.9 us wide against 46.5 us narrow, 1536 tokens (192) 60.8 against 71.1
+// (64-token tiles on four wavefronts against the narrow kernel, 4096 x 4096 with 640 / 1024 / 1536 tokens, 80 / 128 / 192 units: 45.1 / 46.4 / 47.2
+// against 46.3 / 48.0 / 68.5 us; 8192 x 8192 with 320 / 512, 80 / 128: 81.6 / 83.0 against 78.4 / 79.8)
+constexpr long kWideMinUnits = 160;
 constexpr long kWide32MinUnits = 160, kWide32MaxUnits = 448;   // (32-token tile, 512-column group) units: see launch_uniform
 
 // ---- uniform groups (matmul, bmm): `tokens` rows per group.  Which kernel takes which rows is decided by
@@ -554,9 +558,11 @@ int pick_ksplit(long tokens, long n_groups, int m, int k) {
 struct KTilePick { int nt, kw, splits; };
 // Which uniform launches they take.
 //  * From 17 tokens on, while the 64-token x 128-column tiles are at most 768 (1.5 rounds of two workgroups per CU), 384 from 800
-//    tokens on: past that the wide kernels' shared activation tiles win (8192 x 8192 with 768 / 1024 tokens 75.9 -> 70.9 / 83.9 -> 96.2 us,
-//    4096 x 11008 with 512 / 1024 44.9 -> 38.5 / 71.1 -> 76.2; 4096 x 4096 and 11008 x 4096 with 1024 31.4 -> 30.8, 68.3 -> 70.1, 11008 x 4096
-//    with 900 61.0 -> 65.2; 4096 x 2048 with 1280 32.1 -> 27.4).  Small layers whose 16-token passes make the streaming kernel about
+//    tokens on: past that the wide kernels' shared activation tiles win (8192 x 8192 with 704 / 768 / 784 / 1024 tokens 74.6 -> 65.7, 73.0 -> 67.2 /
+//    68.2 -> 80.3, 79.8 -> 92.5 us, 4096 x 11008 with 512 / 576 / 1024 39.6 -> 37.0 / 39.4 -> 45.4, 65.4 -> 73.5; 11008 x 4096 with 768 / 900 / 1024
+//    62.6 -> 55.2 / 61.8 -> 65.3, 65.1 -> 68.6; 4096 x 2048 with 1280 / 1536 / 2048 32.5 -> 26.0, 32.3 -> 30.5 / 33.4 -> 43.3).  Not the best line where
+//    the wide kernel's groups of columns fill few of its launch's slots or all (4096 x 3072 with 1024 / 1100 27.3 -> 30.7 / 43.9 -> 29.0, 8192 x 1024
+//    with 3200 82.0 -> 66.4, 4096 x 4096 with 832 29.3 -> 26.8).  Small layers whose 16-token passes make the streaming kernel about
 //    a workgroup per CU stay with it (4096 x 4096 with 96 / 128 9.8 -> 10.0, 9.9 -> 10.1, 4096 x 2048 with 192 9.8 -> 10.1).  Launches of less than 4M weights and 600 tokens stay with the streaming kernel, whose
 //    eight wavefronts a column block start with less ahead of their first request (1024 x 1024 with 17 .. 512 tokens 5.5 - 6.0 -> 6.2 - 6.4
 //    us, with 640 8.1 -> 6.9).
@@ -678,9 +684,10 @@ UniformPlan decide_uniform(int tokens, int stride, int n_groups, int m, int k, l
   // Groups of hundreds of tokens: 256-token x 256-column tiles whose wavefronts share the dequantised weights.
   // On layers of fewer than 8 column groups of 512 (m < 3584) only: elsewhere the 64-token kernel, since its units go to
   // the XCDs in blocks of column groups x token tiles, is as fast or faster inside this window (4096 x 4096 with 3072 /
-  // 3584 / 4096 tokens 80.5 -> 66.8, 80.7 -> 72.4, 81.7 -> 78.2 us; 4096 x 8192 with 2048 tokens 81.5 -> 78.8; 8192 x 4096
-  // and 11008 x 4096 with 4096 tokens 147.3 -> 145, 193 -> 192 us), while 4096 x 2048 with 8192 tokens, whose four column
-  // groups leave half of a padded tile's slots idle, keeps it (81 against 85 us).  The knob tile256 = 2 lifts the limit.
+  // 3584 / 4096 tokens 73.2 -> 66.4, 75.3 -> 70.1, 76.2 -> 75.1 us; 4096 x 8192 with 2048 tokens 76.4 -> 75.1; 8192 x 4096
+  // and 11008 x 4096 with 4096 tokens 142 -> 140, 188 -> 186 us), while layers whose few column groups leave half of a padded
+  // tile's slots idle keep it (64-token tiles -> this: 4096 x 2048 with 6144 / 8192 tokens 68.9 -> 65.0, 81.5 -> 78.0, 4096 x 1024 with 16384
+  // 144 -> 76, 1024 x 2560 with 6144 28.2 -> 26.6; 4096 x 3072 with 4096 63.3 -> 64.1).  The knob tile256 = 2 lifts the limit.
   if (knobs().tile256 && (cgs < 8 || knobs().tile256 > 1) && wide_enabled() && x_below_4g) {
     const long ncp = (m / 128 + 1) / 2;
     const long min_units = knob_or(knobs().tile256_min_units, kTile256MinUnits);
@@ -695,21 +702,21 @@ UniformPlan decide_uniform(int tokens, int stride, int n_groups, int m, int k, l
   // A launch of at most two 32-token workgroups per CU, but of more than the narrow kernel fills well, is bound by
   // the latency of each workgroup's chain of steps, not by the matrix cores: there the 32-token build of the wide
   // kernel with two steps of weights in flight per wavefront beats both the narrow kernel and 64-token tiles.
-  // Measured (narrow or 64-token -> this): 4096 x 4096 with 640 / 1024 / 1536 / 2048 tokens 45.7 -> 37.2, 46.5 -> 38.2,
-  // 54.5 -> 49.7, 60.8 -> 55.6 us; 4096 x 11008 with 384 / 512 tokens 66 -> 46.7, 54.7 -> 48.5 us; 8192 x 8192 with
-  // 384 / 768 tokens 76.5 -> 66.5, 94.7 -> 86.9 us; 8192 x 28672 with 128 / 256 tokens 79 -> 69.3, 99.5 -> 95.5 us.
-  // At 160 units: 4096 x 4096 with 640 tokens 45 -> 36.7, 8192 x 8192 with 320 tokens 76.5 -> 66.2, 11008 x 4096 with 640
-  // tokens 98.8 -> 89.5 us.  Outside the window it loses: 8192 x 8192 with 288 tokens (144 units) 61.7 -> 65.7 us,
-  // 4096 x 11008 with 160 tokens (110 units) 28.9 -> 37 us, with 768 tokens (528 units) 64 -> 76 us; inside it one
-  // case measured slower: 8192 x 28672 with 96 tokens (168 units) 64 -> 69 us.
+  // Measured against both (narrow / 64-token tiles -> this, up to 256 units on eight wavefronts): 4096 x 4096 with 640 / 1024 tokens (160 / 256
+  // units) 46.3 / 45.1 -> 26.8, 48.0 / 46.4 -> 29.8 us, 8192 x 8192 with 320 (160) 78 / 81 -> 45.2, 8192 x 28672 with 96 (168) 63 / 82 -> 46; on
+  // layers whose 64-token tiles are no launch of one workgroup per CU: 4096 x 2048 with 2048 / 3000 (256 / 376) 49 / 48 -> 35, 69 / 49.4 -> 48.4,
+  // 4096 x 5120 with 1100 (350) 68 / 46.6 -> 46.2.  At the upper end the two are level (4096 x 2048 with 3584 / 3700 51.7 / 50.8 in 64-token
+  // tiles, 51.7 / 52.1 in these, 4096 x 5120 with 1400 / 1500 48.5 / 51.2 and 49.9 / 52.2; a K of 8192 or more would be better off past 400 units,
+  // 8192 x 1024 with 7000 134 against 172).  Below 160 units the K-splitting tiles have all but activations that are not aligned (without
+  // them 4096 x 4096 with 512, 128 units, 25.7 -> 26.5, 8192 x 8192 with 256 / 288 41.5 -> 44.4, 62.4 -> 45.0).
   {
     // (a last tile of any size counts: in a launch of one round its workgroups cost nothing, a separate launch of
     // the narrow kernel for them streams the weights once more)
     const long units32 = (long)n_groups * ((tokens + 31) / 32) * cgs;
     // past the launches that the 32-token build runs with eight wavefronts, 64-token tiles with eight wavefronts
-    // are ahead while they make one workgroup per CU at most (4096 x 4096 with 1280 / 1536 tokens 49.7 -> 44.2,
-    // 50.8 -> 46.0 us; 4096 x 11008 with 384 / 640 tokens 47.2 -> 43.0, 51.4 -> 46.0 us; 8192 x 8192 with 768 tokens 88.7 ->
-    // 72.5 us; 8192 x 28672 with 192 tokens 89.4 -> 73.0 us)
+    // are ahead while they make one workgroup per CU at most (4096 x 4096 with 1280 / 1536 tokens 44.6 -> 37.6,
+    // 45.8 -> 38.9 us; 4096 x 11008 with 384 / 640 tokens 44.1 -> 36.8, 48.6 -> 41.3 us; 8192 x 8192 with 768 tokens 83.5 ->
+    // 67.2 us; 8192 x 28672 with 192 tokens 81.7 -> 65.7 us)
     ks64 = done == 0 && wide_enabled() && k % 128 == 0 && x_below_4g && tokens >= kWideTokens &&
            units32 > knob_or(knobs().wide32_ksplit_max_units, kWide32KSplitMaxUnits) &&
            (long)n_groups * ((tokens + kWideTokens - 1) / kWideTokens) * ((cgs + 7) / 8 * 8) <=
@@ -1847,7 +1854,7 @@ bool lora_fused_can(int n_tokens, int n_adapters, int k, int r, int m) {
 //       up to 8                          up to 2048 0.88, to 3072 0.95 (1.08), past that 1.02 (1.26);
 //       more                             up to 4096 0.82, past that 1.01 (1.37: 1375 tokens over 46 adapters, one chunk of 13312 columns).
 // Of what it takes, one call in 1400 is more than 5 % behind the pair, none more than 7 %.  ldmm, whose other launches hide the host's share, has
-// the same rule: there the whole call takes 0.94 of its time with the pair in a graph, and none of 4374 more than 1.05.
+// the same rule: there the whole call takes 0.94 of its time with the pair in a graph, and the worst of 4374 1.05.
 // Rank 128 never (1.1 - 2.5); below k = 512 some wavefronts have no step.
 bool lora_fused_takes(int n_tokens, int n_adapters, int k, int r, int m) {
   if (!knobs().lora_fused || m == 0 || !lora_fused_can(n_tokens, n_adapters, k, r, m)) return false;
