@@ -6,9 +6,9 @@
 // tile's rows by the whole of A, keeps the intermediate in LDS, and multiplies that by its columns of B.  Workgroups of a tile
 // repeat its first product, which costs them x and A once more from L2; what it saves is the second launch, with its own chain of round
 // trips (tile -> rows and shares of K -> operands) and the shares' way to memory and back, and on the host a launch and a scratch.
-// So the rule that picks it (lora_fused_takes) bounds what a workgroup reads.  Measured against the pair, in a graph / called one by one: 16
-// tokens over 16 adapters of rank 16 on 1024 x 2048 7.0 -> 5.6 / 8.3 -> 5.8 us, 600 over 8 of rank 32 on 2048 x 2048 11.9 -> 10.7 / 11.9 -> 10.6.
-// Of the 5 us, 2 are the routing, 0.8 the first operands, 0.7 the sums, 0.6 the columns of B.
+// So the rule that picks it (lora_fused_takes) bounds what a workgroup reads, and how many columns it has.  Measured against the pair, in a
+// graph / called one by one: 16 tokens over 16 adapters of rank 16 on 1024 x 2048 7.0 -> 5.6 / 8.3 -> 5.8 us, 600 over 8 of rank 32 on
+// 2048 x 2048 11.9 -> 10.7 / 11.9 -> 10.6.  Of the 5 us, 2 are the routing, 0.8 the first operands, 0.7 the sums, 0.6 the columns of B.
 //   * The wavefronts split K in steps of 64.  A step's rows of A (128 r consecutive bytes) and pieces of x (8 rows x 128 bytes a
 //     request, whole lines) come by direct loads to a place in LDS that is the wavefront's own: no barrier in the loop.  A step's operands
 //     are read into registers, the next step's requests go out, then come the MFMAs.
