@@ -1165,21 +1165,20 @@ static bool plan_wide_launch(int prob_n, int n_deltas, int prob_m, int prob_k) {
   return plan_has_wide(prob_n, n_deltas) && !mid_tiles(prob_n, n_deltas, prob_m, prob_k) && prob_k % 128 == 0 && (long)prob_n * prob_k * 2 < (1L << 32) &&
          (long)(prob_n / 48 + 1) * ((prob_m / 128 + 3) / 4) >= knob_or(knobs().plan_wide_min_units, kPlanWideMinUnits);
 }
-// Which planned batches it takes.  All that would go to the streaming kernel alone (2164 random ones, k and m 512 .. 13824, 20 .. 4096 tokens over
-// 2 .. 64 deltas, evenly routed and Zipf: geometric mean 0.82 of its time, worst 1.10; 20 deltas of 3840 x 1152 with 1861 tokens
-// 73 -> 31 us, 5 of 11008 x 4096 with 279 63 -> 36, 32 of 4096 x 4096 with 513 53.5 -> 48).
-// Of those whose hot deltas go to the wide kernel on fewer than 16 column groups of 512 (7764 random ones, m 512 .. 7680, 512 .. 32768 tokens over 1 .. 64
-// deltas: 0.860 of the time, taking each one's better kernel 0.852, all of them 0.880): up to three groups any, which the wide
-// kernel pads to eight (0.45 - 0.85); below 96 tokens per delta any, whose 64-token tiles are half empty (0.67 - 0.98); else as
-// long as the wide kernel's shared activation tiles are not ahead, in units of 64 tokens x 128 columns up to 4096 below eight
-// groups (0.91 - 0.98 there, 0.98 - 1.06 above), 1536 with eight, which fill its order of units without an idle slot (1.01 -
-// 1.13 above; 16 deltas of 4096 x 4096 with 4096 tokens 100 against 114 us), 3072 with more (0.91 - 0.99, 1.02 - 1.14 above).
-// Of those for the wide kernels the ones of
-// few 64-token tiles, the deeper K the more (1027 random ones: 0.76 of the time, 17 of them more than 3 % slower, worst 1.23):
-// up to 256 units of 64 tokens x 128 columns any (0.42 - 0.80: half the CUs had no workgroup), up to one round of 512 from
-// k = 1280 on (0.71 - 0.91), two rounds from k = 2560 on (0.81 - 0.93), three from k = 4500 on (0.91).  Past that, with fewer
-// than 32 tokens a delta and on short K the wide kernels' shared activation tiles and fewer workgroups are ahead (the other 1626:
-// 1.03, up to 1.57; 4096 x 11008 with 2048 tokens over 4 deltas 134 -> 152 us).
+// Which planned batches it takes.  Its time, routing plan included, of the other kernels', in graphs; 43214 random batches: 27681 of 20 .. 4096 tokens over
+// 2 .. 64 deltas, k and m 512 .. 13824, and 15533 of 512 .. 32768 over 1 .. 64, m up to 7680, evenly routed and Zipf.
+//   * All that would go to the streaming kernel alone (10380 that are not routed inside it: 0.77, worst 1.12; 20 deltas of 3840 x 1152 with 1861
+//     tokens 73 -> 31 us, 5 of 11008 x 4096 with 279 63 -> 36, 32 of 4096 x 4096 with 513 53.5 -> 48).
+//   * Of those whose hot deltas go to the wide kernel on fewer than 16 column groups of 512 (7005: 0.869 of the time, taking each one's better
+//     kernel 0.853, all of them 0.871): up to three groups any, which the wide kernel pads to eight (0.33 - 0.96); below 96 tokens per
+//     delta any, whose 64-token tiles are half empty (0.79); else as long as the wide kernel's shared activation tiles are not ahead, in units of 64
+//     tokens x 128 columns up to 4096 below eight groups (0.88; 0.94 to 6144, 0.95 above, up to 1.13), none with eight, which fill its order of
+//     units without an idle slot (0.97 up to 3072, a third of them slower; 1.06 above), 3072 with more (0.92; 0.98 to 5120, 1.06 above).
+//   * Of those for the wide kernels the ones of few 64-token tiles, the deeper K the more (7481 taken: 0.70 of the time, 1 % of them more than 3 %
+//     slower, worst 1.26): up to 256 units of 64 tokens x 128 columns any (0.61: half the CUs had no workgroup), up to one round of 512
+//     from k = 1280 on (0.73), two rounds from k = 2560 on (0.76), three from k = 4500 on (0.78).  Past that, with fewer than 32 tokens a delta and
+//     on short K the wide kernels' shared activation tiles and fewer workgroups are ahead for half of the batches (the other 9027: 1.01, 0.42 .. 1.72;
+//     4096 x 11008 with 2048 tokens over 4 deltas 134 -> 152 us).
 static bool ktile_plan_takes(int prob_n, int n_deltas, int prob_m, int prob_k) {
   if (!knobs().plan_ktile || !ktile_plan_can(prob_n, prob_k)) return false;
   if (knobs().plan_ktile == 2) return true;
